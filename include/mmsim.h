@@ -111,7 +111,10 @@ typedef struct {
                                      MMSIM_E_OVERFLOW (the one-call entry points then try again with more)     */
     int32_t batching_lds_tables;  /* batching simulator: bit 0 latency table, bit 1 models of each group may be
                                      copied to LDS; -1: both, subject to fit                                    */
-    int32_t reserved;
+    int32_t window_lanes;         /* plain simulator, small and middle-sized batches: 8, 16, 32 or 64 requests of a
+                                     placement side by side in a wavefront; -1: 64 placements in a wavefront, one
+                                     request after the other; 0: by the number of simulations.  An option above that
+                                     shapes the one-request-at-a-time kernels selects them as well             */
     int64_t stats_scratch_bytes;  /* scratch of one launch of mmsim_batch_model_stats; 0: 1 GiB                 */
 } mmsim_options;
 void mmsim_options_default(mmsim_options *options);

@@ -59,7 +59,7 @@ class Options(C.Structure):
                 ("counts_in_lds", C.c_int32), ("tile_order_by_slots", C.c_int32), ("sched_groups", C.c_int32),
                 ("segment_requests", C.c_int32), ("sched_spin_limit", C.c_int32), ("skip_ahead", C.c_int32),
                 ("xcd_map", C.c_int32), ("batching_lanes", C.c_int32), ("batching_event_slots", C.c_int32),
-                ("batching_lds_tables", C.c_int32), ("reserved", C.c_int32), ("stats_scratch_bytes", C.c_int64)]
+                ("batching_lds_tables", C.c_int32), ("window_lanes", C.c_int32), ("stats_scratch_bytes", C.c_int64)]
 
 
 class DeviceInfo(C.Structure):

@@ -16,7 +16,12 @@ PKG = os.path.dirname(HERE)
 OUT = os.path.join(PKG, "libmmsim.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
-SOURCES = ["mmsim_api.hip", "sim_mixed.hip", "sim_batching.hip", "sim_scalar.hip", "stats.hip"]
+# object name -> source, flags of its own.  sim_window.hip is compiled once per number of requests side by side (its
+# instances are many; four translation units build in parallel).
+UNITS = {"mmsim_api": ("mmsim_api.hip", []), "window_batch": ("window_batch.hip", []),
+         **{f"sim_window_{w}": ("sim_window.hip", [f"-DMMSIM_WINDOW_LANES={w}"]) for w in (64, 32, 16, 8)},
+         "sim_mixed": ("sim_mixed.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_scalar": ("sim_scalar.hip", []),
+         "stats": ("stats.hip", [])}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -41,9 +46,10 @@ SOURCE_FLAGS = {"sim_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-il
                 "sim_batching.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"]}
 
 
-def _compile(src, extra, src_dir=HERE, obj_dir=OBJ_DIR):
-    obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *extra, "-c", os.path.join(src_dir, src), "-o", obj]
+def _compile(unit, extra, src_dir=HERE, obj_dir=OBJ_DIR):
+    src, own = UNITS[unit]
+    obj = os.path.join(obj_dir, unit + ".o")
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *own, *extra, "-c", os.path.join(src_dir, src), "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{proc.stdout}\n{proc.stderr}")
@@ -53,11 +59,11 @@ def _compile(src, extra, src_dir=HERE, obj_dir=OBJ_DIR):
 
 
 def build(verbose=False, extra_flags=(), src_dir=HERE, out=OUT):
-    """Compiles SOURCES from `src_dir` and links them into `out`."""
+    """Compiles UNITS from `src_dir` and links them into `out`."""
     obj_dir = os.path.join(src_dir, "build")
     os.makedirs(obj_dir, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(5, len(SOURCES))) as pool:
-        results = list(pool.map(lambda s: _compile(s, list(extra_flags), src_dir, obj_dir), SOURCES))
+    with ThreadPoolExecutor(max_workers=min(8, len(UNITS))) as pool:
+        results = list(pool.map(lambda u: _compile(u, list(extra_flags), src_dir, obj_dir), UNITS))
     objs = [o for o, _ in results]
     if verbose:
         for _, w in results:

@@ -20,76 +20,9 @@
 #include <new>
 #include <thread>
 
-#include "mmsim_internal.h"
+#include "mmsim_host.h"
 
 using namespace mmsim;
-
-namespace {
-
-thread_local std::string g_last_error;
-
-int fail(int code, const std::string &msg) {
-    g_last_error = msg;
-    return code;
-}
-
-int hip_fail(hipError_t e, const char *what) {
-    return fail(e == hipErrorOutOfMemory ? MMSIM_E_NOMEM : MMSIM_E_HIP,
-                std::string(what) + ": " + hipGetErrorString(e));
-}
-
-#define HIP_TRY(expr)                                      \
-    do {                                                   \
-        hipError_t e__ = (expr);                           \
-        if (e__ != hipSuccess) return hip_fail(e__, #expr); \
-    } while (0)
-
-// Device memory for a batch comes either from hipMalloc or, while g_arena is set (mmsim_eval_batch_static), from
-// a bump allocator over the library's static device scratch: such buffers are never freed one by one.
-struct Arena {
-    unsigned char *base = nullptr;
-    size_t cap = 0, used = 0;
-    bool overflow = false;
-};
-thread_local Arena *g_arena = nullptr;
-
-template <typename T>
-struct DevBuf {
-    T *p = nullptr;
-    size_t n = 0;
-    bool owned = true;
-    DevBuf() = default;
-    DevBuf(const DevBuf &) = delete;
-    DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { release(); }
-    void release() {
-        if (p && owned) (void)hipFree(p);
-        p = nullptr;
-        n = 0;
-        owned = true;
-    }
-    hipError_t alloc(size_t count) {
-        release();
-        n = count;
-        const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-        if (Arena *ar = g_arena) {
-            const size_t rounded = (bytes + 255) & ~(size_t)255;
-            if (rounded > ar->cap - ar->used) {
-                ar->overflow = true;
-                n = 0;
-                return hipErrorOutOfMemory;
-            }
-            p = reinterpret_cast<T *>(ar->base + ar->used);
-            ar->used += rounded;
-            owned = false;
-            return hipSuccess;
-        }
-        return hipMalloc(reinterpret_cast<void **>(&p), bytes);
-    }
-    size_t bytes() const { return n * sizeof(T); }
-};
-
-}  // namespace
 
 // Device scratch of mmsim_eval_batch_static: every device table and result buffer of one batch is carved out
 // of this array, so that entry point never allocates.  Each GPU the library runs on holds its own copy at its
@@ -99,115 +32,6 @@ static __device__ __align__(256) unsigned char scratch[MMSIM_STATIC_SCRATCH_BYTE
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mutex;
 static unsigned char *g_scratch_ptr[kMaxDevices] = {};  // per device, filled by the first context made on it
-
-struct mmsim_ctx {
-    int device = 0;
-    hipStream_t stream = nullptr;
-    hipDeviceProp_t prop{};
-    int max_lds = 0;
-    unsigned char *scratch = nullptr;     // this device's copy of the static scratch (mmsim_eval_batch_static)
-    hipEvent_t ev_static[2] = {};         // timing events of batches that live in the static scratch
-    mmsim_options opt{};                  // what batches made without options of their own use (mmsim_ctx_set_options)
-};
-
-std::atomic<uint64_t> g_next_workload_id{1};
-
-struct mmsim_workload {
-    mmsim_ctx *ctx = nullptr;
-    uint64_t id = 0;  // unique per mmsim_workload_create: a batch remembers which streams it was made from
-    int64_t R = 0;
-    int32_t M = 0;
-    DevBuf<Req> reqs;
-    std::vector<int32_t> model_num_requests;  // requests per model id (placement independent)
-    int64_t repeats = 0;                      // requests with the model of the request before
-    // arrivals regrouped by model (batching simulator): offsets per model, then per arrival
-    // its time, its deadline time + (double)slo and its index in the stream
-    std::vector<int64_t> mq_off;
-    DevBuf<MqEntry> mq;
-};
-
-// Ordered replica lists per (placement, model): the rows of m_id2g_id.
-struct RepLists {
-    int32_t B = 0, M = 0, Gmax = 0;
-    std::vector<int32_t> num_groups;  // [B]
-    std::vector<int32_t> group_cfg;   // [B][Gmax]
-    std::vector<int64_t> off;         // [B*M+1]
-    std::vector<int32_t> grp;         // group index per replica
-    // models of each group in the order the batching simulator scans them (g_id2m_id);
-    // left empty, they are derived from the replica lists as the reference does (:424-430)
-    std::vector<int64_t> g2m_off;     // [B*Gmax+1]
-    std::vector<int32_t> g2m_m;
-};
-
-struct mmsim_batch {
-    mmsim_ctx *ctx = nullptr;
-    uint32_t flags = 0;
-    int32_t n_seeds = 0, B = 0, M = 0, Gmax = 0, tiles = 0, waves = 0;
-    int32_t smax_bucket = 0, rmax_all = 0, nslots = 0, waves_per_block = 1;
-    size_t lds_bytes = 0;
-    int64_t Rmax = 0, Rtotal = 0;
-    std::vector<int64_t> wl_R;                           // [n_seeds] stream lengths
-    std::vector<uint64_t> wl_id;                         // [n_seeds] ids of the workloads the batch was made from
-    std::vector<std::vector<int32_t>> wl_model_requests;  // [n_seeds][M] requests per model of each stream
-    std::vector<int32_t> pos;  // pos[placement] = tile * 64 + lane it is simulated on
-    // Paired batch (mmsim_eval_pairs): placement p is simulated on stream stream_of[p] only; a tile holds
-    // placements of one stream, and results are laid out as for a single seed.
-    bool paired = false;
-    std::vector<int32_t> stream_of;   // [B]
-    DevBuf<int32_t> tile_seed;        // [tiles]
-    int32_t out_seeds = 1;            // seeds of the result layout: n_seeds, or 1 for a paired batch
-    size_t wave_bytes = 0;     // LDS bytes of one wavefront's region (chunked loop, batching simulator)
-    // Plain simulator, loop over runs: one launch of `sched_groups` workgroups, each owning a set of (tile, stream)
-    // items that its wavefronts simulate segment by segment (clocks parked in `state` between segments).
-    int32_t sched_groups = 0, sched_waves = 0, seg_requests = 0, max_nseg = 1;
-    DevBuf<int32_t> plan;      // wg_off | item_tile | item_seed | item_nslots | item_bytes | item_nseg | part_off | part_bytes
-    DevBuf<double> state;
-
-    DevBuf<Req> streams;
-    DevBuf<int64_t> stream_off;
-    DevBuf<uint32_t> rep32, repx32;
-    DevBuf<uint64_t> rep8;
-    DevBuf<uint8_t> repx;
-    DevBuf<uint8_t> rmax;
-    DevBuf<int32_t> kerr;
-    DevBuf<uint32_t> ginfo;
-    DevBuf<float> lat;
-    DevBuf<int32_t> n_good;
-    DevBuf<double> lat_sum;
-    DevBuf<int32_t> model_good, group_req, group_good;
-    DevBuf<unsigned long long> slot_cnt;      // plain simulator: per-group counts by last clock slot [waves][nslots][64]
-    std::vector<int16_t> group_last_slot;     // [B][Gmax] last clock slot of each group, -1: no such group
-    int32_t group_by_slot = 0, slot_rows = 0; // group_by_slot: the group counts are in slot_cnt (else in group_req / group_good)
-    int32_t group_lds = 0;                    // the kernel keeps the slot counters in LDS while it runs
-    DevBuf<double> finish;
-    DevBuf<uint8_t> good;
-    DevBuf<int64_t> fp_ops;
-    // batching simulator
-    DevBuf<int64_t> mq_off;
-    DevBuf<MqEntry> mq;
-    DevBuf<int32_t> status, batch_sizes;
-    DevBuf<uint16_t> g2m_off, g2m_idx;
-    DevBuf<float> lat_nb;
-    std::vector<uint8_t> hosted;  // [B][M] model has a replica (batching: decides model_num_requests)
-    BatchingArgs bargs{};
-    // device buffers of mmsim_batch_model_stats, made by its first call and kept for the next ones
-    DevBuf<const MqEntry *> st_mq;
-    DevBuf<int64_t> st_i64;   // mq_off | lo | hi | sim_base
-    DevBuf<int32_t> st_i32;   // sim_stream | model_req | model_good
-    DevBuf<double> st_f64;    // the seven double results
-    DevBuf<uint64_t> st_scratch;
-
-    MixedArgs args{};
-    hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-    bool own_events = true;  // false: the context's events (batch in the static scratch)
-    bool ran = false;
-    mmsim_options opt{};     // the options the batch was built with
-
-    ~mmsim_batch() {
-        if (own_events && ev_start) (void)hipEventDestroy(ev_start);
-        if (own_events && ev_stop) (void)hipEventDestroy(ev_stop);
-    }
-};
 
 namespace {
 
@@ -239,25 +63,11 @@ int check_options(const mmsim_options *o) {
         return fail(MMSIM_E_INVALID, "options: negative value");
     if (o->batching_lanes != 0 && o->batching_lanes != 8 && o->batching_lanes != 16 && o->batching_lanes != 32 && o->batching_lanes != 64)
         return fail(MMSIM_E_INVALID, "options: batching_lanes must be 0, 8, 16, 32 or 64");
+    if (o->window_lanes != -1 && o->window_lanes != 0 && o->window_lanes != 8 && o->window_lanes != 16 && o->window_lanes != 32 &&
+        o->window_lanes != 64)
+        return fail(MMSIM_E_INVALID, "options: window_lanes must be -1, 0, 8, 16, 32 or 64");
     if (o->batching_lds_tables < -1 || o->batching_lds_tables > 3) return fail(MMSIM_E_INVALID, "options: batching_lds_tables outside -1..3");
     return MMSIM_OK;
-}
-
-// Runs fn(lo, hi) on slices of [0, n) on up to 16 host threads (one slice per thread; the caller's
-// slices write disjoint memory).  Small ranges run on the calling thread.
-template <class F>
-void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
-    int64_t threads = std::min<int64_t>(16, std::max(1u, std::thread::hardware_concurrency()));
-    threads = std::min<int64_t>(threads, n / std::max<int64_t>(1, min_per_thread));
-    if (threads <= 1) {
-        fn((int64_t)0, n);
-        return;
-    }
-    const int64_t per = (n + threads - 1) / threads;
-    std::vector<std::thread> pool;
-    for (int64_t lo = per; lo < n; lo += per) pool.emplace_back([&fn, lo, per, n] { fn(lo, std::min(n, lo + per)); });
-    fn((int64_t)0, std::min(n, per));
-    for (std::thread &th : pool) th.join();
 }
 
 // group -> models CSR of the C ABI into ordered per-(placement, model) replica lists
@@ -395,6 +205,35 @@ int expand_successors(const mmsim_placements *base, const mmsim_successors *sc, 
     return MMSIM_OK;
 }
 
+}  // namespace
+
+int mmsim::compact_latency(const mmsim_tables *t, bool all_batch_sizes, CompactLatency *out) {
+    const int32_t M = t->M, C = t->C;
+    out->uniform = true;
+    for (int32_t m = 0; m < M && out->uniform; ++m)
+        for (int c = 0; c < C && out->uniform; ++c) {
+            const float *row = t->cfg_lat + ((size_t)m * C + c) * t->Smax * t->NB;
+            for (int k = 1; k < t->cfg_pp[c]; ++k)
+                if (std::memcmp(&row[(size_t)k * t->NB], &row[0], sizeof(float) * (all_batch_sizes ? (size_t)t->NB : 1)) != 0) out->uniform = false;
+        }
+    out->off.assign((size_t)C + 1, 0);
+    for (int c = 0; c < C; ++c) out->off[c + 1] = out->off[c] + (out->uniform ? 1 : t->cfg_pp[c]);
+    out->row = out->off[C] + 1;
+    if (out->row > kMaxLatRow) return fail(MMSIM_E_UNSUPPORTED, "configurations have more than 1022 pipeline stages in total");
+    out->lat.assign((size_t)M * out->row, std::numeric_limits<float>::infinity());
+    for (int32_t m = 0; m < M; ++m)
+        for (int c = 0; c < C; ++c)
+            for (int k = 0; k < (out->uniform ? 1 : t->cfg_pp[c]); ++k) {
+                const float v = t->cfg_lat[(((size_t)m * C + c) * t->Smax + k) * t->NB];
+                if (v != v) return fail(MMSIM_E_INVALID, "tables: a stage latency is NaN");
+                if (v < 0.0f) return fail(MMSIM_E_INVALID, "tables: a stage latency is negative");
+                out->lat[(size_t)m * out->row + out->off[c] + k] = v;
+            }
+    return MMSIM_OK;
+}
+
+namespace {
+
 // Builds every device table of a batch from replica lists and launches nothing.
 int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
                 const RepLists &rl, uint32_t flags, mmsim_batch **out, const int32_t *stream_of = nullptr,
@@ -505,30 +344,15 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     b->nslots = nslots;
 
     phase("slots and replica counts");
-    // ---- compact batch-size-1 latency table.  General form: row of model m = its stage
-    //      latencies for configuration 0, then configuration 1, ... (the cfg_pp[c] real
-    //      stages only).  When every (model, config) has one latency for all its stages the
-    //      row is just one value per configuration.
-    bool uniform_stages = true;  // (the batching kernel reads every batch size's column: all of them must agree)
-    for (int32_t m = 0; m < M && uniform_stages; ++m)
-        for (int c = 0; c < C && uniform_stages; ++c) {
-            const float *row = t->cfg_lat + ((size_t)m * C + c) * t->Smax * t->NB;
-            for (int k = 1; k < t->cfg_pp[c]; ++k)
-                if (std::memcmp(&row[(size_t)k * t->NB], &row[0], sizeof(float) * (batching ? (size_t)t->NB : 1)) != 0) uniform_stages = false;
-        }
-    std::vector<int32_t> lat_off(C + 1, 0);
-    for (int c = 0; c < C; ++c) lat_off[c + 1] = lat_off[c] + (uniform_stages ? 1 : t->cfg_pp[c]);
-    const int32_t lat_row = lat_off[C] + 1;  // one extra entry per model: +inf, the latency of "no such replica"
-    if (lat_row > kMaxLatRow) return fail(MMSIM_E_UNSUPPORTED, "configurations have more than 1022 pipeline stages in total");
-    std::vector<float> lat((size_t)M * lat_row, std::numeric_limits<float>::infinity());
-    for (int32_t m = 0; m < M; ++m)
-        for (int c = 0; c < C; ++c)
-            for (int k = 0; k < (uniform_stages ? 1 : t->cfg_pp[c]); ++k) {
-                const float v = t->cfg_lat[(((size_t)m * C + c) * t->Smax + k) * t->NB];
-                if (v != v) return fail(MMSIM_E_INVALID, "tables: a stage latency is NaN");
-                if (v < 0.0f) return fail(MMSIM_E_INVALID, "tables: a stage latency is negative");
-                lat[(size_t)m * lat_row + lat_off[c] + k] = v;
-            }
+    CompactLatency cl;
+    {
+        const int rc = compact_latency(t, batching, &cl);  // (the batching kernel reads every batch size's column: all must agree)
+        if (rc != MMSIM_OK) return rc;
+    }
+    const bool uniform_stages = cl.uniform;
+    const std::vector<int32_t> &lat_off = cl.off;
+    const int32_t lat_row = cl.row;
+    const std::vector<float> &lat = cl.lat;
 
     // ---- which request loop: bursty streams (most requests repeat the model of the one before) get the loop over runs
     bool runs = false;
@@ -1124,7 +948,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     HIP_TRY(b->streams.alloc((size_t)b->Rtotal));
     for (int s = 0; s < n_seeds; ++s)
         if (wls[s]->R > 0)
-            HIP_TRY(hipMemcpyAsync(b->streams.p + soff[s], wls[s]->reqs.p, sizeof(Req) * (size_t)wls[s]->R,
+            HIP_TRY(hipMemcpyAsync(b->streams.p + soff[s], wls[s]->reqs->p, sizeof(Req) * (size_t)wls[s]->R,
                                    hipMemcpyDeviceToDevice, st));
     HIP_TRY(b->stream_off.alloc(soff.size()));
     HIP_TRY(hipMemcpyAsync(b->stream_off.p, soff.data(), sizeof(int64_t) * soff.size(), hipMemcpyHostToDevice, st));
@@ -1333,6 +1157,23 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     return MMSIM_OK;
 }
 
+// A batch from placements as the caller gave them, for whichever kernel suits it.  events: the batch will be timed
+// (mmsim_batch_sync).
+int make_batch(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_streams, const mmsim_tables *tables,
+               const mmsim_placements *placements, const int32_t *stream_of, uint32_t flags, const mmsim_options *options,
+               bool events, mmsim_batch **out) {
+    int rc = check_tables(tables);
+    if (rc) return rc;
+    rc = check_options(options);
+    if (rc) return rc;
+    rc = build_window(ctx, workloads, n_streams, tables, placements, stream_of, flags, options ? *options : ctx->opt, events, out);
+    if (rc <= 0) return rc;
+    RepLists rl;
+    rc = lists_from_placements(placements, tables->M, tables->C, &rl);
+    if (rc) return rc;
+    return build_batch(ctx, workloads, n_streams, tables, rl, flags, out, stream_of, options);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1480,10 +1321,10 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
             }
     }
     HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(w->reqs.alloc((size_t)R));
+    HIP_TRY(w->reqs->alloc((size_t)R));
     HIP_TRY(w->mq.alloc(known));
     if (R > 0) {
-        HIP_TRY(hipMemcpyAsync(w->reqs.p, host.data(), sizeof(Req) * (size_t)R, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipMemcpyAsync(w->reqs->p, host.data(), sizeof(Req) * (size_t)R, hipMemcpyHostToDevice, ctx->stream));
         if (known > 0) {
             HIP_TRY(hipMemcpyAsync(w->mq.p, mq.data(), sizeof(MqEntry) * known, hipMemcpyHostToDevice, ctx->stream));
         }
@@ -1504,14 +1345,7 @@ int mmsim_batch_create_ex(mmsim_ctx *ctx, const mmsim_workload *const *workloads
                           const mmsim_options *options, mmsim_batch **out) {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "batch_create: null pointer");
     *out = nullptr;
-    int rc = check_tables(tables);
-    if (rc) return rc;
-    rc = check_options(options);
-    if (rc) return rc;
-    RepLists rl;
-    rc = lists_from_placements(placements, tables->M, tables->C, &rl);
-    if (rc) return rc;
-    return build_batch(ctx, workloads, n_seeds, tables, rl, flags, out, nullptr, options);
+    return make_batch(ctx, workloads, n_seeds, tables, placements, nullptr, flags, options, true, out);
 }
 
 int mmsim_batch_create(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
@@ -1524,6 +1358,7 @@ int mmsim_batch_run(mmsim_batch *b) {
     if (!b) return fail(MMSIM_E_INVALID, "batch_run: null batch");
     mmsim_ctx *ctx = b->ctx;
     HIP_TRY(hipSetDevice(ctx->device));
+    if (b->window) return run_window(b);
     if (b->flags & MMSIM_WANT_MODEL_COUNTS)
         HIP_TRY(hipMemsetAsync(b->model_good.p, 0, b->model_good.bytes(), ctx->stream));
     if (b->group_by_slot) {
@@ -1565,6 +1400,7 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) {
     if (wm && (!out->model_num_requests || !out->model_num_good)) return fail(MMSIM_E_INVALID, "batch_fetch: model count arrays missing");
     if (wg && (!out->group_num_requests || !out->group_num_good)) return fail(MMSIM_E_INVALID, "batch_fetch: group count arrays missing");
     HIP_TRY(hipSetDevice(b->ctx->device));
+    if (b->window) return fetch_window(b, out);
     HIP_TRY(hipStreamSynchronize(b->ctx->stream));
 
     if (!(b->flags & MMSIM_BATCHING)) {
@@ -1713,8 +1549,12 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
     for (int s = 0; s < b->out_seeds; ++s)
         for (int32_t p = 0; p < B; ++p) {
             const size_t sim = (size_t)s * B + p;
-            const int64_t wave = (int64_t)s * tiles + b->pos[p] / kWave;
             sim_stream[sim] = b->paired ? b->stream_of[p] : s;
+            if (b->window) {
+                sim_base[sim] = (int64_t)sim * b->Rmax;
+                continue;
+            }
+            const int64_t wave = (int64_t)s * tiles + b->pos[p] / kWave;
             sim_base[sim] = wave * b->Rmax * kWave + b->pos[p] % kWave;
         }
     const size_t cells = (size_t)n_sims * (size_t)M;
@@ -1740,8 +1580,9 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
     HIP_TRY(hipMemcpyAsync(i64, up.data(), sizeof(int64_t) * up.size(), hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(d_i32.p, sim_stream.data(), sizeof(int32_t) * sim_stream.size(), hipMemcpyHostToDevice, st));
     StatsArgs f{};
-    f.finish = b->finish.p;
-    f.good = b->good.p;
+    f.finish = b->window ? b->wargs.finish : b->finish.p;
+    f.good = b->window ? b->wargs.good : b->good.p;
+    f.stride = b->window ? 1 : kWave;
     f.mq = d_mq.p;
     f.mq_off = i64;
     f.lo = i64 + mqo.size();
@@ -1796,9 +1637,9 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) {
     out->slots = b->nslots;
     out->lds_bytes = (int32_t)b->lds_bytes;
     out->requests_total = b->Rtotal;
-    out->table_bytes = (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() +
+    out->table_bytes = b->window ? (int64_t)b->win_in.bytes() : (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() +
                                  b->rmax.bytes() + b->lat.bytes() + b->lat_nb.bytes());
-    out->stream_bytes = (int64_t)b->streams.bytes();
+    out->stream_bytes = b->window ? b->Rtotal * (int64_t)sizeof(Req) : (int64_t)b->streams.bytes();
     out->workgroups = b->sched_groups;
     out->segments = b->max_nseg;
     out->launches = 1;
@@ -1811,7 +1652,8 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) {
 int mmsim_batch_kernel_name(const mmsim_batch *b, char *buf, size_t size) {
     if (!b || !buf || size == 0) return fail(MMSIM_E_INVALID, "batch_kernel_name: null pointer or empty buffer");
     const std::string name = (b->flags & MMSIM_BATCHING) ? sim_batching_kernel_name(b->bargs)
-                                                         : sim_mixed_kernel_name(b->args, b->smax_bucket);
+                             : b->window                   ? sim_window_kernel_name(b->wargs)
+                                                           : sim_mixed_kernel_name(b->args, b->smax_bucket);
     std::snprintf(buf, size, "%s", name.c_str());
     return MMSIM_OK;
 }
@@ -1824,18 +1666,11 @@ namespace {
 int eval_once(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_streams, const mmsim_tables *tables,
               const mmsim_placements *placements, const int32_t *stream_of, uint32_t flags, const mmsim_options *options,
               mmsim_result *out, int *event_slots) {
-    int rc = check_tables(tables);
-    if (rc) return rc;
-    rc = check_options(options);
-    if (rc) return rc;
-    RepLists rl;
-    rc = lists_from_placements(placements, tables->M, tables->C, &rl);
-    if (rc) return rc;
     mmsim_batch *b = nullptr;
-    rc = build_batch(ctx, workloads, n_streams, tables, rl, flags, &b, stream_of, options);
+    int rc = make_batch(ctx, workloads, n_streams, tables, placements, stream_of, flags, options, false, &b);
     if (rc == MMSIM_OK && event_slots) *event_slots = b->bargs.heap_cap;
     if (rc == MMSIM_OK) rc = mmsim_batch_run(b);
-    if (rc == MMSIM_OK) rc = mmsim_batch_sync(b, nullptr);
+    if (rc == MMSIM_OK && !b->window) rc = mmsim_batch_sync(b, nullptr);  // (the fetch waits by itself)
     if (rc == MMSIM_OK) rc = mmsim_batch_fetch(b, out);
     mmsim_batch_destroy(b);
     return rc;
@@ -1964,11 +1799,6 @@ int mmsim_eval_batch_static(mmsim_ctx *ctx, const mmsim_workload *const *workloa
                             mmsim_result *out) {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "eval_batch_static: null pointer");
     if (!ctx->scratch) return fail(MMSIM_E_HIP, "eval_batch_static: the context has no static scratch");
-    int rc = check_tables(tables);
-    if (rc) return rc;
-    RepLists rl;
-    rc = lists_from_placements(placements, tables->M, tables->C, &rl);
-    if (rc) return rc;
     // Every device buffer of the batch is carved out of the device's static scratch (nothing is allocated or
     // freed on the device); the scratch keeps the last call's contents, and what must start at zero is
     // cleared by build_batch / mmsim_batch_run as for any batch.
@@ -1977,7 +1807,7 @@ int mmsim_eval_batch_static(mmsim_ctx *ctx, const mmsim_workload *const *workloa
     arena.cap = MMSIM_STATIC_SCRATCH_BYTES;
     mmsim_batch *b = nullptr;
     g_arena = &arena;
-    rc = build_batch(ctx, workloads, n_seeds, tables, rl, flags, &b);
+    int rc = make_batch(ctx, workloads, n_seeds, tables, placements, nullptr, flags, nullptr, true, &b);
     g_arena = nullptr;
     if (rc != MMSIM_OK && arena.overflow)
         return fail(MMSIM_E_NOMEM, "eval_batch_static: the batch (placements x models x seeds, streams, requested outputs) "

@@ -1,0 +1,275 @@
+// Host-side objects of libmmsim shared by its translation units: error reporting, device memory, and what the
+// opaque handles of the C ABI point at.
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <map>
+#include <memory>
+#include <mutex>
+#include <thread>
+
+#include "mmsim_internal.h"
+
+namespace mmsim {
+
+inline thread_local std::string g_last_error;
+
+inline int fail(int code, const std::string &msg) {
+    g_last_error = msg;
+    return code;
+}
+
+inline int hip_fail(hipError_t e, const char *what) {
+    return fail(e == hipErrorOutOfMemory ? MMSIM_E_NOMEM : MMSIM_E_HIP,
+                std::string(what) + ": " + hipGetErrorString(e));
+}
+
+#define HIP_TRY(expr)                                      \
+    do {                                                   \
+        hipError_t e__ = (expr);                           \
+        if (e__ != hipSuccess) return hip_fail(e__, #expr); \
+    } while (0)
+
+// Device memory for a batch comes either from hipMalloc or, while g_arena is set (mmsim_eval_batch_static), from
+// a bump allocator over the library's static device scratch: such buffers are never freed one by one.
+struct Arena {
+    unsigned char *base = nullptr;
+    size_t cap = 0, used = 0;
+    bool overflow = false;
+};
+inline thread_local Arena *g_arena = nullptr;
+
+template <typename T>
+struct DevBuf {
+    T *p = nullptr;
+    size_t n = 0;
+    bool owned = true;
+    DevBuf() = default;
+    DevBuf(const DevBuf &) = delete;
+    DevBuf &operator=(const DevBuf &) = delete;
+    ~DevBuf() { release(); }
+    void release() {
+        if (p && owned) (void)hipFree(p);
+        p = nullptr;
+        n = 0;
+        owned = true;
+    }
+    hipError_t alloc(size_t count) {
+        release();
+        n = count;
+        const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+        if (Arena *ar = g_arena) {
+            const size_t rounded = (bytes + 255) & ~(size_t)255;
+            if (rounded > ar->cap - ar->used) {
+                ar->overflow = true;
+                n = 0;
+                return hipErrorOutOfMemory;
+            }
+            p = reinterpret_cast<T *>(ar->base + ar->used);
+            ar->used += rounded;
+            owned = false;
+            return hipSuccess;
+        }
+        return hipMalloc(reinterpret_cast<void **>(&p), bytes);
+    }
+    size_t bytes() const { return n * sizeof(T); }
+};
+
+}  // namespace mmsim
+
+
+using namespace mmsim;
+
+namespace mmsim {
+
+// Host memory the GPU copies from and to directly, kept by a context between calls: packed inputs and results pass
+// through it.  Grows on demand; a call that needs more than kMost gives its memory back at the end.
+struct Staging {
+    static constexpr size_t kMost = (size_t)64 << 20;
+    unsigned char *p = nullptr;
+    size_t n = 0;
+    Staging() = default;
+    Staging(const Staging &) = delete;
+    Staging &operator=(const Staging &) = delete;
+    ~Staging() { release(); }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+    }
+    hipError_t ensure(size_t bytes) {
+        if (bytes <= n) return hipSuccess;
+        release();
+        const size_t want = std::max<size_t>(bytes, std::min(kMost, std::max<size_t>((size_t)1 << 20, 2 * bytes)));
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), want, hipHostMallocDefault);
+        if (e != hipSuccess) {
+            p = nullptr;
+            return e;
+        }
+        n = want;
+        return hipSuccess;
+    }
+    void trim() {
+        if (n > kMost) release();
+    }
+};
+
+// Runs fn(lo, hi) on slices of [0, n) on up to 16 host threads (one slice per thread; the caller's
+// slices write disjoint memory).  Small ranges run on the calling thread.
+template <class F>
+void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
+    int64_t threads = std::min<int64_t>(16, std::max(1u, std::thread::hardware_concurrency()));
+    threads = std::min<int64_t>(threads, n / std::max<int64_t>(1, min_per_thread));
+    if (threads <= 1) {
+        fn((int64_t)0, n);
+        return;
+    }
+    const int64_t per = (n + threads - 1) / threads;
+    std::vector<std::thread> pool;
+    for (int64_t lo = per; lo < n; lo += per) pool.emplace_back([&fn, lo, per, n] { fn(lo, std::min(n, lo + per)); });
+    fn((int64_t)0, std::min(n, per));
+    for (std::thread &th : pool) th.join();
+}
+
+}  // namespace mmsim
+
+struct mmsim_ctx {
+    Staging staging;
+    int device = 0;
+    hipStream_t stream = nullptr;
+    hipDeviceProp_t prop{};
+    int max_lds = 0;
+    unsigned char *scratch = nullptr;     // this device's copy of the static scratch (mmsim_eval_batch_static)
+    hipEvent_t ev_static[2] = {};         // timing events of batches that live in the static scratch
+    mmsim_options opt{};                  // what batches made without options of their own use (mmsim_ctx_set_options)
+};
+
+inline std::atomic<uint64_t> g_next_workload_id{1};
+
+struct mmsim_workload {
+    mmsim_ctx *ctx = nullptr;
+    uint64_t id = 0;  // unique per mmsim_workload_create: a batch remembers which streams it was made from
+    int64_t R = 0;
+    int32_t M = 0;
+    std::shared_ptr<DevBuf<Req>> reqs = std::make_shared<DevBuf<Req>>();  // shared with batches that read it in place
+    std::vector<int32_t> model_num_requests;  // requests per model id (placement independent)
+    int64_t repeats = 0;                      // requests with the model of the request before
+    // arrivals regrouped by model (batching simulator): offsets per model, then per arrival
+    // its time, its deadline time + (double)slo and its index in the stream
+    std::vector<int64_t> mq_off;
+    DevBuf<MqEntry> mq;
+};
+
+// Ordered replica lists per (placement, model): the rows of m_id2g_id.
+struct RepLists {
+    int32_t B = 0, M = 0, Gmax = 0;
+    std::vector<int32_t> num_groups;  // [B]
+    std::vector<int32_t> group_cfg;   // [B][Gmax]
+    std::vector<int64_t> off;         // [B*M+1]
+    std::vector<int32_t> grp;         // group index per replica
+    // models of each group in the order the batching simulator scans them (g_id2m_id);
+    // left empty, they are derived from the replica lists as the reference does (:424-430)
+    std::vector<int64_t> g2m_off;     // [B*Gmax+1]
+    std::vector<int32_t> g2m_m;
+};
+
+struct mmsim_batch {
+    mmsim_ctx *ctx = nullptr;
+    uint32_t flags = 0;
+    int32_t n_seeds = 0, B = 0, M = 0, Gmax = 0, tiles = 0, waves = 0;
+    int32_t smax_bucket = 0, rmax_all = 0, nslots = 0, waves_per_block = 1;
+    size_t lds_bytes = 0;
+    int64_t Rmax = 0, Rtotal = 0;
+    std::vector<int64_t> wl_R;                           // [n_seeds] stream lengths
+    std::vector<uint64_t> wl_id;                         // [n_seeds] ids of the workloads the batch was made from
+    std::vector<std::vector<int32_t>> wl_model_requests;  // [n_seeds][M] requests per model of each stream
+    std::vector<int32_t> pos;  // pos[placement] = tile * 64 + lane it is simulated on
+    // Paired batch (mmsim_eval_pairs): placement p is simulated on stream stream_of[p] only; a tile holds
+    // placements of one stream, and results are laid out as for a single seed.
+    bool paired = false;
+    std::vector<int32_t> stream_of;   // [B]
+    DevBuf<int32_t> tile_seed;        // [tiles]
+    int32_t out_seeds = 1;            // seeds of the result layout: n_seeds, or 1 for a paired batch
+    size_t wave_bytes = 0;     // LDS bytes of one wavefront's region (chunked loop, batching simulator)
+    // Plain simulator, loop over runs: one launch of `sched_groups` workgroups, each owning a set of (tile, stream)
+    // items that its wavefronts simulate segment by segment (clocks parked in `state` between segments).
+    int32_t sched_groups = 0, sched_waves = 0, seg_requests = 0, max_nseg = 1;
+    DevBuf<int32_t> plan;      // wg_off | item_tile | item_seed | item_nslots | item_bytes | item_nseg | part_off | part_bytes
+    DevBuf<double> state;
+
+    DevBuf<Req> streams;
+    DevBuf<int64_t> stream_off;
+    DevBuf<uint32_t> rep32, repx32;
+    DevBuf<uint64_t> rep8;
+    DevBuf<uint8_t> repx;
+    DevBuf<uint8_t> rmax;
+    DevBuf<int32_t> kerr;
+    DevBuf<uint32_t> ginfo;
+    DevBuf<float> lat;
+    DevBuf<int32_t> n_good;
+    DevBuf<double> lat_sum;
+    DevBuf<int32_t> model_good, group_req, group_good;
+    DevBuf<unsigned long long> slot_cnt;      // plain simulator: per-group counts by last clock slot [waves][nslots][64]
+    std::vector<int16_t> group_last_slot;     // [B][Gmax] last clock slot of each group, -1: no such group
+    int32_t group_by_slot = 0, slot_rows = 0; // group_by_slot: the group counts are in slot_cnt (else in group_req / group_good)
+    int32_t group_lds = 0;                    // the kernel keeps the slot counters in LDS while it runs
+    DevBuf<double> finish;
+    DevBuf<uint8_t> good;
+    DevBuf<int64_t> fp_ops;
+    // batching simulator
+    DevBuf<int64_t> mq_off;
+    DevBuf<MqEntry> mq;
+    DevBuf<int32_t> status, batch_sizes;
+    DevBuf<uint16_t> g2m_off, g2m_idx;
+    DevBuf<float> lat_nb;
+    std::vector<uint8_t> hosted;  // [B][M] model has a replica (batching: decides model_num_requests)
+    BatchingArgs bargs{};
+    // device buffers of mmsim_batch_model_stats, made by its first call and kept for the next ones
+    DevBuf<const MqEntry *> st_mq;
+    DevBuf<int64_t> st_i64;   // mq_off | lo | hi | sim_base
+    DevBuf<int32_t> st_i32;   // sim_stream | model_req | model_good
+    DevBuf<double> st_f64;    // the seven double results
+    DevBuf<uint64_t> st_scratch;
+
+    // Requests side by side (window_batch.hip): all inputs in one buffer, all outputs in another
+    bool window = false;
+    WindowArgs wargs{};
+    DevBuf<uint8_t> win_in, win_out;
+    std::vector<std::shared_ptr<DevBuf<Req>>> win_streams;
+    size_t win_lat_sum = 0, win_model = 0, win_group = 0, win_finish = 0, win_good = 0;  // offsets in win_out (n_good: 0)
+
+    MixedArgs args{};
+    hipEvent_t ev_start = nullptr, ev_stop = nullptr;
+    bool own_events = true;  // false: the context's events (batch in the static scratch)
+    bool ran = false;
+    mmsim_options opt{};     // the options the batch was built with
+
+    ~mmsim_batch() {
+        if (own_events && ev_start) (void)hipEventDestroy(ev_start);
+        if (own_events && ev_stop) (void)hipEventDestroy(ev_stop);
+    }
+};
+
+namespace mmsim {
+
+// The latency table as the plain simulator's kernels read it: [M][lat_row], per model the latencies of configuration
+// 0, then 1, ... (its cfg_pp[c] stages, or one value per configuration when every (model, configuration) has one
+// latency for all its stages), then one +inf entry, the latency of "no such replica".
+struct CompactLatency {
+    bool uniform = true;
+    int32_t row = 0;
+    std::vector<int32_t> off;  // [C+1]
+    std::vector<float> lat;
+};
+int compact_latency(const mmsim_tables *t, bool all_batch_sizes, CompactLatency *out);
+
+// Builds the batch for the kernel of sim_window.hip if that is the one for it.  Returns MMSIM_OK, an error code, or 1
+// when the batch is for the other kernels (or is not valid: they say what is wrong with it).
+int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
+                 const mmsim_placements *p, const int32_t *stream_of, uint32_t flags, const mmsim_options &o, bool events,
+                 mmsim_batch **out);
+int run_window(mmsim_batch *b);
+int fetch_window(mmsim_batch *b, mmsim_result *out);
+
+}  // namespace mmsim

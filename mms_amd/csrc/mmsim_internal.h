@@ -201,6 +201,56 @@ struct BatchingArgs {
     double *finish;              // [waves][Rmax][64]
     uint8_t *good;               // [waves][Rmax][64]
 };
+// Arguments of the plain simulator's kernel for small and middle-sized batches (sim_window.hip): the lanes of a
+// wavefront hold requests of 64 / lanes placements.
+struct WindowArgs {
+    const Req *const *stream_ptr;    // [streams]
+    const int64_t *stream_len;       // [streams]
+    const int32_t *stream_of;        // paired batches: [B] the one stream of each placement; null: every placement on every stream
+    // the placements as they were given, packed
+    const uint8_t *num_groups;       // [B]
+    const uint8_t *group_cfg;        // [B][Gmax]
+    const uint32_t *entry_off;       // [B+1]
+    const uint32_t *entries;         // model | group << 16
+    const uint8_t *cfg_pp;           // [C] stages of a configuration
+    const uint16_t *lat_off;         // [C] where its latencies start in a model's row of lat
+    const float *lat;                // [M][lat_row]
+    int32_t M, lat_row, B, Gmax, group_words, nslots, tiles, out_seeds;
+    int32_t lanes;                   // requests of a placement side by side: 64, 32, 16 or 8
+    int32_t smax, smax_bucket, pow2_depths, uniform_stages, has_ext;  // smax: most stages of a group
+    int32_t lat_lds_bytes;           // the workgroup's copy of lat (tables with per-stage latencies, if it fits), or 0
+    int32_t place_bytes;             // LDS of one placement; offsets within it (see sim_window.hip):
+    int32_t o_rep, o_ext, o_xi, o_bits, o_gd, o_mcnt;
+    int64_t Rmax;
+    double fixed_overhead;
+    uint32_t flags;
+    // outputs, laid out as the caller's: simulation = seed * B + placement
+    int32_t *n_good;
+    double *lat_sum;
+    int32_t *model_good;             // [L][M]
+    int32_t *group_req, *group_good; // [L][Gmax]
+    double *finish;                  // [L][Rmax]
+    uint8_t *good;                   // [L][Rmax]
+};
+// LDS bytes behind the latency table, per wavefront: requests on their way from the lanes that fetched them to the
+// placements that share the wavefront.
+__host__ __device__ constexpr int window_ring_bytes(int lanes) { return lanes == kWave ? 0 : 2 * kWave * (int)sizeof(Req); }
+constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
+constexpr int64_t kMaxWindowSims = 16384;  // simulations from which on 64 placements share a wavefront
+typedef void (*WindowKernel)(const WindowArgs);
+// The kernel for LANES requests side by side (64, 32, 16, 8), stage bucket smax and the rest of its template arguments.
+template <int LANES>
+WindowKernel window_kernel(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+template <>
+WindowKernel window_kernel<64>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+template <>
+WindowKernel window_kernel<32>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+template <>
+WindowKernel window_kernel<16>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+template <>
+WindowKernel window_kernel<8>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+std::string sim_window_kernel_name(const WindowArgs &args);
+
 // Arguments of the scalar-clock request loop (one placement, device pointers).
 struct ScalarArgs {
     const double *tstamps;            // [R]
@@ -221,13 +271,14 @@ struct ScalarArgs {
 // regrouped by model and the window of request indices that the warm-up trimming leaves.  One launch
 // handles the simulations sim0 .. sim0 + n - 1, one scratch row each.
 struct StatsArgs {
-    const double *finish;           // [waves][Rmax][64]
-    const uint8_t *good;            // [waves][Rmax][64]
+    const double *finish;           // [waves][Rmax][64], or [n_sims][Rmax]
+    const uint8_t *good;            // likewise
     const MqEntry *const *mq;       // [n_streams] model-ordered arrivals of each stream
     const int64_t *mq_off;          // [n_streams][M+1]
     const int64_t *lo, *hi;         // [n_streams] window [lo, hi) of request indices
     const int32_t *sim_stream;      // [n_sims] stream of each simulation
-    const int64_t *sim_base;        // [n_sims] wave * Rmax * 64 + lane: where its column of finish / good starts
+    const int64_t *sim_base;        // [n_sims] where its values of finish / good start: wave * Rmax * 64 + lane, or sim * Rmax
+    int32_t stride;                 // from one request to the next: 64 or 1
     uint64_t *scratch;              // [rows][scratch_pitch] latencies of a stream's requests in model order (all ones: not accepted)
     int64_t scratch_pitch;
     int32_t M, sim0;

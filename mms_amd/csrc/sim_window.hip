@@ -1,0 +1,629 @@
+// Plain (non-batching) request-loop simulation for gfx950, small and middle-sized batches: requests side by side.
+//
+// The request loop of the reference (simulate_requests_mixed, alpa_serve/simulator/controller.py:561-628) is serial
+// in its requests, and sim_mixed.hip walks it that way, 64 placements to a wavefront: the fastest form when there
+// are enough placements to fill the chip (a hundred thousand simulations), and one wavefront's 470 cycles per
+// request when there are not -- a search step of a thousand candidates keeps 16 of the 1024 SIMDs busy.  Here the
+// lanes of a wavefront hold W consecutive REQUESTS of one placement (W = 64, 32, 16 or 8; 64 / W placements to a
+// wavefront), and a block of W requests takes as many steps as its longest chain of requests that really depend on
+// one another, not W.
+//
+// A step evaluates every pending request of the block against the clocks as they are: choice of the group, stage
+// walk, SLO decision.  Which of these verdicts are what the serial loop would find?
+//
+//   Clocks only ever grow, and only when a request is accepted.  Take a pending request j that chose group h, and
+//   let no earlier pending request i that is accepted, or whose verdict is open, list h among its replicas.  Then
+//   whatever the earlier ones do, the clocks of h are the same when j's turn comes, and those of the other groups on
+//   j's list have not become smaller: j still chooses h (ties go to the group listed first, and h won its ties
+//   already) and finds the same times.  Its verdict is final.  A request that does meet such an i waits for the next
+//   step, and counts as open for those behind it.
+//
+// The earliest pending request never waits, so every step settles at least one.  What is left of the dependences of a
+// training workload is about 7 to 17 steps for 64 requests, since bursts that overload a model are mostly rejects,
+// and a run of rejects is settled in one step.
+//
+// "Lists h among its replicas" is a bit mask per (request, replica): before the first step of a block every request
+// sets its bit in the masks of its groups (gm[slot] in LDS), reads back those of its own replicas and keeps the bits
+// of the requests before it.  The tournament that picks the group carries the mask along, so a step decides who has
+// to wait with one ballot ("accepted") and one AND, without another trip to LDS.  Requests that wait and are not
+// accepted so far, and list several groups, may still be accepted by another of their groups: only these can hold up
+// requests that the accepted ones do not hold up (the loop behind the ballot; rare).
+//
+// Times are the same fp64 operations in the reference's order as in sim_mixed.hip; the latency sum is accumulated in
+// arrival order (ordered_sum), so every result equals the serial loop's bit for bit.
+//
+// What bounds it: a lone wavefront per SIMD is one dependent chain per step, LDS read of the replicas' clocks ->
+// tournament -> walk -> ballot -> commit; when several share a SIMD, instruction issue.  Per placement all state is a
+// few KB of LDS and nothing in a step touches global memory; requests are fetched two blocks ahead, replica entries
+// one block ahead.
+//
+// LDS of one placement (byte offsets in WindowArgs, built by the wavefront itself from the packed placement):
+//   clk  [slots+1] f64      stage clocks, a placement's groups laid end to end, and a slot for writes that do not count
+//   gm   [slots+1] u64      mask of the block's requests that list the group whose last slot this is
+//   cnt  [slots+1] u64      requests (low half) and accepted requests (high half) of that group  (OUT >= 1)
+//   rep  [M][4] {u32, f32}  entry word and last-stage latency of the first four replicas, in group order
+//   ext  [..][4] {u32, f32} further replicas, four to a chunk; xi[M]: first chunk | chunks << 16
+//   bits [M][GW] u32        which groups host the model (used while the entries are made)
+//   gd   [Gmax] u32         entry word of every group
+//   mcnt [M] u32            accepted requests per model  (OUT >= 1)
+// Entry word: bits 0-14 LDS address / 8 of the group's last-stage clock, 15-19 stages - 1, 20-29 index of its
+// last-stage latency in the model's row of the latency table, 30 (fourth entry) "there are more", 31 "no such replica": the word then repeats the first
+// replica's (which wins every tie against its copies) or, without any replica, the placement's first slot.
+#include "mmsim_internal.h"
+
+namespace mmsim {
+namespace {
+
+// <wave primitives>
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// whether this lane's bit is set (a scalar mask used as a condition: no instruction)
+__device__ __forceinline__ bool in_mask(uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes); }
+// a request of the stream: a load that only counts as global (through a generic pointer it would be waited for with
+// the LDS accesses)
+__device__ __forceinline__ Req load_global(const Req *p) {
+    const u32x4 v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4 *>(reinterpret_cast<uintptr_t>(p));
+    return Req{__hiloint2double((int)v.y, (int)v.x), (int32_t)v.z, __uint_as_float(v.w)};
+}
+// Marks the places where the lanes' LDS accesses depend on one another: the compiler keeps them on their side (a
+// wavefront's LDS accesses are carried out in order; no instruction).
+__device__ __forceinline__ void wave_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ double vmax(double x, double y) {  // neither is NaN: no input quieting
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+__device__ __forceinline__ double vmin(double x, double y) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+template <typename T>
+__device__ __forceinline__ T lds_get(uint32_t addr) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) T *>(addr);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(uint32_t addr, T v) {
+    *reinterpret_cast<__attribute__((address_space(3))) T *>(addr) = v;
+}
+// waits for a request on its way here, not inside the loops that follow
+__device__ __forceinline__ void arrived_req(Req &r) {
+    uint32_t w[4];
+    __builtin_memcpy(w, &r, 16);
+    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+    __builtin_memcpy(&r, w, 16);
+}
+// In a loop that lanes leave one by one: what loop_enter to loop_leave encloses, with collectives of the lanes still in.
+__device__ __forceinline__ void loop_enter(bool) {}
+__device__ __forceinline__ void loop_leave() {}
+__device__ __forceinline__ uint64_t ballot_in_loop(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ void order_in_loop() { wave_order(); }
+// keeps the compiler from merging what made v with what uses it
+__device__ __forceinline__ void pin(uint32_t &v) { asm volatile("" : "+v"(v)); }
+// LDS atomics whose result nobody waits for
+__device__ __forceinline__ void lds_or_u32(uint32_t addr, uint32_t v) { asm volatile("ds_or_b32 %0, %1" : : "v"(addr), "v"(v) : "memory"); }
+__device__ __forceinline__ void lds_or_u64(uint32_t addr, uint64_t v) { asm volatile("ds_or_b64 %0, %1" : : "v"(addr), "v"(v) : "memory"); }
+__device__ __forceinline__ void lds_add_u32(uint32_t addr, uint32_t v) { asm volatile("ds_add_u32 %0, %1" : : "v"(addr), "v"(v) : "memory"); }
+__device__ __forceinline__ void lds_add_u64(uint32_t addr, uint64_t v) { asm volatile("ds_add_u64 %0, %1" : : "v"(addr), "v"(v) : "memory"); }
+__device__ __forceinline__ uint32_t lds_fetch_add_u32(uint32_t addr, uint32_t v) {
+    return __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(addr), v, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+template <int W>
+__device__ __forceinline__ int shfl_up(int v, int d) { return __shfl_up(v, (unsigned)d, W); }
+template <int W>
+__device__ __forceinline__ int shfl_last(int v) { return __shfl(v, W - 1, W); }
+template <int W>
+__device__ __forceinline__ int shfl_xor(int v, int d) { return __shfl_xor(v, d, W); }
+__device__ __forceinline__ int lane_value(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+
+// S + x of lane 0 of the W lanes, + x of lane 1, ...: one addition after the other, as the serial loop adds.  In and
+// out S is the same in all W lanes.  v_fmac_f64 with a DPP operand that a lane of the row broadcasts computes
+// fma(x_k, 1, S) = S + x_k, one instruction an addition (rows are 16 lanes; 64-bit DPP knows this pattern only), for
+// all placements of the wavefront at once; rows of one placement follow one another.  Lanes outside `lanes` hold zero.  A DPP operand needs two wait
+// states after its register is written (s_nop).
+#define MMSIM_ADD1(K, ROWS) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K " row_mask:" ROWS " bank_mask:0xf\n"
+#define MMSIM_ADD16(ROWS)                                                                                      \
+    MMSIM_ADD1(0, ROWS) MMSIM_ADD1(1, ROWS) MMSIM_ADD1(2, ROWS) MMSIM_ADD1(3, ROWS) MMSIM_ADD1(4, ROWS)          \
+    MMSIM_ADD1(5, ROWS) MMSIM_ADD1(6, ROWS) MMSIM_ADD1(7, ROWS) MMSIM_ADD1(8, ROWS) MMSIM_ADD1(9, ROWS)          \
+    MMSIM_ADD1(10, ROWS) MMSIM_ADD1(11, ROWS) MMSIM_ADD1(12, ROWS) MMSIM_ADD1(13, ROWS) MMSIM_ADD1(14, ROWS)     \
+    MMSIM_ADD1(15, ROWS)
+#define MMSIM_ADD2(K, K2)                                                            \
+    "v_fmac_f64_dpp %0, %2, %3 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n"     \
+    "v_fmac_f64_dpp %1, %2, %3 row_newbcast:" #K2 " row_mask:0xf bank_mask:0xf\n"
+#define MMSIM_ADD_ROWS(ROWS) \
+    asm("s_nop 1\n" MMSIM_ADD16(ROWS) "s_nop 1" : "+v"(s) : "v"(x), "v"(one))
+// what lane 15 of a row holds, into all lanes of the next row (rows named by ROWS)
+template <int ROWS>
+__device__ __forceinline__ double row_carry(double s) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(s), __double2loint(s), 0x142 /* row_bcast:15 */, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(s), __double2hiint(s), 0x142, ROWS, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+template <int W>
+__device__ __forceinline__ double ordered_sum(double s, double x, uint64_t lanes) {
+    const double one = 1.0;
+    if constexpr (W == 64) {
+        if (lanes & 0xFFFFull) MMSIM_ADD_ROWS("0x1");
+        s = row_carry<0x2>(s);
+        if (lanes & 0xFFFF0000ull) MMSIM_ADD_ROWS("0x2");
+        s = row_carry<0x4>(s);
+        if (lanes & 0xFFFF00000000ull) MMSIM_ADD_ROWS("0x4");
+        s = row_carry<0x8>(s);
+        if (lanes & 0xFFFF000000000000ull) MMSIM_ADD_ROWS("0x8");
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(s), 63), __builtin_amdgcn_readlane(__double2loint(s), 63));
+    } else if constexpr (W == 32) {
+        MMSIM_ADD_ROWS("0x5");
+        s = row_carry<0xA>(s);
+        MMSIM_ADD_ROWS("0xa");
+        return __hiloint2double(__shfl(__double2hiint(s), 31, 32), __shfl(__double2loint(s), 31, 32));
+    } else if constexpr (W == 16) {
+        MMSIM_ADD_ROWS("0xf");
+        return s;
+    } else {  // two placements to a row: lanes 0-7 are the first one's, lanes 8-15 the second one's
+        double s2 = s;
+        asm("s_nop 1\n" MMSIM_ADD2(0, 8) MMSIM_ADD2(1, 9) MMSIM_ADD2(2, 10) MMSIM_ADD2(3, 11) MMSIM_ADD2(4, 12) MMSIM_ADD2(5, 13)
+                MMSIM_ADD2(6, 14) MMSIM_ADD2(7, 15) "s_nop 1"
+            : "+v"(s), "+v"(s2)
+            : "v"(x), "v"(one));
+        return (lane_id() & 8) ? s2 : s;
+    }
+}
+#undef MMSIM_ADD_ROWS
+#undef MMSIM_ADD2
+#undef MMSIM_ADD16
+#undef MMSIM_ADD1
+// </wave primitives>
+
+struct Entry {  // a replica, as rep and ext hold it
+    uint32_t d;
+    float l;
+};
+struct Entry4 {
+    Entry e[4];
+};
+__device__ __forceinline__ float as_float(uint32_t v) { return __uint_as_float(v); }
+__device__ __forceinline__ uint32_t as_uint(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ Req fetch_req(uint32_t addr) {
+    const u32x4 v = lds_get<u32x4>(addr);
+    return Req{__hiloint2double((int)v.y, (int)v.x), (int32_t)v.z, as_float(v.w)};
+}
+__device__ __forceinline__ void store_req(uint32_t addr, const Req &r) {
+    lds_put<u32x4>(addr, u32x4{(uint32_t)__double2loint(r.t), (uint32_t)__double2hiint(r.t), (uint32_t)r.m, as_uint(r.slo)});
+}
+__device__ __forceinline__ Entry4 load_entries(uint32_t addr) {  // two 16-byte reads
+    const u32x4 a = lds_get<u32x4>(addr), b = lds_get<u32x4>(addr + 16u);
+    return Entry4{{{a.x, as_float(a.y)}, {a.z, as_float(a.w)}, {b.x, as_float(b.y)}, {b.z, as_float(b.w)}}};
+}
+__device__ __forceinline__ int max2(int x, int y) { return x > y ? x : y; }
+constexpr uint32_t kAddrMask8 = 0x7FFFu;
+constexpr uint32_t kEntryMore = 1u << 30;
+__device__ __forceinline__ uint32_t entry_addr(uint32_t d) { return (d & kAddrMask8) << 3; }
+__device__ __forceinline__ int entry_stages_m1(uint32_t d) { return (int)(d >> 15) & 0x1F; }
+__device__ __forceinline__ uint32_t entry_lat(uint32_t d) { return (d >> 20) & 0x3FFu; }
+__device__ __forceinline__ bool entry_none(uint32_t d) { return (int32_t)d < 0; }
+
+template <int I>
+struct Int {
+    static constexpr int value = I;
+};
+// W: requests (lanes) of one placement.  SMAX: most stages of a group (bucket).  OUTPUTS: anything beyond the scores
+// (a.flags says what).  EXT: some model has more than four replicas.  POW2: every group has 1, 2, 4, ... stages.  UNIFORM: one latency per (model, configuration).
+template <int W, int SMAX, bool OUTPUTS, bool EXT, bool POW2, bool UNIFORM>
+__global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(const WindowArgs a) {
+    constexpr int P = kWave / W;
+    const int lane = lane_id(), j = lane % W, sub = lane / W;
+    const int wv = (int)(threadIdx.x >> 6);
+    // latency table for the per-stage latencies of the walk (general tables only), shared by the workgroup
+    if (!UNIFORM && a.lat_lds_bytes > 0) {
+        for (int i = (int)threadIdx.x; i < a.M * a.lat_row; i += (int)blockDim.x) lds_put<float>((uint32_t)i * 4u, a.lat[i]);
+        __syncthreads();
+    }
+    const int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;  // (seed, tile of P placements)
+    if (unit >= (int64_t)a.tiles * a.out_seeds) return;
+    const int seed_row = (int)(unit / a.tiles);
+    const int b = (int)(unit % a.tiles) * P + sub;
+    const bool mine = b < a.B;
+    // (with a stream of its own for every placement there is one placement to a wavefront: the host sees to that)
+    const int seed = a.stream_of ? lane_value(a.stream_of[mine ? b : 0], 0) : seed_row;
+    const Req *__restrict__ reqs = a.stream_ptr[seed];
+    const uint32_t R = (uint32_t)a.stream_len[seed];
+
+    // LDS: [latency table][per wavefront: two chunks of 64 requests (W < 64)][per placement: its tables and state]
+    const uint32_t ring = (uint32_t)a.lat_lds_bytes + (uint32_t)wv * (uint32_t)window_ring_bytes(W);
+    const uint32_t base = (uint32_t)a.lat_lds_bytes + (blockDim.x >> 6) * (uint32_t)window_ring_bytes(W) +
+                          (uint32_t)(wv * P + sub) * (uint32_t)a.place_bytes;
+    const uint32_t clk = base, rep = base + a.o_rep, ext = base + a.o_ext, xi = base + a.o_xi;
+    const uint32_t bits = base + a.o_bits, gd = base + a.o_gd, mcnt = base + a.o_mcnt;
+    const uint32_t gm_rel = (uint32_t)(a.nslots + SMAX) * 8u, cnt_rel = gm_rel * 2u;  // from a clock to its mask and its counter
+    const uint32_t spare = clk + (uint32_t)a.nslots * 8u;  // SMAX slots for writes that do not count
+    const int M = a.M, GW = a.group_words, Gmax = a.Gmax;
+
+    // ---- the placement's tables
+    for (int k = j; k < (a.nslots + SMAX) * (OUTPUTS ? 3 : 2); k += W) lds_put<uint64_t>(clk + (uint32_t)k * 8u, 0ull);
+    for (int k = j; k < M * GW; k += W) lds_put<uint32_t>(bits + (uint32_t)k * 4u, 0u);
+    if (OUTPUTS)
+        for (int k = j; k < M; k += W) lds_put<uint32_t>(mcnt + (uint32_t)k * 4u, 0u);
+    const int ng = mine ? (int)a.num_groups[b] : 0;
+    {
+        const uint8_t *cfg = a.group_cfg + (size_t)(mine ? b : 0) * Gmax;
+        int slot = 0;
+        for (int g0 = 0; g0 < Gmax; g0 += W) {
+            const int g = g0 + j;
+            int pp = 0, c = 0;
+            if (g < ng) {
+                c = cfg[g];
+                pp = a.cfg_pp[c];
+            }
+            int upto = pp;
+            for (int d = 1; d < W; d *= 2) {
+                const int v = shfl_up<W>(upto, d);
+                if (j >= d) upto += v;
+            }
+            if (g < ng) {
+                const uint32_t last = (uint32_t)(slot + upto - 1);
+                const uint32_t lat_last = (uint32_t)a.lat_off[c] + (UNIFORM ? 0u : (uint32_t)(pp - 1));
+                lds_put<uint32_t>(gd + (uint32_t)g * 4u, (clk + last * 8u) >> 3 | (uint32_t)(pp - 1) << 15 | lat_last << 20);
+            }
+            slot += shfl_last<W>(upto);
+        }
+    }
+    uint32_t ext_used = base + a.o_gd + (uint32_t)Gmax * 4u;  // a word behind gd: chunks of ext given out
+    if (j == 0) lds_put<uint32_t>(ext_used, 0u);
+    wave_order();
+    if (mine)
+        for (uint32_t e = a.entry_off[b] + (uint32_t)j; e < a.entry_off[b + 1]; e += W) {
+            const uint32_t v = a.entries[e], m = v & 0xFFFFu, g = v >> 16;
+            lds_or_u32(bits + (m * (uint32_t)GW + (g >> 5)) * 4u, 1u << (g & 31u));
+        }
+    wave_order();
+    for (int m = j; m < M; m += W) {
+        const uint32_t mb = bits + (uint32_t)(m * GW) * 4u;
+        int n = 0;
+        for (int w = 0; w < GW; ++w) n += __popc(lds_get<uint32_t>(mb + (uint32_t)w * 4u));
+        uint32_t chunk0 = 0;
+        if constexpr (EXT) {
+            const uint32_t chunks = n > 4 ? (uint32_t)(n - 1) / 4u : 0u;
+            if (chunks > 0) chunk0 = lds_fetch_add_u32(ext_used, chunks);
+            lds_put<uint32_t>(xi + (uint32_t)m * 4u, chunk0 | chunks << 16);
+        }
+        Entry first{(clk >> 3) | kEmpty, __builtin_inff()};
+        int k = 0;
+        auto put = [&](const Entry &e) {
+            const uint32_t at = k < 4 ? rep + (uint32_t)(m * 4 + k) * 8u : ext + (chunk0 * 4u + (uint32_t)(k - 4)) * 8u;
+            lds_put<uint32_t>(at, k == 3 && n > 4 ? e.d | kEntryMore : e.d);
+            lds_put<float>(at + 4u, e.l);
+            ++k;
+        };
+        for (int w = 0; w < GW; ++w)
+            for (uint32_t v = lds_get<uint32_t>(mb + (uint32_t)w * 4u); v != 0u; v &= v - 1u) {
+                const uint32_t d = lds_get<uint32_t>(gd + (uint32_t)(w * 32 + __ffs((int)v) - 1) * 4u);
+                const Entry e{d, a.lat[(size_t)m * a.lat_row + entry_lat(d)]};
+                if (k == 0) first = Entry{d | kEmpty, e.l};
+                put(e);
+            }
+        while (k < 4 || (k & 3) != 0) put(first);
+    }
+    wave_order();
+
+    const double overhead = a.fixed_overhead;
+    const uint64_t my_bit = 1ull << lane;
+    // bits of this placement's requests before this one
+    const uint64_t before = (my_bit - 1ull) & ~((1ull << (sub * W)) - 1ull);
+    int32_t n_good = 0;
+    double lat_sum = 0.0;
+    const size_t row = (size_t)seed_row * a.B + (size_t)(mine ? b : 0);  // where the results go
+    double *fin_out = a.finish + row * (size_t)a.Rmax;
+    uint8_t *good_out = a.good + row * (size_t)a.Rmax;
+    const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
+
+    auto load_req = [&](uint32_t i) -> Req {
+        Req r{0.0, -1, 0.0f};
+        if (i < R) r = load_global(reqs + i);
+        return r;
+    };
+    auto load_rep = [&](int m) -> Entry4 { return load_entries(rep + (uint32_t)(m < 0 ? 0 : m) * 32u); };
+    // Requests come 64 at a time, one to a lane.  W == 64: that is a block, fetched two blocks ahead.  Otherwise the
+    // chunks pass through LDS, which deals them to the placements' lanes; the chunk after the one a block is of is in
+    // LDS as well, and the one after that on its way.
+    Req far = load_req((uint32_t)lane);
+    Req cur, nxt;
+    auto store_ring = [&](uint32_t chunk) { store_req(ring + (chunk & 1u) * 1024u + (uint32_t)lane * 16u, far); };
+    auto load_ring = [&](uint32_t i) -> Req { return fetch_req(ring + (i & 127u) * 16u); };
+    if constexpr (W == 64) {
+        cur = far;
+        nxt = load_req(64u + (uint32_t)lane);
+    } else {
+        store_ring(0u);
+        far = load_req(64u + (uint32_t)lane);
+        store_ring(1u);
+        far = load_req(128u + (uint32_t)lane);
+        wave_order();
+        cur = load_ring((uint32_t)j);
+        nxt = load_ring((uint32_t)(W + j));
+    }
+    Entry4 q = load_rep(cur.m);
+    // What a block is like: requests that can be served at all, that list several groups, more than two, more than
+    // four; how deep their groups are.  Worked out a block ahead (a scalar that depends on vector compares is slow to come).
+    uint64_t pend, multis, fours, mores, deep_a, deep_b;
+    auto look = [&]() {
+        pend = ballot(cur.m >= 0 && !entry_none(q.e[0].d));  // (past the end of the stream: m is -1)
+        multis = ballot(!entry_none(q.e[1].d)) & pend;
+        fours = ballot(!entry_none(q.e[2].d)) & pend;
+        if constexpr (EXT) mores = ballot((q.e[3].d & kEntryMore) != 0u) & pend;
+        if constexpr (SMAX > 1) {
+            const int deep = max2(max2(entry_stages_m1(q.e[0].d), entry_stages_m1(q.e[1].d)),
+                                  max2(entry_stages_m1(q.e[2].d), entry_stages_m1(q.e[3].d)));
+            deep_a = ballot(deep >= (SMAX == 4 ? 2 : SMAX == 16 ? 8 : 16)) & pend;
+            if constexpr (SMAX == 16) deep_b = ballot(deep >= 4) & pend;
+            if constexpr (EXT) {  // (the groups behind the fourth are not looked at: as deep as any of the batch)
+                if (a.smax > (SMAX == 4 ? 2 : SMAX == 16 ? 8 : 16)) deep_a |= mores;
+                if (SMAX == 16 && a.smax > 4) deep_b |= mores;
+            }
+        }
+    };
+    look();
+
+    for (uint32_t blk = 0; blk < R; blk += W) {
+        const int m = cur.m;
+        const double arr = cur.t, slo = (double)cur.slo;
+        uint32_t ca[4], word[4];  // what the tournament carries: the entry word, or all that single-stage groups need of it
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            ca[k] = entry_addr(q.e[k].d);
+            word[k] = SMAX == 1 ? ca[k] : q.e[k].d;
+        }
+        Entry4 nrep;
+        Req nn;
+        double best = 0.0, t = 0.0, latency = 0.0;
+        uint32_t chosen = clk;  // the chosen group's entry word (SMAX == 1: the address of its clock)
+        // The block, for requests that list at most NC groups (2, 4, or 5: more than four).
+        auto block = [&](auto NCv) {
+            constexpr int NC = decltype(NCv)::value, N4 = NC > 4 ? 4 : NC;
+            double c[N4];
+#pragma unroll
+            for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
+            // ---- the masks of the block's requests.  (Copies of the first replica set its bit again: harmless.)
+            uint64_t gm[N4];
+            uint32_t x0 = 0, xn = 0;  // chunks of further replicas
+            if constexpr (NC > 4) {
+                const uint32_t v = lds_get<uint32_t>(xi + (uint32_t)(m < 0 ? 0 : m) * 4u);
+                x0 = ext + (v & 0xFFFFu) * 32u;
+                xn = in_mask(pend) ? v >> 16 : 0u;
+            }
+            if (in_mask(pend)) {
+#pragma unroll
+                for (int k = 0; k < N4; ++k) lds_or_u64(ca[k] + gm_rel, my_bit);
+                if constexpr (NC > 4)
+                    for (uint32_t x = 0; x < xn; ++x) {
+                        const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) lds_or_u64(entry_addr(e.e[k].d) + gm_rel, my_bit);
+                    }
+            }
+            wave_order();
+#pragma unroll
+            for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ca[k] + gm_rel) & before;
+            uint64_t gm_ext = 0;  // requests before this one that share any of the groups: holds for every further replica
+            if constexpr (NC > 4) {
+                for (uint32_t x = 0; x < xn; ++x) {
+                    const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
+                }
+                gm_ext = (gm_ext & before) | gm[0] | gm[1] | gm[2] | gm[3];
+            }
+            wave_order();
+#pragma unroll
+            for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ca[k] + gm_rel, 0);  // for the next block
+            if constexpr (NC > 4)
+                for (uint32_t x = 0; x < xn; ++x) {
+                    const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
+                }
+            // ---- fetched ahead: the requests of the block after the next, the replicas of the next
+            nrep = load_rep(nxt.m);
+            if constexpr (W == 64) {
+                nn = load_req(blk + 128u + (uint32_t)j);
+            } else {
+                if ((blk & 63u) == 0u && blk != 0u) {  // a chunk begins: the one after it takes the place of the one before
+                    store_ring(blk / 64u + 1u);
+                    far = load_req(blk + 128u + (uint32_t)lane);
+                    wave_order();
+                }
+                nn = load_ring(blk + 2u * W + (uint32_t)j);
+            }
+            wave_order();
+            // ---- the steps.  Each lane stays in the loop until its verdict is final and leaves with what it found.
+            // D: most stages of a group.
+            auto steps = [&](auto Dv) {
+                constexpr int D = decltype(Dv)::value;
+                struct Cand {
+                    double c;
+                    uint32_t d;
+                    float l;
+                    uint64_t g;
+                };
+                auto first_min = [](const Cand &x, const Cand &y) {
+                    const bool right = y.c < x.c;
+                    return Cand{vmin(x.c, y.c), right ? y.d : x.d, right ? y.l : x.l, right ? y.g : x.g};
+                };
+                bool waits;
+                do {
+                    // ---- choose the replica group: strictly smallest last-stage clock, first listed wins ties (:590-598)
+                    Cand win = first_min(Cand{c[0], word[0], q.e[0].l, gm[0]}, Cand{c[1], word[1], q.e[1].l, gm[1]});
+                    if constexpr (NC > 2)
+                        win = first_min(win, first_min(Cand{c[2], word[2], q.e[2].l, gm[2]}, Cand{c[3], word[3], q.e[3].l, gm[3]}));
+                    if constexpr (NC > 4)
+                        for (uint32_t x = 0; x < xn; ++x) {
+                            const Entry4 e = load_entries(x0 + x * 32u);
+                            Cand y[4];
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                const uint32_t at = entry_addr(e.e[k].d);
+                                y[k] = Cand{lds_get<double>(at), SMAX == 1 ? at : e.e[k].d, e.e[k].l, gm_ext};
+                            }
+                            win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
+                        }
+                    best = win.c;
+                    chosen = win.d;
+                    // a clock that is infinite is never chosen (:590-598)
+                    const double limit = __hiloint2double(best < 1e100 ? __double2hiint(slo) : 0x7FF80000, __double2loint(slo));
+                    const double l_last = (double)win.l;
+                    // ---- walk the stages and decide (:605-613).  All requests read and walk D stages from their group's first
+                    // on and take the time after their last one (what lies behind a shallower group's slots does not matter).
+                    double cv[D];
+                    const uint32_t last = SMAX == 1 ? win.d : entry_addr(win.d);
+                    const int sm1 = SMAX == 1 ? 0 : entry_stages_m1(win.d);
+                    const uint32_t gclk = last - (uint32_t)sm1 * 8u;
+                    if constexpr (SMAX == 1) {
+                        t = vmax(arr, best) + l_last;
+                        cv[0] = t;
+                    } else {
+                        const uint32_t lrow = (uint32_t)m * (uint32_t)a.lat_row + entry_lat(win.d) - (uint32_t)sm1;
+                        float l[UNIFORM ? 1 : D];
+#pragma unroll
+                        for (int k = 0; k < D; ++k) {
+                            cv[k] = lds_get<double>(gclk + (uint32_t)k * 8u);
+                            if constexpr (!UNIFORM)
+                                l[k] = a.lat_lds_bytes > 0 ? lds_get<float>((lrow + (uint32_t)k) * 4u) : a.lat[lrow + (uint32_t)k];
+                        }
+#pragma unroll
+                        for (int k = 0; k < D; ++k) {
+                            cv[k] = vmax(k == 0 ? arr : cv[k > 0 ? k - 1 : 0], cv[k]) + (UNIFORM ? l_last : (double)l[UNIFORM ? 0 : k]);
+                            if (k == 0)
+                                t = cv[0];
+                            else if (!POW2 || (k & (k + 1)) == 0)
+                                t = sm1 >= k ? cv[k] : t;
+                        }
+                    }
+                    latency = (t + overhead) - arr;
+                    const uint64_t accs = ballot_in_loop(latency <= limit);
+                    // ---- whose verdict is final
+                    const uint64_t blockers = win.g & accs;
+                    waits = blockers != 0ull;
+                    uint64_t waiting = ballot_in_loop(waits);
+                    // requests that wait, are not accepted so far and list several groups: they hold up others too
+                    for (uint64_t open = waiting & multis & ~accs; __builtin_expect(open != 0ull, 0);) {
+                        waits = (win.g & (accs | waiting)) != 0ull;
+                        const uint64_t w2 = ballot_in_loop(waits);
+                        open = w2 & ~waiting & multis & ~accs;
+                        waiting = w2;
+                    }
+                    // accepted and final: the clocks (:614-619).  Everybody writes, the others where it does not matter.
+                    uint32_t to = in_mask(accs) ? gclk : spare;
+                    pin(to);
+                    to = waits ? spare : to;
+                    pin(to);
+#pragma unroll
+                    for (int k = 0; k < D; ++k) {
+                        if (k > 0 && (!POW2 || (k & (k - 1)) == 0)) {
+                            to = sm1 >= k ? to : spare;
+                            pin(to);
+                        }
+                        lds_put<double>(to + (uint32_t)k * 8u, cv[k]);
+                    }
+                    order_in_loop();
+#pragma unroll
+                    for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
+                } while (waits);
+            };
+            loop_enter(in_mask(pend));
+            if (in_mask(pend)) {
+                if constexpr (SMAX == 1) {
+                    steps(Int<1>{});
+                } else if constexpr (SMAX == 4) {
+                    if (deep_a == 0ull) steps(Int<2>{});
+                    else steps(Int<4>{});
+                } else if constexpr (SMAX == 16) {
+                    if (deep_a != 0ull) steps(Int<16>{});
+                    else if (deep_b != 0ull) steps(Int<8>{});
+                    else steps(Int<4>{});
+                } else {
+                    if (deep_a == 0ull) steps(Int<16>{});
+                    else steps(Int<32>{});
+                }
+                loop_leave();
+            }
+        };
+        if constexpr (EXT) {
+            if (mores != 0ull) block(Int<5>{});
+            else if (fours != 0ull) block(Int<4>{});
+            else block(Int<2>{});
+        } else {
+            if (fours != 0ull) block(Int<4>{});
+            else block(Int<2>{});
+        }
+        wave_order();
+        const uint64_t found = ballot(best < 1e100) & pend, accepted = ballot(latency <= slo) & found;
+        const bool good = in_mask(accepted);
+        const double took = good ? latency : 0.0;
+        n_good += good ? 1 : 0;
+        if constexpr (OUTPUTS) {
+            if (in_mask(found)) lds_add_u64((SMAX == 1 ? chosen : entry_addr(chosen)) + cnt_rel, good ? 0x100000001ull : 1ull);  // :611, :618
+            if (good) lds_add_u32(mcnt + (uint32_t)m * 4u, 1u);
+        }
+        if constexpr (OUTPUTS)
+            if (want_req && mine && blk + (uint32_t)j < R) {
+                fin_out[blk + (uint32_t)j] = good ? t + overhead : arr;
+                good_out[blk + (uint32_t)j] = good ? 1 : 0;
+            }
+        if constexpr (W == 64) arrived_req(nn);
+        cur = nxt;
+        nxt = nn;
+        q = nrep;
+        look();
+        if (accepted != 0ull) lat_sum = ordered_sum<W>(lat_sum, took, accepted);
+    }
+
+    for (int d = 1; d < W; d *= 2) n_good += shfl_xor<W>(n_good, d);
+    if (!mine) return;
+    if (j == 0) {
+        a.n_good[row] = n_good;
+        a.lat_sum[row] = lat_sum;
+    }
+    if constexpr (OUTPUTS) {
+        if (a.flags & MMSIM_WANT_MODEL_COUNTS)
+            for (int m = j; m < M; m += W) a.model_good[row * (size_t)M + (size_t)m] = (int32_t)lds_get<uint32_t>(mcnt + (uint32_t)m * 4u);
+        if (a.flags & MMSIM_WANT_GROUP_COUNTS)
+            for (int g = j; g < Gmax; g += W) {
+                uint64_t v = 0ull;
+                if (g < ng) v = lds_get<uint64_t>(entry_addr(lds_get<uint32_t>(gd + (uint32_t)g * 4u)) + cnt_rel);
+                a.group_req[row * (size_t)Gmax + (size_t)g] = (int32_t)(uint32_t)v;
+                a.group_good[row * (size_t)Gmax + (size_t)g] = (int32_t)(v >> 32);
+            }
+    }
+}
+
+constexpr int W_ = MMSIM_WINDOW_LANES;  // the file is compiled once for each number of requests side by side
+
+template <int SMAX, bool POW2, bool UNIFORM>
+WindowKernel pick_out(bool outputs, bool ext) {
+    if (outputs) return ext ? sim_window_kernel<W_, SMAX, true, true, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, true, false, POW2, UNIFORM>;
+    return ext ? sim_window_kernel<W_, SMAX, false, true, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, false, false, POW2, UNIFORM>;
+}
+template <int SMAX>
+WindowKernel pick_depths(bool outputs, bool ext, bool pow2, bool uniform) {
+    if (pow2) return uniform ? pick_out<SMAX, true, true>(outputs, ext) : pick_out<SMAX, true, false>(outputs, ext);
+    return uniform ? pick_out<SMAX, false, true>(outputs, ext) : pick_out<SMAX, false, false>(outputs, ext);
+}
+
+}  // namespace
+
+template <>
+WindowKernel window_kernel<MMSIM_WINDOW_LANES>(int smax, bool outputs, bool ext, bool pow2, bool uniform) {
+    switch (smax) {
+        case 1: return pick_out<1, true, true>(outputs, ext);  // one stage: its latency is the configuration's
+        case 4: return pick_depths<4>(outputs, ext, pow2, uniform);
+        case 16: return pick_depths<16>(outputs, ext, pow2, uniform);
+        case 32: return pick_depths<32>(outputs, ext, pow2, uniform);
+        default: return nullptr;
+    }
+}
+
+}  // namespace mmsim

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kStatsThreads) void model_stats_kernel(StatsArgs a)
     long long first_e = 0x7FFFFFFFFFFFFFFFll, last_e = -1;
     Accum acc;
     for (int64_t e = e0 + tid; e < e1; e += kStatsThreads) {
-        const size_t row = (size_t)q[e].idx * kWave;
+        const size_t row = (size_t)q[e].idx * (size_t)a.stride;
         const bool ok = gd[row] != 0;
         const double lat = fin[row] - q[e].t;
         const uint64_t bits = ok ? key_of(lat) : kNotAccepted;

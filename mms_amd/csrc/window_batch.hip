@@ -1,0 +1,351 @@
+// Host side of the kernel that simulates requests side by side (sim_window.hip): which batches it is for, how many
+// requests of a placement share a wavefront, packing, launch, results.
+//
+// The placements travel as they were given, a few bytes per replica: the wavefronts build their own tables (the other
+// kernels' descriptor tables are a kilobyte per placement and model of a tile).  One buffer holds every input and one
+// every output, so a call is one copy in, one launch and one copy out, through the context's pinned staging memory.
+#include <cstring>
+
+#include "mmsim_host.h"
+
+namespace mmsim {
+namespace {
+
+size_t up16(size_t v) { return (v + 15) & ~(size_t)15; }
+
+// Bump layout of a buffer: offset of the next array.
+struct Layout {
+    size_t used = 0;
+    size_t take(size_t bytes) {
+        const size_t at = used;
+        used += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
+};
+
+bool has_outputs(uint32_t flags) {
+    return (flags & (MMSIM_WANT_PER_REQUEST | MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS)) != 0;
+}
+
+hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_bytes, hipStream_t stream) {
+    const bool out = has_outputs(a.flags), ext = a.has_ext != 0, pow2 = a.pow2_depths != 0, uniform = a.uniform_stages != 0;
+    const WindowKernel kern = a.lanes == 64   ? window_kernel<64>(a.smax_bucket, out, ext, pow2, uniform)
+                              : a.lanes == 32 ? window_kernel<32>(a.smax_bucket, out, ext, pow2, uniform)
+                              : a.lanes == 16 ? window_kernel<16>(a.smax_bucket, out, ext, pow2, uniform)
+                                              : window_kernel<8>(a.smax_bucket, out, ext, pow2, uniform);
+    if (!kern || waves_per_block < 1 || waves_per_block > kMaxWindowWaves) return hipErrorInvalidValue;
+    if (lds_bytes > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        if (e != hipSuccess) return e;
+    }
+    const int64_t units = (int64_t)a.tiles * a.out_seeds;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((units + waves_per_block - 1) / waves_per_block)), dim3((unsigned)waves_per_block * kWave),
+                       lds_bytes, stream, a);
+    return hipGetLastError();
+}
+
+struct Shape {
+    int32_t nslots = 1, smax = 1, rmax = 1, ext_cap = 0;
+    bool pow2 = true;  // every group has 1, 2, 4, ... stages
+};
+
+}  // namespace
+
+int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
+                 const mmsim_placements *p, const int32_t *stream_of, uint32_t flags, const mmsim_options &o, bool events,
+                 mmsim_batch **out) {
+    constexpr int kOther = 1;  // the batch is for the other kernels, or they will say what is wrong with it
+    if (o.window_lanes < 0 || (flags & (MMSIM_BATCHING | MMSIM_WANT_OP_COUNT))) return kOther;
+    if (o.window_lanes == 0 && (o.request_loop >= 0 || o.waves_per_cu > 0 || o.counts_in_lds >= 0 || o.tile_order_by_slots >= 0 ||
+                                o.sched_groups > 0 || o.segment_requests > 0 || o.sched_spin_limit >= 0 || o.skip_ahead >= 0 || o.xcd_map >= 0))
+        return kOther;
+    if (!p || !p->num_groups || !p->group_cfg || !p->gm_off || p->B < 1 || p->Gmax < 1 || p->Gmax > MMSIM_MAX_GROUPS) return kOther;
+    if (n_seeds < 1 || !wls || t->M > 65535) return kOther;
+    for (int s = 0; s < n_seeds; ++s)
+        if (!wls[s] || wls[s]->ctx != ctx || wls[s]->M != t->M) return kOther;
+    const int32_t B = p->B, M = t->M, Gmax = p->Gmax, C = t->C;
+    const int32_t out_seeds = stream_of ? 1 : n_seeds;
+    const int64_t sims = (int64_t)B * out_seeds;
+    if (o.window_lanes == 0 && sims > kMaxWindowSims) return kOther;
+    if (stream_of)
+        for (int32_t b = 0; b < B; ++b)
+            if (stream_of[b] < 0 || stream_of[b] >= n_seeds) return kOther;
+    CompactLatency cl;
+    if (compact_latency(t, false, &cl) != MMSIM_OK) return kOther;
+
+    // ---- inputs: one buffer
+    Layout in;
+    int64_t replicas = 0;
+    for (int32_t b = 0; b < B; ++b) {
+        const int32_t G = p->num_groups[b];
+        if (G < 0 || G > Gmax) return kOther;
+        const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+        if (off[G] < off[0] || (off[G] > off[0] && !p->gm_idx)) return kOther;
+        replicas += off[G] - off[0];
+        if (replicas > 0x7FFFFFFF) return kOther;
+    }
+    const size_t at_ptr = in.take(sizeof(void *) * (size_t)n_seeds), at_len = in.take(sizeof(int64_t) * (size_t)n_seeds);
+    const size_t at_so = in.take(stream_of ? sizeof(int32_t) * (size_t)B : 0);
+    const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
+    const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
+    const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
+    HIP_TRY(hipSetDevice(ctx->device));
+    HIP_TRY(ctx->staging.ensure(in.used));
+    unsigned char *host = ctx->staging.p;
+    uint8_t *h_ng = host + at_ng, *h_cfg = host + at_cfg;
+    uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off), *h_ent = reinterpret_cast<uint32_t *>(host + at_ent);
+    {
+        uint32_t at = 0;
+        for (int32_t b = 0; b < B; ++b) {
+            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+            h_off[b] = at;
+            at += (uint32_t)(off[p->num_groups[b]] - off[0]);
+        }
+        h_off[B] = at;
+    }
+    std::atomic<bool> bad{false};
+    std::mutex shape_mutex;
+    Shape shape;
+    parallel_slices(B, 1024, [&](int64_t b0, int64_t b1) {
+        Shape mine;
+        std::vector<uint8_t> count((size_t)M, 0);
+        for (int64_t b = b0; b < b1; ++b) {
+            const int32_t G = p->num_groups[b];
+            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+            const int32_t *cfg = p->group_cfg + (size_t)b * Gmax;
+            uint32_t *ent = h_ent + h_off[b];
+            int32_t slots = 0, chunks = 0;
+            h_ng[b] = (uint8_t)G;
+            for (int32_t g = 0; g < Gmax; ++g) {
+                h_cfg[(size_t)b * Gmax + g] = g < G ? (uint8_t)cfg[g] : 0;
+                if (g >= G) continue;
+                if (cfg[g] < 0 || cfg[g] >= C || off[g + 1] < off[g]) {
+                    bad = true;
+                    return;
+                }
+                const int32_t pp = t->cfg_pp[cfg[g]];
+                slots += pp;
+                mine.pow2 = mine.pow2 && (pp & (pp - 1)) == 0;
+                mine.smax = std::max(mine.smax, pp);
+                for (int64_t x = off[g]; x < off[g + 1]; ++x) {
+                    const int32_t m = p->gm_idx[x];
+                    if (m < 0 || m >= M || count[m] >= MMSIM_MAX_REPLICAS) {
+                        bad = true;
+                        return;
+                    }
+                    *ent++ = (uint32_t)m | (uint32_t)g << 16;
+                    chunks += count[m] >= 4 && (count[m] & 3) == 0;
+                    count[m] += 1;
+                    mine.rmax = std::max<int32_t>(mine.rmax, count[m]);
+                }
+            }
+            if (slots > MMSIM_MAX_SLOTS) {
+                bad = true;
+                return;
+            }
+            mine.nslots = std::max(mine.nslots, slots);
+            mine.ext_cap = std::max(mine.ext_cap, chunks);
+            for (const uint32_t *e = h_ent + h_off[b]; e < ent; ++e) count[*e & 0xFFFFu] = 0;
+        }
+        std::lock_guard<std::mutex> lock(shape_mutex);
+        shape.nslots = std::max(shape.nslots, mine.nslots);
+        shape.smax = std::max(shape.smax, mine.smax);
+        shape.pow2 = shape.pow2 && mine.pow2;
+        shape.rmax = std::max(shape.rmax, mine.rmax);
+        shape.ext_cap = std::max(shape.ext_cap, mine.ext_cap);
+    });
+    if (bad) return kOther;
+
+    // ---- LDS of one placement, lanes per placement, wavefronts per workgroup
+    WindowArgs a{};
+    a.smax = shape.smax;
+    a.smax_bucket = smax_bucket_for(shape.smax);
+    if (a.smax_bucket < 0) return kOther;
+    const bool uniform = cl.uniform || a.smax_bucket == 1;
+    const bool counts = has_outputs(flags);
+    const int group_words = (Gmax + 31) / 32;
+    // (behind the clocks as many slots as a walk has stages, for reads and writes that do not count)
+    size_t place = up16(((size_t)shape.nslots + a.smax_bucket) * 8 * (counts ? 3 : 2));
+    a.o_rep = (int32_t)place;
+    place += (size_t)M * 32;
+    a.o_ext = (int32_t)place;
+    place += (size_t)shape.ext_cap * 32;
+    a.o_xi = (int32_t)place;
+    place = up16(place + (shape.ext_cap > 0 ? (size_t)M * 4 : 0));
+    a.o_bits = (int32_t)place;
+    place = up16(place + (size_t)M * group_words * 4);
+    a.o_gd = (int32_t)place;
+    place = up16(place + ((size_t)Gmax + 1) * 4);
+    a.o_mcnt = (int32_t)place;
+    place = up16(place + (counts ? (size_t)M * 4 : 0));
+    const size_t lds = (size_t)ctx->max_lds, lat_bytes = uniform ? 0 : up16(cl.lat.size() * sizeof(float));
+    if (place > lds) return kOther;
+    const size_t lat_lds = lat_bytes + place <= lds ? lat_bytes : 0;
+    const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
+    auto wave_lds = [&](int lanes) { return place * (size_t)(kWave / lanes) + (size_t)window_ring_bytes(lanes); };
+    auto fits = [&](int lanes) { return lat_lds + wave_lds(lanes) <= lds; };
+    int lanes = o.window_lanes;
+    if (lanes == 0) {
+        // as many placements to a wavefront as it takes to get one wavefront to a SIMD
+        lanes = 64;
+        while (lanes > 8 && sims * lanes / kWave > 4 * cus && fits(lanes / 2)) lanes /= 2;
+    }
+    if (stream_of) lanes = kWave;  // (the placements of a wavefront share a stream)
+    while (lanes < kWave && !fits(lanes)) lanes *= 2;
+    if (!fits(lanes)) return kOther;
+    const int per_wave = kWave / lanes;
+    const int64_t tiles = (B + per_wave - 1) / per_wave, units = tiles * out_seeds;
+    int waves = (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (units + cus - 1) / cus));
+    while (waves > 1 && lat_lds + wave_lds(lanes) * (size_t)waves > lds) --waves;
+
+    std::unique_ptr<mmsim_batch> b(new (std::nothrow) mmsim_batch);
+    if (!b) return fail(MMSIM_E_NOMEM, "host allocation failed");
+    b->ctx = ctx;
+    b->opt = o;
+    b->window = true;
+    b->flags = flags;
+    b->n_seeds = n_seeds;
+    b->B = B;
+    b->M = M;
+    b->Gmax = Gmax;
+    b->paired = stream_of != nullptr;
+    b->out_seeds = out_seeds;
+    b->tiles = (int32_t)tiles;
+    b->waves = (int32_t)units;
+    b->smax_bucket = a.smax_bucket;
+    b->rmax_all = shape.rmax;
+    b->nslots = shape.nslots;
+    b->waves_per_block = waves;
+    b->lds_bytes = lat_lds + wave_lds(lanes) * (size_t)waves;
+    if (stream_of) b->stream_of.assign(stream_of, stream_of + B);
+    const Req **h_ptr = reinterpret_cast<const Req **>(host + at_ptr);
+    int64_t *h_len = reinterpret_cast<int64_t *>(host + at_len);
+    for (int s = 0; s < n_seeds; ++s) {
+        b->wl_R.push_back(wls[s]->R);
+        b->wl_id.push_back(wls[s]->id);
+        b->wl_model_requests.push_back(wls[s]->model_num_requests);
+        b->win_streams.push_back(wls[s]->reqs);  // (the workload may be destroyed before the batch)
+        h_ptr[s] = wls[s]->reqs->p;
+        h_len[s] = wls[s]->R;
+        b->Rmax = std::max(b->Rmax, wls[s]->R);
+        b->Rtotal += wls[s]->R;
+    }
+    if (stream_of) std::memcpy(host + at_so, stream_of, sizeof(int32_t) * (size_t)B);
+    for (int32_t c = 0; c < C; ++c) {
+        (host + at_pp)[c] = (uint8_t)t->cfg_pp[c];
+        reinterpret_cast<uint16_t *>(host + at_loff)[c] = (uint16_t)cl.off[c];
+    }
+    std::memcpy(host + at_lat, cl.lat.data(), sizeof(float) * cl.lat.size());
+
+    // ---- outputs: one buffer, laid out as the caller's arrays
+    Layout res;
+    const size_t L = (size_t)sims;
+    res.take(sizeof(int32_t) * L);
+    b->win_lat_sum = res.take(sizeof(double) * L);
+    b->win_model = res.take((flags & MMSIM_WANT_MODEL_COUNTS) ? sizeof(int32_t) * L * M : 0);
+    b->win_group = res.take((flags & MMSIM_WANT_GROUP_COUNTS) ? 2 * sizeof(int32_t) * L * Gmax : 0);
+    b->win_finish = res.take((flags & MMSIM_WANT_PER_REQUEST) ? sizeof(double) * L * (size_t)b->Rmax : 0);
+    b->win_good = res.take((flags & MMSIM_WANT_PER_REQUEST) ? L * (size_t)b->Rmax : 0);
+
+    HIP_TRY(b->win_in.alloc(in.used));
+    HIP_TRY(b->win_out.alloc(res.used));
+    HIP_TRY(hipMemcpyAsync(b->win_in.p, host, in.used, hipMemcpyHostToDevice, ctx->stream));
+    if (events) {
+        if (g_arena) {
+            b->own_events = false;
+            b->ev_start = ctx->ev_static[0];
+            b->ev_stop = ctx->ev_static[1];
+        } else {
+            HIP_TRY(hipEventCreate(&b->ev_start));
+            HIP_TRY(hipEventCreate(&b->ev_stop));
+        }
+        HIP_TRY(hipStreamSynchronize(ctx->stream));  // a batch that is kept: the staging memory serves other calls before its run
+        ctx->staging.trim();
+    }
+    const uint8_t *d = b->win_in.p;
+    a.stream_ptr = reinterpret_cast<const Req *const *>(d + at_ptr);
+    a.stream_len = reinterpret_cast<const int64_t *>(d + at_len);
+    a.stream_of = stream_of ? reinterpret_cast<const int32_t *>(d + at_so) : nullptr;
+    a.num_groups = d + at_ng;
+    a.group_cfg = d + at_cfg;
+    a.entry_off = reinterpret_cast<const uint32_t *>(d + at_off);
+    a.entries = reinterpret_cast<const uint32_t *>(d + at_ent);
+    a.cfg_pp = d + at_pp;
+    a.lat_off = reinterpret_cast<const uint16_t *>(d + at_loff);
+    a.lat = reinterpret_cast<const float *>(d + at_lat);
+    a.M = M;
+    a.lat_row = cl.row;
+    a.B = B;
+    a.Gmax = Gmax;
+    a.group_words = group_words;
+    a.nslots = shape.nslots;
+    a.tiles = (int32_t)tiles;
+    a.out_seeds = out_seeds;
+    a.lanes = lanes;
+    a.pow2_depths = shape.pow2 ? 1 : 0;
+    a.uniform_stages = uniform ? 1 : 0;
+    a.has_ext = shape.ext_cap > 0 ? 1 : 0;
+    a.lat_lds_bytes = (int32_t)lat_lds;
+    a.place_bytes = (int32_t)place;
+    a.Rmax = b->Rmax;
+    a.fixed_overhead = t->fixed_overhead;
+    a.flags = flags;
+    uint8_t *r = b->win_out.p;
+    a.n_good = reinterpret_cast<int32_t *>(r);
+    a.lat_sum = reinterpret_cast<double *>(r + b->win_lat_sum);
+    a.model_good = reinterpret_cast<int32_t *>(r + b->win_model);
+    a.group_req = reinterpret_cast<int32_t *>(r + b->win_group);
+    a.group_good = a.group_req + L * Gmax;
+    a.finish = reinterpret_cast<double *>(r + b->win_finish);
+    a.good = r + b->win_good;
+    b->wargs = a;
+    *out = b.release();
+    return MMSIM_OK;
+}
+
+std::string sim_window_kernel_name(const WindowArgs &a) {
+    auto tf = [](bool v) { return v ? ", true" : ", false"; };
+    return "sim_window_kernel<" + std::to_string(a.lanes) + ", " + std::to_string(a.smax_bucket) + tf(has_outputs(a.flags)) + tf(a.has_ext != 0) +
+           tf(a.pow2_depths != 0) + tf(a.uniform_stages != 0) + ">";
+}
+
+int run_window(mmsim_batch *b) {
+    if (b->ev_start) HIP_TRY(hipEventRecord(b->ev_start, b->ctx->stream));
+    HIP_TRY(launch_window(b->wargs, b->waves_per_block, b->lds_bytes, b->ctx->stream));
+    if (b->ev_stop) HIP_TRY(hipEventRecord(b->ev_stop, b->ctx->stream));
+    b->ran = true;
+    return MMSIM_OK;
+}
+
+int fetch_window(mmsim_batch *b, mmsim_result *out) {
+    const bool wm = b->flags & MMSIM_WANT_MODEL_COUNTS, wg = b->flags & MMSIM_WANT_GROUP_COUNTS,
+               wr = (b->flags & MMSIM_WANT_PER_REQUEST) && out->finish && out->good;
+    hipStream_t st = b->ctx->stream;
+    const size_t L = (size_t)b->B * b->out_seeds, M = (size_t)b->M, G = (size_t)b->Gmax, Rm = (size_t)b->Rmax;
+    Staging &stage = b->ctx->staging;
+    HIP_TRY(stage.ensure(b->win_finish));
+    HIP_TRY(hipMemcpyAsync(stage.p, b->win_out.p, b->win_finish, hipMemcpyDeviceToHost, st));
+    if (wr && Rm > 0) {
+        HIP_TRY(hipMemcpyAsync(out->finish, b->win_out.p + b->win_finish, sizeof(double) * L * Rm, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(out->good, b->win_out.p + b->win_good, L * Rm, hipMemcpyDeviceToHost, st));
+    }
+    HIP_TRY(hipStreamSynchronize(st));
+    const int32_t *ng = reinterpret_cast<const int32_t *>(stage.p);
+    for (size_t l = 0; l < L; ++l) out->n_good[l] = ng[l];
+    std::memcpy(out->latency_sum, stage.p + b->win_lat_sum, sizeof(double) * L);
+    if (out->status) std::memset(out->status, 0, sizeof(int32_t) * L);
+    if (wm) {
+        std::memcpy(out->model_num_good, stage.p + b->win_model, sizeof(int32_t) * L * M);
+        for (size_t l = 0; l < L; ++l)
+            std::memcpy(out->model_num_requests + l * M,
+                        b->wl_model_requests[(size_t)(b->paired ? b->stream_of[l] : (int32_t)(l / (size_t)b->B))].data(), sizeof(int32_t) * M);
+    }
+    if (wg) {
+        std::memcpy(out->group_num_requests, stage.p + b->win_group, sizeof(int32_t) * L * G);
+        std::memcpy(out->group_num_good, stage.p + b->win_group + sizeof(int32_t) * L * G, sizeof(int32_t) * L * G);
+    }
+    stage.trim();
+    return MMSIM_OK;
+}
+
+}  // namespace mmsim

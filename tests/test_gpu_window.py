@@ -1,0 +1,104 @@
+"""The plain simulator with requests side by side (sim_window.hip) against the CPU oracle, bit for bit: every number of
+requests side by side, at the sizes where it can go wrong -- streams that end inside a block or a chunk of requests,
+batches that do not fill a wavefront, models with more replicas than one and two fetches hold, depths that are powers of
+two and others, tables with a latency per stage, infinite latencies and odd SLOs."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from mms_amd import _lib, engine as E
+from mms_amd.placement_policy.base_policy import ModelPlacement
+from mms_amd.profiling import LatencyMemData, ParallelConfig, ProfilingResult
+from helpers import assert_batch_matches, oracle_batch
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = _lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS
+
+
+def _problem(seed, depths, uniform, M, groups, B, hosts):
+    rng = np.random.default_rng(seed)
+    pcs = [ParallelConfig(1, 1, d) for d in depths]
+    profiles = []
+    for m in range(M):
+        para = {}
+        for pc in pcs:
+            if rng.random() < 0.04:
+                continue                                   # no profile: an infinite latency
+            total = rng.uniform(0.05, 0.3)
+            stages = np.full(pc.pp, total / pc.pp) if uniform else rng.dirichlet(np.ones(pc.pp)) * total
+            para[pc] = LatencyMemData({1: [float(x) for x in stages]}, {1: [0.0] * pc.pp}, [1.0] * pc.pp)
+        profiles.append(ProfilingResult(f"m{m}", para, 0, 0))
+    sols = []
+    for _ in range(B):
+        n = int(rng.integers(1, groups + 1))
+        sols.append(ModelPlacement([pcs[int(rng.integers(len(pcs)))] for _ in range(n)],
+                                   [[int(x) for x in rng.choice(M, size=int(rng.integers(0, hosts + 1)), replace=False)] for _ in range(n)]))
+    return profiles, sols
+
+
+def _stream(seed, R, M, load):
+    rng = np.random.default_rng(seed)
+    gaps = rng.exponential(0.02 / load, size=R)
+    gaps[rng.random(R) < 0.2] = 0.0
+    ids = np.repeat(rng.integers(-1, M, R + 1), rng.geometric(0.4, R + 1))[:R].astype(np.int32)
+    slos = rng.uniform(0.1, 0.8, R).astype(np.float32)
+    slos[rng.random(R) < 0.02] = np.inf
+    slos[rng.random(R) < 0.02] = np.nan
+    return SimpleNamespace(tstamps=np.cumsum(gaps), model_ids=ids, slos=slos)
+
+
+@pytest.mark.parametrize("lanes", [64, 32, 16, 8])
+@pytest.mark.parametrize("depths,uniform,groups,hosts", [((1,), True, 6, 4), ((1,), True, 40, 5), ((1, 2, 4), True, 5, 4), ((1, 3, 4), False, 9, 5),
+                                                        ((1, 2, 4, 8, 16), True, 7, 4), ((2, 5, 11), False, 12, 5), ((8, 32), True, 6, 4), ((7, 20), True, 6, 5)])
+def test_requests_side_by_side(lanes, depths, uniform, groups, hosts):
+    eng = E.Engine.default()
+    M = 5 if groups > 6 else 9
+    lengths = (0, 1, lanes - 1, lanes + 1, 127, 128, 1500)
+    streams = [_stream(100 * lanes + k, R, M, 1.0 + k) for k, R in enumerate(lengths)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    for B, flags in ((1, COUNTS | _lib.WANT_PER_REQUEST), (64 // lanes + 1, COUNTS), (131, 0)):
+        profiles, sols = _problem(B + sum(depths), depths, uniform, M, groups, B, hosts)
+        table = E.LatencyTable(profiles, [1])
+        packed = E.pack_placements(sols, table)
+        batch = E.Batch(eng, dws, table, packed, flags, options=dict(window_lanes=lanes))
+        assert batch.kernel_name().startswith(f"sim_window_kernel<{lanes},")
+        for _ in range(2):                                 # a second run starts from scratch again
+            batch.run()
+            batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k, st in enumerate(streams):
+            ref = oracle_batch(st, table, packed, want_per_request=bool(flags & _lib.WANT_PER_REQUEST))
+            if flags & _lib.WANT_PER_REQUEST:
+                R = len(st.tstamps)
+                assert np.array_equal(out["good"][k][:, :R], ref["good"]) and np.array_equal(out["finish"][k][:, :R], ref["finish"])
+            assert_batch_matches(out, ref, k, packed[0], where=f"{lanes} lanes, B={B}, stream {k}")
+    for dw in dws:
+        dw.close()
+
+
+def test_replaced_placements_and_the_kept_streams():
+    """eval_pairs on this kernel (one placement to a wavefront), and a batch that outlives the workloads it was made from."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(5, (1, 2, 4), True, 6, 5, 37, 4)
+    table = E.LatencyTable(profiles, [1])
+    packed = E.pack_placements(sols, table)
+    streams = [_stream(40 + k, R, 6, 2.0) for k, R in enumerate((700, 1, 333))]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, 6) for s in streams]
+    of = np.arange(len(sols)) % 3
+    got = E.eval_pairs(eng, dws, table, packed, of, COUNTS)
+    batch = E.Batch(eng, dws, table, packed, COUNTS)
+    for dw in dws:
+        dw.close()
+    batch.run()
+    batch.sync()
+    full = batch.fetch()
+    batch.close()
+    for k, st in enumerate(streams):
+        ref = oracle_batch(st, table, packed)
+        assert_batch_matches(full, ref, k, packed[0], where=f"stream {k}")
+        mine = np.flatnonzero(of == k)
+        for key in ("n_good", "latency_sum", "model_num_good", "group_num_requests"):
+            assert np.array_equal(got[key][mine], full[key][k][mine]), key
