@@ -105,7 +105,8 @@ typedef struct {
     int32_t xcd_map;              /* chunked loop: 0 = seeds innermost in the workgroup numbering; -1 / 1: all
                                      seeds of a tile group on one XCD                                           */
     int32_t batching_lanes;       /* batching simulator: 8, 16, 32 or 64 simulations per wavefront; 0: the widest
-                                     that still gives a CU eight wavefronts                                    */
+                                     that still gives a CU eight wavefronts, and fewer than 8 if the batch
+                                     leaves the chip room                                                       */
     int32_t batching_event_slots; /* batching simulator: idle-event slots per simulation (a multiple of eight);
                                      0: from the group count.  Too few makes a simulation stop with
                                      MMSIM_E_OVERFLOW (the one-call entry points then try again with more)     */

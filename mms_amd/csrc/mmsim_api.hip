@@ -378,6 +378,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     int heap_cap = 0, heap_min = 0, heap_pref = 0;  // batching simulator: event slots per lane (chosen, least, preferred)
     std::function<size_t(int, int)> batching_bytes_for;
     int blanes = kWave;  // batching simulator: lanes of a wavefront that simulate
+    int tile_sims = kWave;  // simulations of a tile
     // Wavefronts per workgroup: no more than it takes to give every CU its share of the
     // batch (a small batch is spread over the CUs, one wavefront per workgroup), and
     // no more than fit in LDS.  Option waves_per_cu (1..8) sets the number instead.
@@ -500,6 +501,32 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         size_for(blanes);
         if (heap_cap < heap_min) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: per-wavefront state does not fit in LDS (too many models/stages/groups)");
         batching_bytes_for = bytes_for;
+        tile_sims = blanes;
+        if (blanes == 8 && o.batching_lanes == 0 && !g_arena && !(flags & MMSIM_WANT_PER_REQUEST)) {
+            // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
+            // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
+            // devices, ms at 8 / 4 / 2 / 1 simulations: 1024 placements 16.5 / 13.5 / 11.3 / 9.4, 4096: 17.1 / 14.7 /
+            // 12.7 / 19.5 (two rounds), 8192: 17.7 / 15.7 / 25).  Rows of the device tables and of the counts are 64 wide
+            // whatever a tile holds; a microsecond of a request's time (what is gained) makes up for a few kilobytes
+            // of them.  The per-request outputs and the tables of a call without allocations stay dense.
+            const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
+            const size_t least = bytes_for(8, std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7)));  // (event slots are trimmed below)
+            const int64_t per_cu = std::max<int64_t>(1, std::max(std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / least)),
+                                                                 2 * std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / 2 / least))));
+            const int64_t counts = ((flags & MMSIM_WANT_MODEL_COUNTS) ? M : 0) + ((flags & MMSIM_WANT_GROUP_COUNTS) ? 2 * Gmax : 0);
+            int64_t members = 0;
+            for (int32_t p = 0; p < B; ++p) members = std::max(members, rl.off[(size_t)(p + 1) * M] - rl.off[(size_t)p * M]);
+            const int64_t tile_bytes = ((int64_t)M * std::max(rmax_all - kPackedReplicas, 0) + 8 * (int64_t)Gmax +
+                                        2 * members) * kWave +
+                                       counts * 4 * kWave * b->out_seeds;
+            int64_t longest = 0;
+            for (int s = 0; s < n_seeds; ++s) longest = std::max(longest, wls[s]->R);
+            for (int sims = tile_sims / 2; sims >= 1; sims /= 2) {
+                const int64_t tiles = (B + sims - 1) / sims;
+                if (tiles * b->out_seeds > per_cu * cus || tiles * tile_bytes > 4000 * longest) break;
+                tile_sims = sims;
+            }
+        }
         wpb = (int)std::min<size_t>(kMaxWavesPerBlockBatching, (size_t)ctx->max_lds / wave_bytes);
     }
 
@@ -550,7 +577,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
             if (by_slots && slots_of[x] != slots_of[y]) return slots_of[x] > slots_of[y];
             return expected[x] > expected[y];
         });
-        const int32_t tl = batching ? blanes : kWave;  // placements per tile
+        const int32_t tl = tile_sims;  // placements per tile
         b->pos.assign(B, 0);
         int32_t tile = -1, in_tile = tl;
         for (int32_t k = 0; k < B; ++k) {
@@ -738,12 +765,11 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     std::vector<uint32_t> rep32, repx32;
     std::vector<uint64_t> rep8;
     std::vector<uint8_t> repx;
-    // Tiles of eight simulations (octets): a row of rep8 is read as 64 descriptors instead, one per lane of the
-    // wavefront -- lane 8 * simulation + j holds the descriptor of the j-th replica (kEmpty: none); the second half
-    // of the row is not used.
+    // Octet tiles: rep8 holds descriptors instead, a row of 8 * tile_sims of them per (tile, model) -- word
+    // 8 * simulation + j is the descriptor of the j-th replica (kEmpty: none).
     const bool octets = batching && blanes == 8;
     if (batching) {
-        rep8.assign((size_t)b->tiles * M * kWave, octets ? ((uint64_t)kEmpty << 32 | kEmpty) : none8);
+        rep8.assign((size_t)b->tiles * M * (octets ? tile_sims * 4 : kWave), octets ? ((uint64_t)kEmpty << 32 | kEmpty) : none8);
         repx.assign((size_t)b->tiles * M * RX * kWave, (uint8_t)Gmax);
     } else {
         rep32.resize((size_t)b->tiles * M * 2 * kWave * 4);
@@ -803,7 +829,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 const int j = (int)(x - lo);
                 if (batching) {
                     if (j < kPackedReplicas && octets)
-                        reinterpret_cast<uint32_t *>(rep8.data())[((size_t)tile * M + m) * 2 * kWave + (size_t)lane * 8 + (size_t)j] =
+                        reinterpret_cast<uint32_t *>(rep8.data())[(((size_t)tile * M + m) * tile_sims + (size_t)lane) * 8 + (size_t)j] =
                             ginfo[((size_t)tile * (Gmax + 1) + g) * kWave + lane];
                     else if (j < kPackedReplicas)
                         word = (word & ~(0xFFull << (8 * j))) | ((uint64_t)g << (8 * j));
@@ -898,7 +924,10 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
         const size_t g2m_b = ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
         const size_t cap = (size_t)ctx->max_lds;
+        // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
         const int tiles_here = std::max(1, b->tiles);
+        const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
+        const int wanted = (int)std::min<int64_t>(2 * kMaxWavesPerBlockBatching, std::max<int64_t>(1, ((int64_t)b->waves + cus - 1) / cus));
         // Fewer event slots (down to G+8) are accepted when that puts more wavefronts on a CU.
         const int wpb_max = kMaxWavesPerBlockBatching;
         const int heap_try_min = std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7));
@@ -915,9 +944,9 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                     if ((want_lat && !(allowed & 1)) || (want_g2m && !(allowed & 2))) continue;
                     const size_t per = wb + (want_g2m ? g2m_b : 0), shared = want_lat ? lat_b : 0;
                     if (shared + per > cap / per_cu) continue;
-                    const int w = (int)std::min<size_t>(std::min(wpb_max, tiles_here), (cap / per_cu - shared) / per);
-                    if (per_cu * w > best_total) {
-                        best_total = per_cu * w;
+                    const int w = (int)std::min<size_t>(std::min({wpb_max, tiles_here, wanted}), (cap / per_cu - shared) / per);
+                    if (std::min(per_cu * w, wanted) > best_total) {
+                        best_total = std::min(per_cu * w, wanted);
                         best_w = w;
                         best_heap = hc;
                         batching_lat_lds = shared;
@@ -1137,6 +1166,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         q.lat_lds_bytes = (int32_t)batching_lat_lds;
         q.g2m_in_lds = batching_g2m_lds;
         q.lane_stride = blanes;
+        q.tile_sims = tile_sims;
         q.uniform_stages = uniform_stages ? 1 : 0;
         q.tile_seed = b->tile_seed.p;
         q.paired = b->paired ? 1 : 0;

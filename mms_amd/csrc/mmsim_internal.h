@@ -172,7 +172,7 @@ struct BatchingArgs {
     const int64_t *stream_off;   // [n_seeds+1]
     const int64_t *mq_off;       // [n_seeds][M+1] offsets into mq of the arrivals of each model
     const MqEntry *mq;           // model-ordered arrivals of all seeds, plus kMqPadding zeroed entries at the end
-    const uint64_t *rep8;        // as in MixedArgs
+    const uint64_t *rep8;        // as in MixedArgs; octet tiles: descriptors, [tiles][M][8 * tile_sims] u32
     const uint8_t *repx;
     const uint32_t *ginfo;       // [tiles][Gmax+1][64]
     const uint16_t *g2m_off;     // [tiles][Gmax+1][64] start of each group's model list
@@ -185,6 +185,7 @@ struct BatchingArgs {
     int32_t lat_lds_bytes;       // > 0: the workgroup keeps a copy of lat in LDS (that many bytes, 16-aligned)
     int32_t g2m_in_lds;          // 1: each wavefront keeps its g2m_off / g2m_idx rows in LDS
     int32_t lane_stride;         // 64, 32 or 16: lanes of a wavefront that simulate; pitch of the per-lane LDS arrays
+    int32_t tile_sims;           // simulations of a tile: lane_stride, or fewer in an octet tile (1, 2 or 4)
     int32_t uniform_stages;      // 1: a configuration's stages all have the same latencies and lat holds them once ([M][lat_row][NB], one row per configuration)
     const int32_t *tile_seed;    // as in MixedArgs
     int32_t paired;

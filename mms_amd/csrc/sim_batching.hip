@@ -12,7 +12,9 @@
 // tiles: a wavefront carries 64, 32, 16 or 8 simulations ("lanes" below),
 // whichever puts most wavefronts on a CU; with 8, each simulation is worked on
 // by an octet of lanes that hold the same state, take the same branches and
-// split the scans among them.
+// split the scans among them.  Batches that leave the chip room put 4, 2 or 1
+// simulations into such a wavefront instead of 8 (BatchingArgs::tile_sims): the
+// events of its octets then wait for fewer others.
 //
 // State of a lane:
 //   * stage clocks clk[slot][lane] in LDS, as in the plain simulator; a
@@ -254,11 +256,15 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const int64_t R = a.stream_off[seed + 1] - off;
     const Req *__restrict__ reqs = a.streams + off;
     const uint64_t *__restrict__ rep_tile = a.rep8 + (size_t)tile * M * kWave + sl;
-    // octets: the row of a model holds a descriptor per lane (the j-th replica's group for lane 8 * simulation + j)
-    const uint32_t *__restrict__ repd_tile = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 2 * kWave + lane;
+    // octets: the row of a model holds a descriptor per lane (the j-th replica's group for lane 8 * simulation + j), of
+    // as many lanes as the tile's simulations have; what the others read belongs to a simulation that is not theirs, and they
+    // are dead
+    const uint32_t row_lanes = 8u * (uint32_t)a.tile_sims;
+    const uint32_t *__restrict__ repd_tile = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * row_lanes +
+                                             ((uint32_t)lane & (row_lanes - 1u));
     auto row_of = [&](int mx) -> uint64_t {
         const size_t mr = (size_t)(mx < 0 ? 0 : mx);
-        if constexpr (OCT) return repd_tile[mr * 2 * kWave];
+        if constexpr (OCT) return repd_tile[mr * row_lanes];
         return rep_tile[mr * kWave];
     };
     const uint8_t *__restrict__ repx_tile = a.repx + (size_t)tile * M * a.rep_extra * kWave + sl;
@@ -281,7 +287,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     double my_cm = __builtin_inf();  // SH: the earliest event time of chunk oj (this lane's place in its octet)
     static_assert(!SH || OCT, "registers for the event slots' bookkeeping go with octets");
     double next_due = __builtin_inf();  // the earliest of them (+inf if none): arrivals before it skip the event list
-    int dead = sim ? 0 : 1;  // nonzero: this lane simulates nothing (more): out of event slots, unsupported input, or a spare lane of a narrow tile
+    // nonzero: this lane simulates nothing (more): out of event slots, unsupported input, a spare lane of a narrow
+    // tile, or an octet beyond the tile's simulations
+    int dead = sim && sl < a.tile_sims ? 0 : 1;
 
     const uint32_t none = (uint32_t)Gmax;
     Req blk_req = {0.0, -1, 0.0f};  // this lane's request of the current block of 64

@@ -7,6 +7,7 @@ accumulated in service order on the GPU and in arrival order by the oracle, so
 it is compared to 1e-12 relative.
 """
 import os
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -346,3 +347,37 @@ def test_batching_on_the_small_configs_too(eng):
     for s, st in enumerate(streams):
         ref = oracle_batch(st, table, packed, batching=True, want_per_request=True)
         _check(out, ref, s, per_request=True)
+
+
+@pytest.mark.parametrize("B,n_streams,sims", [(1, 1, 1), (7, 3, 1), (66, 31, 1), (65, 33, 2), (67, 60, 2), (67, 61, 4), (67, 120, 4), (70, 236, 8)])
+def test_simulations_of_an_octet_tile(eng, B, n_streams, sims):
+    """Batches with few simulations put 1, 2 or 4 of them into a wavefront instead of 8 (a CU runs eight such wavefronts):
+    the oracle's counts whatever the number, with streams of odd lengths and a last tile that is not full."""
+    cfg = make_config(5, B)
+    table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
+    packed = E.pack_placements(cfg.placements, table)
+    st = cfg.stream(0)
+    rng = np.random.default_rng(B)
+    streams = []
+    for k in range(n_streams):
+        lo, R = int(rng.integers(0, 20000)), 3000 if k == 0 else int(rng.integers(1, 400))
+        streams.append(SimpleNamespace(tstamps=st.tstamps[lo:lo + R] - st.tstamps[lo], model_ids=st.model_ids[lo:lo + R],
+                                       slos=st.slos[lo:lo + R]))
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, cfg.num_models) for s in streams]
+    for flags in (0, _lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS):
+        batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING)
+        if flags == 0:
+            assert batch.info()["waves"] == -(-B // sims) * n_streams
+        for _ in range(2):
+            batch.run()
+            batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k in sorted({0, 1, n_streams // 2, n_streams - 1} & set(range(n_streams))):
+            ref = oracle_batch(streams[k], table, packed, batching=True)
+            for key in ("n_good", "model_num_requests", "model_num_good", "group_num_requests", "group_num_good"):
+                if key in out:
+                    assert np.array_equal(out[key][k], ref[key]), (B, k, key)
+            assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
+    for dw in dws:
+        dw.close()
