@@ -186,9 +186,18 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     auto fits = [&](int lanes) { return lat_lds + wave_lds(lanes) <= lds; };
     int lanes = o.window_lanes;
     if (lanes == 0) {
-        // as many placements to a wavefront as it takes to get one wavefront to a SIMD
+        // LDS holds the state of so many placements at once; what is left over would run after them, and two rounds
+        // take longer than 64 placements to a wavefront (20000 requests: 8192 placements of 128 models on 64 devices,
+        // of which 4600 fit, 11.9 ms at best against 10.2 ms; 16384 of 64 models, of which 10000 fit, 13.7 against 9.7 ms).
+        if (sims > cus * (int64_t)((lds - lat_lds) / place)) return kOther;
+        // As many requests side by side as leave two wavefronts to a SIMD, four where a group is one stage: a step is a
+        // dependent chain that the other wavefronts fill, and more of them share the issue slots.  20000 requests, ms
+        // at 64 / 32 / 16 / 8 lanes: 4096 placements of 128 models 7.2 / 6.4 / 6.9 / 8.0; 8192 of 64 models
+        // 9.3 / 9.4 / 7.5 / 8.0; 8192 four-stage pipelines 7.4 / 6.1 / 6.0 / 6.8; single devices, 4096: 2.2 / 2.5 / 3.3
+        // / 4.6, 8192: 3.9 / 3.7 / 3.9 / 5.2.
+        const int64_t most = (a.smax_bucket == 1 ? 16 : 8) * cus;
         lanes = 64;
-        while (lanes > 8 && sims * lanes / kWave > 4 * cus && fits(lanes / 2)) lanes /= 2;
+        while (lanes > 8 && sims * lanes / kWave > most && fits(lanes / 2)) lanes /= 2;
     }
     if (stream_of) lanes = kWave;  // (the placements of a wavefront share a stream)
     while (lanes < kWave && !fits(lanes)) lanes *= 2;
