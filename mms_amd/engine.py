@@ -164,14 +164,18 @@ def pack_placements(sols: Sequence, table: LatencyTable):
     B = len(sols)
     num_groups = np.fromiter((len(s.group_configs) for s in sols), np.int32, B)
     Gmax = max(int(num_groups.max()) if B else 1, 1)
-    # two flat passes over all groups of all placements, scattered into the padded [B][Gmax] arrays row by row
+    # flat passes over all groups of all placements, scattered into the padded [B][Gmax] arrays row by row
     total_groups = int(num_groups.sum()) if B else 0
     has = np.arange(Gmax)[None, :] < num_groups[:, None]
     group_cfg = np.zeros((B, Gmax), np.int32)
     sizes = np.zeros((B, Gmax), np.int64)
-    group_cfg[has] = np.fromiter(map(table.config_id, chain.from_iterable(s.group_configs for s in sols)),
-                                 np.int32, total_groups)
-    sizes[has] = np.fromiter(map(len, chain.from_iterable(s.group_models for s in sols)), np.int64, total_groups)
+    cfgs = list(chain.from_iterable(s.group_configs for s in sols))
+    try:
+        group_cfg[has] = np.fromiter(map(table.index.get, cfgs), np.int32, total_groups)
+    except TypeError:       # the table does not know all of them yet
+        group_cfg[has] = np.fromiter(map(table.config_id, cfgs), np.int32, total_groups)
+    models = list(chain.from_iterable(s.group_models for s in sols))
+    sizes[has] = np.fromiter(map(len, models), np.int64, total_groups)
     gm_off = np.zeros((B, Gmax + 1), np.int64)
     np.cumsum(sizes, axis=1, out=gm_off[:, 1:])
     per_sol = gm_off[:, -1].copy()
@@ -179,8 +183,14 @@ def pack_placements(sols: Sequence, table: LatencyTable):
     np.cumsum(per_sol[:-1], out=base[1:])
     gm_off += base[:, None]
     total = int(per_sol.sum())
-    gm_idx = np.fromiter(chain.from_iterable(chain.from_iterable(s.group_models) for s in sols),
-                         np.int32, total)
+    gm_idx = None
+    if len(table.prof_ress) <= 256:     # model ids as bytes: 8.9 ms for 400000, np.fromiter takes 13.9
+        try:
+            gm_idx = np.frombuffer(bytes(chain.from_iterable(models)), np.uint8, total).astype(np.int32)
+        except (TypeError, ValueError):     # an id that is no byte (the library says what is wrong with it)
+            pass
+    if gm_idx is None:
+        gm_idx = np.fromiter(chain.from_iterable(models), np.int32, total)
     return num_groups, group_cfg, gm_off, gm_idx
 
 

@@ -308,7 +308,7 @@ class PlacementEvaluator:
         R = len(self.workload)
         goodput = out["n_good"][0] / R
         latency_mean = out["latency_sum"][0] / R
-        replicas = np.fromiter((sum(len(x) for x in s.group_models) for s in sols), np.int64, len(sols))
+        replicas = np.fromiter((sum(map(len, s.group_models)) for s in sols), np.int64, len(sols))
         scores = goodput - latency_mean / 10000 + replicas / 1000000
         return [float(x) for x in scores]
 

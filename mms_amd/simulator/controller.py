@@ -21,7 +21,7 @@ from mms_amd import _lib, engine as _engine
 from mms_amd.profiling import ProfilingResult
 from mms_amd.simulator.workload import (DEFAULT_WARMUP, PerModelStatsResult,
                                         StatsResult, Workload)
-from mms_amd.util import ServingCase, batchsize_config, eps, inf
+from mms_amd.util import ServingCase, batchsize_config, eps
 from mms_amd.simulator.event_sim import Client, Controller, GroupManager, simulate_one_case  # noqa: F401
 
 
@@ -145,13 +145,20 @@ def approximate_one_case_one_placement(placement, model_names, prof_ress, model_
 def replacement_cuts(placement, arrivals):
     """Index ranges of the segments of a ModelPlacementWithReplacement: a new segment starts at the
     first arrival strictly later than the next change time (controller.py:345-365)."""
-    change_times = list(placement.start_times[1:]) + [inf]
+    arrivals = np.asarray(arrivals)
+    in_order = bool(np.all(arrivals[1:] >= arrivals[:-1]) and np.all(arrivals[:1] == arrivals[:1]))  # (and no NaN)
     cuts = [0]
-    pt = 0
-    for i in range(len(arrivals)):
-        if arrivals[i] > change_times[pt]:
-            cuts.append(i)
-            pt += 1
+    at = 0          # an arrival starts one segment at most
+    for time in placement.start_times[1:]:
+        if in_order:
+            at += int(np.searchsorted(arrivals[at:], time, side="right"))
+        else:
+            later = np.flatnonzero(arrivals[at:] > time)
+            at = at + int(later[0]) if len(later) else len(arrivals)
+        if at >= len(arrivals):
+            break
+        cuts.append(at)
+        at += 1
     cuts.append(len(arrivals))
     return list(zip(cuts[:-1], cuts[1:]))
 

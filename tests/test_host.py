@@ -369,3 +369,45 @@ def test_add_model_normalized_is_add_model_then_normalize():
         assert got == want
         assert type(got.group_models) is tuple and all(type(r) is tuple for r in got.group_models)
         assert got.add_model_normalized(0, 99) == got.add_model(0, 99).normalize()
+
+
+def test_replacement_cuts_are_the_scans():
+    """replacement_cuts against the reference's scan over the arrivals (controller.py:345-365): ties, arrivals and change
+    times out of order, NaN and infinities, more changes than arrivals."""
+    from types import SimpleNamespace
+    from mms_amd.simulator.controller import replacement_cuts
+
+    def scan(starts, arrivals):
+        change_times, cuts = list(starts[1:]) + [float("inf")], [0]
+        for i in range(len(arrivals)):
+            if arrivals[i] > change_times[len(cuts) - 1]:
+                cuts.append(i)
+        cuts.append(len(arrivals))
+        return list(zip(cuts[:-1], cuts[1:]))
+
+    rng = np.random.default_rng(3)
+    for trial in range(2000):
+        arrivals = rng.integers(0, 8, int(rng.integers(0, 12))).astype(float)
+        starts = [0.0] + list(rng.integers(-1, 9, int(rng.integers(0, 5))).astype(float)) + [float("nan")] * (trial % 11 == 0)
+        if trial % 3:
+            arrivals.sort()
+        if trial % 7 == 0 and len(arrivals):
+            arrivals[rng.integers(len(arrivals))] = (float("nan"), float("inf"), float("-inf"))[trial % 3]
+        assert replacement_cuts(SimpleNamespace(start_times=starts), arrivals) == scan(starts, arrivals), (starts, arrivals)
+
+
+@pytest.mark.parametrize("models", [3, 256, 257, 300])
+def test_packing_keeps_every_id(models):
+    """pack_placements with ids that fit a byte and ids that do not, ids as numpy integers, ids no table has."""
+    from mms_amd.engine import LatencyTable, pack_placements
+    from mms_amd.placement_policy.base_policy import ModelPlacement
+    from mms_amd.profiling import ParallelConfig
+    one, two = ParallelConfig(1, 1, 1), ParallelConfig(1, 1, 2)
+    table = LatencyTable([None] * models, [1])
+    sols = [ModelPlacement([one, two, one], [[0, models - 1], [], [np.int64(1)]]), ModelPlacement([], []),
+            ModelPlacement([two], [[2, models + 44, -5]])]
+    for _ in range(2):      # the second time the table knows all configurations
+        groups, cfg, off, idx = pack_placements(sols, table)
+        assert groups.tolist() == [3, 0, 1] and cfg.tolist() == [[0, 1, 0], [0, 0, 0], [1, 0, 0]]
+        assert off.tolist() == [[0, 2, 2, 3], [3, 3, 3, 3], [3, 6, 6, 6]]
+        assert idx.dtype == np.int32 and idx.tolist() == [0, models - 1, 1, 2, models + 44, -5]
