@@ -443,6 +443,14 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
             // D: most stages of a group.
             auto steps = [&](auto Dv) {
                 constexpr int D = decltype(Dv)::value;
+                // The stages behind the first NEAR are read, walked and written by the lanes that chose a group with
+                // so many, in a branch that most steps skip.  A wavefront on its own (W == 64) takes up to eight
+                // without a branch, as the stages are a shorter chain than the branch; wavefronts that share a
+                // SIMD (W < 64) gain from four stages on, as they share its issue slots.  20000 requests, against
+                // all stages in every lane: 4096 placements of groups up to 16 deep 6.44 -> 5.11 ms, up to 8 deep
+                // 5.02 -> 4.81 ms; 1025 placements, W == 64, up to 16 deep 3.60 -> 3.20 ms (2.88 -> 2.98 ms up to 8
+                // deep, where only the registers of the unused deep path differ).
+                constexpr int NEAR = W == 64 ? 8 : 4;
                 struct Cand {
                     double c;
                     uint32_t d;
@@ -475,7 +483,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     // a clock that is infinite is never chosen (:590-598)
                     const double limit = __hiloint2double(best < 1e100 ? __double2hiint(slo) : 0x7FF80000, __double2loint(slo));
                     const double l_last = (double)win.l;
-                    // ---- walk the stages and decide (:605-613).  All requests read and walk D stages from their group's first
+                    // ---- walk the stages and decide (:605-613).  All requests read and walk the near stages from their group's first
                     // on and take the time after their last one (what lies behind a shallower group's slots does not matter).
                     double cv[D];
                     const uint32_t last = SMAX == 1 ? win.d : entry_addr(win.d);
@@ -487,19 +495,43 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     } else {
                         const uint32_t lrow = (uint32_t)m * (uint32_t)a.lat_row + entry_lat(win.d) - (uint32_t)sm1;
                         float l[UNIFORM ? 1 : D];
-#pragma unroll
-                        for (int k = 0; k < D; ++k) {
+                        auto read = [&](int k) {
                             cv[k] = lds_get<double>(gclk + (uint32_t)k * 8u);
                             if constexpr (!UNIFORM)
                                 l[k] = a.lat_lds_bytes > 0 ? lds_get<float>((lrow + (uint32_t)k) * 4u) : a.lat[lrow + (uint32_t)k];
-                        }
-#pragma unroll
-                        for (int k = 0; k < D; ++k) {
+                        };
+                        auto pass = [&](int k) {
                             cv[k] = vmax(k == 0 ? arr : cv[k > 0 ? k - 1 : 0], cv[k]) + (UNIFORM ? l_last : (double)l[UNIFORM ? 0 : k]);
                             if (k == 0)
                                 t = cv[0];
                             else if (!POW2 || (k & (k + 1)) == 0)
                                 t = sm1 >= k ? cv[k] : t;
+                        };
+#pragma unroll
+                        for (int k = 0; k < (D < 8 ? D : 8); ++k) read(k);
+#pragma unroll
+                        for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) pass(k);
+                        if constexpr (D > NEAR) {
+                            if (sm1 >= NEAR) {
+#pragma unroll
+                                for (int k = NEAR; k < (D < 8 ? D : 8); ++k) pass(k);
+                                if constexpr (D > 8) {
+                                    if (sm1 >= 8) {
+#pragma unroll
+                                        for (int k = 8; k < (D < 16 ? D : 16); ++k) read(k);
+#pragma unroll
+                                        for (int k = 8; k < (D < 16 ? D : 16); ++k) pass(k);
+                                        if constexpr (D > 16) {
+                                            if (sm1 >= 16) {
+#pragma unroll
+                                                for (int k = 16; k < D; ++k) read(k);
+#pragma unroll
+                                                for (int k = 16; k < D; ++k) pass(k);
+                                            }
+                                        }
+                                    }
+                                }
+                            }
                         }
                     }
                     latency = (t + overhead) - arr;
@@ -515,18 +547,32 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                         open = w2 & ~waiting & multis & ~accs;
                         waiting = w2;
                     }
-                    // accepted and final: the clocks (:614-619).  Everybody writes, the others where it does not matter.
+                    // accepted and final: the clocks (:614-619).  Everybody writes the near stages, the others where it does
+                    // not matter.
                     uint32_t to = in_mask(accs) ? gclk : spare;
                     pin(to);
                     to = waits ? spare : to;
                     pin(to);
-#pragma unroll
-                    for (int k = 0; k < D; ++k) {
+                    auto commit = [&](int k) {
                         if (k > 0 && (!POW2 || (k & (k - 1)) == 0)) {
                             to = sm1 >= k ? to : spare;
                             pin(to);
                         }
                         lds_put<double>(to + (uint32_t)k * 8u, cv[k]);
+                    };
+#pragma unroll
+                    for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) commit(k);
+                    if constexpr (D > NEAR) {
+                        if (to == gclk && sm1 >= NEAR) {
+#pragma unroll
+                            for (int k = NEAR; k < (D < 8 ? D : 8); ++k) commit(k);
+                            if constexpr (D > 8) {
+                                if (sm1 >= 8) {
+#pragma unroll
+                                    for (int k = 8; k < D; ++k) commit(k);
+                                }
+                            }
+                        }
                     }
                     order_in_loop();
 #pragma unroll
