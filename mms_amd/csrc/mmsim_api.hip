@@ -502,7 +502,9 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         if (heap_cap < heap_min) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: per-wavefront state does not fit in LDS (too many models/stages/groups)");
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
-        if (blanes == 8 && o.batching_lanes == 0 && !g_arena && !(flags & MMSIM_WANT_PER_REQUEST)) {
+        if (blanes == 8 && o.batching_lanes == 0 && B == 1) {
+            tile_sims = 1;  // (no more tiles than otherwise)
+        } else if (blanes == 8 && o.batching_lanes == 0 && !g_arena && !(flags & MMSIM_WANT_PER_REQUEST)) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
             // devices, ms at 8 / 4 / 2 / 1 simulations: 1024 placements 16.5 / 13.5 / 11.3 / 9.4, 4096: 17.1 / 14.7 /
