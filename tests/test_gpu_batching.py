@@ -381,3 +381,25 @@ def test_simulations_of_an_octet_tile(eng, B, n_streams, sims):
             assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
     for dw in dws:
         dw.close()
+
+
+@pytest.mark.parametrize("sizes", [[1], [1, 2, 4], [1, 2, 3, 5, 8], [1, 2, 4, 8, 16, 32, 64, 128], [1, 2, 3, 5, 8, 9, 17, 30]])
+@pytest.mark.parametrize("groups", [1, 8, 30])
+def test_one_simulation_to_a_wavefront(eng, sizes, groups):
+    """A single placement has a wavefront to itself, whose octets look at eight arrivals at a time: the oracle's flags and
+    finish times with equal arrival instants, streams that end inside a window or a block, models with more replicas
+    than an octet has lanes, and batch sizes that share latency columns."""
+    most = 0
+    for seed in range(12):
+        c = random_case(7_000_000 + 1000 * groups + 100 * len(sizes) + seed, max_m=2 + seed % 9, max_g=groups, max_s=1 + seed % 8,
+                        max_r=(1, 8, 9, 63, 64, 65, 130, 200, 400, 400, 700, 700)[seed], nb=len(sizes), load=1.0 + 3 * (seed % 9),
+                        inf_slo=False, tie_prob=0.05 * (seed % 8), p_member=0.3 + 0.1 * (seed % 7))
+        f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
+            c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], sizes)
+        fin, good, cnt = _single(eng, c, sizes)
+        assert np.array_equal(good, g0), seed
+        assert np.array_equal(fin.view(np.uint64), f0.view(np.uint64)), seed
+        for a, b in zip(cnt, c0):
+            assert np.array_equal(a, b), seed
+        most = max(most, int((c["m2g"] >= 0).sum(axis=1).max()))
+    assert most > 8 or groups < 30
