@@ -480,6 +480,21 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (wave_bytes <= (size_t)ctx->max_lds) break;
             }
         };
+        // Rows of the device tables and of the counts are 64 wide whatever a tile holds; the microsecond or two of a
+        // request's time that narrow tiles gain makes up for a few kilobytes of them.  The per-request outputs and the
+        // tables of a call without allocations stay dense.
+        auto affordable = [&](int sims) {
+            if (g_arena || (flags & MMSIM_WANT_PER_REQUEST)) return false;
+            const int64_t counts = ((flags & MMSIM_WANT_MODEL_COUNTS) ? M : 0) + ((flags & MMSIM_WANT_GROUP_COUNTS) ? 2 * Gmax : 0);
+            int64_t members = 0;
+            for (int32_t p = 0; p < B; ++p) members = std::max(members, rl.off[(size_t)(p + 1) * M] - rl.off[(size_t)p * M]);
+            const int64_t tile_bytes = ((int64_t)M * std::max(rmax_all - kPackedReplicas, 0) + 8 * (int64_t)Gmax +
+                                        2 * members) * kWave +
+                                       counts * 4 * kWave * b->out_seeds;
+            int64_t longest = 0;
+            for (int s = 0; s < n_seeds; ++s) longest = std::max(longest, wls[s]->R);
+            return (B + sims - 1) / sims * tile_bytes <= 4000 * longest;
+        };
         // Simulations per wavefront.  The loops between two arrivals run per lane and are bound by
         // latency (LDS and memory round trips), so a wavefront takes nearly as long with 8 simulations
         // as with 64 while its LDS footprint grows with their number: narrow tiles (32, 16 or 8 lanes
@@ -497,6 +512,10 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (blanes == 8 || (per_cu >= 8 && waves >= 8 * cus)) break;
                 blanes /= 2;
             }
+            // Octets beat 16 lanes even in several rounds (3000 requests, 48 models on 24 devices: 32768 simulations
+            // 14.0 -> 9.5 ms, 131072 50 -> 28 ms); 32 lanes, where a CU has room for eight such wavefronts, are level with
+            // them (16 models on 8 devices, 65536: 11.4 against 11.8 ms).
+            if (blanes == 16 && affordable(8)) blanes = 8;
         }
         size_for(blanes);
         if (heap_cap < heap_min) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: per-wavefront state does not fit in LDS (too many models/stages/groups)");
@@ -504,28 +523,18 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         tile_sims = blanes;
         if (blanes == 8 && o.batching_lanes == 0 && B == 1) {
             tile_sims = 1;  // (no more tiles than otherwise)
-        } else if (blanes == 8 && o.batching_lanes == 0 && !g_arena && !(flags & MMSIM_WANT_PER_REQUEST)) {
+        } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
             // devices, ms at 8 / 4 / 2 / 1 simulations: 1024 placements 16.5 / 13.5 / 11.3 / 9.4, 4096: 17.1 / 14.7 /
-            // 12.7 / 19.5 (two rounds), 8192: 17.7 / 15.7 / 25).  Rows of the device tables and of the counts are 64 wide
-            // whatever a tile holds; a microsecond of a request's time (what is gained) makes up for a few kilobytes
-            // of them.  The per-request outputs and the tables of a call without allocations stay dense.
+            // 12.7 / 19.5 (two rounds), 8192: 17.7 / 15.7 / 25).
             const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
             const size_t least = bytes_for(8, std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7)));  // (event slots are trimmed below)
             const int64_t per_cu = std::max<int64_t>(1, std::max(std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / least)),
                                                                  2 * std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / 2 / least))));
-            const int64_t counts = ((flags & MMSIM_WANT_MODEL_COUNTS) ? M : 0) + ((flags & MMSIM_WANT_GROUP_COUNTS) ? 2 * Gmax : 0);
-            int64_t members = 0;
-            for (int32_t p = 0; p < B; ++p) members = std::max(members, rl.off[(size_t)(p + 1) * M] - rl.off[(size_t)p * M]);
-            const int64_t tile_bytes = ((int64_t)M * std::max(rmax_all - kPackedReplicas, 0) + 8 * (int64_t)Gmax +
-                                        2 * members) * kWave +
-                                       counts * 4 * kWave * b->out_seeds;
-            int64_t longest = 0;
-            for (int s = 0; s < n_seeds; ++s) longest = std::max(longest, wls[s]->R);
             for (int sims = tile_sims / 2; sims >= 1; sims /= 2) {
                 const int64_t tiles = (B + sims - 1) / sims;
-                if (tiles * b->out_seeds > per_cu * cus || tiles * tile_bytes > 4000 * longest) break;
+                if (tiles * b->out_seeds > per_cu * cus || !affordable(sims)) break;
                 tile_sims = sims;
             }
         }
