@@ -1909,9 +1909,32 @@ int mmsim_simulate_requests_mixed(mmsim_ctx *ctx, double *finish, uint8_t *good,
     mmsim_batch *b = nullptr;
     const mmsim_workload *wls[1] = {wl};
     const uint32_t flags = MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST;
-    rc = build_batch(ctx, wls, 1, &t, rl, flags, &b);
+    // Rows that list their groups in ascending order are what a placement's groups and models say (every row that
+    // approximate_one_case_one_placement makes): the kernel with the requests side by side may take them.
+    bool ascending = true;
+    for (int32_t m = 0; m < M && ascending; ++m)
+        for (int64_t x = rl.off[m] + 1; x < rl.off[m + 1]; ++x) ascending = ascending && rl.grp[(size_t)x] > rl.grp[(size_t)x - 1];
+    if (ascending) {
+        std::vector<int64_t> gm_off((size_t)G + 1, 0);
+        std::vector<int32_t> gm_idx(rl.grp.size() + 1);
+        for (int32_t g : rl.grp) gm_off[(size_t)g + 1] += 1;
+        for (int32_t g = 0; g < G; ++g) gm_off[(size_t)g + 1] += gm_off[(size_t)g];
+        std::vector<int64_t> at(gm_off.begin(), gm_off.end() - 1);
+        for (int32_t m = 0; m < M; ++m)
+            for (int64_t x = rl.off[m]; x < rl.off[m + 1]; ++x) gm_idx[(size_t)at[(size_t)rl.grp[(size_t)x]]++] = m;
+        mmsim_placements p{};
+        p.B = 1;
+        p.Gmax = G;
+        p.num_groups = rl.num_groups.data();
+        p.group_cfg = rl.group_cfg.data();
+        p.gm_off = gm_off.data();
+        p.gm_idx = gm_idx.data();
+        rc = make_batch(ctx, wls, 1, &t, &p, nullptr, flags, nullptr, false, &b);
+    } else {
+        rc = build_batch(ctx, wls, 1, &t, rl, flags, &b);
+    }
     if (rc == MMSIM_OK) rc = mmsim_batch_run(b);
-    if (rc == MMSIM_OK) rc = mmsim_batch_sync(b, nullptr);
+    if (rc == MMSIM_OK && !b->window) rc = mmsim_batch_sync(b, nullptr);  // (a window batch's fetch waits)
     if (rc == MMSIM_OK) {
         int64_t ng = 0;
         double ls = 0.0;

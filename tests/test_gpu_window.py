@@ -10,6 +10,7 @@ import pytest
 from mms_amd import _lib, engine as E
 from mms_amd.placement_policy.base_policy import ModelPlacement
 from mms_amd.profiling import LatencyMemData, ParallelConfig, ProfilingResult
+from oracle import oracle_c
 from helpers import assert_batch_matches, oracle_batch
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +103,29 @@ def test_replaced_placements_and_the_kept_streams():
         mine = np.flatnonzero(of == k)
         for key in ("n_good", "latency_sum", "model_num_good", "group_num_requests"):
             assert np.array_equal(got[key][mine], full[key][k][mine]), key
+
+
+@pytest.mark.parametrize("order", ["ascending", "descending", "repeated"])
+def test_replica_tables_of_one_placement(order):
+    """simulate_requests_mixed: tables whose rows list their groups in ascending order go through the requests side by
+    side, others (another order decides ties, a group may be named twice) through the loop over requests."""
+    eng = E.Engine.default()
+    for seed in range(10):
+        rng = np.random.default_rng(1000 + seed)
+        M, G, R = int(rng.integers(1, 7)), int(rng.integers(1, 12)), (0, 1, 63, 64, 65, 500)[seed % 6]
+        st = _stream(seed, R, M, 2.0)
+        stages = rng.integers(1, 6, G).astype(np.int32)
+        lat = np.zeros((M, G, int(stages.max())), np.float32)
+        for g in range(G):
+            lat[:, g, :stages[g]] = rng.uniform(0.01, 0.2, (M, stages[g]))
+        m2g = np.full((M, G), -1, np.int32)
+        for m in range(M):
+            row = np.flatnonzero(rng.random(G) < 0.6)
+            row = row[::-1] if order == "descending" else np.repeat(row, 2)[:G] if order == "repeated" else row
+            m2g[m, :len(row)] = row
+        fin, good = np.empty(R), np.empty(R, bool)
+        counts = E.simulate_requests_mixed(eng, fin, good, st.tstamps, st.model_ids, st.slos, m2g, stages, lat)
+        f0, g0, c0 = oracle_c.simulate_requests_mixed(st.tstamps, st.model_ids, st.slos, m2g, stages, lat)[:3]
+        assert np.array_equal(good, g0) and np.array_equal(fin.view(np.uint64), f0.view(np.uint64)), seed
+        for x, y in zip(counts, c0):
+            assert np.array_equal(x, y), seed
