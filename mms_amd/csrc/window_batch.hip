@@ -332,6 +332,7 @@ int fetch_window(mmsim_batch *b, mmsim_result *out) {
     hipStream_t st = b->ctx->stream;
     const size_t L = (size_t)b->B * b->out_seeds, M = (size_t)b->M, G = (size_t)b->Gmax, Rm = (size_t)b->Rmax;
     Staging &stage = b->ctx->staging;
+    if (b->win_finish > stage.n) HIP_TRY(hipStreamSynchronize(st));  // the inputs may still be on their way out of it
     HIP_TRY(stage.ensure(b->win_finish));
     HIP_TRY(hipMemcpyAsync(stage.p, b->win_out.p, b->win_finish, hipMemcpyDeviceToHost, st));
     if (wr && Rm > 0) {
