@@ -42,7 +42,11 @@ FLAGS = [
 # Blocks that are only reached by a branch start on a 64-byte boundary: a taken branch costs a lone wavefront
 # tens of cycles, less when its target starts an instruction cache line (measured: -1 % in the counts mode; 32- and
 # 128-byte boundaries, aligning every block, and switching block placement or tail duplication off are all slower).
-SOURCE_FLAGS = {"sim_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
+# Requests side by side (20000 requests; 1025 four-stage pipelines / 4096 of them / 1025 and 4096 mixed groups / 4096 single
+# devices): default 2.91 / 4.36 / 2.95 / 4.84 / 2.17 ms, with max-ilp 2.69 / 4.23 / 2.86 / 4.79 / 2.17, with the aligned
+# blocks as well 2.70 / 4.13 / 2.90 / 4.71 / 2.16, with these alone no change; iterative-ilp fails on it.
+SOURCE_FLAGS = {"sim_window.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
+                "sim_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_batching.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"]}
 
 
