@@ -80,7 +80,9 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         const int32_t G = p->num_groups[b];
         if (G < 0 || G > Gmax) return kOther;
         const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-        if (off[G] < off[0] || (off[G] > off[0] && !p->gm_idx)) return kOther;
+        for (int32_t g = 0; g < G; ++g)  // (what is written below has room for off[G] - off[0] entries)
+            if (off[g + 1] < off[g]) return kOther;
+        if (off[G] > off[0] && !p->gm_idx) return kOther;
         replicas += off[G] - off[0];
         if (replicas > 0x7FFFFFFF) return kOther;
     }
@@ -119,7 +121,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             for (int32_t g = 0; g < Gmax; ++g) {
                 h_cfg[(size_t)b * Gmax + g] = g < G ? (uint8_t)cfg[g] : 0;
                 if (g >= G) continue;
-                if (cfg[g] < 0 || cfg[g] >= C || off[g + 1] < off[g]) {
+                if (cfg[g] < 0 || cfg[g] >= C) {
                     bad = true;
                     return;
                 }

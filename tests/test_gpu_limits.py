@@ -153,6 +153,24 @@ def test_more_items_than_one_workgroup_can_own(eng, opts):
     dw.close()
 
 
+def test_offsets_that_go_back_are_refused(eng):
+    """gm_off that rises and falls again inside a placement: its last offset says less than its groups list, so it is
+    looked at before anything is packed by it (here 64 * M entries would go where there is room for one)."""
+    pc = ParallelConfig(1, 1, 1)
+    M = 20000
+    table = E.LatencyTable([synthetic_profile("m", 0.1, [pc])] * M, [1])
+    table.config_id(pc)
+    idx = np.tile(np.arange(M, dtype=np.int32), 64)
+    packed = (np.array([2], np.int32), np.zeros((1, 2), np.int32), np.array([[0, len(idx), 1]], np.int64), idx)
+    dw = E.DeviceWorkload(eng, *_stream(M), M)
+    for static in (False, True):
+        with pytest.raises(_lib.MmsimError) as err:
+            E.eval_batch(eng, [dw], table, packed, static=static)
+        assert err.value.code == _lib.E_INVALID and "gm_off not monotone" in str(err.value)
+    dw.close()
+    _still_works(eng)
+
+
 def test_options_are_validated(eng):
     for bad in (dict(request_loop=2), dict(waves_per_cu=9), dict(batching_lanes=12), dict(segment_requests=-5),
                 dict(batching_lds_tables=4)):
