@@ -34,8 +34,14 @@ hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_by
                               : a.lanes == 16 ? window_kernel<16>(a.smax_bucket, out, ext, pow2, uniform)
                                               : window_kernel<8>(a.smax_bucket, out, ext, pow2, uniform);
     if (!kern || waves_per_block < 1 || waves_per_block > kMaxWindowWaves) return hipErrorInvalidValue;
+    // The kernel takes LDS addresses as numbers from 0 on: its dynamic LDS starts there as long as nothing static lies
+    // before it.
+    hipFuncAttributes attr;
+    hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(kern));
+    if (e != hipSuccess) return e;
+    if (attr.sharedSizeBytes != 0) return hipErrorInvalidKernelFile;
     if (lds_bytes > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         if (e != hipSuccess) return e;
     }
     const int64_t units = (int64_t)a.tiles * a.out_seeds;
@@ -322,7 +328,9 @@ std::string sim_window_kernel_name(const WindowArgs &a) {
 
 int run_window(mmsim_batch *b) {
     if (b->ev_start) HIP_TRY(hipEventRecord(b->ev_start, b->ctx->stream));
-    HIP_TRY(launch_window(b->wargs, b->waves_per_block, b->lds_bytes, b->ctx->stream));
+    const hipError_t e = launch_window(b->wargs, b->waves_per_block, b->lds_bytes, b->ctx->stream);
+    if (e == hipErrorInvalidKernelFile) return fail(MMSIM_E_HIP, "simulation kernel: dynamic LDS does not start at address 0");
+    if (e != hipSuccess) return hip_fail(e, "sim_window launch");
     if (b->ev_stop) HIP_TRY(hipEventRecord(b->ev_stop, b->ctx->stream));
     b->ran = true;
     return MMSIM_OK;

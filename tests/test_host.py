@@ -34,6 +34,19 @@ def test_library_loads_and_exports_every_declared_symbol():
     assert lib.mmsim_abi_version() == int(re.search(r"#define MMSIM_ABI_VERSION (\d+)", header).group(1))
 
 
+def test_kernels_that_address_lds_by_number_have_it_from_0_on():
+    """The plain simulator's kernels take LDS addresses as numbers from 0 on, which holds while nothing static lies
+    before the dynamic LDS: the metadata of the built kernels says so (the launch looks as well and refuses)."""
+    code = open(_lib.LIB_PATH, "rb").read()
+    found = {}
+    for m in re.finditer(rb"\.group_segment_fixed_size(.)(?:(?!\.group_segment_fixed_size).)*?\.symbol..?(_Z\w+?)\.kd", code, re.S):
+        found[m.group(2).decode()] = m.group(1)[0]      # (one byte: below 128)
+    sizes = {k: v for k, v in found.items() if "sim_window_kernel" in k or "sim_mixed_kernel" in k}
+    assert sum("sim_window_kernel" in k for k in sizes) >= 4 * 26 and any("sim_mixed_kernel" in k for k in sizes)
+    assert any(v != 0 for k, v in found.items() if "model_stats_kernel" in k)      # (one that has some)
+    assert set(sizes.values()) == {0}
+
+
 def test_no_device_means_a_loud_error_not_a_fallback():
     import torch
     if torch.cuda.is_available():
