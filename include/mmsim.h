@@ -325,7 +325,8 @@ int mmsim_eval_successors(mmsim_ctx *ctx, const mmsim_workload *const *workloads
  * mmsim_eval_batch, bit for bit, but every device table and result buffer of
  * the batch lives in a static device array of MMSIM_STATIC_SCRATCH_BYTES that
  * the library holds on each GPU it runs on until the process ends: no
- * hipMalloc, no hipFree.  A batch that needs more (many placements x models,
+ * hipMalloc, no hipFree, and no pinned host memory either (hipHostMalloc,
+ * hipHostFree).  A batch that needs more (many placements x models,
  * several long streams, per-request outputs) is refused with MMSIM_E_NOMEM
  * and a message that names the limit.  All calls on one GPU share that GPU's
  * array: calls that overlap on one GPU race, from whichever contexts or

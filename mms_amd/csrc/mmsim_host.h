@@ -242,6 +242,7 @@ struct mmsim_batch {
     MixedArgs args{};
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     bool own_events = true;  // false: the context's events (batch in the static scratch)
+    bool in_scratch = false; // the batch lives in the static scratch: nothing is allocated for it, pinned memory included
     bool ran = false;
     mmsim_options opt{};     // the options the batch was built with
 

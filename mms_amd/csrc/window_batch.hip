@@ -3,7 +3,8 @@
 //
 // The placements travel as they were given, a few bytes per replica: the wavefronts build their own tables (the other
 // kernels' descriptor tables are a kilobyte per placement and model of a tile).  One buffer holds every input and one
-// every output, so a call is one copy in, one launch and one copy out, through the context's pinned staging memory.
+// every output, so a call is one copy in, one launch and one copy out, through the context's pinned staging memory
+// (mmsim_eval_batch_static, which must not call the runtime's allocators: through ordinary memory).
 #include <cstring>
 
 #include "mmsim_host.h"
@@ -98,8 +99,12 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
     const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
     HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(ctx->staging.ensure(in.used));
-    unsigned char *host = ctx->staging.p;
+    std::vector<unsigned char> plain;  // (read until the wait below)
+    if (g_arena)
+        plain.resize(in.used);
+    else
+        HIP_TRY(ctx->staging.ensure(in.used));
+    unsigned char *host = g_arena ? plain.data() : ctx->staging.p;
     uint8_t *h_ng = host + at_ng, *h_cfg = host + at_cfg;
     uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off), *h_ent = reinterpret_cast<uint32_t *>(host + at_ent);
     {
@@ -270,6 +275,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     if (events) {
         if (g_arena) {
             b->own_events = false;
+            b->in_scratch = true;
             b->ev_start = ctx->ev_static[0];
             b->ev_stop = ctx->ev_static[1];
         } else {
@@ -277,7 +283,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             HIP_TRY(hipEventCreate(&b->ev_stop));
         }
         HIP_TRY(hipStreamSynchronize(ctx->stream));  // a batch that is kept: the staging memory serves other calls before its run
-        ctx->staging.trim();
+        if (!g_arena) ctx->staging.trim();
     }
     const uint8_t *d = b->win_in.p;
     a.stream_ptr = reinterpret_cast<const Req *const *>(d + at_ptr);
@@ -342,29 +348,35 @@ int fetch_window(mmsim_batch *b, mmsim_result *out) {
     hipStream_t st = b->ctx->stream;
     const size_t L = (size_t)b->B * b->out_seeds, M = (size_t)b->M, G = (size_t)b->Gmax, Rm = (size_t)b->Rmax;
     Staging &stage = b->ctx->staging;
-    if (b->win_finish > stage.n) HIP_TRY(hipStreamSynchronize(st));  // the inputs may still be on their way out of it
-    HIP_TRY(stage.ensure(b->win_finish));
-    HIP_TRY(hipMemcpyAsync(stage.p, b->win_out.p, b->win_finish, hipMemcpyDeviceToHost, st));
+    std::vector<unsigned char> plain;
+    if (b->in_scratch) {
+        plain.resize(b->win_finish);
+    } else {
+        if (b->win_finish > stage.n) HIP_TRY(hipStreamSynchronize(st));  // the inputs may still be on their way out of it
+        HIP_TRY(stage.ensure(b->win_finish));
+    }
+    unsigned char *host = b->in_scratch ? plain.data() : stage.p;
+    HIP_TRY(hipMemcpyAsync(host, b->win_out.p, b->win_finish, hipMemcpyDeviceToHost, st));
     if (wr && Rm > 0) {
         HIP_TRY(hipMemcpyAsync(out->finish, b->win_out.p + b->win_finish, sizeof(double) * L * Rm, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipMemcpyAsync(out->good, b->win_out.p + b->win_good, L * Rm, hipMemcpyDeviceToHost, st));
     }
     HIP_TRY(hipStreamSynchronize(st));
-    const int32_t *ng = reinterpret_cast<const int32_t *>(stage.p);
+    const int32_t *ng = reinterpret_cast<const int32_t *>(host);
     for (size_t l = 0; l < L; ++l) out->n_good[l] = ng[l];
-    std::memcpy(out->latency_sum, stage.p + b->win_lat_sum, sizeof(double) * L);
+    std::memcpy(out->latency_sum, host + b->win_lat_sum, sizeof(double) * L);
     if (out->status) std::memset(out->status, 0, sizeof(int32_t) * L);
     if (wm) {
-        std::memcpy(out->model_num_good, stage.p + b->win_model, sizeof(int32_t) * L * M);
+        std::memcpy(out->model_num_good, host + b->win_model, sizeof(int32_t) * L * M);
         for (size_t l = 0; l < L; ++l)
             std::memcpy(out->model_num_requests + l * M,
                         b->wl_model_requests[(size_t)(b->paired ? b->stream_of[l] : (int32_t)(l / (size_t)b->B))].data(), sizeof(int32_t) * M);
     }
     if (wg) {
-        std::memcpy(out->group_num_requests, stage.p + b->win_group, sizeof(int32_t) * L * G);
-        std::memcpy(out->group_num_good, stage.p + b->win_group + sizeof(int32_t) * L * G, sizeof(int32_t) * L * G);
+        std::memcpy(out->group_num_requests, host + b->win_group, sizeof(int32_t) * L * G);
+        std::memcpy(out->group_num_good, host + b->win_group + sizeof(int32_t) * L * G, sizeof(int32_t) * L * G);
     }
-    stage.trim();
+    if (!b->in_scratch) stage.trim();
     return MMSIM_OK;
 }
 

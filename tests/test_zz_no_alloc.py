@@ -6,6 +6,11 @@ row, the second with a smaller input, so that what the first call left in the st
 show if anything that must start at zero were not cleared.  Collected last (file name): a failure
 here must not hide the other tests.
 """
+import json
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -78,3 +83,41 @@ def test_static_entry_point_refuses_what_does_not_fit():
     got = E.eval_batch(eng, dw, table, packed, 0, static=True)
     ref = E.eval_batch(eng, dw, table, packed, 0, static=False)
     _same(got, ref, "after a refusal")
+
+
+_COUNT = """
+import ctypes, json, sys
+counter = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)      # before the library, so that its calls come here
+counter.allocator_calls.restype = ctypes.c_long
+from mms_amd import _lib, engine as E
+from mms_amd.synthetic import make_config
+eng = E.Engine.default()
+cfg = make_config(2, 64)
+table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
+st = cfg.stream(0)
+dw = [E.DeviceWorkload(eng, st.tstamps[:900], st.model_ids[:900], st.slos[:900], cfg.num_models)]
+packed = E.pack_placements(cfg.placements, table)
+def calls(static, flags):
+    before = counter.allocator_calls()
+    E.eval_batch(eng, dw, table, packed, flags, static=static)
+    return counter.allocator_calls() - before
+every = _lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS | _lib.WANT_PER_REQUEST
+first = [calls(True, f) for f in (0, every)]
+plain = calls(False, 0)
+again = [calls(True, f) for f in (0, every)]
+eng.set_options(window_lanes=-1)      # the kernels that take one request after the other
+print(json.dumps([first, plain, again, [calls(True, f) for f in (0, every)], calls(False, 0)]))
+"""
+
+
+def test_static_entry_point_calls_no_allocator(tmp_path):
+    """Neither device memory nor pinned host memory is allocated or freed inside the call, the context's first one
+    included (a process of its own, in which the library's calls of the allocators are counted)."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    lib = str(tmp_path / "alloc_counter.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", os.path.join(here, "alloc_counter.c"), "-o", lib, "-ldl"], check=True)
+    out = subprocess.run([sys.executable, "-c", _COUNT, lib], cwd=os.path.dirname(here), capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    first, plain, again, one_by_one, plain2 = json.loads(out.stdout.splitlines()[-1])
+    assert plain > 0 and plain2 > 0          # the count sees the ordinary entry point's
+    assert first == again == one_by_one == [0, 0]
