@@ -1663,6 +1663,7 @@ void mmsim_batch_destroy(mmsim_batch *b) {
     if (b->ctx) {
         (void)hipSetDevice(b->ctx->device);
         (void)hipStreamSynchronize(b->ctx->stream);
+        if (b->window && !b->in_scratch) b->ctx->staging.trim();  // (of a call that failed on the way)
     }
     delete b;
 }

@@ -80,41 +80,17 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     CompactLatency cl;
     if (compact_latency(t, false, &cl) != MMSIM_OK) return kOther;
 
-    // ---- inputs: one buffer
-    Layout in;
+    // ---- what the placements are like (nothing is packed before the batch is known to be for this kernel)
     int64_t replicas = 0;
     for (int32_t b = 0; b < B; ++b) {
         const int32_t G = p->num_groups[b];
         if (G < 0 || G > Gmax) return kOther;
         const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-        for (int32_t g = 0; g < G; ++g)  // (what is written below has room for off[G] - off[0] entries)
+        for (int32_t g = 0; g < G; ++g)  // (what is packed below has room for off[G] - off[0] entries)
             if (off[g + 1] < off[g]) return kOther;
         if (off[G] > off[0] && !p->gm_idx) return kOther;
         replicas += off[G] - off[0];
         if (replicas > 0x7FFFFFFF) return kOther;
-    }
-    const size_t at_ptr = in.take(sizeof(void *) * (size_t)n_seeds), at_len = in.take(sizeof(int64_t) * (size_t)n_seeds);
-    const size_t at_so = in.take(stream_of ? sizeof(int32_t) * (size_t)B : 0);
-    const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
-    const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
-    const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
-    HIP_TRY(hipSetDevice(ctx->device));
-    std::vector<unsigned char> plain;  // (read until the wait below)
-    if (g_arena)
-        plain.resize(in.used);
-    else
-        HIP_TRY(ctx->staging.ensure(in.used));
-    unsigned char *host = g_arena ? plain.data() : ctx->staging.p;
-    uint8_t *h_ng = host + at_ng, *h_cfg = host + at_cfg;
-    uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off), *h_ent = reinterpret_cast<uint32_t *>(host + at_ent);
-    {
-        uint32_t at = 0;
-        for (int32_t b = 0; b < B; ++b) {
-            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-            h_off[b] = at;
-            at += (uint32_t)(off[p->num_groups[b]] - off[0]);
-        }
-        h_off[B] = at;
     }
     std::atomic<bool> bad{false};
     std::mutex shape_mutex;
@@ -126,12 +102,8 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             const int32_t G = p->num_groups[b];
             const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
             const int32_t *cfg = p->group_cfg + (size_t)b * Gmax;
-            uint32_t *ent = h_ent + h_off[b];
             int32_t slots = 0, chunks = 0;
-            h_ng[b] = (uint8_t)G;
-            for (int32_t g = 0; g < Gmax; ++g) {
-                h_cfg[(size_t)b * Gmax + g] = g < G ? (uint8_t)cfg[g] : 0;
-                if (g >= G) continue;
+            for (int32_t g = 0; g < G; ++g) {
                 if (cfg[g] < 0 || cfg[g] >= C) {
                     bad = true;
                     return;
@@ -140,17 +112,16 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
                 slots += pp;
                 mine.pow2 = mine.pow2 && (pp & (pp - 1)) == 0;
                 mine.smax = std::max(mine.smax, pp);
-                for (int64_t x = off[g]; x < off[g + 1]; ++x) {
-                    const int32_t m = p->gm_idx[x];
-                    if (m < 0 || m >= M || count[m] >= MMSIM_MAX_REPLICAS) {
-                        bad = true;
-                        return;
-                    }
-                    *ent++ = (uint32_t)m | (uint32_t)g << 16;
-                    chunks += count[m] >= 4 && (count[m] & 3) == 0;
-                    count[m] += 1;
-                    mine.rmax = std::max<int32_t>(mine.rmax, count[m]);
+            }
+            for (int64_t x = off[0]; x < off[G]; ++x) {
+                const int32_t m = p->gm_idx[x];
+                if (m < 0 || m >= M || count[m] >= MMSIM_MAX_REPLICAS) {
+                    bad = true;
+                    return;
                 }
+                chunks += count[m] >= 4 && (count[m] & 3) == 0;
+                count[m] += 1;
+                mine.rmax = std::max<int32_t>(mine.rmax, count[m]);
             }
             if (slots > MMSIM_MAX_SLOTS) {
                 bad = true;
@@ -158,7 +129,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             }
             mine.nslots = std::max(mine.nslots, slots);
             mine.ext_cap = std::max(mine.ext_cap, chunks);
-            for (const uint32_t *e = h_ent + h_off[b]; e < ent; ++e) count[*e & 0xFFFFu] = 0;
+            for (int64_t x = off[0]; x < off[G]; ++x) count[p->gm_idx[x]] = 0;
         }
         std::lock_guard<std::mutex> lock(shape_mutex);
         shape.nslots = std::max(shape.nslots, mine.nslots);
@@ -219,6 +190,52 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     const int64_t tiles = (B + per_wave - 1) / per_wave, units = tiles * out_seeds;
     int waves = (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (units + cus - 1) / cus));
     while (waves > 1 && lat_lds + wave_lds(lanes) * (size_t)waves > lds) --waves;
+
+    // ---- inputs: one buffer
+    Layout in;
+    const size_t at_ptr = in.take(sizeof(void *) * (size_t)n_seeds), at_len = in.take(sizeof(int64_t) * (size_t)n_seeds);
+    const size_t at_so = in.take(stream_of ? sizeof(int32_t) * (size_t)B : 0);
+    const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
+    const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
+    const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
+    HIP_TRY(hipSetDevice(ctx->device));
+    std::vector<unsigned char> plain;  // (read until the wait below)
+    if (g_arena)
+        plain.resize(in.used);
+    else
+        HIP_TRY(ctx->staging.ensure(in.used));
+    struct Trim {  // the memory of a batch that is not made after all
+        Staging *staging;
+        hipStream_t stream;
+        ~Trim() {
+            if (!staging) return;
+            if (staging->n > Staging::kMost) (void)hipStreamSynchronize(stream);  // (the inputs may be on their way out of it)
+            staging->trim();
+        }
+    } unless_made{g_arena ? nullptr : &ctx->staging, ctx->stream};
+    unsigned char *host = g_arena ? plain.data() : ctx->staging.p;
+    uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off);
+    {
+        uint32_t at = 0;
+        for (int32_t b = 0; b < B; ++b) {
+            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+            h_off[b] = at;
+            at += (uint32_t)(off[p->num_groups[b]] - off[0]);
+        }
+        h_off[B] = at;
+    }
+    parallel_slices(B, 1024, [&](int64_t b0, int64_t b1) {
+        for (int64_t b = b0; b < b1; ++b) {
+            const int32_t G = p->num_groups[b];
+            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+            uint8_t *cfg = host + at_cfg + (size_t)b * Gmax;
+            uint32_t *ent = reinterpret_cast<uint32_t *>(host + at_ent) + h_off[b];
+            host[at_ng + (size_t)b] = (uint8_t)G;
+            for (int32_t g = 0; g < Gmax; ++g) cfg[g] = g < G ? (uint8_t)p->group_cfg[(size_t)b * Gmax + g] : 0;
+            for (int32_t g = 0; g < G; ++g)
+                for (int64_t x = off[g]; x < off[g + 1]; ++x) *ent++ = (uint32_t)p->gm_idx[x] | (uint32_t)g << 16;
+        }
+    });
 
     std::unique_ptr<mmsim_batch> b(new (std::nothrow) mmsim_batch);
     if (!b) return fail(MMSIM_E_NOMEM, "host allocation failed");
@@ -322,6 +339,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     a.finish = reinterpret_cast<double *>(r + b->win_finish);
     a.good = r + b->win_good;
     b->wargs = a;
+    unless_made.staging = nullptr;
     *out = b.release();
     return MMSIM_OK;
 }

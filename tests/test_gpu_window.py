@@ -129,3 +129,55 @@ def test_replica_tables_of_one_placement(order):
         assert np.array_equal(good, g0) and np.array_equal(fin.view(np.uint64), f0.view(np.uint64)), seed
         for x, y in zip(counts, c0):
             assert np.array_equal(x, y), seed
+
+
+def test_batches_beyond_the_lds_of_the_chip():
+    """LDS holds the state of so many placements at once; one more and the whole batch goes to the kernels that take one
+    request after the other, with the same results, and the next call is not affected."""
+    eng = E.Engine.default()
+    info = eng.device_info()
+    M = 900
+    profiles, sols = _problem(11, (1, 2), True, M, 3, 200, 6)
+    table = E.LatencyTable(profiles, [1])
+    st = _stream(7, 400, M, 3.0)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, M)
+    # 32 bytes per model for the first four replicas and 4 for its groups, and some hundred bytes beside them
+    at_least = info["lds_bytes_per_block"] // (36 * M + 600) * info["compute_units"]
+    at_most = info["lds_bytes_per_block"] // (36 * M) * info["compute_units"]
+    ref = oracle_batch(st, table, E.pack_placements(sols, table))
+    for B, kernel in ((at_least, "sim_window_kernel<"), (at_most + 1, "sim_mixed_kernel<"), (at_least, "sim_window_kernel<")):
+        packed = E.pack_placements([sols[b % len(sols)] for b in range(B)], table)
+        batch = E.Batch(eng, [dw], table, packed, 0)
+        assert batch.kernel_name().startswith(kernel), (B, batch.kernel_name())
+        batch.close()
+        out = E.eval_batch(eng, [dw], table, packed)
+        for key in ("n_good", "latency_sum"):
+            assert np.array_equal(out[key][0], ref[key][np.arange(B) % len(sols)]), (B, key)
+    dw.close()
+
+
+@pytest.mark.parametrize("lanes", [64, 32, 16, 8])
+def test_latency_tables_that_do_not_fit_beside_a_placement(lanes):
+    """A table with a latency per stage, larger than LDS: the stage walk reads it from memory."""
+    eng = E.Engine.default()
+    M, depths = 80, tuple(range(1, 33))      # rows of 528 latencies and one more: 165 KB
+    profiles, sols = _problem(lanes, depths, False, M, 7, 40, 12)
+    table = E.LatencyTable(profiles, [1])
+    for p in profiles:
+        for pc in p.para_dict:
+            table.config_id(pc)
+    packed = E.pack_placements(sols, table)
+    assert table.arrays()[0].shape[2] == 32 and 4 * M * (sum(depths) + 1) > eng.device_info()["lds_bytes_per_block"]
+    streams = [_stream(60 + k, R, M, 4.0) for k, R in enumerate((1000, lanes + 1))]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    for flags in (0, COUNTS):
+        batch = E.Batch(eng, dws, table, packed, flags, options=dict(window_lanes=lanes))
+        assert batch.kernel_name().endswith("false>") and batch.info()["lds_bytes"] < 4 * M * sum(depths)
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k, st in enumerate(streams):
+            assert_batch_matches(out, oracle_batch(st, table, packed), k, packed[0], where=f"{lanes} lanes, stream {k}")
+    for dw in dws:
+        dw.close()
