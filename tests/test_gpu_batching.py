@@ -403,3 +403,38 @@ def test_one_simulation_to_a_wavefront(eng, sizes, groups):
             assert np.array_equal(a, b), seed
         most = max(most, int((c["m2g"] >= 0).sum(axis=1).max()))
     assert most > 8 or groups < 30
+
+
+@pytest.mark.parametrize("flags,octets", [(0, True), (_lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS, False)])
+def test_octets_in_place_of_sixteen_lanes(eng, flags, octets):
+    """32768 simulations of a small problem: sixteen of them to a wavefront give every SIMD two wavefronts, octets take
+    half the time, and are chosen while the 64-wide rows of their tables are small beside the streams (they are not with
+    counts of 64 short streams)."""
+    from mms_amd.profiling import ParallelConfig, synthetic_profile
+    from mms_amd.placement_policy import ModelPlacement
+    rng = np.random.default_rng(3)
+    M, G, B, n_streams, R, sizes = 8, 6, 512, 64, 250, [1, 2, 4]
+    pcs = [ParallelConfig(1, 1, 1), ParallelConfig(1, 1, 2)]
+    profiles = [synthetic_profile(f"m{m}", 0.05 + 0.02 * m, pcs, batch_sizes=sizes, batch_slope=0.2) for m in range(M)]
+    sols = [ModelPlacement([pcs[int(rng.integers(2))] for _ in range(G)], [sorted(rng.choice(M, 3, replace=False).tolist()) for _ in range(G)])
+            for _ in range(B)]
+    table = E.LatencyTable(profiles, sizes)
+    packed = E.pack_placements(sols, table)
+    streams = [SimpleNamespace(tstamps=np.cumsum(rng.exponential(0.01, R + k)), model_ids=rng.integers(0, M, R + k).astype(np.int32),
+                               slos=rng.uniform(0.2, 1.0, R + k).astype(np.float32)) for k in range(n_streams)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING)
+    name, waves = batch.kernel_name(), batch.info()["waves"]
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    assert waves == B * n_streams // (8 if octets else 16) and name.split(", ")[3] == ("true" if octets else "false"), (waves, name)
+    for k in (0, 31, 63):
+        ref = oracle_batch(streams[k], table, packed, batching=True)
+        for key in ("n_good", "model_num_requests", "model_num_good", "group_num_requests", "group_num_good"):
+            if key in out:
+                assert np.array_equal(out[key][k], ref[key]), (k, key)
+        assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
+    for dw in dws:
+        dw.close()
