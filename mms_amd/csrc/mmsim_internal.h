@@ -237,8 +237,9 @@ struct WindowArgs {
 // placements that share the wavefront.
 __host__ __device__ constexpr int window_ring_bytes(int lanes) { return lanes == kWave ? 0 : 2 * kWave * (int)sizeof(Req); }
 constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
-// More simulations than this put 64 placements to a wavefront (20000 requests, 16384 four-stage pipelines of 32 models:
-// 8.0 ms with requests side by side, 7.6 ms so; 8192: 6.0 against 7.6 ms).
+// More simulations than this put 64 placements to a wavefront, whatever they are (20000 requests, best number of lanes against
+// that: 16384 single devices 6.8 against 6.5 ms, two-stage pipelines 8.9 / 8.9, four-stage ones 7.9 / 7.8; 24576: 10.4 / 7.0,
+// 13.8 / 9.4, 12.5 / 8.2; build_window says when fewer do).
 constexpr int64_t kMaxWindowSims = 12288;
 typedef void (*WindowKernel)(const WindowArgs);
 // The kernel for LANES requests side by side (64, 32, 16, 8), stage bucket smax and the rest of its template arguments.

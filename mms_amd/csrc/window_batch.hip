@@ -54,6 +54,7 @@ hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_by
 struct Shape {
     int32_t nslots = 1, smax = 1, rmax = 1, ext_cap = 0;
     bool pow2 = true;  // every group has 1, 2, 4, ... stages
+    int64_t depths = 0;  // stages of the group of every replica, added up
 };
 
 }  // namespace
@@ -112,6 +113,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
                 slots += pp;
                 mine.pow2 = mine.pow2 && (pp & (pp - 1)) == 0;
                 mine.smax = std::max(mine.smax, pp);
+                mine.depths += (off[g + 1] - off[g]) * pp;
             }
             for (int64_t x = off[0]; x < off[G]; ++x) {
                 const int32_t m = p->gm_idx[x];
@@ -137,6 +139,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         shape.pow2 = shape.pow2 && mine.pow2;
         shape.rmax = std::max(shape.rmax, mine.rmax);
         shape.ext_cap = std::max(shape.ext_cap, mine.ext_cap);
+        shape.depths += mine.depths;
     });
     if (bad) return kOther;
 
@@ -168,28 +171,56 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
     auto wave_lds = [&](int lanes) { return place * (size_t)(kWave / lanes) + (size_t)window_ring_bytes(lanes); };
     auto fits = [&](int lanes) { return lat_lds + wave_lds(lanes) <= lds; };
+    auto waves_for = [&](int l) {  // wavefronts of a workgroup
+        const int64_t units = (B + kWave / l - 1) / (kWave / l) * out_seeds;
+        int waves = (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (units + cus - 1) / cus));
+        while (waves > 1 && lat_lds + wave_lds(l) * (size_t)waves > lds) --waves;
+        return waves;
+    };
+    auto at_once = [&](int l) {  // placements on the chip at once, in workgroups of so many wavefronts
+        const int waves = waves_for(l);
+        return cus * (int64_t)(lds / (lat_lds + wave_lds(l) * (size_t)waves)) * waves * (kWave / l);
+    };
     int lanes = o.window_lanes;
     if (lanes == 0) {
-        // LDS holds the state of so many placements at once; what is left over would run after them, and two rounds
-        // take longer than 64 placements to a wavefront (20000 requests: 8192 placements of 128 models on 64 devices,
-        // of which 4600 fit, 11.9 ms at best against 10.2 ms; 16384 of 64 models, of which 10000 fit, 13.7 against 9.7 ms).
-        if (sims > cus * (int64_t)((lds - lat_lds) / place)) return kOther;
-        // As many requests side by side as leave two wavefronts to a SIMD, four where a group is one stage: a step is a
-        // dependent chain that the other wavefronts fill, and more of them share the issue slots.  20000 requests, ms
-        // at 64 / 32 / 16 / 8 lanes: 4096 placements of 128 models 7.2 / 6.4 / 6.9 / 8.0; 8192 of 64 models
-        // 9.3 / 9.4 / 7.5 / 8.0; 8192 four-stage pipelines 7.4 / 6.1 / 6.0 / 6.8; single devices, 4096: 2.2 / 2.5 / 3.3
-        // / 4.6, 8192: 3.9 / 3.7 / 3.9 / 5.2.
-        const int64_t most = (a.smax_bucket == 1 ? 16 : 8) * cus;
-        lanes = 64;
-        while (lanes > 8 && sims * lanes / kWave > most && fits(lanes / 2)) lanes /= 2;
+        // Up to how many simulations, and how many requests side by side.  Measured on some 500 batches (12000 or 20000
+        // requests at 1 to 12 a second and model; 1025 to 12288 placements of 16 to 300 models on 16 to 64 devices, in
+        // groups of 1 to 32 stages); below: milliseconds at 64 / 32 / 16 / 8 lanes against 64 placements to a wavefront.
+        //
+        // A step is longer the deeper the groups are, while with 64 placements to a wavefront the depth costs little; what
+        // counts is between the mean and the deepest.  Groups of 2 to 16 devices (3.5 and 16 stages), 8192: 7.1 / 6.7 / 5.3
+        // / 5.8 against 6.0, 12288: 9.4 / 8.8 / 6.8 / 10.7; 16-stage pipelines, 4096: 7.8 / 5.6 / 4.9 / 5.3 against 5.7,
+        // 8192: 14.7 / 9.9 / 7.1 / 5.9; 1 to 8 stages (3.2), 12288: 7.5 / 6.3 / 5.1 / 8.7 against 5.7.  Depths other than
+        // 1, 2, 4, 8 and 16 are slow in the other kernel (6.4 and 12 stages, 12288: 11.7 / 9.7 / 7.7 / 12.2 against 10.7),
+        // and paired batches fill its tiles with what one stream has.
+        const double depth = (shape.smax + (replicas > 0 ? (double)shape.depths / (double)replicas : 1.0)) / 2;
+        const bool any_depth = stream_of || !shape.pow2 || shape.smax > 16;
+        if (sims > (any_depth || depth <= 6 ? kMaxWindowSims : depth <= 10 ? 8192 : 4096)) return kOther;
+        lanes = kWave;
+        if (sims > at_once(kWave)) {
+            // More than LDS holds at once: the wavefronts with one placement each, which follow one another freely (8192 of
+            // 300 models: 2.1 / 3.0 / 4.8 / 7.7 against 4.6; of 128 models, at worst, 5.7 / 5.1 / 5.8 / 7.3 against 5.2; 12288:
+            // 3.0 to 8.5 against 4.5 to 6.1).
+            if (sims > 8192 || !fits(kWave)) return kOther;
+        } else {
+            // As many requests side by side as leave three wavefronts to a SIMD (the registers of the kernels for up to 16
+            // stages hold three or four), four of the single-stage kernel, two of deep groups.  Four-stage pipelines, 3000:
+            // 3.6 / 4.2 / 4.5 / 5.6, 6000: 5.6 / 4.9 / 5.7 / 6.2, 12288: 10.2 / 9.3 / 7.2 / 7.8; single stages, 4096: 2.6 / 2.8
+            // / 3.8 / 5.0, 8192: 4.5 / 4.2 / 4.4 / 5.7; 32-stage pipelines, 12288: 45 / 29 / 19 / 15 against 25.
+            // A narrower wavefront needs more LDS, for its placements and for the requests on their way to them: where it would
+            // take two rounds, up to twice as many wavefronts stay (5000 placements of 128 models, 5.1 / 6.4), unless the
+            // groups are deep (11000 32-stage pipelines, in two rounds either way, 16 lanes 26, 8 lanes 24).
+            const int64_t most = (a.smax_bucket == 1 ? 16 : depth <= 10 ? 12 : 8) * cus;
+            while (lanes > 8 && sims * lanes / kWave > most && fits(lanes / 2) &&
+                   (sims <= at_once(lanes / 2) || sims * lanes / kWave > 2 * most || depth > 10))
+                lanes /= 2;
+        }
     }
     if (stream_of) lanes = kWave;  // (the placements of a wavefront share a stream)
     while (lanes < kWave && !fits(lanes)) lanes *= 2;
     if (!fits(lanes)) return kOther;
-    const int per_wave = kWave / lanes;
+    const int per_wave = kWave / lanes, waves = waves_for(lanes);
     const int64_t tiles = (B + per_wave - 1) / per_wave, units = tiles * out_seeds;
-    int waves = (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (units + cus - 1) / cus));
-    while (waves > 1 && lat_lds + wave_lds(lanes) * (size_t)waves > lds) --waves;
 
     // ---- inputs: one buffer
     Layout in;

@@ -132,8 +132,9 @@ def test_replica_tables_of_one_placement(order):
 
 
 def test_batches_beyond_the_lds_of_the_chip():
-    """LDS holds the state of so many placements at once; one more and the whole batch goes to the kernels that take one
-    request after the other, with the same results, and the next call is not affected."""
+    """LDS holds the state of so many placements at once; more follow one another with one placement to a wavefront, and
+    batches beyond 8192 go to the kernels that take one request after the other, with the same results; the next call is
+    not affected."""
     eng = E.Engine.default()
     info = eng.device_info()
     M = 900
@@ -145,7 +146,8 @@ def test_batches_beyond_the_lds_of_the_chip():
     at_least = info["lds_bytes_per_block"] // (36 * M + 600) * info["compute_units"]
     at_most = info["lds_bytes_per_block"] // (36 * M) * info["compute_units"]
     ref = oracle_batch(st, table, E.pack_placements(sols, table))
-    for B, kernel in ((at_least, "sim_window_kernel<"), (at_most + 1, "sim_mixed_kernel<"), (at_least, "sim_window_kernel<")):
+    for B, kernel in ((at_least, "sim_window_kernel<"), (at_most + 1, "sim_window_kernel<64,"), (8193, "sim_mixed_kernel<"),
+                      (at_least, "sim_window_kernel<")):
         packed = E.pack_placements([sols[b % len(sols)] for b in range(B)], table)
         batch = E.Batch(eng, [dw], table, packed, 0)
         assert batch.kernel_name().startswith(kernel), (B, batch.kernel_name())
@@ -181,3 +183,28 @@ def test_latency_tables_that_do_not_fit_beside_a_placement(lanes):
             assert_batch_matches(out, oracle_batch(st, table, packed), k, packed[0], where=f"{lanes} lanes, stream {k}")
     for dw in dws:
         dw.close()
+
+
+@pytest.mark.parametrize("stages,B,kernel", [(1, 4096, "window_kernel<64"), (1, 4097, "window_kernel<32"), (1, 8194, "window_kernel<16"),
+                                            (1, 12288, "window_kernel<16"), (1, 12289, "mixed_kernel<"), (4, 3072, "window_kernel<64"),
+                                            (4, 3073, "window_kernel<32"), (4, 6146, "window_kernel<16"), (4, 12288, "window_kernel<16"),
+                                            (4, 12289, "mixed_kernel<"), (8, 8192, "window_kernel<16"), (8, 8193, "mixed_kernel<"),
+                                            (16, 4096, "window_kernel<32"), (16, 4097, "mixed_kernel<"), (3, 12288, "window_kernel<16"),
+                                            (32, 12288, "window_kernel<8"), (32, 12289, "mixed_kernel<")])
+def test_which_batches_have_their_requests_side_by_side(stages, B, kernel):
+    """The number of simulations and the depth of the groups decide (kernels of either side of every line)."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(stages, (stages,), True, 4, 2, 64, 3)
+    table = E.LatencyTable(profiles, [1])
+    st = _stream(stages, 130, 4, 2.0)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, 4)
+    of = np.arange(B) % len(sols)
+    batch = E.Batch(eng, [dw], table, E.pack_placements([sols[b] for b in of], table), 0)
+    assert batch.kernel_name().startswith("sim_" + kernel), batch.kernel_name()
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    dw.close()
+    ref = oracle_batch(st, table, E.pack_placements(sols, table))
+    assert np.array_equal(out["n_good"][0], ref["n_good"][of]) and np.array_equal(out["latency_sum"][0], ref["latency_sum"][of])
