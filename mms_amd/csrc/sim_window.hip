@@ -54,7 +54,6 @@
 namespace mmsim {
 namespace {
 
-// <wave primitives>
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
@@ -97,11 +96,6 @@ __device__ __forceinline__ void arrived_req(Req &r) {
     asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
     __builtin_memcpy(&r, w, 16);
 }
-// In a loop that lanes leave one by one: what loop_enter to loop_leave encloses, with collectives of the lanes still in.
-__device__ __forceinline__ void loop_enter(bool) {}
-__device__ __forceinline__ void loop_leave() {}
-__device__ __forceinline__ uint64_t ballot_in_loop(bool p) { return __builtin_amdgcn_ballot_w64(p); }
-__device__ __forceinline__ void order_in_loop() { wave_order(); }
 // keeps the compiler from merging what made v with what uses it
 __device__ __forceinline__ void pin(uint32_t &v) { asm volatile("" : "+v"(v)); }
 // LDS atomics whose result nobody waits for
@@ -177,7 +171,6 @@ __device__ __forceinline__ double ordered_sum(double s, double x, uint64_t lanes
 #undef MMSIM_ADD2
 #undef MMSIM_ADD16
 #undef MMSIM_ADD1
-// </wave primitives>
 
 struct Entry {  // a replica, as rep and ext hold it
     uint32_t d;
@@ -535,15 +528,15 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                         }
                     }
                     latency = (t + overhead) - arr;
-                    const uint64_t accs = ballot_in_loop(latency <= limit);
+                    const uint64_t accs = ballot(latency <= limit);
                     // ---- whose verdict is final
                     const uint64_t blockers = win.g & accs;
                     waits = blockers != 0ull;
-                    uint64_t waiting = ballot_in_loop(waits);
+                    uint64_t waiting = ballot(waits);
                     // requests that wait, are not accepted so far and list several groups: they hold up others too
                     for (uint64_t open = waiting & multis & ~accs; __builtin_expect(open != 0ull, 0);) {
                         waits = (win.g & (accs | waiting)) != 0ull;
-                        const uint64_t w2 = ballot_in_loop(waits);
+                        const uint64_t w2 = ballot(waits);
                         open = w2 & ~waiting & multis & ~accs;
                         waiting = w2;
                     }
@@ -574,12 +567,11 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                             }
                         }
                     }
-                    order_in_loop();
+                    wave_order();
 #pragma unroll
                     for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
                 } while (waits);
             };
-            loop_enter(in_mask(pend));
             if (in_mask(pend)) {
                 if constexpr (SMAX == 1) {
                     steps(Int<1>{});
@@ -594,7 +586,6 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     if (deep_a == 0ull) steps(Int<16>{});
                     else steps(Int<32>{});
                 }
-                loop_leave();
             }
         };
         if constexpr (EXT) {
