@@ -1231,7 +1231,7 @@ void mmsim_options_default(mmsim_options *o) {
     o->skip_ahead = o->xcd_map = o->batching_lds_tables = -1;
 }
 
-int mmsim_ctx_set_options(mmsim_ctx *ctx, const mmsim_options *options) {
+int mmsim_ctx_set_options(mmsim_ctx *ctx, const mmsim_options *options) try {
     if (!ctx) return fail(MMSIM_E_INVALID, "ctx_set_options: null context");
     int rc = check_options(options);
     if (rc) return rc;
@@ -1240,9 +1240,11 @@ int mmsim_ctx_set_options(mmsim_ctx *ctx, const mmsim_options *options) {
     else
         mmsim_options_default(&ctx->opt);
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
-int mmsim_ctx_create(int device, mmsim_ctx **out) {
+int mmsim_ctx_create(int device, mmsim_ctx **out) try {
     if (!out) return fail(MMSIM_E_INVALID, "ctx_create: out is null");
     *out = nullptr;
     int count = 0;
@@ -1279,6 +1281,8 @@ int mmsim_ctx_create(int device, mmsim_ctx **out) {
     }
     *out = c.release();
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 void mmsim_ctx_destroy(mmsim_ctx *ctx) {
@@ -1293,7 +1297,7 @@ void mmsim_ctx_destroy(mmsim_ctx *ctx) {
     delete ctx;
 }
 
-int mmsim_ctx_device_info(mmsim_ctx *ctx, mmsim_device_info *out) {
+int mmsim_ctx_device_info(mmsim_ctx *ctx, mmsim_device_info *out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "device_info: null pointer");
     std::memset(out, 0, sizeof(*out));
     std::snprintf(out->name, sizeof(out->name), "%s", ctx->prop.name);
@@ -1303,10 +1307,12 @@ int mmsim_ctx_device_info(mmsim_ctx *ctx, mmsim_device_info *out) {
     out->lds_bytes_per_block = ctx->max_lds;
     out->hbm_bytes = (int64_t)ctx->prop.totalGlobalMem;
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *tstamps, const int32_t *model_ids,
-                          const float *slos, mmsim_workload **out) {
+                          const float *slos, mmsim_workload **out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "workload_create: null pointer");
     *out = nullptr;
     if (R < 0 || M < 1) return fail(MMSIM_E_INVALID, "workload_create: R must be >= 0 and M >= 1");
@@ -1373,6 +1379,8 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
     }
     *out = w.release();
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 void mmsim_workload_destroy(mmsim_workload *wl) {
@@ -1383,19 +1391,23 @@ void mmsim_workload_destroy(mmsim_workload *wl) {
 
 int mmsim_batch_create_ex(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
                           const mmsim_tables *tables, const mmsim_placements *placements, uint32_t flags,
-                          const mmsim_options *options, mmsim_batch **out) {
+                          const mmsim_options *options, mmsim_batch **out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "batch_create: null pointer");
     *out = nullptr;
     return make_batch(ctx, workloads, n_seeds, tables, placements, nullptr, flags, options, true, out);
+} catch (...) {
+    return caught();
 }
 
 int mmsim_batch_create(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
                        const mmsim_tables *tables, const mmsim_placements *placements, uint32_t flags,
-                       mmsim_batch **out) {
+                       mmsim_batch **out) try {
     return mmsim_batch_create_ex(ctx, workloads, n_seeds, tables, placements, flags, nullptr, out);
+} catch (...) {
+    return caught();
 }
 
-int mmsim_batch_run(mmsim_batch *b) {
+int mmsim_batch_run(mmsim_batch *b) try {
     if (!b) return fail(MMSIM_E_INVALID, "batch_run: null batch");
     mmsim_ctx *ctx = b->ctx;
     HIP_TRY(hipSetDevice(ctx->device));
@@ -1421,18 +1433,22 @@ int mmsim_batch_run(mmsim_batch *b) {
     HIP_TRY(hipEventRecord(b->ev_stop, ctx->stream));
     b->ran = true;
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
-int mmsim_batch_sync(mmsim_batch *b, float *kernel_ms) {
+int mmsim_batch_sync(mmsim_batch *b, float *kernel_ms) try {
     if (!b) return fail(MMSIM_E_INVALID, "batch_sync: null batch");
     if (!b->ran) return fail(MMSIM_E_INVALID, "batch_sync: batch was never run");
     HIP_TRY(hipSetDevice(b->ctx->device));
     HIP_TRY(hipEventSynchronize(b->ev_stop));
     if (kernel_ms) HIP_TRY(hipEventElapsedTime(kernel_ms, b->ev_start, b->ev_stop));
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
-int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) {
+int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
     if (!b || !out) return fail(MMSIM_E_INVALID, "batch_fetch: null pointer");
     if (!b->ran) return fail(MMSIM_E_INVALID, "batch_fetch: batch was never run");
     if (!out->n_good || !out->latency_sum) return fail(MMSIM_E_INVALID, "batch_fetch: n_good and latency_sum are required");
@@ -1550,10 +1566,12 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) {
                                  ? "a simulation ran out of idle-event slots; its results are invalid (pass status[] to see which)"
                                  : "a simulation hit an input the batching simulator does not support (all replica clocks infinite)");
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloads, int32_t n_streams,
-                            const int64_t *skip, mmsim_model_stats *out) {
+                            const int64_t *skip, mmsim_model_stats *out) try {
     if (!b || !workloads || !skip || !out) return fail(MMSIM_E_INVALID, "batch_model_stats: null pointer");
     if (!b->ran) return fail(MMSIM_E_INVALID, "batch_model_stats: batch was never run");
     if (!(b->flags & MMSIM_WANT_PER_REQUEST))
@@ -1656,6 +1674,8 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
                             out->latency_std, out->latency_p90, out->latency_p99};
     for (int k = 0; k < 7; ++k) std::memcpy(o64[k], h_f64.data() + (size_t)k * cells, sizeof(double) * cells);
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 void mmsim_batch_destroy(mmsim_batch *b) {
@@ -1668,7 +1688,7 @@ void mmsim_batch_destroy(mmsim_batch *b) {
     delete b;
 }
 
-int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) {
+int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {
     if (!b || !out) return fail(MMSIM_E_INVALID, "batch_get_info: null pointer");
     out->lanes = b->B * b->out_seeds;
     out->waves = b->waves;
@@ -1689,15 +1709,19 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) {
     out->event_slots = (b->flags & MMSIM_BATCHING) ? b->bargs.heap_cap : 0;
     out->reserved = 0;
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
-int mmsim_batch_kernel_name(const mmsim_batch *b, char *buf, size_t size) {
+int mmsim_batch_kernel_name(const mmsim_batch *b, char *buf, size_t size) try {
     if (!b || !buf || size == 0) return fail(MMSIM_E_INVALID, "batch_kernel_name: null pointer or empty buffer");
     const std::string name = (b->flags & MMSIM_BATCHING) ? sim_batching_kernel_name(b->bargs)
                              : b->window                   ? sim_window_kernel_name(b->wargs)
                                                            : sim_mixed_kernel_name(b->args, b->smax_bucket);
     std::snprintf(buf, size, "%s", name.c_str());
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 namespace {
@@ -1812,14 +1836,16 @@ int eval_with_retry(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int3
 
 int mmsim_eval_batch(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
                      const mmsim_tables *tables, const mmsim_placements *placements, uint32_t flags,
-                     mmsim_result *out) {
+                     mmsim_result *out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "eval_batch: null pointer");
     return eval_with_retry(ctx, workloads, n_seeds, tables, placements, nullptr, flags, out);
+} catch (...) {
+    return caught();
 }
 
 int mmsim_eval_successors(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
                           const mmsim_tables *tables, const mmsim_placements *base, const mmsim_successors *successors,
-                          uint32_t flags, mmsim_result *out) {
+                          uint32_t flags, mmsim_result *out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "eval_successors: null pointer");
     int rc = check_tables(tables);
     if (rc) return rc;
@@ -1827,18 +1853,22 @@ int mmsim_eval_successors(mmsim_ctx *ctx, const mmsim_workload *const *workloads
     rc = expand_successors(base, successors, tables->M, &all);
     if (rc) return rc;
     return mmsim_eval_batch(ctx, workloads, n_seeds, tables, &all.view, flags, out);
+} catch (...) {
+    return caught();
 }
 
 int mmsim_eval_pairs(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_streams,
                      const mmsim_tables *tables, const mmsim_placements *placements, const int32_t *stream_of,
-                     uint32_t flags, mmsim_result *out) {
+                     uint32_t flags, mmsim_result *out) try {
     if (!ctx || !out || !stream_of) return fail(MMSIM_E_INVALID, "eval_pairs: null pointer");
     return eval_with_retry(ctx, workloads, n_streams, tables, placements, stream_of, flags, out);
+} catch (...) {
+    return caught();
 }
 
 int mmsim_eval_batch_static(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int32_t n_seeds,
                             const mmsim_tables *tables, const mmsim_placements *placements, uint32_t flags,
-                            mmsim_result *out) {
+                            mmsim_result *out) try {
     if (!ctx || !out) return fail(MMSIM_E_INVALID, "eval_batch_static: null pointer");
     if (!ctx->scratch) return fail(MMSIM_E_HIP, "eval_batch_static: the context has no static scratch");
     // Every device buffer of the batch is carved out of the device's static scratch (nothing is allocated or
@@ -1848,9 +1878,11 @@ int mmsim_eval_batch_static(mmsim_ctx *ctx, const mmsim_workload *const *workloa
     arena.base = ctx->scratch;
     arena.cap = MMSIM_STATIC_SCRATCH_BYTES;
     mmsim_batch *b = nullptr;
-    g_arena = &arena;
-    int rc = make_batch(ctx, workloads, n_seeds, tables, placements, nullptr, flags, nullptr, true, &b);
-    g_arena = nullptr;
+    int rc;
+    {
+        ArenaScope scope(&arena);
+        rc = make_batch(ctx, workloads, n_seeds, tables, placements, nullptr, flags, nullptr, true, &b);
+    }
     if (rc != MMSIM_OK && arena.overflow)
         return fail(MMSIM_E_NOMEM, "eval_batch_static: the batch (placements x models x seeds, streams, requested outputs) "
                                    "needs more device scratch than the static " +
@@ -1860,6 +1892,8 @@ int mmsim_eval_batch_static(mmsim_ctx *ctx, const mmsim_workload *const *workloa
     if (rc == MMSIM_OK) rc = mmsim_batch_fetch(b, out);
     mmsim_batch_destroy(b);  // frees nothing on the device: the buffers belong to the scratch
     return rc;
+} catch (...) {
+    return caught();
 }
 
 int mmsim_simulate_requests_mixed(mmsim_ctx *ctx, double *finish, uint8_t *good, const double *tstamps,
@@ -1867,7 +1901,7 @@ int mmsim_simulate_requests_mixed(mmsim_ctx *ctx, double *finish, uint8_t *good,
                                   const int32_t *num_stages, const float *stage_latency, int64_t num_requests,
                                   int32_t M, int32_t G, int32_t Smax, double fixed_overhead,
                                   int32_t *model_num_requests, int32_t *model_num_good_requests,
-                                  int32_t *group_num_requests, int32_t *group_num_good_requests) {
+                                  int32_t *group_num_requests, int32_t *group_num_good_requests) try {
     if (!ctx) return fail(MMSIM_E_INVALID, "simulate_requests_mixed: null context");
     if (M < 1 || G < 1 || Smax < 1 || num_requests < 0) return fail(MMSIM_E_INVALID, "simulate_requests_mixed: bad size");
     if (!m_id2g_id || !num_stages || !stage_latency || !model_num_requests || !model_num_good_requests ||
@@ -1908,6 +1942,7 @@ int mmsim_simulate_requests_mixed(mmsim_ctx *ctx, double *finish, uint8_t *good,
     rc = mmsim_workload_create(ctx, num_requests, M, tstamps, model_ids, slos, &wl);
     if (rc) return rc;
     mmsim_batch *b = nullptr;
+    const std::unique_ptr<mmsim_workload, void (*)(mmsim_workload *)> keep(wl, mmsim_workload_destroy);
     const mmsim_workload *wls[1] = {wl};
     const uint32_t flags = MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST;
     // Rows that list their groups in ascending order are what a placement's groups and models say (every row that
@@ -1951,8 +1986,9 @@ int mmsim_simulate_requests_mixed(mmsim_ctx *ctx, double *finish, uint8_t *good,
         rc = mmsim_batch_fetch(b, &r);
     }
     mmsim_batch_destroy(b);
-    mmsim_workload_destroy(wl);
     return rc;
+} catch (...) {
+    return caught();
 }
 
 int mmsim_simulate_requests(mmsim_ctx *ctx, double *finish, uint8_t *good, const double *tstamps,
@@ -1960,7 +1996,7 @@ int mmsim_simulate_requests(mmsim_ctx *ctx, double *finish, uint8_t *good, const
                             const float *group_max_latency, const float *group_sum_latency, int64_t num_requests,
                             int32_t M, int32_t G, double fixed_overhead,
                             int32_t *model_num_requests, int32_t *model_num_good_requests,
-                            int32_t *group_num_requests, int32_t *group_num_good_requests) {
+                            int32_t *group_num_requests, int32_t *group_num_good_requests) try {
     if (!ctx) return fail(MMSIM_E_INVALID, "simulate_requests: null context");
     if (M < 1 || G < 1 || num_requests < 0) return fail(MMSIM_E_INVALID, "simulate_requests: bad size");
     if (!m_id2g_id || !group_max_latency || !group_sum_latency || !model_num_requests || !model_num_good_requests ||
@@ -2036,6 +2072,8 @@ int mmsim_simulate_requests(mmsim_ctx *ctx, double *finish, uint8_t *good, const
     std::memcpy(group_num_requests, cnt.data() + 2 * (size_t)M, sizeof(int32_t) * (size_t)G);
     std::memcpy(group_num_good_requests, cnt.data() + 2 * (size_t)M + G, sizeof(int32_t) * (size_t)G);
     return MMSIM_OK;
+} catch (...) {
+    return caught();
 }
 
 int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8_t *good, const double *tstamps,
@@ -2044,7 +2082,7 @@ int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8
                                            const float *stage_latency, const int32_t *batch_sizes, int64_t num_requests,
                                            int32_t M, int32_t G, int32_t Smax, int32_t NB, double fixed_overhead,
                                            int32_t *model_num_requests, int32_t *model_num_good_requests,
-                                           int32_t *group_num_requests, int32_t *group_num_good_requests) {
+                                           int32_t *group_num_requests, int32_t *group_num_good_requests) try {
     if (!ctx) return fail(MMSIM_E_INVALID, "simulate_requests_mixed_batching: null context");
     if (M < 1 || G < 1 || Smax < 1 || NB < 1 || num_requests < 0)
         return fail(MMSIM_E_INVALID, "simulate_requests_mixed_batching: bad size");
@@ -2095,6 +2133,7 @@ int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8
     mmsim_workload *wl = nullptr;
     rc = mmsim_workload_create(ctx, num_requests, M, tstamps, model_ids, slos, &wl);
     if (rc) return rc;
+    const std::unique_ptr<mmsim_workload, void (*)(mmsim_workload *)> keep(wl, mmsim_workload_destroy);
     const mmsim_workload *wls[1] = {wl};
     const uint32_t flags = MMSIM_BATCHING | MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST;
     // (a simulation that runs out of idle-event slots is run again with twice as many, as in mmsim_eval_batch)
@@ -2122,8 +2161,9 @@ int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8
         mmsim_batch_destroy(b);
         if (rc != MMSIM_E_OVERFLOW) break;
     }
-    mmsim_workload_destroy(wl);
     return rc;
+} catch (...) {
+    return caught();
 }
 
 }  // extern "C"

@@ -4,9 +4,11 @@
 
 #include <algorithm>
 #include <atomic>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 #include "mmsim_internal.h"
@@ -18,6 +20,16 @@ inline thread_local std::string g_last_error;
 inline int fail(int code, const std::string &msg) {
     g_last_error = msg;
     return code;
+}
+
+// What an entry point returns for an exception that reached it (host memory or threads that were not to be had): none
+// leaves the C ABI.
+inline int caught() noexcept {
+    try {
+        return fail(MMSIM_E_NOMEM, "host allocation failed");
+    } catch (...) {
+        return MMSIM_E_NOMEM;  // (not even the message: the one before stays)
+    }
 }
 
 inline int hip_fail(hipError_t e, const char *what) {
@@ -39,6 +51,10 @@ struct Arena {
     bool overflow = false;
 };
 inline thread_local Arena *g_arena = nullptr;
+struct ArenaScope {
+    explicit ArenaScope(Arena *a) { g_arena = a; }
+    ~ArenaScope() { g_arena = nullptr; }
+};
 
 template <typename T>
 struct DevBuf {
@@ -116,7 +132,8 @@ struct Staging {
 };
 
 // Runs fn(lo, hi) on slices of [0, n) on up to 16 host threads (one slice per thread; the caller's
-// slices write disjoint memory).  Small ranges run on the calling thread.
+// slices write disjoint memory).  Small ranges run on the calling thread.  What a slice throws is thrown to the caller
+// when all have ended; a slice for which there is no thread runs on the calling one.
 template <class F>
 void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
     int64_t threads = std::min<int64_t>(16, std::max(1u, std::thread::hardware_concurrency()));
@@ -126,10 +143,28 @@ void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
         return;
     }
     const int64_t per = (n + threads - 1) / threads;
+    std::mutex thrown_mutex;
+    std::exception_ptr thrown;
+    auto slice = [&](int64_t lo) noexcept {
+        try {
+            fn(lo, std::min(n, lo + per));
+        } catch (...) {
+            std::lock_guard<std::mutex> lock(thrown_mutex);
+            if (!thrown) thrown = std::current_exception();
+        }
+    };
     std::vector<std::thread> pool;
-    for (int64_t lo = per; lo < n; lo += per) pool.emplace_back([&fn, lo, per, n] { fn(lo, std::min(n, lo + per)); });
-    fn((int64_t)0, std::min(n, per));
+    pool.reserve((size_t)threads);
+    for (int64_t lo = per; lo < n; lo += per) {
+        try {
+            pool.emplace_back(slice, lo);
+        } catch (const std::system_error &) {
+            slice(lo);
+        }
+    }
+    slice(0);
     for (std::thread &th : pool) th.join();
+    if (thrown) std::rethrow_exception(thrown);
 }
 
 }  // namespace mmsim

@@ -171,6 +171,23 @@ def test_offsets_that_go_back_are_refused(eng):
     _still_works(eng)
 
 
+def test_host_memory_that_is_not_to_be_had_is_an_error_code(eng):
+    """No C++ exception leaves the C ABI: a stream of 2^31 - 1 models needs 26 GB of host memory for its lists, and the
+    process may have one more."""
+    import resource
+    before = resource.getrlimit(resource.RLIMIT_AS)
+    in_use = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+    none = np.zeros(0)
+    resource.setrlimit(resource.RLIMIT_AS, (in_use + (1 << 30), before[1]))
+    try:
+        with pytest.raises(_lib.MmsimError) as err:
+            E.DeviceWorkload(eng, none, none, none, 0x7FFFFFFF)
+    finally:
+        resource.setrlimit(resource.RLIMIT_AS, before)
+    assert err.value.code == _lib.E_NOMEM and "host allocation failed" in str(err.value)
+    _still_works(eng)
+
+
 def test_options_are_validated(eng):
     for bad in (dict(request_loop=2), dict(waves_per_cu=9), dict(batching_lanes=12), dict(segment_requests=-5),
                 dict(batching_lds_tables=4)):

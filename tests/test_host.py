@@ -3,6 +3,8 @@ workload generation and statistics, helpers."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -45,6 +47,15 @@ def test_kernels_that_address_lds_by_number_have_it_from_0_on():
     assert sum("sim_window_kernel" in k for k in sizes) >= 4 * 26 and any("sim_mixed_kernel" in k for k in sizes)
     assert any(v != 0 for k, v in found.items() if "model_stats_kernel" in k)      # (one that has some)
     assert set(sizes.values()) == {0}
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_exceptions_of_host_threads_reach_the_caller(tmp_path):
+    exe = str(tmp_path / "slices_throw")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "slices_throw.cpp"), "-o", exe], check=True)
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert proc.returncode == 0 and proc.stdout == "ok\n", (proc.returncode, proc.stderr)
 
 
 def test_no_device_means_a_loud_error_not_a_fallback():
