@@ -105,8 +105,9 @@ typedef struct {
     int32_t xcd_map;              /* chunked loop: 0 = seeds innermost in the workgroup numbering; -1 / 1: all
                                      seeds of a tile group on one XCD                                           */
     int32_t batching_lanes;       /* batching simulator: 8, 16, 32 or 64 simulations per wavefront; 0: the widest
-                                     that still gives a CU eight wavefronts, and fewer than 8 if the batch
-                                     leaves the chip room                                                       */
+                                     that still gives a CU eight wavefronts; 8 rather than 16 unless the 64-wide
+                                     rows of their tables and counts are large beside the streams; 4, 2 or 1 if
+                                     the batch leaves the chip room for such wavefronts                        */
     int32_t batching_event_slots; /* batching simulator: idle-event slots per simulation (a multiple of eight);
                                      0: from the group count.  Too few makes a simulation stop with
                                      MMSIM_E_OVERFLOW (the one-call entry points then try again with more)     */
@@ -114,8 +115,9 @@ typedef struct {
                                      copied to LDS; -1: both, subject to fit                                    */
     int32_t window_lanes;         /* plain simulator, small and middle-sized batches: 8, 16, 32 or 64 requests of a
                                      placement side by side in a wavefront; -1: 64 placements in a wavefront, one
-                                     request after the other; 0: by the number of simulations.  An option above that
-                                     shapes the one-request-at-a-time kernels selects them as well             */
+                                     request after the other; 0: by the number of simulations and the depth of the
+                                     groups.  An option above that shapes the one-request-at-a-time kernels
+                                     selects them as well                                                      */
     int64_t stats_scratch_bytes;  /* scratch of one launch of mmsim_batch_model_stats; 0: 1 GiB                 */
 } mmsim_options;
 void mmsim_options_default(mmsim_options *options);

@@ -526,8 +526,8 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
-            // devices, ms at 8 / 4 / 2 / 1 simulations: 1024 placements 16.5 / 13.5 / 11.3 / 9.4, 4096: 17.1 / 14.7 /
-            // 12.7 / 19.5 (two rounds), 8192: 17.7 / 15.7 / 25).
+            // devices, ms at 8 / 4 / 2 / 1 simulations, a single one in the kernel that looks at eight arrivals at once: 1024
+            // placements 16.6 / 13.8 / 11.4 / 7.4, 4096: 17.3 / 14.8 / 12.7 / 16.0 (two rounds), 8192: 17.7 / 15.8 / 25).
             const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
             const size_t least = bytes_for(8, std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7)));  // (event slots are trimmed below)
             const int64_t per_cu = std::max<int64_t>(1, std::max(std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / least)),
