@@ -115,8 +115,9 @@ typedef struct {
                                      copied to LDS; -1: both, subject to fit                                    */
     int32_t window_lanes;         /* plain simulator, small and middle-sized batches: 8, 16, 32 or 64 requests of a
                                      placement side by side in a wavefront; -1: 64 placements in a wavefront, one
-                                     request after the other; 0: by the number of simulations and the depth of the
-                                     groups.  An option above that shapes the one-request-at-a-time kernels
+                                     request after the other; 0: by the number of simulations, the depth of the
+                                     groups and, in the one-call entry points, what
+                                     packing costs.  An option above that shapes the one-request-at-a-time kernels
                                      selects them as well                                                      */
     int64_t stats_scratch_bytes;  /* scratch of one launch of mmsim_batch_model_stats; 0: 1 GiB                 */
 } mmsim_options;

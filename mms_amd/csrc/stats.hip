@@ -5,9 +5,9 @@
 //
 // One workgroup of 1024 threads per (simulation, model); its threads share the model's requests, which
 // the per-model lists of the stream name (index and arrival time).  The first pass gathers the model's
-// latencies out of the simulation's column of finish[wave][request][64] / good (one 8-byte element per
-// 512-byte row: read once; simulations of one wavefront run side by side, so the rows are shared in L2)
-// into a contiguous scratch row, all ones for requests that were not accepted, and counts, sums and bins
+// latencies out of the simulation's row of finish / good, or out of its column of finish[wave][request][64]
+// (one 8-byte element per 512-byte row: read once; simulations of one wavefront run side by side, so the
+// rows are shared in L2; 64 x 1.0 M requests: 2.07 ms from rows, 2.17 ms from columns), into a contiguous scratch row, all ones for requests that were not accepted, and counts, sums and bins
 // the top byte on the way; every thread later reads back only what it wrote itself.
 //
 // Percentiles are order statistics: sorted[int(q * n)] (workload.py:344-346), found exactly with a

@@ -81,17 +81,67 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     CompactLatency cl;
     if (compact_latency(t, false, &cl) != MMSIM_OK) return kOther;
 
-    // ---- what the placements are like (nothing is packed before the batch is known to be for this kernel)
+    // Beyond what the chip's LDS holds at once in any case (see below): known before anything is packed.
+    const size_t lds = (size_t)ctx->max_lds;
+    const int group_words = (Gmax + 31) / 32;
+    const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
+    const size_t place_least = (size_t)M * 32 + (size_t)M * group_words * 4;
+    if (place_least > lds) return kOther;
+    // A call that evaluates a batch once packs it for the other kernel at about 18 ns per placement and model, and for this
+    // one at a tenth of that; the other kernel runs 0.5 us per request.  Where that is the faster one (the lines below), it is
+    // by a quarter of its time or so and worth its packing with streams of more than a sixth of placements x models.  Whole
+    // calls, 3000 / 12000 / 50000 requests, against the other kernel: 12288 placements in groups of 2 to 16 devices, 32
+    // models, 2.4 / 7.8 / 29 against 8.3 / 12.9 / 32 ms; 5000 16-stage pipelines, 16 models, 2.0 / 7.3 / 29 against 4.2 /
+    // 7.8 / 26; 12288 placements of 128 models, twice what LDS holds, 2.7 / 7.1 / 25 against 29 / 34 / 53.
+    // In the static scratch the batch stays here too: the other kernel's tables are a hundred times as large.
+    int64_t longest = 0;
+    for (int s = 0; s < n_seeds; ++s) longest = std::max(longest, wls[s]->R);
+    const bool packing_counts = g_arena || (!events && (int64_t)B * M >= 6 * longest);
+    const int64_t most_in_rounds = packing_counts ? kMaxWindowSims : 8192;  // simulations that LDS does not hold at once
+    if (o.window_lanes == 0 && sims > most_in_rounds && sims > cus * (int64_t)(lds / place_least)) return kOther;
+
+    // ---- inputs: one buffer
+    Layout in;
     int64_t replicas = 0;
     for (int32_t b = 0; b < B; ++b) {
         const int32_t G = p->num_groups[b];
         if (G < 0 || G > Gmax) return kOther;
         const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-        for (int32_t g = 0; g < G; ++g)  // (what is packed below has room for off[G] - off[0] entries)
-            if (off[g + 1] < off[g]) return kOther;
-        if (off[G] > off[0] && !p->gm_idx) return kOther;
+        if (off[G] < off[0] || (off[G] > off[0] && !p->gm_idx) || off[G] - off[0] > (int64_t)M * MMSIM_MAX_REPLICAS) return kOther;
         replicas += off[G] - off[0];
         if (replicas > 0x7FFFFFFF) return kOther;
+    }
+    const size_t at_ptr = in.take(sizeof(void *) * (size_t)n_seeds), at_len = in.take(sizeof(int64_t) * (size_t)n_seeds);
+    const size_t at_so = in.take(stream_of ? sizeof(int32_t) * (size_t)B : 0);
+    const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
+    const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
+    const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
+    HIP_TRY(hipSetDevice(ctx->device));
+    std::vector<unsigned char> plain;  // (read until the wait below)
+    if (g_arena)
+        plain.resize(in.used);
+    else
+        HIP_TRY(ctx->staging.ensure(in.used));
+    struct Trim {  // the memory of a batch that is not made after all
+        Staging *staging;
+        hipStream_t stream;
+        ~Trim() {
+            if (!staging) return;
+            if (staging->n > Staging::kMost) (void)hipStreamSynchronize(stream);  // (the inputs may be on their way out of it)
+            staging->trim();
+        }
+    } unless_made{g_arena ? nullptr : &ctx->staging, ctx->stream};
+    unsigned char *host = g_arena ? plain.data() : ctx->staging.p;
+    uint8_t *h_ng = host + at_ng, *h_cfg = host + at_cfg;
+    uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off), *h_ent = reinterpret_cast<uint32_t *>(host + at_ent);
+    {
+        uint32_t at = 0;
+        for (int32_t b = 0; b < B; ++b) {
+            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
+            h_off[b] = at;
+            at += (uint32_t)(off[p->num_groups[b]] - off[0]);
+        }
+        h_off[B] = at;
     }
     std::atomic<bool> bad{false};
     std::mutex shape_mutex;
@@ -103,9 +153,13 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             const int32_t G = p->num_groups[b];
             const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
             const int32_t *cfg = p->group_cfg + (size_t)b * Gmax;
+            uint32_t *ent = h_ent + h_off[b];  // (room for off[G] - off[0])
             int32_t slots = 0, chunks = 0;
-            for (int32_t g = 0; g < G; ++g) {
-                if (cfg[g] < 0 || cfg[g] >= C) {
+            h_ng[b] = (uint8_t)G;
+            for (int32_t g = 0; g < Gmax; ++g) {
+                h_cfg[(size_t)b * Gmax + g] = g < G ? (uint8_t)cfg[g] : 0;
+                if (g >= G) continue;
+                if (cfg[g] < 0 || cfg[g] >= C || off[g + 1] < off[g] || off[g + 1] > off[G]) {
                     bad = true;
                     return;
                 }
@@ -114,16 +168,17 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
                 mine.pow2 = mine.pow2 && (pp & (pp - 1)) == 0;
                 mine.smax = std::max(mine.smax, pp);
                 mine.depths += (off[g + 1] - off[g]) * pp;
-            }
-            for (int64_t x = off[0]; x < off[G]; ++x) {
-                const int32_t m = p->gm_idx[x];
-                if (m < 0 || m >= M || count[m] >= MMSIM_MAX_REPLICAS) {
-                    bad = true;
-                    return;
+                for (int64_t x = off[g]; x < off[g + 1]; ++x) {
+                    const int32_t m = p->gm_idx[x];
+                    if (m < 0 || m >= M || count[m] >= MMSIM_MAX_REPLICAS) {
+                        bad = true;
+                        return;
+                    }
+                    *ent++ = (uint32_t)m | (uint32_t)g << 16;
+                    chunks += count[m] >= 4 && (count[m] & 3) == 0;
+                    count[m] += 1;
+                    mine.rmax = std::max<int32_t>(mine.rmax, count[m]);
                 }
-                chunks += count[m] >= 4 && (count[m] & 3) == 0;
-                count[m] += 1;
-                mine.rmax = std::max<int32_t>(mine.rmax, count[m]);
             }
             if (slots > MMSIM_MAX_SLOTS) {
                 bad = true;
@@ -131,7 +186,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             }
             mine.nslots = std::max(mine.nslots, slots);
             mine.ext_cap = std::max(mine.ext_cap, chunks);
-            for (int64_t x = off[0]; x < off[G]; ++x) count[p->gm_idx[x]] = 0;
+            for (const uint32_t *e = h_ent + h_off[b]; e < ent; ++e) count[*e & 0xFFFFu] = 0;
         }
         std::lock_guard<std::mutex> lock(shape_mutex);
         shape.nslots = std::max(shape.nslots, mine.nslots);
@@ -150,7 +205,6 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     if (a.smax_bucket < 0) return kOther;
     const bool uniform = cl.uniform || a.smax_bucket == 1;
     const bool counts = has_outputs(flags);
-    const int group_words = (Gmax + 31) / 32;
     // (behind the clocks as many slots as a walk has stages, for reads and writes that do not count)
     size_t place = up16(((size_t)shape.nslots + a.smax_bucket) * 8 * (counts ? 3 : 2));
     a.o_rep = (int32_t)place;
@@ -165,10 +219,9 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     place = up16(place + ((size_t)Gmax + 1) * 4);
     a.o_mcnt = (int32_t)place;
     place = up16(place + (counts ? (size_t)M * 4 : 0));
-    const size_t lds = (size_t)ctx->max_lds, lat_bytes = uniform ? 0 : up16(cl.lat.size() * sizeof(float));
+    const size_t lat_bytes = uniform ? 0 : up16(cl.lat.size() * sizeof(float));
     if (place > lds) return kOther;
     const size_t lat_lds = lat_bytes + place <= lds ? lat_bytes : 0;
-    const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
     auto wave_lds = [&](int lanes) { return place * (size_t)(kWave / lanes) + (size_t)window_ring_bytes(lanes); };
     auto fits = [&](int lanes) { return lat_lds + wave_lds(lanes) <= lds; };
     auto waves_for = [&](int l) {  // wavefronts of a workgroup
@@ -193,26 +246,28 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         // 8192: 14.7 / 9.9 / 7.1 / 5.9; 1 to 8 stages (3.2), 12288: 7.5 / 6.3 / 5.1 / 8.7 against 5.7.  Depths other than
         // 1, 2, 4, 8 and 16 are slow in the other kernel (6.4 and 12 stages, 12288: 11.7 / 9.7 / 7.7 / 12.2 against 10.7),
         // and paired batches fill its tiles with what one stream has.
-        const double depth = (shape.smax + (replicas > 0 ? (double)shape.depths / (double)replicas : 1.0)) / 2;
-        const bool any_depth = stream_of || !shape.pow2 || shape.smax > 16;
+        const double mean = replicas > 0 ? (double)shape.depths / (double)replicas : 1.0, depth = (shape.smax + mean) / 2;
+        const bool any_depth = packing_counts || stream_of || !shape.pow2 || shape.smax > 16;
         if (sims > (any_depth || depth <= 6 ? kMaxWindowSims : depth <= 10 ? 8192 : 4096)) return kOther;
+        // More than LDS holds at once: the wavefronts with one placement each, which follow one another freely (8192 of 300
+        // models: 2.1 / 3.0 / 4.8 / 7.7 against 4.6; of 128 models, at worst, 5.7 / 5.1 / 5.8 / 7.3 against 5.2; 12288: 3.0 to
+        // 8.5 against 4.5 to 6.1), but narrower ones with deep groups, whose steps are long.
         lanes = kWave;
-        if (sims > at_once(kWave)) {
-            // More than LDS holds at once: the wavefronts with one placement each, which follow one another freely (8192 of
-            // 300 models: 2.1 / 3.0 / 4.8 / 7.7 against 4.6; of 128 models, at worst, 5.7 / 5.1 / 5.8 / 7.3 against 5.2; 12288:
-            // 3.0 to 8.5 against 4.5 to 6.1).
-            if (sims > 8192 || !fits(kWave)) return kOther;
-        } else {
+        const bool rounds = sims > at_once(kWave);
+        if (rounds && (sims > most_in_rounds || !fits(kWave))) return kOther;
+        // (12288 16-stage pipelines of 64 models: 3000 requests 2.7 against 9.1 with the packing, 12000: 9.7 / 13.5, 50000: 37 / 31)
+        if (rounds && depth > 10 && shape.pow2 && shape.smax <= 16 && !g_arena && (int64_t)B * M < 20 * longest) return kOther;
+        if (!rounds || depth > 10) {
             // As many requests side by side as leave three wavefronts to a SIMD (the registers of the kernels for up to 16
             // stages hold three or four), four of the single-stage kernel, two of deep groups.  Four-stage pipelines, 3000:
             // 3.6 / 4.2 / 4.5 / 5.6, 6000: 5.6 / 4.9 / 5.7 / 6.2, 12288: 10.2 / 9.3 / 7.2 / 7.8; single stages, 4096: 2.6 / 2.8
-            // / 3.8 / 5.0, 8192: 4.5 / 4.2 / 4.4 / 5.7; 32-stage pipelines, 12288: 45 / 29 / 19 / 15 against 25.
-            // A narrower wavefront needs more LDS, for its placements and for the requests on their way to them: where it would
-            // take two rounds, up to twice as many wavefronts stay (5000 placements of 128 models, 5.1 / 6.4), unless the
-            // groups are deep (11000 32-stage pipelines, in two rounds either way, 16 lanes 26, 8 lanes 24).
-            const int64_t most = (a.smax_bucket == 1 ? 16 : depth <= 10 ? 12 : 8) * cus;
+            // / 3.8 / 5.0, 8192: 4.5 / 4.2 / 4.4 / 5.7; eight-stage pipelines, 12288: 14.8 / 10.0 / 6.9 / 6.1; 32-stage ones 45 / 29
+            // / 19 / 15.  A narrower wavefront needs more LDS, for its placements and for the requests on their way to them:
+            // where it would take two rounds instead of one, up to twice as many wavefronts stay (5000 placements of 128
+            // models, 5.1 / 6.4).
+            const int64_t most = (a.smax_bucket == 1 ? 16 : mean > 7 ? 8 : 12) * cus;
             while (lanes > 8 && sims * lanes / kWave > most && fits(lanes / 2) &&
-                   (sims <= at_once(lanes / 2) || sims * lanes / kWave > 2 * most || depth > 10))
+                   (sims <= at_once(lanes / 2) || sims * lanes / kWave > 2 * most || (depth > 10 && sims > at_once(lanes))))
                 lanes /= 2;
         }
     }
@@ -221,52 +276,6 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     if (!fits(lanes)) return kOther;
     const int per_wave = kWave / lanes, waves = waves_for(lanes);
     const int64_t tiles = (B + per_wave - 1) / per_wave, units = tiles * out_seeds;
-
-    // ---- inputs: one buffer
-    Layout in;
-    const size_t at_ptr = in.take(sizeof(void *) * (size_t)n_seeds), at_len = in.take(sizeof(int64_t) * (size_t)n_seeds);
-    const size_t at_so = in.take(stream_of ? sizeof(int32_t) * (size_t)B : 0);
-    const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
-    const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
-    const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
-    HIP_TRY(hipSetDevice(ctx->device));
-    std::vector<unsigned char> plain;  // (read until the wait below)
-    if (g_arena)
-        plain.resize(in.used);
-    else
-        HIP_TRY(ctx->staging.ensure(in.used));
-    struct Trim {  // the memory of a batch that is not made after all
-        Staging *staging;
-        hipStream_t stream;
-        ~Trim() {
-            if (!staging) return;
-            if (staging->n > Staging::kMost) (void)hipStreamSynchronize(stream);  // (the inputs may be on their way out of it)
-            staging->trim();
-        }
-    } unless_made{g_arena ? nullptr : &ctx->staging, ctx->stream};
-    unsigned char *host = g_arena ? plain.data() : ctx->staging.p;
-    uint32_t *h_off = reinterpret_cast<uint32_t *>(host + at_off);
-    {
-        uint32_t at = 0;
-        for (int32_t b = 0; b < B; ++b) {
-            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-            h_off[b] = at;
-            at += (uint32_t)(off[p->num_groups[b]] - off[0]);
-        }
-        h_off[B] = at;
-    }
-    parallel_slices(B, 1024, [&](int64_t b0, int64_t b1) {
-        for (int64_t b = b0; b < b1; ++b) {
-            const int32_t G = p->num_groups[b];
-            const int64_t *off = p->gm_off + (size_t)b * (Gmax + 1);
-            uint8_t *cfg = host + at_cfg + (size_t)b * Gmax;
-            uint32_t *ent = reinterpret_cast<uint32_t *>(host + at_ent) + h_off[b];
-            host[at_ng + (size_t)b] = (uint8_t)G;
-            for (int32_t g = 0; g < Gmax; ++g) cfg[g] = g < G ? (uint8_t)p->group_cfg[(size_t)b * Gmax + g] : 0;
-            for (int32_t g = 0; g < G; ++g)
-                for (int64_t x = off[g]; x < off[g + 1]; ++x) *ent++ = (uint32_t)p->gm_idx[x] | (uint32_t)g << 16;
-        }
-    });
 
     std::unique_ptr<mmsim_batch> b(new (std::nothrow) mmsim_batch);
     if (!b) return fail(MMSIM_E_NOMEM, "host allocation failed");

@@ -85,6 +85,24 @@ def test_static_entry_point_refuses_what_does_not_fit():
     _same(got, ref, "after a refusal")
 
 
+def test_static_entry_point_takes_large_batches_of_small_tables():
+    """9900 placements of 100 models in eight-stage groups: the kernel with requests side by side takes them in 2 MB, the
+    tables of the others would not fit the scratch beside their results."""
+    from mms_amd.placement_policy.base_policy import ModelPlacement
+    from mms_amd.profiling import ParallelConfig, synthetic_profile
+    eng = E.Engine.default()
+    M, pc = 100, ParallelConfig(1, 1, 8)
+    table = E.LatencyTable([synthetic_profile(f"m{m}", 0.1 + 0.001 * m, [pc]) for m in range(M)], [1])
+    rng = np.random.default_rng(1)
+    sols = [ModelPlacement([pc, pc], [rng.choice(M, 5, replace=False).tolist() for _ in range(2)]) for _ in range(100)]
+    packed = E.pack_placements([sols[b % 100] for b in range(9900)], table)
+    dw = [E.DeviceWorkload(eng, np.cumsum(rng.exponential(0.002, 500)), rng.integers(0, M, 500).astype(np.int32),
+                           np.full(500, 0.5, np.float32), M)]
+    got = E.eval_batch(eng, dw, table, packed, 0, static=True)
+    _same(got, E.eval_batch(eng, dw, table, packed, 0), "100 models")
+    _same({k: v[:, :100] for k, v in got.items()}, E.eval_batch(eng, dw, table, E.pack_placements(sols, table)), "the first hundred")
+
+
 _COUNT = """
 import ctypes, json, sys
 counter = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)      # before the library, so that its calls come here
