@@ -20,7 +20,8 @@ OBJ_DIR = os.path.join(HERE, "build")
 # instances are many; four translation units build in parallel).
 UNITS = {"mmsim_api": ("mmsim_api.hip", []), "window_batch": ("window_batch.hip", []),
          **{f"sim_window_{w}": ("sim_window.hip", [f"-DMMSIM_WINDOW_LANES={w}"]) for w in (64, 32, 16, 8)},
-         "sim_mixed": ("sim_mixed.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_scalar": ("sim_scalar.hip", []),
+         "sim_mixed": ("sim_mixed.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_batching_solo": ("sim_batching_solo.hip", []),
+         "sim_scalar": ("sim_scalar.hip", []),
          "stats": ("stats.hip", [])}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -47,6 +48,7 @@ FLAGS = [
 # blocks as well 2.70 / 4.13 / 2.90 / 4.71 / 2.16, with these alone no change; iterative-ilp fails on it.
 SOURCE_FLAGS = {"sim_window.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
+                "sim_batching_solo.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_batching.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"]}
 
 

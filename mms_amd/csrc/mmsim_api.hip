@@ -875,6 +875,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     std::vector<uint16_t> g2m_off, g2m_idx;
     std::vector<float> lat_nb;
     int members_max = 1;
+    bool g2m_ascending = true;  // every group lists its models in ascending order, each once
     if (batching) {
         b->hosted.assign((size_t)B * M, 0);
         std::vector<std::vector<int32_t>> lists(Gmax);
@@ -886,6 +887,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (!rl.g2m_off.empty())
                     dst.assign(rl.g2m_m.begin() + rl.g2m_off[(size_t)p * Gmax + g], rl.g2m_m.begin() + rl.g2m_off[(size_t)p * Gmax + g + 1]);
                 total += dst.size();
+                for (size_t x = 1; x < dst.size(); ++x) g2m_ascending = g2m_ascending && dst[x] > dst[x - 1];
             }
             for (int32_t m = 0; m < M; ++m) {
                 const int64_t lo = rl.off[(size_t)p * M + m], hi = rl.off[(size_t)p * M + m + 1];
@@ -931,9 +933,10 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     //      idle SIMD loses more than one that reads these tables through the caches.
     size_t batching_lat_lds = 0;
     int batching_g2m_lds = 0;
+    const bool solo = batching && blanes == 8 && tile_sims == 1 && g2m_ascending && batching_solo_fits(M, t->NB, heap_cap, Gmax);
     if (batching) {
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
-        const size_t g2m_b = ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
+        const size_t g2m_b = solo ? 0 : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
         const size_t cap = (size_t)ctx->max_lds;
         // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
         const int tiles_here = std::max(1, b->tiles);
@@ -941,12 +944,12 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         const int wanted = (int)std::min<int64_t>(2 * kMaxWavesPerBlockBatching, std::max<int64_t>(1, ((int64_t)b->waves + cus - 1) / cus));
         // Fewer event slots (down to G+8) are accepted when that puts more wavefronts on a CU.
         const int wpb_max = kMaxWavesPerBlockBatching;
-        const int heap_try_min = std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7));
+        const int heap_try_min = solo ? heap_cap : std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7));  // (its event slots are registers)
         int best_w = 0, best_total = 0, best_heap = heap_cap;
         // option batching_lds_tables (bit 0: latency table, bit 1: group lists) fixes which tables may go to LDS
         const int allowed = o.batching_lds_tables >= 0 ? (o.batching_lds_tables & 3) : 3;
         for (int hc = heap_cap; hc >= heap_try_min; hc -= 8) {
-            const size_t wb = batching_bytes_for(blanes, hc);
+            const size_t wb = solo ? batching_solo_bytes(nslots, M) : batching_bytes_for(blanes, hc);
             for (int per_cu = 1; per_cu <= 2; ++per_cu)  // workgroups meant to share a CU (each gets that share of LDS)
                 for (int opt = 0; opt < 4; ++opt) {      // both, lists only, table only, neither: the first that gives most wavefronts
                     // (the lists before the table: a selection reads them in two dependent steps, while the table is
@@ -966,7 +969,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 }
         }
         heap_cap = best_heap;
-        wave_bytes = batching_bytes_for(blanes, heap_cap);
+        wave_bytes = solo ? batching_solo_bytes(nslots, M) : batching_bytes_for(blanes, heap_cap);
         wpb = std::max(1, best_w);
         if (batching_g2m_lds) wave_bytes += g2m_b;
         b->waves_per_block = std::min(wpb, b->tiles);
@@ -1178,6 +1181,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         q.g2m_in_lds = batching_g2m_lds;
         q.lane_stride = blanes;
         q.tile_sims = tile_sims;
+        q.solo = solo ? 1 : 0;
         q.uniform_stages = uniform_stages ? 1 : 0;
         q.tile_seed = b->tile_seed.p;
         q.paired = b->paired ? 1 : 0;

@@ -186,6 +186,7 @@ struct BatchingArgs {
     int32_t g2m_in_lds;          // 1: each wavefront keeps its g2m_off / g2m_idx rows in LDS
     int32_t lane_stride;         // 64, 32, 16 or 8 (octets): lanes of a wavefront that simulate; pitch of the per-lane LDS arrays
     int32_t tile_sims;           // simulations of a tile: lane_stride, or fewer in an octet tile (1, 2 or 4)
+    int32_t solo;                // 1: tile_sims is 1 and the kernel for one simulation to a wavefront runs
     int32_t uniform_stages;      // 1: a configuration's stages all have the same latencies and lat holds them once ([M][lat_row][NB], one row per configuration)
     const int32_t *tile_seed;    // as in MixedArgs
     int32_t paired;
@@ -295,6 +296,11 @@ constexpr int64_t kStatsScratchBytes = (int64_t)1 << 30;  // scratch rows of one
 
 hipError_t launch_sim_scalar(const ScalarArgs &args, hipStream_t stream, std::string *err);
 
+// One simulation to a wavefront (sim_batching_solo.hip), for tables, event slots and models that its lanes hold.
+constexpr bool batching_solo_fits(int M, int NB, int heap_cap, int Gmax) { return M <= 512 && NB <= 8 && heap_cap <= 64 && Gmax <= 64; }
+constexpr size_t batching_solo_bytes(int nslots, int M) { return (size_t)((nslots + 4) & ~1) * 8 + (size_t)M * 16; }  // LDS of a wavefront (three clocks more than there are)
+hipError_t launch_sim_batching_solo(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream);
+std::string sim_batching_solo_kernel_name(const BatchingArgs &args);
 hipError_t launch_sim_batching(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream,
                                std::string *err);
 

@@ -14,7 +14,8 @@
 // by an octet of lanes that hold the same state, take the same branches and
 // split the scans among them.  Batches that leave the chip room put 4, 2 or 1
 // simulations into such a wavefront instead of 8 (BatchingArgs::tile_sims): the
-// events of its octets then wait for fewer others.
+// events of its octets then wait for fewer others.  (One simulation: sim_batching_solo.hip,
+// where its tables fit the lanes.)
 //
 // State of a lane:
 //   * stage clocks clk[slot][lane] in LDS, as in the plain simulator; a
@@ -151,10 +152,7 @@ __device__ __forceinline__ lds_vu32 *as_lds_vu32(void *p) { return (lds_vu32 *)p
 // SH (octets only): at most 64 event slots per simulation.  Which slots are in use is a 64-bit mask in registers
 // and lane c of an octet keeps the earliest time of chunk c in a register: neither the free-slot stack nor the
 // chunk minima are read from LDS.
-// SOLO (octets only): one simulation to a wavefront.  All octets hold its state and do the same, except that
-// each looks at an arrival of its own: eight arrivals are looked at in the time of one, and those at which nothing
-// happens but a place in a queue (three in four on the benchmark's bursty streams) cost no more than that.
-template <int NBT, bool LATLDS, bool G2MLDS, bool OCT, bool UNIF, bool SH, bool SOLO>
+template <int NBT, bool LATLDS, bool G2MLDS, bool OCT, bool UNIF, bool SH>
 __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching_kernel(const BatchingArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
 
@@ -172,7 +170,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     // simulations per wavefront (64, 32, 16 or 8): pitch of the per-simulation LDS arrays.  Octets mean 8: a constant
     // there, so that the index arithmetic is shifts, not multiplications
     const int LS = OCT ? 8 : a.lane_stride;
-    const int sl = SOLO ? 0 : OCT ? lane >> 3 : lane;  // this lane's simulation within the tile
+    const int sl = OCT ? lane >> 3 : lane;  // this lane's simulation within the tile
     const int oj = OCT ? lane & 7 : 0;      // this lane's place in its octet
     const int fill = OCT ? kWave : LS;      // lanes that fill the wavefront's shared LDS arrays
 
@@ -282,8 +280,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     double *fin_out = a.finish + (size_t)wave * a.Rmax * kWave + sl;
     uint8_t *good_out = a.good + (size_t)wave * a.Rmax * kWave + sl;
     const double overhead = a.fixed_overhead;
-
-    auto arrived_of = [&](int mx) { return (__attribute__((address_space(3))) uint32_t *)(arrived + mx); };
 
     int32_t n_good = 0;
     double lat_sum = 0.0;
@@ -858,101 +854,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         }
     };
 
-    if constexpr (SOLO) {
-        // Windows of eight arrivals, one to an octet.  A look at a window finds the first arrival at which something
-        // happens: an event is due, or its group is idle.  Those before it only join their queues; then it is dealt
-        // with, by all octets, and the rest of the window is looked at again, since clocks have changed.  Requests
-        // are fetched a block ahead, replica rows a window ahead.
-        const int oct = lane >> 3;
-        auto fetch_block = [&](int64_t i) -> Req {
-            Req r = {0.0, -1, 0.0f};
-            if (i + lane < R) r = reqs[i + lane];
-            return r;
-        };
-        auto row_word = [&](int mx) -> uint32_t { return repd_tile[(size_t)(mx < 0 ? 0 : mx) * row_lanes]; };
-        blk_req = fetch_block(0);
-        Req blk_next = fetch_block(kWave);
-        int m_next = __shfl(blk_req.m, oct);
-        uint32_t d_next = row_word(m_next);
-        for (int64_t w0 = 0; w0 < R && !dead; w0 += 8) {
-            const int from = (int)(w0 & 63) + oct;  // the lane that holds this octet's request
-            const int m = m_next;
-            const uint32_t dj = d_next;
-            const double t = __hiloint2double(__shfl(__double2hiint(blk_req.t), from), __shfl(__double2loint(blk_req.t), from));
-            if ((w0 & 63) == 56) {
-                blk_req = blk_next;
-                blk_next = fetch_block(w0 + 8 + kWave);
-            }
-            m_next = __shfl(blk_req.m, (from + 8) & 63);  // (past the end of the stream: -1)
-            d_next = row_word(m_next);
-            const bool in = w0 + oct < R;
-            const bool valid = (int32_t)dj >= 0 && m >= 0;
-            const uint32_t vb = oct_ballot(valid);
-            const bool hosted = (vb & 1u) != 0, longer = (vb >> 7) != 0;  // longer: the list may go on
-            const uint32_t last = desc_last_slot(dj), first = last - desc_stages_m1(dj);
-            int cur = 0;      // octets before this one are settled
-            int seen_due = -1;  // the octet whose due events have been seen to
-            for (;;) {
-                const double c = clk[last * LS], cf = clk[first * LS];  // slot 0 for a lane without a replica: not used
-                const double mn = oct_min(valid ? c : __builtin_inf());
-                int selj = __ffs((int)oct_ballot(valid && c == mn)) - 1;
-                const bool found = hosted && mn < 1e100;
-                const bool idle = found && ((oct_ballot(t >= cf) >> (selj & 7)) & 1u) != 0;
-                const bool happens = in && oct >= cur && ((next_due <= t && oct > seen_due) || idle || (hosted && (!found || longer)));
-                const uint64_t hb = __builtin_amdgcn_ballot_w64(happens);
-                const int f = hb != 0ull ? (__ffsll((long long)hb) - 1) >> 3 : 8;
-                if (in && oct >= cur && oct < f && oj == 0 && m >= 0)
-                    __hip_atomic_fetch_add(arrived_of(m), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                if (want_req && in && oct >= cur && oct < f && oj == 0 && !hosted) {
-                    fin_out[(size_t)(w0 + oct) * kWave] = t;
-                    good_out[(size_t)(w0 + oct) * kWave] = 0;
-                }
-                __builtin_amdgcn_wave_barrier();
-                if (f == 8) break;
-                cur = f;
-                const int fl = f << 3;
-                const double tf = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(t), fl), __builtin_amdgcn_readlane(__double2loint(t), fl));
-                if (next_due <= tf && f > seen_due) {  // events first; the arrival is looked at again after them
-                    due_events(tf);
-                    seen_due = f;
-                    if (dead) break;
-                    continue;
-                }
-                const int mf = __builtin_amdgcn_readlane(m, fl);
-                const double best0 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(mn), fl), __builtin_amdgcn_readlane(__double2loint(mn), fl));
-                double best = best0 < 1e100 ? best0 : 1e100;
-                uint32_t dsel = kEmpty;
-                bool ready = __builtin_amdgcn_readlane((int)idle, fl) != 0;
-                if (__builtin_amdgcn_readlane((int)found, fl) != 0)
-                    dsel = (uint32_t)__builtin_amdgcn_readlane((int)dj, fl + __builtin_amdgcn_readlane(selj, fl));
-                if (__builtin_amdgcn_readlane((int)longer, fl) != 0)
-                    for (int x = 0; x < a.rep_extra; ++x) {
-                        const uint32_t g = repx_tile[((size_t)mf * a.rep_extra + x) * kWave];
-                        if (g == none) break;
-                        const uint32_t d2 = a.ginfo[((size_t)tile * (Gmax + 1) + g) * kWave];
-                        const double c2 = clk[desc_last_slot(d2) * LS];
-                        if (c2 < best) {
-                            best = c2;
-                            dsel = d2;
-                            ready = tf >= clk[(desc_last_slot(d2) - desc_stages_m1(d2)) * LS];
-                        }
-                    }
-                const uint32_t so_far = arrived[mf];
-                __builtin_amdgcn_wave_barrier();
-                arrived[mf] = so_far + 1u;  // (every lane writes the same)
-                __builtin_amdgcn_wave_barrier();
-                cur = f + 1;
-                if (dsel == kEmpty) {  // every replica's clock is infinite (see below)
-                    dead = MMSIM_E_UNSUPPORTED;
-                    break;
-                }
-                if (ready) {
-                    handle(tf, mf, dsel);
-                    if (dead) break;
-                }
-            }
-        }
-    } else {
     for (int64_t i0 = 0; i0 < R; i0 += kWave) {
     {
         const int64_t at = i0 + lane < R ? i0 + lane : R - 1;
@@ -1101,7 +1002,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         }
     }
     }
-    }
     // ---- drain (:781-787)
     while (!dead && nfree < a.heap_cap) {
         double ti, others;
@@ -1122,9 +1022,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     }
 }
 
-// One simulation to a wavefront: the kernel in which each octet looks at an arrival of its own.
-bool batching_solo(const BatchingArgs &a) { return a.lane_stride == 8 && a.tile_sims == 1 && a.heap_cap <= 64 && a.NB <= 8; }
-
 }  // namespace
 
 hipError_t launch_sim_batching(const BatchingArgs &args, int wpb, size_t lds_bytes, hipStream_t stream,
@@ -1132,25 +1029,25 @@ hipError_t launch_sim_batching(const BatchingArgs &args, int wpb, size_t lds_byt
     hipError_t e = hipSuccess;
     if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.NB > kMaxLatencyColumns || (args.heap_cap & 7) != 0) {
         e = hipErrorInvalidValue;
+    } else if (args.solo) {
+        e = launch_sim_batching_solo(args, wpb, lds_bytes, stream);
     } else {
         const bool ll = args.lat_lds_bytes > 0, gl = args.g2m_in_lds != 0;
         const bool oct = args.lane_stride == 8, unif = args.uniform_stages != 0;
-        const bool small_heap = oct && args.heap_cap <= 64, solo = batching_solo(args);
+        const bool small_heap = oct && args.heap_cap <= 64;
         void (*kern)(const BatchingArgs) = nullptr;
-#define MMSIM_PICK4(NBT, O, U, S, SOLO)                                                                                     \
-    (ll ? (gl ? sim_batching_kernel<NBT, true, true, O, U, S, SOLO> : sim_batching_kernel<NBT, true, false, O, U, S, SOLO>) \
-        : (gl ? sim_batching_kernel<NBT, false, true, O, U, S, SOLO> : sim_batching_kernel<NBT, false, false, O, U, S, SOLO>))
-#define MMSIM_PICK3(NBT, O, S, SOLO) (unif ? MMSIM_PICK4(NBT, O, true, S, SOLO) : MMSIM_PICK4(NBT, O, false, S, SOLO))
-#define MMSIM_PICK(NBT, SOLO)                                                                                           \
-    kern = !oct         ? MMSIM_PICK3(NBT, false, false, false)                                                         \
-           : small_heap ? (SOLO && solo ? MMSIM_PICK3(NBT, true, true, SOLO) : MMSIM_PICK3(NBT, true, true, false))     \
-                        : MMSIM_PICK3(NBT, true, false, false)
+#define MMSIM_PICK4(NBT, O, U, S)                                                                              \
+    (ll ? (gl ? sim_batching_kernel<NBT, true, true, O, U, S> : sim_batching_kernel<NBT, true, false, O, U, S>) \
+        : (gl ? sim_batching_kernel<NBT, false, true, O, U, S> : sim_batching_kernel<NBT, false, false, O, U, S>))
+#define MMSIM_PICK3(NBT, O, S) (unif ? MMSIM_PICK4(NBT, O, true, S) : MMSIM_PICK4(NBT, O, false, S))
+#define MMSIM_PICK(NBT) \
+    kern = !oct ? MMSIM_PICK3(NBT, false, false) : small_heap ? MMSIM_PICK3(NBT, true, true) : MMSIM_PICK3(NBT, true, false)
         if (args.NB <= 4)
-            MMSIM_PICK(4, true);
+            MMSIM_PICK(4);
         else if (args.NB <= 8)
-            MMSIM_PICK(8, true);
+            MMSIM_PICK(8);
         else
-            MMSIM_PICK(16, false);
+            MMSIM_PICK(16);
 #undef MMSIM_PICK
 #undef MMSIM_PICK3
 #undef MMSIM_PICK4
@@ -1169,11 +1066,12 @@ hipError_t launch_sim_batching(const BatchingArgs &args, int wpb, size_t lds_byt
 
 // The template instance launch_sim_batching picks for these arguments, as profilers print it.
 std::string sim_batching_kernel_name(const BatchingArgs &args) {
+    if (args.solo) return sim_batching_solo_kernel_name(args);
     const int nbt = args.NB <= 4 ? 4 : args.NB <= 8 ? 8 : 16;
     auto tf = [](bool v) { return v ? "true" : "false"; };
     return "sim_batching_kernel<" + std::to_string(nbt) + ", " + tf(args.lat_lds_bytes > 0) + ", " + tf(args.g2m_in_lds != 0) +
            ", " + tf(args.lane_stride == 8) + ", " + tf(args.uniform_stages != 0) + ", " +
-           tf(args.lane_stride == 8 && args.heap_cap <= 64) + ", " + tf(batching_solo(args)) + ">";
+           tf(args.lane_stride == 8 && args.heap_cap <= 64) + ">";
 }
 
 }  // namespace mmsim

@@ -1,0 +1,558 @@
+// Batching request-loop simulation for gfx950, one simulation to a wavefront.
+//
+// The same loop as sim_batching.hip (simulate_requests_mixed_batching, alpa_serve/simulator/controller.py:631-798), for
+// batches that leave the chip room for a wavefront per simulation.  There is one flow of control, so what it turns on is
+// scalar, and the lanes hold what it looks things up in, in registers:
+//
+//   lane e  event slot e: time and group of a pending idle event (:728, :739-740).  The earliest is found by comparing
+//           all lanes with the earliest time, which is kept exact (one minimum over the wavefront when an event is
+//           taken, none when one is added).
+//   lane g  the models of group g, a bit per model.  Which models have waiting requests is a scalar mask, so whether
+//           a group that became idle has anything to do is one AND, and only when several of its models wait are
+//           the ranks of their heads looked at (:654-664).
+//   lane j  entry j of the queue a batch is taken from, sixteen of them, and latency column j (:666-704).
+//
+// Latency sums are kept by place in the queue, as the octets there keep them, so that they are equal bit for bit.
+//
+// Arrivals are looked at eight at a time, one to an octet of lanes (lane 8 i + j: the j-th replica of arrival i's model):
+// those at which nothing happens but a place in a queue cost no more than that.  Events that are due are seen to before
+// an arrival is looked at, since the clocks it is judged by may change.
+//
+// What bounds it: one dependent chain per event or arrival, on a wavefront that has its SIMD to itself: instructions
+// (4 cycles each, whatever they do), a taken branch (20 to 30 cycles until the instructions at its target are there), and
+// two trips to LDS and one to memory per batch.  Hence masks in scalars and look-ups in registers instead of lists in
+// LDS, clocks of the window's replicas kept in registers as they change, and paths laid out so that what happens most falls
+// through.  30000 requests, 48 models on 24 devices, 128 placements: 25.0 ms with the octets of sim_batching.hip each
+// looking at an arrival of its own (per arrival 226 instructions, 18 of them branches, 1746 cycles), 15.7 ms here (155, 14,
+// 1123).  Tried, no gain: the queue entries of arrivals touched a window ahead (20.4 / 20.5 ms at the time).
+//
+// LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: where
+// its arrivals start in the stream's lists, head, arrivals so far, rank of the head.
+#include "mmsim_internal.h"
+
+namespace mmsim {
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ T lds_get(uint32_t addr) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) T *>(addr);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(uint32_t addr, T v) {
+    *reinterpret_cast<__attribute__((address_space(3))) T *>(addr) = v;
+}
+// Marks the places where the lanes' LDS accesses depend on one another (a wavefront's LDS accesses are carried out in
+// order; no instruction).
+__device__ __forceinline__ void wave_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bool rarely(bool p) { return __builtin_expect(p, 0); }  // (a branch that is not taken costs little)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ int first_of(uint64_t lanes) { return __builtin_ctzll(lanes); }  // (lanes: not 0)
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ double uni(double v) { return __hiloint2double(uni(__double2hiint(v)), uni(__double2loint(v))); }
+__device__ __forceinline__ int lane_value(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
+__device__ __forceinline__ float lane_value(float v, int l) { return __uint_as_float(lane_value(__float_as_uint(v), l)); }
+__device__ __forceinline__ double lane_value(double v, int l) {
+    return __hiloint2double(lane_value(__double2hiint(v), l), lane_value(__double2loint(v), l));
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int l) {
+    return (uint64_t)lane_value((uint32_t)(v >> 32), l) << 32 | lane_value((uint32_t)v, l);
+}
+__device__ __forceinline__ double max_nn(double x, double y) {  // neither is NaN: no input quieting
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+__device__ __forceinline__ int ilog2i(int v) { return 31 - __clz(v); }
+
+// bit j = the predicate of lane j of the octet
+__device__ __forceinline__ uint32_t oct_ballot(bool p) { return (uint32_t)(ballot(p) >> (threadIdx.x & 56u)) & 0xFFu; }
+// Smallest value of the octet, in all of its lanes; of the wavefront, as a scalar.  A DPP operand needs two wait states
+// after the write of its register (s_nop 1).  All lanes must be active.
+__device__ __forceinline__ uint32_t oct_min(uint32_t v) {
+    asm("s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+    asm volatile(
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n"
+        "s_nop 1\n"
+        "v_min_u32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n"
+        "s_nop 1\n"
+        : "+v"(v));
+    return lane_value(v, 63);
+}
+// Doubles that are never negative nor NaN order as their bit patterns do: the smallest high word, then the smallest low
+// word among the lanes that have it (clocks and event times start at +0 and only grow; +inf is allowed).
+__device__ __forceinline__ double oct_min(double v) {
+    const uint32_t hi = (uint32_t)__double2hiint(v), mh = oct_min(hi);
+    const uint32_t ml = oct_min(hi == mh ? (uint32_t)__double2loint(v) : 0xFFFFFFFFu);
+    return __hiloint2double((int)mh, (int)ml);
+}
+__device__ __forceinline__ double wave_min(double v) {
+    const uint32_t hi = (uint32_t)__double2hiint(v), lo = (uint32_t)__double2loint(v), mh = wave_min(hi);
+    const uint64_t at = ballot(hi == mh);
+    uint32_t ml = lane_value(lo, first_of(at));
+    if (rarely((at & (at - 1)) != 0)) ml = wave_min(hi == mh ? lo : 0xFFFFFFFFu);
+    return __hiloint2double((int)mh, (int)ml);
+}
+
+// LATLDS: the latency table is in LDS.  UNIF: every (model,
+// configuration) has the same latencies in all of its stages, held once.  OUTPUTS: anything beyond the scores (a.flags
+// says what).  MW: 64-bit words that hold a bit per model.
+template <bool LATLDS, bool UNIF, bool OUTPUTS, int MW>
+__global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching_solo_kernel(const BatchingArgs a) {
+    const int lane = (int)(threadIdx.x & 63), oct = lane >> 3;
+    const int wv = uni((int)(threadIdx.x >> 6));
+    const unsigned grid_seeds = a.paired ? 1u : (unsigned)a.n_seeds;
+    const int tile = (int)(blockIdx.x / grid_seeds) * (int)(blockDim.x >> 6) + wv;
+    const int M = a.M, NB = a.NB;
+    if (LATLDS) {
+        const int n = M * a.lat_row * NB;
+        for (int i = (int)threadIdx.x; i < n; i += (int)blockDim.x) lds_put<float>((uint32_t)i * 4u, a.lat[i]);
+        __syncthreads();
+    }
+    if (tile >= a.tiles) return;
+    // paired batches: the tile's own stream; otherwise every tile on every stream
+    const int seed = a.paired ? a.tile_seed[tile] : (int)(blockIdx.x % grid_seeds);
+    const bool want_model = OUTPUTS && (a.flags & MMSIM_WANT_MODEL_COUNTS) != 0;
+    const bool want_group = OUTPUTS && (a.flags & MMSIM_WANT_GROUP_COUNTS) != 0;
+    const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
+    const uint32_t clk = (uint32_t)a.lat_lds_bytes + (uint32_t)wv * (uint32_t)a.wave_lds_bytes;
+    const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {first arrival, head, arrivals so far, rank of the head}
+
+    const int wave = a.paired ? tile : seed * a.tiles + tile;  // where this (tile, stream) pair's results go
+    const int64_t off = a.stream_off[seed], R = a.stream_off[seed + 1] - off;
+    const Req *__restrict__ reqs = a.streams + off;
+    const int64_t *__restrict__ mo = a.mq_off + (size_t)seed * (M + 1);
+    const MqEntry *__restrict__ mq = a.mq + mo[0];
+    const uint32_t *__restrict__ rows = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 8 + (lane & 7);
+    const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra * kWave;
+    const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1) * kWave;
+    int32_t *model_good = a.model_good + (size_t)wave * M * kWave;
+    int32_t *group_req = a.group_req + (size_t)wave * a.Gmax * kWave, *group_good = a.group_good + (size_t)wave * a.Gmax * kWave;
+    double *fin_out = a.finish + (size_t)wave * a.Rmax * kWave;
+    uint8_t *good_out = a.good + (size_t)wave * a.Rmax * kWave;
+    const double overhead = a.fixed_overhead, inf = __builtin_inf();
+    auto lat_at = [&](uint32_t i) -> float { return LATLDS ? lds_get<float>(i * 4u) : a.lat[i]; };
+
+    // ---- state
+    for (int s = lane; s < a.nslots; s += kWave) lds_put<double>(clk + (uint32_t)s * 8u, 0.0);
+    for (int m = lane; m < M; m += kWave)
+        lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{(uint32_t)(mo[m] - mo[0]), 0u, 0u, (uint32_t)a.mq[mo[m]].rank});
+    uint64_t members[MW] = {};  // lane g: models of group g
+    if (lane < a.Gmax) {
+        const uint16_t *first = a.g2m_off + (size_t)tile * (a.Gmax + 1) * kWave + (size_t)lane * kWave;
+        const uint16_t *list = a.g2m_idx + (size_t)tile * a.members_max * kWave;
+        for (int x = first[0]; x < (int)first[kWave]; ++x) {
+            const int m = list[(size_t)x * kWave];
+#pragma unroll
+            for (int i = 0; i < MW; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
+        }
+    }
+    uint64_t waiting[MW] = {};  // models with waiting requests
+    double ev_t = inf;          // lane e: event slot e
+    uint32_t ev_d = 0;
+    uint64_t used = 0;          // event slots that hold an event
+    int nfree = a.heap_cap;
+    double next_due = inf;      // the earliest event's time
+    int32_t n_good = 0;
+    double lat_sum = 0.0;       // of the batch members this lane accounts for
+    int dead = 0;
+    const int cand = a.batch_sizes[lane < NB ? lane : NB - 1], cand_col = ilog2i(cand);  // lane q: batch size q and its latency column
+    const bool sizes_pow2 = ballot(lane < NB && cand != 1 << lane) == 0ull;
+    wave_order();
+
+    // The window of arrivals being looked at: where the lane's replica has its clocks of the last and of the first stage,
+    // and these clocks, kept as they change.  (Lanes without a replica: slot 0, not used.)
+    uint32_t last = clk;
+    double c_last = 0.0, c_first = 0.0;
+
+    auto set_waiting = [&](int m, bool on) {
+#pragma unroll
+        for (int i = 0; i < MW; ++i) {
+            const uint64_t bit = MW == 1 || m >> 6 == i ? 1ull << (m & 63) : 0ull;
+            waiting[i] = on ? waiting[i] | bit : waiting[i] & ~bit;
+        }
+    };
+
+    // :654-664 -- among the models of group g with a waiting request, the one whose head arrived first; of several that
+    // arrived at the same time the first of the (ascending) list
+    auto select_model = [&](uint32_t g) -> int {
+        uint64_t cand[MW];
+        int n = 0, only = -1;
+#pragma unroll
+        for (int i = 0; i < MW; ++i) {
+            cand[i] = waiting[i] & lane_value(members[i], (int)g);
+            n += __builtin_popcountll(cand[i]);
+            if (cand[i] != 0ull) only = 64 * i + first_of(cand[i]);
+        }
+        if (n <= 1) return only;
+        uint32_t rank[MW], least = 0xFFFFFFFFu;
+#pragma unroll
+        for (int i = 0; i < MW; ++i) {
+            rank[i] = 0xFFFFFFFFu;
+            if (cand[i] >> lane & 1ull) rank[i] = lds_get<uint32_t>(queues + (uint32_t)(64 * i + lane) * 16u + 12u);
+            least = rank[i] < least ? rank[i] : least;
+        }
+        least = wave_min(least);
+        int pick = -1;
+#pragma unroll
+        for (int i = MW - 1; i >= 0; --i) {
+            const uint64_t at = ballot(rank[i] == least);
+            if (at != 0ull) pick = 64 * i + first_of(at);
+        }
+        return pick;
+    };
+
+    // takes the lexicographically smallest (time, group) event, which is due at time T == next_due: its descriptor, which
+    // orders like the group's index
+    auto take_event = [&](double T) -> uint32_t {
+        uint64_t at = ballot(ev_t == T) & used;
+        int slot = first_of(at);
+        uint32_t d = lane_value(ev_d, slot);
+        for (at &= at - 1; rarely(at != 0ull); at &= at - 1) {  // several at that time
+            const int s2 = first_of(at);
+            const uint32_t d2 = lane_value(ev_d, s2);
+            if (d2 < d) {
+                d = d2;
+                slot = s2;
+            }
+        }
+        if (lane == slot) ev_t = inf;
+        used &= ~(1ull << slot);
+        nfree += 1;
+        next_due = wave_min(ev_t);
+        return d;
+    };
+
+    // :706-732 with :674-704 inlined; the reference's recursion on "nothing servable" is the outer loop
+    auto handle = [&](double t0, int m, uint32_t d) {
+        const uint32_t g = desc_group(d);
+        const int stages = (int)desc_stages_m1(d) + 1;
+        const uint32_t gclk = clk + (desc_last_slot(d) - desc_stages_m1(d)) * 8u;
+        double c0[4];  // clocks of the group's first four stages (or of what lies behind a shallower group's)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c0[u] = lds_get<double>(gclk + (uint32_t)u * 8u);
+        // fn(k, clock) for the stages in turn.  Nested, so that a shallow group leaves with one branch taken.
+        auto walk = [&](auto &&fn) {
+            fn(0, c0[0]);
+            if (stages > 1) {
+                fn(1, c0[1]);
+                if (stages > 2) {
+                    fn(2, c0[2]);
+                    if (stages > 3) {
+                        fn(3, c0[3]);
+                        for (int k = 4; k < stages; ++k) fn(k, lds_get<double>(gclk + (uint32_t)k * 8u));
+                    }
+                }
+            }
+        };
+        for (;;) {
+            const uint32_t lat_mg = ((uint32_t)m * (uint32_t)a.lat_row + desc_lat_off(d)) * (uint32_t)NB;
+            const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
+            const uint32_t base = uni(queue.x), arr = uni(queue.z);
+            uint32_t h = uni(queue.y);  // arr - h > 0: the caller saw a waiting request
+            // lane j takes entry j from the head of the queue on, whether it has arrived yet or not
+            const MqEntry *ep = mq + (size_t)base + h + (lane & 15);
+            double2 hv = *reinterpret_cast<const double2 *>(ep);
+            int2 ir = *reinterpret_cast<const int2 *>(&ep->idx);
+            // when a batch started now leaves the last stage, lane j: latency column j (:666-672)
+            const int col_j = (lane & 7) < NB ? lane & 7 : NB - 1;
+            const float lu = UNIF ? lat_at(lat_mg + (uint32_t)col_j) : 0.0f;
+            double tcol = t0;
+            walk([&](int k, double c) { tcol = max_nn(c, tcol) + (double)(UNIF ? lu : lat_at(lat_mg + (uint32_t)(k * NB + col_j))); });
+            const double alone = lane_value(tcol, 0) + overhead;
+            // drop heads that cannot meet their deadline even alone (:677-686)
+            bool found = false;
+            uint32_t first = 0;  // place of the head that leads the batch, in the model's list
+            int kfirst = 0;      // and among the entries fetched
+            double deadline = 0.0;
+            for (;;) {
+                const int avail = (int)(arr - h) < 8 ? (int)(arr - h) : 8;
+                const uint64_t pass = ballot(lane < avail && alone <= hv.y);
+                const int k = pass != 0ull ? first_of(pass) : avail;  // the heads before k are dropped
+                if (want_req && lane < k) {
+                    fin_out[(size_t)ir.x * kWave] = hv.x;
+                    good_out[(size_t)ir.x * kWave] = 0;
+                }
+                if (want_group && lane == 0) group_req[g * kWave] += k;
+                if (pass != 0ull) {
+                    found = true;
+                    kfirst = k;
+                    first = h + (uint32_t)k;
+                    deadline = lane_value(hv.y, k);
+                    h = first + 1u;
+                    break;
+                }
+                h += (uint32_t)avail;
+                if (h == arr) break;  // (else there are more than eight)
+                ep = mq + (size_t)base + h + (lane & 15);
+                hv = *reinterpret_cast<const double2 *>(ep);
+                ir = *reinterpret_cast<const int2 *>(&ep->idx);
+            }
+            if (!found) {  // :709-713
+                const int32_t next_rank = mq[(size_t)base + h].rank;
+                set_waiting(m, false);
+                const int m_next = select_model(g);
+                lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, h);
+                lds_put<uint32_t>(queues + (uint32_t)m * 16u + 12u, (uint32_t)next_rank);
+                wave_order();
+                m = m_next;
+                if (m < 0) return;
+                continue;
+            }
+            // grow the batch while the first request still meets its deadline (:693-702): lane b tests batch size b, the
+            // batch is the last size before the first one that fails
+            double tc = tcol;
+            if (rarely(!sizes_pow2)) tc = __hiloint2double(__shfl(__double2hiint(tcol), cand_col), __shfl(__double2loint(tcol), cand_col));
+            const bool ok = lane == 0 || (lane < NB && cand - 1 <= (int)(arr - h) && tc + overhead <= deadline);
+            const int sizes = first_of(~ballot(ok));  // (NB < 64)
+            const int bs = lane_value(cand, sizes - 1), col = lane_value(cand_col, sizes - 1);
+            // run it (:715-732)
+            const int kb = kfirst + bs;  // the rank of the arrival after the batch
+            const uint32_t next_rank = kb < 16 ? (uint32_t)lane_value(ir.y, kb) : (uint32_t)mq[(size_t)base + first + (uint32_t)bs].rank;
+            double t = t0 + overhead, idle_at = 0.0;
+            const float lb = UNIF ? lane_value(lu, col) : 0.0f;
+            walk([&](int k, double c) {
+                t = max_nn(t, c) + (double)(UNIF ? lb : lat_at(lat_mg + (uint32_t)(k * NB + col)));
+                lds_put<double>(gclk + (uint32_t)k * 8u, t);
+                if (k == 0) idle_at = uni(t);
+            });
+            const bool of_group = last == clk + desc_last_slot(d) * 8u;
+            c_last = of_group ? t : c_last;
+            c_first = of_group ? idle_at : c_first;
+            const uint32_t left = first + (uint32_t)bs;  // the batch is the arrivals first .. first+bs-1 of the model
+            lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, left);
+            lds_put<uint32_t>(queues + (uint32_t)m * 16u + 12u, next_rank);
+            wave_order();
+            if (left == arr) set_waiting(m, false);
+            // (sums by place in the queue, see above)
+            if (lane >= kfirst && lane < kfirst + bs && lane < 8) lat_sum += t - hv.x;
+            for (int k = 8; rarely(k < kb); ++k) {
+                const double at = k < 16 ? lane_value(hv.x, k) : mq[(size_t)base + first + (uint32_t)(k - kfirst)].t;
+                if (lane == 0) lat_sum += t - at;
+            }
+            if (want_req) {
+                if (lane >= kfirst && lane < kb && lane < 16) {
+                    fin_out[(size_t)ir.x * kWave] = t;
+                    good_out[(size_t)ir.x * kWave] = 1;
+                }
+                for (int k = 16 + lane; k < kb; k += kWave) {
+                    const int32_t r = mq[(size_t)base + first + (uint32_t)(k - kfirst)].idx;
+                    fin_out[(size_t)r * kWave] = t;
+                    good_out[(size_t)r * kWave] = 1;
+                }
+            }
+            n_good += bs;
+            if (want_group && lane == 0) {
+                group_req[g * kWave] += bs;
+                group_good[g * kWave] += bs;
+            }
+            if (want_model && lane == 0) model_good[(size_t)m * kWave] += bs;
+            if (rarely(nfree == 0)) {
+                dead = MMSIM_E_OVERFLOW;
+                return;
+            }
+            nfree -= 1;
+            const int slot = first_of(~used);
+            used |= 1ull << slot;
+            if (lane == slot) {
+                ev_t = idle_at;
+                ev_d = d;
+            }
+            next_due = idle_at < next_due ? idle_at : next_due;
+            return;
+        }
+    };
+
+    // idle events that are due at time tstamp (:739-744)
+    auto due_events = [&](double tstamp) {
+        while ((int)(next_due <= tstamp) & (int)(used != 0ull)) {
+            const double T = next_due;
+            const uint32_t d = take_event(T);
+            const int m = select_model(desc_group(d));
+            if (m < 0) break;  // the popped event is dropped, later due events stay (:742-743)
+            handle(T, m, d);
+            if (rarely(dead != 0)) break;
+        }
+    };
+
+    // ---- the arrivals: windows of eight.  Requests are fetched a block of 64 ahead, replica rows a window ahead.
+    auto fetch_block = [&](int64_t i) -> Req {
+        Req r = {0.0, -1, 0.0f};
+        if (i + lane < R) r = reqs[i + lane];
+        return r;
+    };
+    auto row_word = [&](int m) -> uint32_t { return rows[(size_t)(m < 0 ? 0 : m) * 8]; };
+    Req block = fetch_block(0), block_next = fetch_block(kWave);
+    int m_next = __shfl(block.m, oct);
+    uint32_t d_next = row_word(m_next);
+    for (int64_t w0 = 0; w0 < R && !dead; w0 += 8) {
+        const int from = (int)(w0 & 63) + oct;  // the lane that holds this octet's request
+        const int n = R - w0 < 8 ? (int)(R - w0) : 8;
+        const int m = m_next;
+        const uint32_t dj = d_next;
+        const double t = __hiloint2double(__shfl(__double2hiint(block.t), from), __shfl(__double2loint(block.t), from));
+        if ((w0 & 63) == 56) {
+            block = block_next;
+            block_next = fetch_block(w0 + 8 + kWave);
+        }
+        m_next = __shfl(block.m, (from + 8) & 63);  // (past the end of the stream: -1)
+        d_next = row_word(m_next);
+        const bool valid = (int32_t)dj >= 0 && m >= 0;
+        const uint32_t vb = oct_ballot(valid);
+        const bool hosted = (vb & 1u) != 0, longer = (vb >> 7) != 0;  // longer: the list may go on
+        last = clk + desc_last_slot(dj) * 8u;
+        c_last = lds_get<double>(last);
+        c_first = lds_get<double>(last - desc_stages_m1(dj) * 8u);
+        int cur = 0;        // arrivals before this one are settled
+        int seen_due = -1;  // the arrival whose due events have been seen to
+        while (cur < n) {
+            const double t_cur = lane_value(t, cur * 8);
+            if ((int)(next_due <= t_cur) & (int)(cur > seen_due)) {  // events first (:739-744)
+                due_events(t_cur);
+                seen_due = cur;
+                if (rarely(dead != 0)) break;
+            }
+            const double mn = oct_min(valid ? c_last : inf);
+            const uint32_t least = oct_ballot(valid && c_last == mn), free = oct_ballot(t >= c_first);
+            const int selj = __ffs((int)least) - 1;  // the first listed of those with the smallest last-stage clock
+            const bool found = hosted & (mn < 1e100), idle = found & (((free >> (selj & 7)) & 1u) != 0);
+            const bool special = hosted & (!found | longer), due = (next_due <= t) & (oct > seen_due);
+            const bool happens = (oct >= cur) & (oct < n) & (due | idle | special);
+            const uint64_t hb = ballot(happens);
+            const int f = hb != 0ull ? first_of(hb) >> 3 : n;
+            if (oct >= cur && oct < f && (lane & 7) == 0 && m >= 0)
+                __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u + 8u), 1u,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            if (want_req && oct >= cur && oct < f && (lane & 7) == 0 && !hosted) {
+                fin_out[(size_t)(w0 + oct) * kWave] = t;
+                good_out[(size_t)(w0 + oct) * kWave] = 0;
+            }
+            wave_order();
+            for (; cur < f; ++cur) {
+                const int mc = lane_value(m, cur * 8);
+                if (mc >= 0) set_waiting(mc, true);
+            }
+            if (f == n) break;
+            const int fl = f * 8;
+            const double tf = lane_value(t, fl);
+            if ((int)(next_due <= tf) & (int)(f > seen_due)) continue;  // its events first
+            // the arrival joins its queue, and its group turns to it if it is idle (:746-778)
+            const int mf = lane_value(m, fl);
+            uint32_t dsel = kEmpty;
+            bool ready = lane_value((int)idle, fl) != 0;
+            const uint32_t listed = lane_value(dj, fl + (lane_value(selj, fl) & 7));
+            if (lane_value((int)found, fl) != 0) dsel = listed;
+            if (rarely(lane_value((int)longer, fl) != 0)) {
+                const double best0 = lane_value(mn, fl);
+                double best = best0 < 1e100 ? best0 : 1e100;
+                for (int x = 0; x < a.rep_extra; ++x) {
+                    const uint32_t g = more_replicas[((size_t)mf * a.rep_extra + x) * kWave];
+                    if (g == (uint32_t)a.Gmax) break;
+                    const uint32_t d2 = ginfo[(size_t)g * kWave];
+                    const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
+                    if (c2 < best) {
+                        best = c2;
+                        dsel = d2;
+                        ready = tf >= uni(lds_get<double>(clk + (desc_last_slot(d2) - desc_stages_m1(d2)) * 8u));
+                    }
+                }
+            }
+            dsel = uni(dsel);
+            if (lane == 0)
+                __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)mf * 16u + 8u), 1u,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            wave_order();
+            set_waiting(mf, true);
+            cur = f + 1;
+            if (rarely(dsel == kEmpty)) {  // every replica's clock is infinite (sim_batching.hip says when)
+                dead = MMSIM_E_UNSUPPORTED;
+                break;
+            }
+            if (ready) {
+                handle(tf, mf, dsel);
+                if (rarely(dead != 0)) break;
+            }
+        }
+    }
+    // ---- drain (:781-787)
+    while (!dead && used != 0ull) {
+        const double T = next_due;
+        const uint32_t d = take_event(T);
+        const int m = select_model(desc_group(d));
+        if (m >= 0) handle(T, m, d);
+    }
+
+    for (int k = 1; k < 8; k *= 2) lat_sum += __hiloint2double(__shfl_xor(__double2hiint(lat_sum), k), __shfl_xor(__double2loint(lat_sum), k));
+    if (lane == 0) {
+        const size_t out = (size_t)wave * kWave;
+        a.n_good[out] = n_good;
+        a.lat_sum[out] = lat_sum;
+        a.status[out] = dead;
+    }
+}
+
+bool solo_outputs(const BatchingArgs &a) {
+    return (a.flags & (MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST)) != 0;
+}
+
+}  // namespace
+
+hipError_t launch_sim_batching_solo(const BatchingArgs &args, int wpb, size_t lds_bytes, hipStream_t stream) {
+    const bool ll = args.lat_lds_bytes > 0, unif = args.uniform_stages != 0, outputs = solo_outputs(args);
+    if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.tile_sims != 1 || !batching_solo_fits(args.M, args.NB, args.heap_cap, args.Gmax)) return hipErrorInvalidValue;
+    void (*kern)(const BatchingArgs) = nullptr;
+#define MMSIM_PICK3(L, U, O)                                       \
+    (args.M <= 64    ? sim_batching_solo_kernel<L, U, O, 1>          \
+     : args.M <= 128 ? sim_batching_solo_kernel<L, U, O, 2>          \
+     : args.M <= 256 ? sim_batching_solo_kernel<L, U, O, 4>          \
+                     : sim_batching_solo_kernel<L, U, O, 8>)
+#define MMSIM_PICK2(L, U) (outputs ? MMSIM_PICK3(L, U, true) : MMSIM_PICK3(L, U, false))
+#define MMSIM_PICK(L) (unif ? MMSIM_PICK2(L, true) : MMSIM_PICK2(L, false))
+    kern = ll ? MMSIM_PICK(true) : MMSIM_PICK(false);
+#undef MMSIM_PICK3
+#undef MMSIM_PICK2
+#undef MMSIM_PICK
+    // The kernel takes LDS addresses as numbers from 0 on: its dynamic LDS starts there as long as nothing static lies
+    // before it.
+    hipFuncAttributes attr;
+    hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(kern));
+    if (e != hipSuccess) return e;
+    if (attr.sharedSizeBytes != 0) return hipErrorInvalidKernelFile;
+    if (lds_bytes > 64 * 1024) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        if (e != hipSuccess) return e;
+    }
+    const unsigned tile_groups = (unsigned)((args.tiles + wpb - 1) / wpb);
+    hipLaunchKernelGGL(kern, dim3(tile_groups * (unsigned)(args.paired ? 1 : args.n_seeds)), dim3(wpb * kWave), lds_bytes, stream, args);
+    return hipGetLastError();
+}
+
+std::string sim_batching_solo_kernel_name(const BatchingArgs &args) {
+    return std::string("sim_batching_solo_kernel<") + (args.lat_lds_bytes > 0 ? "true, " : "false, ") +
+           (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.M <= 64 ? "1>" : args.M <= 128 ? "2>" : args.M <= 256 ? "4>" : "8>");
+}
+
+}  // namespace mmsim

@@ -405,6 +405,37 @@ def test_one_simulation_to_a_wavefront(eng, sizes, groups):
     assert most > 8 or groups < 30
 
 
+@pytest.mark.parametrize("M", [1, 64, 65, 128, 129, 256, 257, 512, 513])
+def test_models_of_one_simulation(eng, M):
+    """The models that wait are bits of one, two, four or eight words (more models: the kernel of wider tiles): the oracle's flags
+    and finish times where a word ends, with heads that arrived at the same instant in different words."""
+    rng = np.random.default_rng(M)
+    G, R, sizes = 5, 1200, [1, 2, 4]
+    c = random_case(8_000_000 + M, max_m=1, max_g=1, max_r=1)       # (keys; every value is made here)
+    member = rng.random((G, M)) < 0.5
+    member[:, M - 1] = True
+    c["m2g"], c["g2m"] = np.full((M, G), -1, np.int32), np.full((G, M), -1, np.int32)
+    for m in range(M):
+        gs = np.flatnonzero(member[:, m])
+        c["m2g"][m, :len(gs)] = gs
+    for g in range(G):
+        ms = np.flatnonzero(member[g])
+        c["g2m"][g, :len(ms)] = ms
+    c["num_stages"] = np.array([1, 2, 4, 7, 1], np.int32)
+    c["lat"] = (rng.uniform(0.01, 0.05, (M, G, 7, 1)) * np.array([1.0, 1.3, 1.9])).astype(np.float32)
+    gaps = rng.exponential(0.01, R)
+    gaps[rng.random(R) < 0.6] = 0.0
+    c["tstamps"], c["slos"] = np.cumsum(gaps), rng.uniform(0.1, 2.0, R).astype(np.float32)
+    c["model_ids"] = rng.choice([0, M // 2, M - 1] + list(range(M)), R).astype(np.int32)
+    f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
+        c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], sizes)
+    fin, good, cnt = _single(eng, c, sizes)
+    assert np.array_equal(good, g0) and np.array_equal(fin.view(np.uint64), f0.view(np.uint64))
+    for a, b in zip(cnt, c0):
+        assert np.array_equal(a, b)
+    assert 0 < g0.sum() < R
+
+
 @pytest.mark.parametrize("flags,octets", [(0, True), (_lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS, False)])
 def test_octets_in_place_of_sixteen_lanes(eng, flags, octets):
     """32768 simulations of a small problem: sixteen of them to a wavefront give every SIMD two wavefronts, octets take
