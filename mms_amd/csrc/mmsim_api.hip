@@ -379,6 +379,8 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     std::function<size_t(int, int)> batching_bytes_for;
     int blanes = kWave;  // batching simulator: lanes of a wavefront that simulate
     int tile_sims = kWave;  // simulations of a tile
+    bool solo = false;      // batching simulator: a wavefront for each simulation
+    int row = kWave;        // width of the rows of the device tables and results
     // Wavefronts per workgroup: no more than it takes to give every CU its share of the
     // batch (a small batch is spread over the CUs, one wavefront per workgroup), and
     // no more than fit in LDS.  Option waves_per_cu (1..8) sets the number instead.
@@ -521,8 +523,20 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         if (heap_cap < heap_min) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: per-wavefront state does not fit in LDS (too many models/stages/groups)");
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
-        if (blanes == 8 && o.batching_lanes == 0 && B == 1) {
+        const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(M, t->NB, heap_cap, Gmax) && rl.models_ascend();
+        // A wavefront for each simulation (sim_batching_solo.hip): as long as there are no more than twice as many as the
+        // chip takes at once (30000 requests, 48 models on 24 devices, a CU takes 20; ms with octets / with these: 2048
+        // simulations 54 / 53, 3072 132 / 62, 4096 133 / 73, 8192 161 / 125, 10240 197 / 149, 16384 200 / 226).  Streams of
+        // a few hundred requests are over within a millisecond and keep fewer wavefronts (4020 simulations of 200
+        // requests, the whole call: 1.3 / 1.0 ms, of 1000: 2.6 / 1.5).
+        const int64_t solo_per_cu = std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
+        int64_t requests = 0;
+        for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
+        if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
+        } else if (can_solo && requests >= (int64_t)512 * n_seeds &&
+                   (int64_t)B * b->out_seeds <= 2 * solo_per_cu * std::max(1, ctx->prop.multiProcessorCount)) {
+            tile_sims = 1;
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
@@ -538,6 +552,8 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 tile_sims = sims;
             }
         }
+        solo = can_solo && tile_sims == 1;
+        row = solo ? 1 : kWave;
         wpb = (int)std::min<size_t>(kMaxWavesPerBlockBatching, (size_t)ctx->max_lds / wave_bytes);
     }
 
@@ -599,7 +615,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 tile_nslots.push_back(1);
                 tile_stream.push_back(b->paired ? stream_of[p] : 0);
             }
-            b->pos[p] = tile * kWave + in_tile++;
+            b->pos[p] = tile * row + in_tile++;
             tile_nslots[tile] = std::max(tile_nslots[tile], slots_of[p]);
         }
         b->tiles = tile + 1;
@@ -757,13 +773,14 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     }
 
     phase("schedule");
-    // ---- per lane group descriptors [tiles][Gmax+1][64]; row Gmax stays empty
-    std::vector<uint32_t> ginfo((size_t)b->tiles * (Gmax + 1) * kWave, kEmpty);
+    // ---- per lane group descriptors [tiles][Gmax+1][64] (a wavefront for each simulation: [1]); row Gmax stays empty
+    b->row = row;
+    std::vector<uint32_t> ginfo((size_t)b->tiles * (Gmax + 1) * row, kEmpty);
     for (int32_t p = 0; p < B; ++p) {
-        const int tile = b->pos[p] / kWave, lane = b->pos[p] % kWave;
+        const int tile = b->pos[p] / row, lane = b->pos[p] % row;
         for (int32_t g = 0; g < rl.num_groups[p]; ++g) {
             const int32_t c = rl.group_cfg[(size_t)p * Gmax + g];
-            ginfo[((size_t)tile * (Gmax + 1) + g) * kWave + lane] =
+            ginfo[((size_t)tile * (Gmax + 1) + g) * row + lane] =
                 pack_desc(slot0[(size_t)p * Gmax + g], (uint32_t)t->cfg_pp[c], (uint32_t)lat_off[c], (uint32_t)g);
         }
     }
@@ -781,7 +798,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     const bool octets = batching && blanes == 8;
     if (batching) {
         rep8.assign((size_t)b->tiles * M * (octets ? tile_sims * 4 : kWave), octets ? ((uint64_t)kEmpty << 32 | kEmpty) : none8);
-        repx.assign((size_t)b->tiles * M * RX * kWave, (uint8_t)Gmax);
+        repx.assign((size_t)b->tiles * M * RX * row, (uint8_t)Gmax);
     } else {
         rep32.resize((size_t)b->tiles * M * 2 * kWave * 4);
         repx32.resize((size_t)b->tiles * M * RX * kWave);
@@ -819,16 +836,16 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     std::vector<int32_t> by_tile(B);
     {
         std::vector<int32_t> at((size_t)b->tiles + 1, 0);
-        for (int32_t p = 0; p < B; ++p) at[(size_t)(b->pos[p] / kWave) + 1] += 1;
+        for (int32_t p = 0; p < B; ++p) at[(size_t)(b->pos[p] / row) + 1] += 1;
         for (int32_t k = 0; k < b->tiles; ++k) at[(size_t)k + 1] += at[(size_t)k];
         std::vector<int32_t> fill(at.begin(), at.end() - 1);
-        for (int32_t p = 0; p < B; ++p) by_tile[(size_t)fill[(size_t)(b->pos[p] / kWave)]++] = p;
+        for (int32_t p = 0; p < B; ++p) by_tile[(size_t)fill[(size_t)(b->pos[p] / row)]++] = p;
         tile_begin = std::move(at);
     }
     parallel_slices(b->tiles, 8, [&](int64_t t0, int64_t t1) {
     for (int64_t k = tile_begin[(size_t)t0]; k < tile_begin[(size_t)t1]; ++k) {
         const int32_t p = by_tile[(size_t)k];
-        const int tile = b->pos[p] / kWave, lane = b->pos[p] % kWave;
+        const int tile = b->pos[p] / row, lane = b->pos[p] % row;
         for (int32_t m = 0; m < M; ++m) {
             const int64_t lo = rl.off[(size_t)p * M + m], hi = rl.off[(size_t)p * M + m + 1];
             uint8_t &rm = rmax[(size_t)tile * M + m];
@@ -841,11 +858,11 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (batching) {
                     if (j < kPackedReplicas && octets)
                         reinterpret_cast<uint32_t *>(rep8.data())[(((size_t)tile * M + m) * tile_sims + (size_t)lane) * 8 + (size_t)j] =
-                            ginfo[((size_t)tile * (Gmax + 1) + g) * kWave + lane];
+                            ginfo[((size_t)tile * (Gmax + 1) + g) * row + lane];
                     else if (j < kPackedReplicas)
                         word = (word & ~(0xFFull << (8 * j))) | ((uint64_t)g << (8 * j));
                     else
-                        repx[(((size_t)tile * M + m) * RX + (size_t)(j - kPackedReplicas)) * kWave + lane] = (uint8_t)g;
+                        repx[(((size_t)tile * M + m) * RX + (size_t)(j - kPackedReplicas)) * row + lane] = (uint8_t)g;
                 } else {
                     const int32_t c = rl.group_cfg[(size_t)p * Gmax + g];
                     const int pp = t->cfg_pp[c];
@@ -875,7 +892,6 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     std::vector<uint16_t> g2m_off, g2m_idx;
     std::vector<float> lat_nb;
     int members_max = 1;
-    bool g2m_ascending = true;  // every group lists its models in ascending order, each once
     if (batching) {
         b->hosted.assign((size_t)B * M, 0);
         std::vector<std::vector<int32_t>> lists(Gmax);
@@ -887,7 +903,6 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (!rl.g2m_off.empty())
                     dst.assign(rl.g2m_m.begin() + rl.g2m_off[(size_t)p * Gmax + g], rl.g2m_m.begin() + rl.g2m_off[(size_t)p * Gmax + g + 1]);
                 total += dst.size();
-                for (size_t x = 1; x < dst.size(); ++x) g2m_ascending = g2m_ascending && dst[x] > dst[x - 1];
             }
             for (int32_t m = 0; m < M; ++m) {
                 const int64_t lo = rl.off[(size_t)p * M + m], hi = rl.off[(size_t)p * M + m + 1];
@@ -901,17 +916,17 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
             if (total > 65535) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: more than 65535 (group, model) pairs in a placement");
             members_max = std::max<int>(members_max, (int)total);
         }
-        g2m_off.assign((size_t)b->tiles * (Gmax + 1) * kWave, 0);
-        g2m_idx.assign((size_t)b->tiles * members_max * kWave, 0);
+        g2m_off.assign((size_t)b->tiles * (Gmax + 1) * row, 0);
+        g2m_idx.assign((size_t)b->tiles * members_max * row, 0);
         for (int32_t p = 0; p < B; ++p) {
-            const int tile = b->pos[p] / kWave, lane = b->pos[p] % kWave;
+            const int tile = b->pos[p] / row, lane = b->pos[p] % row;
             uint16_t at = 0;
             for (int32_t g = 0; g <= Gmax; ++g) {
-                g2m_off[((size_t)tile * (Gmax + 1) + g) * kWave + lane] = at;
+                g2m_off[((size_t)tile * (Gmax + 1) + g) * row + lane] = at;
                 if (g < rl.num_groups[p])
                     for (int32_t m : all[(size_t)p * Gmax + g]) {
                         if (m < 0 || m >= M) return fail(MMSIM_E_INVALID, "group model list names a model outside 0..M-1");
-                        g2m_idx[((size_t)tile * members_max + at) * kWave + lane] = (uint16_t)m;
+                        g2m_idx[((size_t)tile * members_max + at) * row + lane] = (uint16_t)m;
                         ++at;
                     }
             }
@@ -933,7 +948,6 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     //      idle SIMD loses more than one that reads these tables through the caches.
     size_t batching_lat_lds = 0;
     int batching_g2m_lds = 0;
-    const bool solo = batching && blanes == 8 && tile_sims == 1 && g2m_ascending && batching_solo_fits(M, t->NB, heap_cap, Gmax);
     if (batching) {
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
         const size_t g2m_b = solo ? 0 : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
@@ -941,7 +955,8 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
         const int tiles_here = std::max(1, b->tiles);
         const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
-        const int wanted = (int)std::min<int64_t>(2 * kMaxWavesPerBlockBatching, std::max<int64_t>(1, ((int64_t)b->waves + cus - 1) / cus));
+        const int most_shares = solo ? kSoloWavesPerCu / kMaxWavesPerBlockBatching : 2;  // workgroups to a CU
+        const int wanted = (int)std::min<int64_t>(most_shares * kMaxWavesPerBlockBatching, std::max<int64_t>(1, ((int64_t)b->waves + cus - 1) / cus));
         // Fewer event slots (down to G+8) are accepted when that puts more wavefronts on a CU.
         const int wpb_max = kMaxWavesPerBlockBatching;
         const int heap_try_min = solo ? heap_cap : std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7));  // (its event slots are registers)
@@ -950,7 +965,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         const int allowed = o.batching_lds_tables >= 0 ? (o.batching_lds_tables & 3) : 3;
         for (int hc = heap_cap; hc >= heap_try_min; hc -= 8) {
             const size_t wb = solo ? batching_solo_bytes(nslots, M) : batching_bytes_for(blanes, hc);
-            for (int per_cu = 1; per_cu <= 2; ++per_cu)  // workgroups meant to share a CU (each gets that share of LDS)
+            for (int per_cu = 1; per_cu <= most_shares; ++per_cu)  // workgroups meant to share a CU (each gets that share of LDS)
                 for (int opt = 0; opt < 4; ++opt) {      // both, lists only, table only, neither: the first that gives most wavefronts
                     // (the lists before the table: a selection reads them in two dependent steps, while the table is
                     // read beside the queue's entries, which come from memory anyway; measured 2.19 s against 2.42 s)
@@ -1050,7 +1065,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         HIP_TRY(b->batch_sizes.alloc((size_t)t->NB));
         HIP_TRY(hipMemcpyAsync(b->batch_sizes.p, t->batch_sizes, sizeof(int32_t) * (size_t)t->NB, hipMemcpyHostToDevice, st));
     }
-    const size_t lanes_padded = (size_t)b->waves * kWave;
+    const size_t lanes_padded = (size_t)b->waves * row;
     HIP_TRY(b->status.alloc(lanes_padded));
     HIP_TRY(b->n_good.alloc(lanes_padded));
     HIP_TRY(b->lat_sum.alloc(lanes_padded));
@@ -1474,8 +1489,8 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
             return fail(MMSIM_E_HIP, "simulation kernel: the schedule completed " + std::to_string(kerrs[1]) + " of " +
                                          std::to_string(b->waves) + " (tile, stream) items; results are invalid");
     }
-    const int32_t B = b->B, M = b->M, Gmax = b->Gmax, tiles = b->tiles;
-    const size_t lanes_padded = (size_t)b->waves * kWave;
+    const int32_t B = b->B, M = b->M, Gmax = b->Gmax, tiles = b->tiles, row_w = b->row;
+    const size_t lanes_padded = (size_t)b->waves * row_w;
     std::vector<int32_t> ng(lanes_padded);
     std::vector<double> ls(lanes_padded);
     HIP_TRY(hipMemcpy(ng.data(), b->n_good.p, sizeof(int32_t) * lanes_padded, hipMemcpyDeviceToHost));
@@ -1494,7 +1509,7 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
     }
     for (int s = 0; s < b->out_seeds; ++s)
         for (int32_t p = 0; p < B; ++p) {
-            const size_t src = (size_t)s * tiles * kWave + b->pos[p];
+            const size_t src = (size_t)s * tiles * row_w + b->pos[p];
             out->n_good[(size_t)s * B + p] = ng[src];
             out->latency_sum[(size_t)s * B + p] = ls[src];
             if (out->status) out->status[(size_t)s * B + p] = st_host.empty() ? 0 : st_host[src];
@@ -1507,9 +1522,9 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
         HIP_TRY(hipMemcpy(h.data(), dev.p, dev.bytes(), hipMemcpyDeviceToHost));
         for (int s = 0; s < b->out_seeds; ++s)
             for (int32_t p = 0; p < B; ++p) {
-                const size_t wave = (size_t)s * tiles + b->pos[p] / kWave;
+                const size_t wave = (size_t)s * tiles + b->pos[p] / row_w;
                 for (int32_t x = 0; x < width; ++x)
-                    dst[((size_t)s * B + p) * width + x] = h[(wave * width + x) * kWave + b->pos[p] % kWave];
+                    dst[((size_t)s * B + p) * width + x] = h[(wave * width + x) * row_w + b->pos[p] % row_w];
             }
         return MMSIM_OK;
     };
@@ -1528,10 +1543,10 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
         const size_t rows = (size_t)b->slot_rows;
         for (int s = 0; s < b->out_seeds; ++s)
             for (int32_t p = 0; p < B; ++p) {
-                const size_t wave = (size_t)s * tiles + b->pos[p] / kWave;
+                const size_t wave = (size_t)s * tiles + b->pos[p] / row_w;
                 for (int32_t g = 0; g < Gmax; ++g) {
                     const int slot = b->group_last_slot[(size_t)p * Gmax + g];
-                    const unsigned long long v = slot < 0 ? 0ull : h[(wave * rows + slot) * kWave + b->pos[p] % kWave];
+                    const unsigned long long v = slot < 0 ? 0ull : h[(wave * rows + slot) * row_w + b->pos[p] % row_w];
                     out->group_num_requests[((size_t)s * B + p) * Gmax + g] = (int32_t)(v & 0xFFFFFFFFull);
                     out->group_num_good[((size_t)s * B + p) * Gmax + g] = (int32_t)(v >> 32);
                 }
@@ -1544,23 +1559,23 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
     }
     if (wr && b->Rmax > 0) {
         const size_t Rm = (size_t)b->Rmax;
-        std::vector<double> hf(Rm * kWave);
-        std::vector<uint8_t> hg(Rm * kWave);
-        std::vector<int32_t> owner((size_t)tiles * kWave, -1);  // placement simulated on each lane
+        std::vector<double> hf(Rm * row_w);
+        std::vector<uint8_t> hg(Rm * row_w);
+        std::vector<int32_t> owner((size_t)tiles * row_w, -1);  // placement simulated on each lane
         for (int32_t p = 0; p < B; ++p) owner[b->pos[p]] = p;
         for (int s = 0; s < b->out_seeds; ++s)
             for (int32_t tile = 0; tile < tiles; ++tile) {
                 const size_t wave = (size_t)s * tiles + tile;
-                HIP_TRY(hipMemcpy(hf.data(), b->finish.p + wave * Rm * kWave, sizeof(double) * Rm * kWave, hipMemcpyDeviceToHost));
-                HIP_TRY(hipMemcpy(hg.data(), b->good.p + wave * Rm * kWave, Rm * kWave, hipMemcpyDeviceToHost));
-                for (int l = 0; l < kWave; ++l) {
-                    const int32_t p = owner[(size_t)tile * kWave + l];
+                HIP_TRY(hipMemcpy(hf.data(), b->finish.p + wave * Rm * row_w, sizeof(double) * Rm * row_w, hipMemcpyDeviceToHost));
+                HIP_TRY(hipMemcpy(hg.data(), b->good.p + wave * Rm * row_w, Rm * row_w, hipMemcpyDeviceToHost));
+                for (int l = 0; l < row_w; ++l) {
+                    const int32_t p = owner[(size_t)tile * row_w + l];
                     if (p < 0) continue;
                     const size_t Rs = (size_t)b->wl_R[(size_t)(b->paired ? b->stream_of[p] : s)];
                     const size_t row = ((size_t)s * B + (size_t)p) * Rm;
                     for (size_t i = 0; i < Rs; ++i) {
-                        out->finish[row + i] = hf[i * kWave + l];
-                        out->good[row + i] = hg[i * kWave + l];
+                        out->finish[row + i] = hf[i * row_w + l];
+                        out->good[row + i] = hg[i * row_w + l];
                     }
                 }
             }
@@ -1617,8 +1632,8 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
                 sim_base[sim] = (int64_t)sim * b->Rmax;
                 continue;
             }
-            const int64_t wave = (int64_t)s * tiles + b->pos[p] / kWave;
-            sim_base[sim] = wave * b->Rmax * kWave + b->pos[p] % kWave;
+            const int64_t wave = (int64_t)s * tiles + b->pos[p] / b->row;
+            sim_base[sim] = wave * b->Rmax * b->row + b->pos[p] % b->row;
         }
     const size_t cells = (size_t)n_sims * (size_t)M;
     // (the buffers belong to the batch: the first call makes them, later calls allocate nothing)
@@ -1645,7 +1660,7 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
     StatsArgs f{};
     f.finish = b->window ? b->wargs.finish : b->finish.p;
     f.good = b->window ? b->wargs.good : b->good.p;
-    f.stride = b->window ? 1 : kWave;
+    f.stride = b->window ? 1 : b->row;
     f.mq = d_mq.p;
     f.mq_off = i64;
     f.lo = i64 + mqo.size();

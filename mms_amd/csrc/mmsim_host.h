@@ -207,6 +207,12 @@ struct RepLists {
     // left empty, they are derived from the replica lists as the reference does (:424-430)
     std::vector<int64_t> g2m_off;     // [B*Gmax+1]
     std::vector<int32_t> g2m_m;
+    bool models_ascend() const {  // every group lists its models in ascending order
+        for (size_t g = 0; g + 1 < g2m_off.size(); ++g)
+            for (int64_t x = g2m_off[g] + 1; x < g2m_off[g + 1]; ++x)
+                if (g2m_m[(size_t)x] <= g2m_m[(size_t)x - 1]) return false;
+        return true;
+    }
 };
 
 struct mmsim_batch {
@@ -219,7 +225,8 @@ struct mmsim_batch {
     std::vector<int64_t> wl_R;                           // [n_seeds] stream lengths
     std::vector<uint64_t> wl_id;                         // [n_seeds] ids of the workloads the batch was made from
     std::vector<std::vector<int32_t>> wl_model_requests;  // [n_seeds][M] requests per model of each stream
-    std::vector<int32_t> pos;  // pos[placement] = tile * 64 + lane it is simulated on
+    int32_t row = kWave;       // width of the rows of the device tables and results: 64, or 1 if every simulation has a wavefront
+    std::vector<int32_t> pos;  // pos[placement] = tile * row + lane it is simulated on
     // Paired batch (mmsim_eval_pairs): placement p is simulated on stream stream_of[p] only; a tile holds
     // placements of one stream, and results are laid out as for a single seed.
     bool paired = false;

@@ -147,12 +147,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const int64_t *__restrict__ mo = a.mq_off + (size_t)seed * (M + 1);
     const MqEntry *__restrict__ mq = a.mq + mo[0];
     const uint32_t *__restrict__ rows = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 8 + (lane & 7);
-    const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra * kWave;
-    const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1) * kWave;
-    int32_t *model_good = a.model_good + (size_t)wave * M * kWave;
-    int32_t *group_req = a.group_req + (size_t)wave * a.Gmax * kWave, *group_good = a.group_good + (size_t)wave * a.Gmax * kWave;
-    double *fin_out = a.finish + (size_t)wave * a.Rmax * kWave;
-    uint8_t *good_out = a.good + (size_t)wave * a.Rmax * kWave;
+    const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra;
+    const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1);
+    int32_t *model_good = a.model_good + (size_t)wave * M;
+    int32_t *group_req = a.group_req + (size_t)wave * a.Gmax, *group_good = a.group_good + (size_t)wave * a.Gmax;
+    double *fin_out = a.finish + (size_t)wave * a.Rmax;
+    uint8_t *good_out = a.good + (size_t)wave * a.Rmax;
     const double overhead = a.fixed_overhead, inf = __builtin_inf();
     auto lat_at = [&](uint32_t i) -> float { return LATLDS ? lds_get<float>(i * 4u) : a.lat[i]; };
 
@@ -162,10 +162,10 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{(uint32_t)(mo[m] - mo[0]), 0u, 0u, (uint32_t)a.mq[mo[m]].rank});
     uint64_t members[MW] = {};  // lane g: models of group g
     if (lane < a.Gmax) {
-        const uint16_t *first = a.g2m_off + (size_t)tile * (a.Gmax + 1) * kWave + (size_t)lane * kWave;
-        const uint16_t *list = a.g2m_idx + (size_t)tile * a.members_max * kWave;
-        for (int x = first[0]; x < (int)first[kWave]; ++x) {
-            const int m = list[(size_t)x * kWave];
+        const uint16_t *first = a.g2m_off + (size_t)tile * (a.Gmax + 1) + lane;
+        const uint16_t *list = a.g2m_idx + (size_t)tile * a.members_max;
+        for (int x = first[0]; x < (int)first[1]; ++x) {
+            const int m = list[x];
 #pragma unroll
             for (int i = 0; i < MW; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
         }
@@ -293,10 +293,10 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 const uint64_t pass = ballot(lane < avail && alone <= hv.y);
                 const int k = pass != 0ull ? first_of(pass) : avail;  // the heads before k are dropped
                 if (want_req && lane < k) {
-                    fin_out[(size_t)ir.x * kWave] = hv.x;
-                    good_out[(size_t)ir.x * kWave] = 0;
+                    fin_out[ir.x] = hv.x;
+                    good_out[ir.x] = 0;
                 }
-                if (want_group && lane == 0) group_req[g * kWave] += k;
+                if (want_group && lane == 0) group_req[g] += k;
                 if (pass != 0ull) {
                     found = true;
                     kfirst = k;
@@ -355,21 +355,21 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             }
             if (want_req) {
                 if (lane >= kfirst && lane < kb && lane < 16) {
-                    fin_out[(size_t)ir.x * kWave] = t;
-                    good_out[(size_t)ir.x * kWave] = 1;
+                    fin_out[ir.x] = t;
+                    good_out[ir.x] = 1;
                 }
                 for (int k = 16 + lane; k < kb; k += kWave) {
                     const int32_t r = mq[(size_t)base + first + (uint32_t)(k - kfirst)].idx;
-                    fin_out[(size_t)r * kWave] = t;
-                    good_out[(size_t)r * kWave] = 1;
+                    fin_out[r] = t;
+                    good_out[r] = 1;
                 }
             }
             n_good += bs;
             if (want_group && lane == 0) {
-                group_req[g * kWave] += bs;
-                group_good[g * kWave] += bs;
+                group_req[g] += bs;
+                group_good[g] += bs;
             }
-            if (want_model && lane == 0) model_good[(size_t)m * kWave] += bs;
+            if (want_model && lane == 0) model_good[m] += bs;
             if (rarely(nfree == 0)) {
                 dead = MMSIM_E_OVERFLOW;
                 return;
@@ -447,8 +447,8 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u + 8u), 1u,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             if (want_req && oct >= cur && oct < f && (lane & 7) == 0 && !hosted) {
-                fin_out[(size_t)(w0 + oct) * kWave] = t;
-                good_out[(size_t)(w0 + oct) * kWave] = 0;
+                fin_out[w0 + oct] = t;
+                good_out[w0 + oct] = 0;
             }
             wave_order();
             for (; cur < f; ++cur) {
@@ -469,9 +469,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 const double best0 = lane_value(mn, fl);
                 double best = best0 < 1e100 ? best0 : 1e100;
                 for (int x = 0; x < a.rep_extra; ++x) {
-                    const uint32_t g = more_replicas[((size_t)mf * a.rep_extra + x) * kWave];
+                    const uint32_t g = more_replicas[(size_t)mf * a.rep_extra + x];
                     if (g == (uint32_t)a.Gmax) break;
-                    const uint32_t d2 = ginfo[(size_t)g * kWave];
+                    const uint32_t d2 = ginfo[g];
                     const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
                     if (c2 < best) {
                         best = c2;
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 
     for (int k = 1; k < 8; k *= 2) lat_sum += __hiloint2double(__shfl_xor(__double2hiint(lat_sum), k), __shfl_xor(__double2loint(lat_sum), k));
     if (lane == 0) {
-        const size_t out = (size_t)wave * kWave;
+        const size_t out = (size_t)wave;
         a.n_good[out] = n_good;
         a.lat_sum[out] = lat_sum;
         a.status[out] = dead;

@@ -436,6 +436,36 @@ def test_models_of_one_simulation(eng, M):
     assert 0 < g0.sum() < R
 
 
+@pytest.mark.parametrize("B,n_streams,R,solo", [(71, 29, 511, False), (71, 29, 512, True), (320, 32, 513, True), (321, 32, 513, False)])
+def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, solo):
+    """Up to forty simulations to a CU have a wavefront each, unless their streams are short: the oracle's counts and
+    traces on both sides of either line."""
+    cfg = make_config(5, B)
+    table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
+    packed = E.pack_placements(cfg.placements, table)
+    st = cfg.stream(0)
+    cut = [slice(997 * k, 997 * k + R) for k in range(n_streams)]
+    streams = [SimpleNamespace(tstamps=(st.tstamps[c] - st.tstamps[c.start]) / 3, model_ids=st.model_ids[c], slos=st.slos[c]) for c in cut]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, cfg.num_models) for s in streams]
+    counts = _lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS
+    for flags in (0, counts, counts | _lib.WANT_PER_REQUEST):
+        batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING)
+        name, waves = batch.kernel_name(), batch.info()["waves"]
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        batch.close()
+        assert name.startswith("sim_batching_solo" if solo else "sim_batching_kernel") and (waves == B * n_streams) == solo
+        for k in (0, n_streams - 1):
+            ref = oracle_batch(streams[k], table, packed, batching=True, want_per_request=True)
+            if flags:
+                _check(out, ref, k, per_request=bool(flags & _lib.WANT_PER_REQUEST))
+            assert np.array_equal(out["n_good"][k], ref["n_good"]) and np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
+            assert 0 < ref["n_good"].sum() < B * R
+    for dw in dws:
+        dw.close()
+
+
 @pytest.mark.parametrize("flags,octets", [(0, True), (_lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS, False)])
 def test_octets_in_place_of_sixteen_lanes(eng, flags, octets):
     """32768 simulations of a small problem: sixteen of them to a wavefront give every SIMD two wavefronts, octets take
