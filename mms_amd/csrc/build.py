@@ -1,4 +1,4 @@
-"""Builds libmmsim.so (HIP, gfx950 only) into the package folder.
+"""Builds libmmsim.so (HIP, gfx950 only) and _objects.so (host) into the package folder.
 
     python -m mms_amd.csrc.build        # or: from mms_amd.csrc.build import build; build()
 
@@ -9,11 +9,13 @@ off, then linked into one shared library next to the Python package, where
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 OUT = os.path.join(PKG, "libmmsim.so")
+OBJECTS = os.path.join(PKG, "_objects.so")   # Python extension: objects.cpp
 OBJ_DIR = os.path.join(HERE, "build")
 
 # object name -> source, flags of its own.  sim_window.hip is compiled once per number of requests side by side (its
@@ -64,6 +66,16 @@ def _compile(unit, extra, src_dir=HERE, obj_dir=OBJ_DIR):
     return obj, "\n".join(warn)
 
 
+def build_objects(src_dir=HERE, out=OBJECTS):
+    """Compiles objects.cpp, host code for this interpreter, into `out`."""
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_paths()["include"],
+           os.path.join(src_dir, "objects.cpp"), "-o", out]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for objects.cpp:\n{proc.stdout}\n{proc.stderr}")
+    return out
+
+
 def build(verbose=False, extra_flags=(), src_dir=HERE, out=OUT):
     """Compiles UNITS from `src_dir` and links them into `out`."""
     obj_dir = os.path.join(src_dir, "build")
@@ -84,3 +96,4 @@ def build(verbose=False, extra_flags=(), src_dir=HERE, out=OUT):
 
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_objects())

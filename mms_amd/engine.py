@@ -17,6 +17,7 @@ from typing import List, Sequence
 import numpy as np
 
 from mms_amd import _lib
+from mms_amd import _objects   # built by `python -m mms_amd.csrc.build`
 from mms_amd.util import FIXED_OVERHEAD, STAGE_PENALTY
 
 
@@ -161,6 +162,12 @@ class LatencyTable:
 
 def pack_placements(sols: Sequence, table: LatencyTable):
     """ModelPlacement list -> (num_groups[B], group_cfg[B][Gmax], gm_off[B][Gmax+1], gm_idx)."""
+    plain = _objects.pack(sols, table.index, table.config_id)
+    if plain is not None:
+        Gmax = plain[0]
+        num_groups, group_cfg, gm_off, gm_idx = (np.frombuffer(x, t) for x, t in zip(plain[1:], (np.int32, np.int32, np.int64, np.int32)))
+        return num_groups, group_cfg.reshape(-1, Gmax), gm_off.reshape(-1, Gmax + 1), gm_idx
+    # rows that are no lists or tuples, ids that are no ints
     B = len(sols)
     num_groups = np.fromiter((len(s.group_configs) for s in sols), np.int32, B)
     Gmax = max(int(num_groups.max()) if B else 1, 1)
@@ -192,6 +199,23 @@ def pack_placements(sols: Sequence, table: LatencyTable):
     if gm_idx is None:
         gm_idx = np.fromiter(chain.from_iterable(models), np.int32, total)
     return num_groups, group_cfg, gm_off, gm_idx
+
+
+def count_models(sols: Sequence):
+    """Replicas of each ModelPlacement."""
+    plain = _objects.count_models(sols)
+    if plain is not None:
+        return np.frombuffer(plain, np.int64)
+    return np.fromiter((sum(map(len, s.group_models)) for s in sols), np.int64, len(sols))
+
+
+def request_arrays(requests: Sequence, name2id: dict):
+    """(model ids int32, -1: unknown model; latency objectives float32) of a list of requests."""
+    plain = _objects.request_arrays(requests, name2id)
+    if plain is not None:
+        return np.frombuffer(plain[0], np.int32), np.frombuffer(plain[1], np.float32)
+    return (np.array([name2id.get(r.model_name, -1) for r in requests], dtype=np.int32),
+            np.array([r.slo for r in requests], dtype=np.float32))
 
 
 def _result_arrays(flags, n_seeds, B, M, Gmax, Rmax):

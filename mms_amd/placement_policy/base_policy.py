@@ -249,8 +249,7 @@ class PlacementEvaluator:
         names = tuple(name2prof.keys())
         profs = tuple(name2prof.values())
         name2id = {n: i for i, n in enumerate(names)}
-        model_ids = np.array([name2id.get(r.model_name, -1) for r in wl.requests], dtype=np.int32)
-        slos = np.array([r.slo for r in wl.requests], dtype=np.float32)
+        model_ids, slos = _engine.request_arrays(wl.requests, name2id)
         wl.cached_data = (model_ids, slos, names, profs)
         self._names = names
         self._num_requests_per_model = np.bincount(model_ids[model_ids >= 0], minlength=len(names))
@@ -308,8 +307,7 @@ class PlacementEvaluator:
         R = len(self.workload)
         goodput = out["n_good"][0] / R
         latency_mean = out["latency_sum"][0] / R
-        replicas = np.fromiter((sum(map(len, s.group_models)) for s in sols), np.int64, len(sols))
-        scores = goodput - latency_mean / 10000 + replicas / 1000000
+        scores = goodput - latency_mean / 10000 + _engine.count_models(sols) / 1000000
         return [float(x) for x in scores]
 
     def get_stats(self, sols: List[ModelPlacement]):

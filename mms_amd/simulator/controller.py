@@ -259,9 +259,7 @@ def approximate_one_case(case: ServingCase, seed: int = 0, warmup: int = DEFAULT
         # model id == registration order (:331-334)
         model_names, prof_ress = zip(*controller.name2profiling.items())
         name2id = {name: i for i, name in enumerate(model_names)}
-        model_ids = np.array([name2id.get(r.model_name, -1) for r in workload.requests],
-                             dtype=np.int32)
-        slos = np.array([r.slo for r in workload.requests], dtype=np.float32)
+        model_ids, slos = _engine.request_arrays(workload.requests, name2id)
         if workload.enable_simulator_cache:
             workload.cached_data = (model_ids, slos, model_names, prof_ress)
 
