@@ -524,18 +524,18 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
         const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(M, t->NB, heap_cap, Gmax) && rl.models_ascend();
-        // A wavefront for each simulation (sim_batching_solo.hip): as long as there are no more than twice as many as the
-        // chip takes at once (30000 requests, 48 models on 24 devices, a CU takes 20; ms with octets / with these: 2048
-        // simulations 54 / 53, 3072 132 / 62, 4096 133 / 73, 8192 161 / 125, 10240 197 / 149, 16384 200 / 226).  Streams of
-        // a few hundred requests are over within a millisecond and keep fewer wavefronts (4020 simulations of 200
-        // requests, the whole call: 1.3 / 1.0 ms, of 1000: 2.6 / 1.5).
+        // A wavefront for each simulation (sim_batching_solo.hip) up to 64 of them to a CU, of which it takes 20 at once.  ms
+        // with octets / with these, 150000 requests, 96 models on 48 devices: 2048 simulations 54 / 39, 3072 132 / 46, 4096 133
+        // / 52, 8192 161 / 90, 16384 200 / 157; 30000 requests at a lower load, 48 models on 24 devices: 8192 61 / 40, 16384 73 /
+        // 67, 65536 216 / 235 (the octets of a wavefront share the cost of a step).  Streams of a few hundred requests are over
+        // within a millisecond and keep fewer wavefronts (16384 simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
         const int64_t solo_per_cu = std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         int64_t requests = 0;
         for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
         if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
         } else if (can_solo && requests >= (int64_t)512 * n_seeds &&
-                   (int64_t)B * b->out_seeds <= 2 * solo_per_cu * std::max(1, ctx->prop.multiProcessorCount)) {
+                   (int64_t)B * b->out_seeds <= 64 * solo_per_cu / kSoloWavesPerCu * std::max(1, ctx->prop.multiProcessorCount)) {
             tile_sims = 1;
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two

@@ -298,7 +298,10 @@ hipError_t launch_sim_scalar(const ScalarArgs &args, hipStream_t stream, std::st
 
 // One simulation to a wavefront (sim_batching_solo.hip), for tables, event slots and models that its lanes hold.
 constexpr bool batching_solo_fits(int M, int NB, int heap_cap, int Gmax) { return M <= 512 && NB <= 8 && heap_cap <= 64 && Gmax <= 64; }
-constexpr size_t batching_solo_bytes(int nslots, int M) { return (size_t)((nslots + 4) & ~1) * 8 + (size_t)M * 16; }  // LDS of a wavefront (three clocks more than there are)
+constexpr int kSoloRowsInLds = 128;  // up to so many models their replicas' descriptors are in LDS (halves: 8 x 2 bytes)
+constexpr size_t batching_solo_bytes(int nslots, int M) {  // LDS of a wavefront (three clocks more than there are)
+    return (size_t)((nslots + 4) & ~1) * 8 + (size_t)M * (M <= kSoloRowsInLds ? 32 : 16);
+}
 constexpr int kSoloWavesPerCu = 20;  // that share a CU: five to a SIMD, by their registers
 hipError_t launch_sim_batching_solo(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream);
 std::string sim_batching_solo_kernel_name(const BatchingArgs &args);

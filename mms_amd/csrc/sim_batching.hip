@@ -153,8 +153,8 @@ __device__ __forceinline__ lds_vu32 *as_lds_vu32(void *p) { return (lds_vu32 *)p
 // and lane c of an octet keeps the earliest time of chunk c in a register: neither the free-slot stack nor the
 // chunk minima are read from LDS.
 // OUTPUTS: anything beyond the scores (a.flags says what).  Fixed at compile time, since the scalar branches around what
-// is not asked for cost more than what they skip: 30000 requests, 48 models on 24 devices, 2048 placements on 4 streams
-// 165.8 -> 161.3 ms (28.7 -> 24.4 branches per arrival).
+// is not asked for cost more than what they skip: 150000 requests, 96 models on 48 devices, 2048 placements on 4 streams
+// 165.8 -> 161.3 ms (15 % fewer branches, 12 % fewer scalar instructions).
 template <int NBT, bool LATLDS, bool G2MLDS, bool OCT, bool UNIF, bool SH, bool OUTPUTS>
 __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching_kernel(const BatchingArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];

@@ -18,16 +18,23 @@
 // those at which nothing happens but a place in a queue cost no more than that.  Events that are due are seen to before
 // an arrival is looked at, since the clocks it is judged by may change.
 //
-// What bounds it: one dependent chain per event or arrival, on a wavefront that has its SIMD to itself: instructions
-// (4 cycles each, whatever they do), a taken branch (20 to 30 cycles until the instructions at its target are there), and
-// two trips to LDS and one to memory per batch.  Hence masks in scalars and look-ups in registers instead of lists in
-// LDS, clocks of the window's replicas kept in registers as they change, and paths laid out so that what happens most falls
-// through.  30000 requests, 48 models on 24 devices, 128 placements: 25.0 ms with the octets of sim_batching.hip each
-// looking at an arrival of its own (per arrival 226 instructions, 18 of them branches, 1746 cycles), 15.7 ms here (155, 14,
-// 1123).  Tried, no gain: the queue entries of arrivals touched a window ahead (20.4 / 20.5 ms at the time).
+// What bounds it: one dependent chain per event or arrival.  A wavefront that has its SIMD to itself pays for instructions
+// (4 cycles each, whatever they do), taken branches (20 to 30 cycles until the instructions at the target are there), two
+// trips to LDS and one to memory per batch; five of them on a SIMD pay for scalar instructions (one in four cycles for all
+// of them).  Hence masks in scalars and look-ups in registers instead of lists in LDS, clocks of the window's replicas kept
+// in registers as they change, conditions of a window's octets as bits of one mask, and paths laid out so that what happens
+// most falls through.
 //
-// LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: where
-// its arrivals start in the stream's lists, head, arrivals so far, rank of the head.
+// Measured.  30000 requests, 48 models on 24 devices, 128 placements: 25.0 ms with the octets of sim_batching.hip each
+// looking at an arrival of its own (per arrival 226 instructions, 18 of them branches, 1746 cycles), 14.2 ms here (117, 11,
+// 939).  150000 requests, 96 models on 48 devices, 2048 placements on 4 streams: 161 ms with octets, 90 ms here; of these
+// 34 ms since conditions are masks (44 scalar instructions per arrival -> 28), joins of a window's models one reduction
+// (octets_or), dropped requests a loop of its own, the next window's rows in LDS.  Tried, no gain: the queue entries of
+// arrivals touched a window ahead; the batch's times worked out beside the look at its deadline (14.2 -> 14.6, 90 -> 97 ms: its
+// writes by one lane cost more than the chain); six wavefronts to a SIMD.
+//
+// LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
+// its head and of its next arrival in the stream's lists, rank of the head; up to 128 models also their replicas.
 #include "mmsim_internal.h"
 
 namespace mmsim {
@@ -68,10 +75,13 @@ __device__ __forceinline__ double max_nn(double x, double y) {  // neither is Na
     asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
     return r;
 }
+// whether this lane's bit is set (a scalar mask used as a condition: no instruction)
+__device__ __forceinline__ bool in_mask(uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes); }
+constexpr uint64_t kFirstOfOctets = 0x0101010101010101ull;
+// of each octet, the first of its lanes that are in the mask
+__device__ __forceinline__ uint64_t first_of_octets(uint64_t lanes) { return lanes & ~((lanes | kFirstOfOctets << 7) - kFirstOfOctets); }
 __device__ __forceinline__ int ilog2i(int v) { return 31 - __clz(v); }
 
-// bit j = the predicate of lane j of the octet
-__device__ __forceinline__ uint32_t oct_ballot(bool p) { return (uint32_t)(ballot(p) >> (threadIdx.x & 56u)) & 0xFFu; }
 // Smallest value of the octet, in all of its lanes; of the wavefront, as a scalar.  A DPP operand needs two wait states
 // after the write of its register (s_nop 1).  All lanes must be active.
 __device__ __forceinline__ uint32_t oct_min(uint32_t v) {
@@ -102,6 +112,23 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t v) {
         : "+v"(v));
     return lane_value(v, 63);
 }
+// Each word or'ed over the octets (whose lanes hold the same).  All lanes must be active.
+#define MMSIM_OR(W, HOW) "v_or_b32_dpp %" #W ", %" #W ", %" #W " " HOW " bank_mask:0xf\n"
+#define MMSIM_OR2(HOW) MMSIM_OR(0, HOW) MMSIM_OR(1, HOW) "s_nop 0\n"
+#define MMSIM_OR4(HOW) MMSIM_OR(0, HOW) MMSIM_OR(1, HOW) MMSIM_OR(2, HOW) MMSIM_OR(3, HOW)
+__device__ __forceinline__ void octets_or(uint32_t (&v)[2]) {
+    asm volatile("s_nop 1\n" MMSIM_OR2("row_shr:8 row_mask:0xf") MMSIM_OR2("row_bcast:15 row_mask:0xa") MMSIM_OR2("row_bcast:31 row_mask:0xc")
+                 : "+v"(v[0]), "+v"(v[1]));
+    for (uint32_t &x : v) x = lane_value(x, 63);
+}
+__device__ __forceinline__ void octets_or(uint32_t (&v)[4]) {
+    asm volatile("s_nop 1\n" MMSIM_OR4("row_shr:8 row_mask:0xf") MMSIM_OR4("row_bcast:15 row_mask:0xa") MMSIM_OR4("row_bcast:31 row_mask:0xc")
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+    for (uint32_t &x : v) x = lane_value(x, 63);
+}
+#undef MMSIM_OR4
+#undef MMSIM_OR2
+#undef MMSIM_OR
 // Doubles that are never negative nor NaN order as their bit patterns do: the smallest high word, then the smallest low
 // word among the lanes that have it (clocks and event times start at +0 and only grow; +inf is allowed).
 __device__ __forceinline__ double oct_min(double v) {
@@ -139,14 +166,16 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const bool want_group = OUTPUTS && (a.flags & MMSIM_WANT_GROUP_COUNTS) != 0;
     const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
     const uint32_t clk = (uint32_t)a.lat_lds_bytes + (uint32_t)wv * (uint32_t)a.wave_lds_bytes;
-    const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {first arrival, head, arrivals so far, rank of the head}
+    const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {-, head, behind the last arrival so far: places in the stream's lists; rank of the head}
 
     const int wave = a.paired ? tile : seed * a.tiles + tile;  // where this (tile, stream) pair's results go
     const int64_t off = a.stream_off[seed], R = a.stream_off[seed + 1] - off;
     const Req *__restrict__ reqs = a.streams + off;
     const int64_t *__restrict__ mo = a.mq_off + (size_t)seed * (M + 1);
     const MqEntry *__restrict__ mq = a.mq + mo[0];
-    const uint32_t *__restrict__ rows = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 8 + (lane & 7);
+    const uint32_t *__restrict__ rows = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 8;
+    constexpr bool ROWSLDS = 64 * MW <= kSoloRowsInLds;
+    const uint32_t rows16 = queues + (uint32_t)M * 16u;  // [M][8] the descriptors' low halves, if they are in LDS
     const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra;
     const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1);
     int32_t *model_good = a.model_good + (size_t)wave * M;
@@ -159,7 +188,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     // ---- state
     for (int s = lane; s < a.nslots; s += kWave) lds_put<double>(clk + (uint32_t)s * 8u, 0.0);
     for (int m = lane; m < M; m += kWave)
-        lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{(uint32_t)(mo[m] - mo[0]), 0u, 0u, (uint32_t)a.mq[mo[m]].rank});
+        lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{0u, (uint32_t)(mo[m] - mo[0]), (uint32_t)(mo[m] - mo[0]), (uint32_t)a.mq[mo[m]].rank});
+    if constexpr (ROWSLDS)
+        for (int x = lane; x < M * 8; x += kWave) lds_put<uint16_t>(rows16 + (uint32_t)x * 2u, (uint16_t)((rows[x] & 0x1FFFu) | (rows[x] >> 16 & 0x8000u)));
     uint64_t members[MW] = {};  // lane g: models of group g
     if (lane < a.Gmax) {
         const uint16_t *first = a.g2m_off + (size_t)tile * (a.Gmax + 1) + lane;
@@ -170,11 +201,15 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             for (int i = 0; i < MW; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
         }
     }
+    uint64_t hosting = 0;  // groups that host a model
+#pragma unroll
+    for (int i = 0; i < MW; ++i) hosting |= ballot(members[i] != 0ull);
+    const uint32_t group = lane < a.Gmax ? ginfo[lane] : 0u;  // lane g: descriptor of group g
     uint64_t waiting[MW] = {};  // models with waiting requests
     double ev_t = inf;          // lane e: event slot e
     uint32_t ev_d = 0;
     uint64_t used = 0;          // event slots that hold an event
-    int nfree = a.heap_cap;
+    const uint64_t slots = ~0ull >> (64 - a.heap_cap);
     double next_due = inf;      // the earliest event's time
     int32_t n_good = 0;
     double lat_sum = 0.0;       // of the batch members this lane accounts for
@@ -191,8 +226,23 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     auto set_waiting = [&](int m, bool on) {
 #pragma unroll
         for (int i = 0; i < MW; ++i) {
-            const uint64_t bit = MW == 1 || m >> 6 == i ? 1ull << (m & 63) : 0ull;
+            uint64_t bit = 1ull << (m & 63);
+            if (MW > 1) asm("s_cmp_eq_u32 %1, %2\ns_cselect_b64 %0, %3, 0" : "=s"(bit) : "s"(m >> 6), "n"(i), "s"(bit) : "scc");
             waiting[i] = on ? waiting[i] | bit : waiting[i] & ~bit;
+        }
+    };
+
+    // the models m of these octets wait
+    auto add_waiting = [&](int m, uint64_t lanes) {
+        if constexpr (MW <= 2) {
+            uint32_t bits[2 * MW];
+#pragma unroll
+            for (int i = 0; i < 2 * MW; ++i) bits[i] = in_mask(lanes & ballot(m >> 5 == i)) ? 1u << (m & 31) : 0u;
+            octets_or(bits);
+#pragma unroll
+            for (int i = 0; i < MW; ++i) waiting[i] |= (uint64_t)bits[2 * i + 1] << 32 | bits[2 * i];
+        } else {
+            for (lanes &= kFirstOfOctets; lanes != 0ull; lanes &= lanes - 1) set_waiting(lane_value(m, first_of(lanes)), true);
         }
     };
 
@@ -212,7 +262,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 #pragma unroll
         for (int i = 0; i < MW; ++i) {
             rank[i] = 0xFFFFFFFFu;
-            if (cand[i] >> lane & 1ull) rank[i] = lds_get<uint32_t>(queues + (uint32_t)(64 * i + lane) * 16u + 12u);
+            if (in_mask(cand[i])) rank[i] = lds_get<uint32_t>(queues + (uint32_t)(64 * i + lane) * 16u + 12u);
             least = rank[i] < least ? rank[i] : least;
         }
         least = wave_min(least);
@@ -241,7 +291,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         }
         if (lane == slot) ev_t = inf;
         used &= ~(1ull << slot);
-        nfree += 1;
         next_due = wave_min(ev_t);
         return d;
     };
@@ -255,15 +304,18 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 #pragma unroll
         for (int u = 0; u < 4; ++u) c0[u] = lds_get<double>(gclk + (uint32_t)u * 8u);
         // fn(k, clock) for the stages in turn.  Nested, so that a shallow group leaves with one branch taken.
+        // (The number of stages anew, or the compiler keeps each comparison as a mask of lanes.)
         auto walk = [&](auto &&fn) {
+            int n = stages;
+            asm("" : "+s"(n));
             fn(0, c0[0]);
-            if (stages > 1) {
+            if (n > 1) {
                 fn(1, c0[1]);
-                if (stages > 2) {
+                if (n > 2) {
                     fn(2, c0[2]);
-                    if (stages > 3) {
+                    if (n > 3) {
                         fn(3, c0[3]);
-                        for (int k = 4; k < stages; ++k) fn(k, lds_get<double>(gclk + (uint32_t)k * 8u));
+                        for (int k = 4; k < n; ++k) fn(k, lds_get<double>(gclk + (uint32_t)k * 8u));
                     }
                 }
             }
@@ -271,48 +323,46 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         for (;;) {
             const uint32_t lat_mg = ((uint32_t)m * (uint32_t)a.lat_row + desc_lat_off(d)) * (uint32_t)NB;
             const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
-            const uint32_t base = uni(queue.x), arr = uni(queue.z);
-            uint32_t h = uni(queue.y);  // arr - h > 0: the caller saw a waiting request
-            // lane j takes entry j from the head of the queue on, whether it has arrived yet or not
-            const MqEntry *ep = mq + (size_t)base + h + (lane & 15);
-            double2 hv = *reinterpret_cast<const double2 *>(ep);
-            int2 ir = *reinterpret_cast<const int2 *>(&ep->idx);
-            // when a batch started now leaves the last stage, lane j: latency column j (:666-672)
             const int col_j = (lane & 7) < NB ? lane & 7 : NB - 1;
             const float lu = UNIF ? lat_at(lat_mg + (uint32_t)col_j) : 0.0f;
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t arr = uni(queue.z);
+            uint32_t h = uni(queue.y);  // arr - h > 0: the caller saw a waiting request
+            // lane j takes entry j from the head of the queue on, whether it has arrived yet or not
+            const MqEntry *ep = mq + (size_t)h + (lane & 15);
+            double2 hv = *reinterpret_cast<const double2 *>(ep);
+            int rank = ep->rank, idx = want_req ? ep->idx : 0;
+            __builtin_amdgcn_sched_barrier(0);
+            // when a batch started now leaves the last stage, lane j: latency column j (:666-672)
             double tcol = t0;
             walk([&](int k, double c) { tcol = max_nn(c, tcol) + (double)(UNIF ? lu : lat_at(lat_mg + (uint32_t)(k * NB + col_j))); });
-            const double alone = lane_value(tcol, 0) + overhead;
-            // drop heads that cannot meet their deadline even alone (:677-686)
-            bool found = false;
-            uint32_t first = 0;  // place of the head that leads the batch, in the model's list
-            int kfirst = 0;      // and among the entries fetched
-            double deadline = 0.0;
-            for (;;) {
-                const int avail = (int)(arr - h) < 8 ? (int)(arr - h) : 8;
-                const uint64_t pass = ballot(lane < avail && alone <= hv.y);
-                const int k = pass != 0ull ? first_of(pass) : avail;  // the heads before k are dropped
+            tcol += overhead;
+            const double alone = lane_value(tcol, 0);
+            // drop heads that cannot meet their deadline even alone (:677-686): up to eight at a time
+            auto first_that_can = [&](int avail) -> int {  // avail: none of them
+                const uint64_t pass = ballot(lane < avail) & ballot(alone <= hv.y);
+                const int k = pass != 0ull ? first_of(pass) : avail;
                 if (want_req && lane < k) {
-                    fin_out[ir.x] = hv.x;
-                    good_out[ir.x] = 0;
+                    fin_out[idx] = hv.x;
+                    good_out[idx] = 0;
                 }
                 if (want_group && lane == 0) group_req[g] += k;
-                if (pass != 0ull) {
-                    found = true;
-                    kfirst = k;
-                    first = h + (uint32_t)k;
-                    deadline = lane_value(hv.y, k);
-                    h = first + 1u;
-                    break;
-                }
+                return k;
+            };
+            auto waiting_heads = [&]() -> int { return (int)(arr - h) < 8 ? (int)(arr - h) : 8; };
+            int avail = waiting_heads(), kfirst = first_that_can(avail);  // kfirst: place of the one that leads the batch, among the entries fetched
+            while (kfirst == avail) {
                 h += (uint32_t)avail;
                 if (h == arr) break;  // (else there are more than eight)
-                ep = mq + (size_t)base + h + (lane & 15);
+                ep = mq + (size_t)h + (lane & 15);
                 hv = *reinterpret_cast<const double2 *>(ep);
-                ir = *reinterpret_cast<const int2 *>(&ep->idx);
+                rank = ep->rank;
+                if (want_req) idx = ep->idx;
+                avail = waiting_heads();
+                kfirst = first_that_can(avail);
             }
-            if (!found) {  // :709-713
-                const int32_t next_rank = mq[(size_t)base + h].rank;
+            if (h == arr) {  // none of them (:709-713)
+                const int32_t next_rank = mq[(size_t)h].rank;
                 set_waiting(m, false);
                 const int m_next = select_model(g);
                 lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, h);
@@ -322,16 +372,19 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 if (m < 0) return;
                 continue;
             }
+            const uint32_t first = h + (uint32_t)kfirst;  // its place in the model's list
+            const double deadline = lane_value(hv.y, kfirst);
             // grow the batch while the first request still meets its deadline (:693-702): lane b tests batch size b, the
             // batch is the last size before the first one that fails
             double tc = tcol;
             if (rarely(!sizes_pow2)) tc = __hiloint2double(__shfl(__double2hiint(tcol), cand_col), __shfl(__double2loint(tcol), cand_col));
-            const bool ok = lane == 0 || (lane < NB && cand - 1 <= (int)(arr - h) && tc + overhead <= deadline);
-            const int sizes = first_of(~ballot(ok));  // (NB < 64)
+            const uint64_t fits = ballot(lane < NB) & ballot(cand <= (int)(arr - first)) & ballot(tc <= deadline);
+            const int sizes = first_of(~(fits | 1ull));  // (NB < 64)
             const int bs = lane_value(cand, sizes - 1), col = lane_value(cand_col, sizes - 1);
             // run it (:715-732)
             const int kb = kfirst + bs;  // the rank of the arrival after the batch
-            const uint32_t next_rank = kb < 16 ? (uint32_t)lane_value(ir.y, kb) : (uint32_t)mq[(size_t)base + first + (uint32_t)bs].rank;
+            uint32_t next_rank = (uint32_t)lane_value(rank, kb & 15);
+            if (rarely(kb >= 16)) next_rank = uni((uint32_t)mq[(size_t)first + (uint32_t)bs].rank);
             double t = t0 + overhead, idle_at = 0.0;
             const float lb = UNIF ? lane_value(lu, col) : 0.0f;
             walk([&](int k, double c) {
@@ -350,16 +403,16 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             // (sums by place in the queue, see above)
             if (lane >= kfirst && lane < kfirst + bs && lane < 8) lat_sum += t - hv.x;
             for (int k = 8; rarely(k < kb); ++k) {
-                const double at = k < 16 ? lane_value(hv.x, k) : mq[(size_t)base + first + (uint32_t)(k - kfirst)].t;
+                const double at = k < 16 ? lane_value(hv.x, k) : mq[(size_t)first + (uint32_t)(k - kfirst)].t;
                 if (lane == 0) lat_sum += t - at;
             }
             if (want_req) {
                 if (lane >= kfirst && lane < kb && lane < 16) {
-                    fin_out[ir.x] = t;
-                    good_out[ir.x] = 1;
+                    fin_out[idx] = t;
+                    good_out[idx] = 1;
                 }
                 for (int k = 16 + lane; k < kb; k += kWave) {
-                    const int32_t r = mq[(size_t)base + first + (uint32_t)(k - kfirst)].idx;
+                    const int32_t r = mq[(size_t)first + (uint32_t)(k - kfirst)].idx;
                     fin_out[r] = t;
                     good_out[r] = 1;
                 }
@@ -370,11 +423,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 group_good[g] += bs;
             }
             if (want_model && lane == 0) model_good[m] += bs;
-            if (rarely(nfree == 0)) {
+            if (rarely(used == slots)) {  // nothing more happens; the arrivals' loop looks at `dead` once a window
                 dead = MMSIM_E_OVERFLOW;
+                used = 0ull;
+                next_due = inf;
                 return;
             }
-            nfree -= 1;
             const int slot = first_of(~used);
             used |= 1ull << slot;
             if (lane == slot) {
@@ -388,13 +442,13 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 
     // idle events that are due at time tstamp (:739-744)
     auto due_events = [&](double tstamp) {
-        while ((int)(next_due <= tstamp) & (int)(used != 0ull)) {
+        while (next_due <= tstamp) {
+            if (rarely(used == 0ull)) break;  // (tstamp: +inf)
             const double T = next_due;
             const uint32_t d = take_event(T);
             const int m = select_model(desc_group(d));
             if (m < 0) break;  // the popped event is dropped, later due events stay (:742-743)
             handle(T, m, d);
-            if (rarely(dead != 0)) break;
         }
     };
 
@@ -404,101 +458,111 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         if (i + lane < R) r = reqs[i + lane];
         return r;
     };
-    auto row_word = [&](int m) -> uint32_t { return rows[(size_t)(m < 0 ? 0 : m) * 8]; };
+    auto row_word = [&](int m) -> uint32_t {
+        const uint32_t at = (uint32_t)(m < 0 ? 0 : m) * 8u + (uint32_t)(lane & 7);
+        if constexpr (ROWSLDS) return (uint32_t)(int32_t)lds_get<int16_t>(rows16 + at * 2u);
+        return rows[at];
+    };
+    auto time_of = [&](const Req &r, int l) -> double { return __hiloint2double(__shfl(__double2hiint(r.t), l), __shfl(__double2loint(r.t), l)); };
     Req block = fetch_block(0), block_next = fetch_block(kWave);
-    int m_next = __shfl(block.m, oct);
-    uint32_t d_next = row_word(m_next);
+    // of the next window, and the models of the one after it
+    int m1 = __shfl(block.m, oct), m2 = __shfl(block.m, 8 + oct);
+    uint32_t d1 = row_word(m1);
+    double t1 = time_of(block, oct);
     for (int64_t w0 = 0; w0 < R && !dead; w0 += 8) {
         const int from = (int)(w0 & 63) + oct;  // the lane that holds this octet's request
         const int n = R - w0 < 8 ? (int)(R - w0) : 8;
-        const int m = m_next;
-        const uint32_t dj = d_next;
-        const double t = __hiloint2double(__shfl(__double2hiint(block.t), from), __shfl(__double2loint(block.t), from));
+        const int m = m1;
+        const uint32_t dj = d1;
+        const double t = t1;
+        last = clk + desc_last_slot(dj) * 8u;
+        c_last = lds_get<double>(last);
+        c_first = lds_get<double>(last - desc_stages_m1(dj) * 8u);
         if ((w0 & 63) == 56) {
             block = block_next;
             block_next = fetch_block(w0 + 8 + kWave);
         }
-        m_next = __shfl(block.m, (from + 8) & 63);  // (past the end of the stream: -1)
-        d_next = row_word(m_next);
-        const bool valid = (int32_t)dj >= 0 && m >= 0;
-        const uint32_t vb = oct_ballot(valid);
-        const bool hosted = (vb & 1u) != 0, longer = (vb >> 7) != 0;  // longer: the list may go on
-        last = clk + desc_last_slot(dj) * 8u;
-        c_last = lds_get<double>(last);
-        c_first = lds_get<double>(last - desc_stages_m1(dj) * 8u);
-        int cur = 0;        // arrivals before this one are settled
-        int seen_due = -1;  // the arrival whose due events have been seen to
+        m1 = m2;
+        d1 = row_word(m1);  // (past the end of the stream: -1)
+        t1 = time_of(block, (from + 8) & 63);
+        m2 = __shfl((w0 & 63) == 48 ? block_next.m : block.m, (from + 16) & 63);
+        const bool valid = ((int32_t)dj >= 0) & (m >= 0);
+        const uint64_t valids = ballot((int32_t)dj >= 0) & ballot(m >= 0), known = ballot(m >= 0);
+        const uint64_t hosted = valids & kFirstOfOctets, longer = valids >> 7 & kFirstOfOctets;  // longer: the list may go on
+        const uint64_t here = ~0ull >> (64 - 8 * n);
+        int cur = 0;             // arrivals before this one are settled
+        uint64_t unseen = ~0ull;  // arrivals whose due events have not been seen to
         while (cur < n) {
-            const double t_cur = lane_value(t, cur * 8);
-            if ((int)(next_due <= t_cur) & (int)(cur > seen_due)) {  // events first (:739-744)
-                due_events(t_cur);
-                seen_due = cur;
-                if (rarely(dead != 0)) break;
+            uint64_t due = ballot(next_due <= t) & unseen;
+            if ((due >> (cur * 8) & 1ull) != 0ull) {  // events first (:739-744)
+                due_events(lane_value(t, cur * 8));
+                unseen = ~0xFFull << (cur * 8);
+                due = ballot(next_due <= t) & unseen;
             }
             const double mn = oct_min(valid ? c_last : inf);
-            const uint32_t least = oct_ballot(valid && c_last == mn), free = oct_ballot(t >= c_first);
-            const int selj = __ffs((int)least) - 1;  // the first listed of those with the smallest last-stage clock
-            const bool found = hosted & (mn < 1e100), idle = found & (((free >> (selj & 7)) & 1u) != 0);
-            const bool special = hosted & (!found | longer), due = (next_due <= t) & (oct > seen_due);
-            const bool happens = (oct >= cur) & (oct < n) & (due | idle | special);
-            const uint64_t hb = ballot(happens);
-            const int f = hb != 0ull ? first_of(hb) >> 3 : n;
-            if (oct >= cur && oct < f && (lane & 7) == 0 && m >= 0)
+            const uint64_t found = ballot(mn < 1e100);
+            // the first listed of those with the smallest last-stage clock
+            const uint64_t selected = first_of_octets(ballot(c_last == mn) & valids);
+            const uint64_t idle = selected & found & ballot(t >= c_first), special = hosted & (~found | longer);
+            const uint64_t left = here & ~0ull << (cur * 8), happens = left & (due | idle | special);
+            // those before the first at which something happens join their queues, and that one unless it has events first
+            uint64_t joining = left;
+            int f = n;
+            if (happens != 0ull) {
+                f = first_of(happens) >> 3;
+                joining &= (((due >> (f * 8) & 1ull) != 0ull ? 1ull : 0x100ull) << (f * 8)) - 1ull;
+            }
+            if (in_mask(joining & known & kFirstOfOctets))
                 __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u + 8u), 1u,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            if (want_req && oct >= cur && oct < f && (lane & 7) == 0 && !hosted) {
+            if (want_req && in_mask(joining & kFirstOfOctets & ~hosted)) {
                 fin_out[w0 + oct] = t;
                 good_out[w0 + oct] = 0;
             }
             wave_order();
-            for (; cur < f; ++cur) {
-                const int mc = lane_value(m, cur * 8);
-                if (mc >= 0) set_waiting(mc, true);
-            }
-            if (f == n) break;
+            add_waiting(m, joining & known);
+            cur = f;
+            if (happens == 0ull) break;
             const int fl = f * 8;
+            if ((due >> fl & 1ull) != 0ull) continue;
+            // its group turns to the arrival if it is idle (:746-778)
+            cur = f + 1;
             const double tf = lane_value(t, fl);
-            if ((int)(next_due <= tf) & (int)(f > seen_due)) continue;  // its events first
-            // the arrival joins its queue, and its group turns to it if it is idle (:746-778)
             const int mf = lane_value(m, fl);
-            uint32_t dsel = kEmpty;
-            bool ready = lane_value((int)idle, fl) != 0;
-            const uint32_t listed = lane_value(dj, fl + (lane_value(selj, fl) & 7));
-            if (lane_value((int)found, fl) != 0) dsel = listed;
-            if (rarely(lane_value((int)longer, fl) != 0)) {
-                const double best0 = lane_value(mn, fl);
-                double best = best0 < 1e100 ? best0 : 1e100;
-                for (int x = 0; x < a.rep_extra; ++x) {
-                    const uint32_t g = more_replicas[(size_t)mf * a.rep_extra + x];
-                    if (g == (uint32_t)a.Gmax) break;
-                    const uint32_t d2 = ginfo[g];
-                    const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
-                    if (c2 < best) {
-                        best = c2;
-                        dsel = d2;
-                        ready = tf >= uni(lds_get<double>(clk + (desc_last_slot(d2) - desc_stages_m1(d2)) * 8u));
+            uint32_t dsel = lane_value(dj, first_of(selected >> fl) + fl);
+            if (ROWSLDS) dsel = lane_value(group, first_of(ballot((group & 0x1FFFu) == (dsel & 0x1FFFu)) & hosting));
+            bool ready = (idle >> fl & 0xFFull) != 0ull;
+            if (rarely((special >> fl & 1ull) != 0ull)) {
+                double best = lane_value(mn, fl);
+                if (!(best < 1e100)) {
+                    best = 1e100;
+                    dsel = kEmpty;
+                    ready = false;
+                }
+                if ((longer >> fl & 1ull) != 0ull)
+                    for (int x = 0; x < a.rep_extra; ++x) {
+                        const uint32_t g = more_replicas[(size_t)mf * a.rep_extra + x];
+                        if (g == (uint32_t)a.Gmax) break;
+                        const uint32_t d2 = ginfo[g];
+                        const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
+                        if (c2 < best) {
+                            best = c2;
+                            dsel = d2;
+                            ready = tf >= uni(lds_get<double>(clk + (desc_last_slot(d2) - desc_stages_m1(d2)) * 8u));
+                        }
                     }
+                dsel = uni(dsel);
+                if (rarely(dsel == kEmpty)) {  // every replica's clock is infinite (sim_batching.hip says when)
+                    dead = MMSIM_E_UNSUPPORTED;
+                    used = 0ull;
+                    break;
                 }
             }
-            dsel = uni(dsel);
-            if (lane == 0)
-                __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)mf * 16u + 8u), 1u,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            wave_order();
-            set_waiting(mf, true);
-            cur = f + 1;
-            if (rarely(dsel == kEmpty)) {  // every replica's clock is infinite (sim_batching.hip says when)
-                dead = MMSIM_E_UNSUPPORTED;
-                break;
-            }
-            if (ready) {
-                handle(tf, mf, dsel);
-                if (rarely(dead != 0)) break;
-            }
+            if (ready) handle(tf, mf, dsel);
         }
     }
     // ---- drain (:781-787)
-    while (!dead && used != 0ull) {
+    while (used != 0ull && !dead) {
         const double T = next_due;
         const uint32_t d = take_event(T);
         const int m = select_model(desc_group(d));

@@ -436,9 +436,9 @@ def test_models_of_one_simulation(eng, M):
     assert 0 < g0.sum() < R
 
 
-@pytest.mark.parametrize("B,n_streams,R,solo", [(71, 29, 511, False), (71, 29, 512, True), (320, 32, 513, True), (321, 32, 513, False)])
+@pytest.mark.parametrize("B,n_streams,R,solo", [(71, 29, 511, False), (71, 29, 512, True), (512, 32, 513, True), (513, 32, 513, False)])
 def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, solo):
-    """Up to forty simulations to a CU have a wavefront each, unless their streams are short: the oracle's counts and
+    """Up to sixty-four simulations to a CU have a wavefront each, unless their streams are short: the oracle's counts and
     traces on both sides of either line."""
     cfg = make_config(5, B)
     table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
