@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <functional>
 #include <limits>
@@ -233,6 +234,30 @@ int mmsim::compact_latency(const mmsim_tables *t, bool all_batch_sizes, CompactL
 }
 
 namespace {
+
+// How busy the streams keep the groups, about: requests of a second, times the time a group needs for one (the longest of
+// its stages, alone in its batch, over the models as often as they are asked for), over the groups of a placement.
+double offered_load(const mmsim_workload *const *wls, int32_t n_streams, const mmsim_tables *t, const RepLists &rl) {
+    double requests = 0.0, seconds = 0.0;
+    std::vector<double> weight(t->M, 0.0), busy(t->C, 0.0);
+    for (int s = 0; s < n_streams; ++s) {
+        seconds += wls[s]->span;
+        for (int32_t m = 0; m < t->M; ++m) {
+            weight[m] += (double)wls[s]->model_num_requests[m];
+            requests += (double)wls[s]->model_num_requests[m];
+        }
+    }
+    for (int32_t c = 0; c < t->C; ++c)
+        for (int32_t m = 0; m < t->M; ++m) {
+            float longest = 0.0f;
+            for (int k = 0; k < t->cfg_pp[c]; ++k) longest = std::max(longest, t->cfg_lat[(((size_t)m * t->C + c) * t->Smax + k) * t->NB]);
+            if (std::isfinite(longest)) busy[c] += weight[m] / requests * (double)longest;
+        }
+    double a_second = 0.0;  // requests that the groups of all placements take in a second
+    for (int32_t p = 0; p < rl.B; ++p)
+        for (int32_t g = 0; g < rl.num_groups[p]; ++g) a_second += 1.0 / std::max(1e-9, busy[rl.group_cfg[(size_t)p * rl.Gmax + g]]);
+    return a_second > 0.0 && seconds > 0.0 ? requests / seconds * rl.B / a_second : 0.0;
+}
 
 // Builds every device table of a batch from replica lists and launches nothing.
 int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
@@ -524,25 +549,28 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
         const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(M, t->NB, heap_cap, Gmax) && rl.models_ascend();
-        // A wavefront for each simulation (sim_batching_solo.hip) up to 64 of them to a CU, of which it takes 20 at once.  ms
-        // with octets / with these, 150000 requests, 96 models on 48 devices: 2048 simulations 54 / 39, 3072 132 / 46, 4096 133
-        // / 52, 8192 161 / 90, 16384 200 / 157; 30000 requests at a lower load, 48 models on 24 devices: 8192 61 / 40, 16384 73 /
-        // 67, 65536 216 / 235 (the octets of a wavefront share the cost of a step).  Streams of a few hundred requests are over
-        // within a millisecond and keep fewer wavefronts (16384 simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
-        const int64_t solo_per_cu = std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
+        // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them; beyond that,
+        // up to 64, if the groups are busy.  ms with octets / with these, 150000 requests, 96 models on 48 devices, all of them
+        // busy: 2048 simulations 54 / 39, 3072 132 / 46, 4096 133 / 52, 8192 161 / 90, 16384 200 / 157; 30000 requests, 48 models
+        // on 24 devices, half of them: 8192 61 / 40, 16384 73 / 67, 65536 216 / 235; 23108 requests, 5 models on 49 devices, a
+        // tenth, where nearly every request is a batch and the octets of a wavefront share the cost of their events: 4096 164 /
+        // 116, 8192 181 / 202.  Streams of a few hundred requests are over within a millisecond and keep fewer wavefronts (16384
+        // simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
+        const int64_t cus = std::max(1, ctx->prop.multiProcessorCount), sims = (int64_t)B * b->out_seeds;
+        const int64_t at_once = cus * std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         int64_t requests = 0;
         for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
+        const bool all_solo = can_solo && requests >= (int64_t)512 * n_seeds &&
+                              (sims <= at_once || (sims <= at_once * 64 / kSoloWavesPerCu && offered_load(wls, n_seeds, t, rl) >= 0.5));
         if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
-        } else if (can_solo && requests >= (int64_t)512 * n_seeds &&
-                   (int64_t)B * b->out_seeds <= 64 * solo_per_cu / kSoloWavesPerCu * std::max(1, ctx->prop.multiProcessorCount)) {
+        } else if (all_solo) {
             tile_sims = 1;
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
             // devices, ms at 8 / 4 / 2 / 1 simulations, a single one in the kernel that looks at eight arrivals at once: 1024
             // placements 16.6 / 13.8 / 11.4 / 7.4, 4096: 17.3 / 14.8 / 12.7 / 16.0 (two rounds), 8192: 17.7 / 15.8 / 25).
-            const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
             const size_t least = bytes_for(8, std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7)));  // (event slots are trimmed below)
             const int64_t per_cu = std::max<int64_t>(1, std::max(std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / least)),
                                                                  2 * std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / 2 / least))));
@@ -1356,6 +1384,7 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
         if (i > 0 && host[i].m == host[i - 1].m) w->repeats += 1;
         if (i > 0 && tstamps[i] < tstamps[i - 1]) sorted = false;
     }
+    if (R > 0) w->span = std::max(0.0, tstamps[R - 1] - tstamps[0]);
     w->mq_off.assign((size_t)M + 1, 0);
     for (int32_t m = 0; m < M; ++m) w->mq_off[m + 1] = w->mq_off[m] + w->model_num_requests[m];
     const size_t known = (size_t)w->mq_off[M];

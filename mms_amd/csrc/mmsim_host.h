@@ -189,6 +189,7 @@ struct mmsim_workload {
     int32_t M = 0;
     std::shared_ptr<DevBuf<Req>> reqs = std::make_shared<DevBuf<Req>>();  // shared with batches that read it in place
     std::vector<int32_t> model_num_requests;  // requests per model id (placement independent)
+    double span = 0.0;                        // from the first arrival to the last
     int64_t repeats = 0;                      // requests with the model of the request before
     // arrivals regrouped by model (batching simulator): offsets per model, then per arrival
     // its time, its deadline time + (double)slo and its index in the stream

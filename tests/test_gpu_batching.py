@@ -436,16 +436,17 @@ def test_models_of_one_simulation(eng, M):
     assert 0 < g0.sum() < R
 
 
-@pytest.mark.parametrize("B,n_streams,R,solo", [(71, 29, 511, False), (71, 29, 512, True), (512, 32, 513, True), (513, 32, 513, False)])
-def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, solo):
-    """Up to sixty-four simulations to a CU have a wavefront each, unless their streams are short: the oracle's counts and
-    traces on both sides of either line."""
+@pytest.mark.parametrize("B,n_streams,R,pace,solo", [(71, 29, 511, 3.0, False), (71, 29, 512, 3.0, True), (512, 32, 513, 3.0, True), (513, 32, 513, 3.0, False),
+                                                     (160, 32, 520, 0.01, True), (161, 32, 520, 0.01, False)])
+def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, pace, solo):
+    """Twenty simulations to a CU, or sixty-four if their groups are busy, have a wavefront each, unless their streams are
+    short: the oracle's counts and traces on both sides of each line."""
     cfg = make_config(5, B)
     table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
     packed = E.pack_placements(cfg.placements, table)
     st = cfg.stream(0)
     cut = [slice(997 * k, 997 * k + R) for k in range(n_streams)]
-    streams = [SimpleNamespace(tstamps=(st.tstamps[c] - st.tstamps[c.start]) / 3, model_ids=st.model_ids[c], slos=st.slos[c]) for c in cut]
+    streams = [SimpleNamespace(tstamps=(st.tstamps[c] - st.tstamps[c.start]) / pace, model_ids=st.model_ids[c], slos=st.slos[c]) for c in cut]
     dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, cfg.num_models) for s in streams]
     counts = _lib.WANT_MODEL_COUNTS | _lib.WANT_GROUP_COUNTS
     for flags in (0, counts, counts | _lib.WANT_PER_REQUEST):
