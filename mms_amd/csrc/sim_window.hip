@@ -39,6 +39,10 @@
 // block, 53 % of them issuing (418 instructions) and 46 % waiting; 4096 placements, four wavefronts to a SIMD, 5.6 ms,
 // 4800 cycles a block, 40 % issuing, 32 % waiting to issue, 28 % for LDS.  (One request after the other, 64 placements to
 // a wavefront: 24 ms either way.)
+// Few instructions to a step count most where a wavefront is alone.  That a block's second four replicas are in registers like
+// the first, instead of being fetched for every step (only blocks with a ninth do that), and that the words that the walk
+// needs are ready for it took, 108000 requests: 700 placements of single-device groups, a model in 25 on more than four of them, 6.1
+// -> 5.3 ms, 1025 placements of groups up to 16 deep 15.5 -> 13.1 ms, 600 of four-stage pipelines 10.4 -> 9.65 ms.
 //
 // LDS of one placement (byte offsets in WindowArgs, built by the wavefront itself from the packed placement):
 //   clk  [slots+SMAX] f64   stage clocks, a placement's groups laid end to end, and SMAX slots for what does not count
@@ -50,7 +54,7 @@
 //   gd   [Gmax] u32         entry word of every group
 //   mcnt [M] u32            accepted requests per model  (OUTPUTS)
 // Entry word: bits 0-14 LDS address / 8 of the group's last-stage clock, 15-19 stages - 1, 20-29 index of its
-// last-stage latency in the model's row of the latency table, 30 (fourth entry) "there are more", 31 "no such replica":
+// last-stage latency in the model's row of the latency table, 30 "there are more" (fourth entry), "more than eight" (third), 31 "no such replica":
 // the word then repeats the first replica's (which wins every tie against its copies) or, without any replica, the
 // placement's first slot.
 #include "mmsim_internal.h"
@@ -65,10 +69,10 @@ __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_bal
 __device__ __forceinline__ bool in_mask(uint64_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes); }
 // a request of the stream: a load that only counts as global (through a generic pointer it would be waited for with
 // the LDS accesses)
-__device__ __forceinline__ Req load_global(const Req *p) {
-    const u32x4 v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4 *>(reinterpret_cast<uintptr_t>(p));
-    return Req{__hiloint2double((int)v.y, (int)v.x), (int32_t)v.z, __uint_as_float(v.w)};
+__device__ __forceinline__ u32x4 load_global(const Req *p) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) u32x4 *>(reinterpret_cast<uintptr_t>(p));
 }
+__device__ __forceinline__ Req as_req(const u32x4 &v) { return Req{__hiloint2double((int)v.y, (int)v.x), (int32_t)v.z, __uint_as_float(v.w)}; }
 // Marks the places where the lanes' LDS accesses depend on one another: the compiler keeps them on their side (a
 // wavefront's LDS accesses are carried out in order; no instruction).
 __device__ __forceinline__ void wave_order() {
@@ -94,12 +98,7 @@ __device__ __forceinline__ void lds_put(uint32_t addr, T v) {
     *reinterpret_cast<__attribute__((address_space(3))) T *>(addr) = v;
 }
 // waits for a request on its way here, not inside the loops that follow
-__device__ __forceinline__ void arrived_req(Req &r) {
-    uint32_t w[4];
-    __builtin_memcpy(w, &r, 16);
-    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
-    __builtin_memcpy(&r, w, 16);
-}
+__device__ __forceinline__ void arrived(u32x4 &r) { asm volatile("" : "+v"(r)); }
 // keeps the compiler from merging what made v with what uses it
 __device__ __forceinline__ void pin(uint32_t &v) { asm volatile("" : "+v"(v)); }
 // LDS atomics whose result nobody waits for
@@ -184,14 +183,6 @@ struct Entry4 {
     Entry e[4];
 };
 __device__ __forceinline__ float as_float(uint32_t v) { return __uint_as_float(v); }
-__device__ __forceinline__ uint32_t as_uint(float v) { return __float_as_uint(v); }
-__device__ __forceinline__ Req fetch_req(uint32_t addr) {
-    const u32x4 v = lds_get<u32x4>(addr);
-    return Req{__hiloint2double((int)v.y, (int)v.x), (int32_t)v.z, as_float(v.w)};
-}
-__device__ __forceinline__ void store_req(uint32_t addr, const Req &r) {
-    lds_put<u32x4>(addr, u32x4{(uint32_t)__double2loint(r.t), (uint32_t)__double2hiint(r.t), (uint32_t)r.m, as_uint(r.slo)});
-}
 __device__ __forceinline__ Entry4 load_entries(uint32_t addr) {  // two 16-byte reads
     const u32x4 a = lds_get<u32x4>(addr), b = lds_get<u32x4>(addr + 16u);
     return Entry4{{{a.x, as_float(a.y)}, {a.z, as_float(a.w)}, {b.x, as_float(b.y)}, {b.z, as_float(b.w)}}};
@@ -293,7 +284,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         int k = 0;
         auto put = [&](const Entry &e) {
             const uint32_t at = k < 4 ? rep + (uint32_t)(m * 4 + k) * 8u : ext + (chunk0 * 4u + (uint32_t)(k - 4)) * 8u;
-            lds_put<uint32_t>(at, k == 3 && n > 4 ? e.d | kEntryMore : e.d);
+            lds_put<uint32_t>(at, (k == 3 && n > 4) || (k == 2 && n > 8) ? e.d | kEntryMore : e.d);
             lds_put<float>(at + 4u, e.l);
             ++k;
         };
@@ -319,8 +310,8 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     uint8_t *good_out = a.good + row * (size_t)a.Rmax;
     const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
 
-    auto load_req = [&](uint32_t i) -> Req {
-        Req r{0.0, -1, 0.0f};
+    auto load_req = [&](uint32_t i) -> u32x4 {
+        u32x4 r{0u, 0u, ~0u, 0u};
         if (i < R) r = load_global(reqs + i);
         return r;
     };
@@ -328,31 +319,37 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     // Requests come 64 at a time, one to a lane.  W == 64: that is a block, fetched two blocks ahead.  Otherwise the
     // chunks pass through LDS, which deals them to the placements' lanes; the chunk after the one a block is of is in
     // LDS as well, and the one after that on its way.
-    Req far = load_req((uint32_t)lane);
-    Req cur, nxt;
-    auto store_ring = [&](uint32_t chunk) { store_req(ring + (chunk & 1u) * 1024u + (uint32_t)lane * 16u, far); };
-    auto load_ring = [&](uint32_t i) -> Req { return fetch_req(ring + (i & 127u) * 16u); };
+    u32x4 far = load_req((uint32_t)lane);
+    Req cur;
+    u32x4 nxt;
+    auto store_ring = [&](uint32_t chunk) { lds_put<u32x4>(ring + (chunk & 1u) * 1024u + (uint32_t)lane * 16u, far); };
+    auto load_ring = [&](uint32_t i) -> u32x4 { return lds_get<u32x4>(ring + (i & 127u) * 16u); };
     if constexpr (W == 64) {
-        cur = far;
         nxt = load_req(64u + (uint32_t)lane);
+        arrived(far);  // (here, or the first step of every block waits for what is on its way then)
+        arrived(nxt);
+        cur = as_req(far);
     } else {
         store_ring(0u);
         far = load_req(64u + (uint32_t)lane);
         store_ring(1u);
         far = load_req(128u + (uint32_t)lane);
         wave_order();
-        cur = load_ring((uint32_t)j);
+        cur = as_req(load_ring((uint32_t)j));
         nxt = load_ring((uint32_t)(W + j));
     }
     Entry4 q = load_rep(cur.m);
     // What a block is like: requests that can be served at all, that list several groups, more than two, more than
     // four; how deep their groups are.  Worked out a block ahead (a scalar that depends on vector compares is slow to come).
-    uint64_t pend, multis, fours, mores, deep_a, deep_b;
+    uint64_t pend, multis, fours, mores, eights, deep_a, deep_b;
     auto look = [&]() {
         pend = ballot(cur.m >= 0 && !entry_none(q.e[0].d));  // (past the end of the stream: m is -1)
         multis = ballot(!entry_none(q.e[1].d)) & pend;
         fours = ballot(!entry_none(q.e[2].d)) & pend;
-        if constexpr (EXT) mores = ballot((q.e[3].d & kEntryMore) != 0u) & pend;
+        if constexpr (EXT) {
+            mores = ballot((q.e[3].d & kEntryMore) != 0u) & pend;
+            eights = ballot((q.e[2].d & kEntryMore) != 0u) & pend;
+        }
         if constexpr (SMAX > 1) {
             const int deep = max2(max2(entry_stages_m1(q.e[0].d), entry_stages_m1(q.e[1].d)),
                                   max2(entry_stages_m1(q.e[2].d), entry_stages_m1(q.e[3].d)));
@@ -366,22 +363,33 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     };
     look();
 
+    // What a step needs of an entry word, ready for it: the address of the group's first clock and, from bit 18 on, stages - 1;
+    // of a single stage the address, of several latencies the word itself.
+    auto walk_word = [](uint32_t d) -> uint32_t {
+        if constexpr (SMAX > 1 && !UNIFORM) return d;
+        return SMAX == 1 ? entry_addr(d) : (entry_addr(d) - (uint32_t)entry_stages_m1(d) * 8u) | (uint32_t)entry_stages_m1(d) << 18;
+    };
+    auto first_clock = [](uint32_t w) -> uint32_t {
+        if constexpr (SMAX > 1 && !UNIFORM) return entry_addr(w) - (uint32_t)entry_stages_m1(w) * 8u;
+        return SMAX == 1 ? w : w & 0x3FFFFu;
+    };
+    auto stages_m1 = [](uint32_t w) -> int { return SMAX == 1 ? 0 : UNIFORM ? (int)(w >> 18) : entry_stages_m1(w); };
     for (uint32_t blk = 0; blk < R; blk += W) {
         const int m = cur.m;
         const double arr = cur.t, slo = (double)cur.slo;
-        uint32_t ca[4], word[4];  // what the tournament carries: the entry word, or all that single-stage groups need of it
+        uint32_t ca[4], word[4];  // what the tournament carries of an entry word
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             ca[k] = entry_addr(q.e[k].d);
-            word[k] = SMAX == 1 ? ca[k] : q.e[k].d;
+            word[k] = walk_word(q.e[k].d);
         }
         Entry4 nrep;
-        Req nn;
+        u32x4 nn;
         double best = 0.0, t = 0.0, latency = 0.0;
-        uint32_t chosen = clk;  // the chosen group's entry word (SMAX == 1: the address of its clock)
-        // The block, for requests that list at most NC groups (2, 4, or 5: more than four).
+        uint32_t chosen = SMAX > 1 && !UNIFORM ? clk >> 3 : clk;  // the chosen group's walk word
+        // The block, for requests that list at most NC groups (2, 4, 8, or 9: more than eight).
         auto block = [&](auto NCv) {
-            constexpr int NC = decltype(NCv)::value, N4 = NC > 4 ? 4 : NC;
+            constexpr int NC = decltype(NCv)::value, N4 = NC > 4 ? 4 : NC, NX = NC == 8 ? 4 : 0;
             double c[N4];
 #pragma unroll
             for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
@@ -393,10 +401,36 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                 x0 = ext + (v & 0xFFFFu) * 32u;
                 xn = in_mask(pend) ? v >> 16 : 0u;
             }
+            // up to eight: the second four like the first, in registers (of a request without: copies of its first, which
+            // never beat it)
+            Entry4 more = q;
+            uint32_t xa[4], xword[4];
+            double cx[4];
+            if constexpr (NX > 0) {
+                if (xn > 0u) more = load_entries(x0);
+                else more.e[1] = more.e[2] = more.e[3] = more.e[0];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    xa[k] = entry_addr(more.e[k].d);
+                    xword[k] = walk_word(more.e[k].d);
+                    cx[k] = lds_get<double>(xa[k]);
+                }
+            }
+            uint32_t ga[N4];
+#pragma unroll
+            for (int k = 0; k < N4; ++k) {
+                ga[k] = ca[k] + gm_rel;
+                pin(ga[k]);
+            }
             if (in_mask(pend)) {
 #pragma unroll
-                for (int k = 0; k < N4; ++k) lds_or_u64(ca[k] + gm_rel, my_bit);
-                if constexpr (NC > 4)
+                for (int k = 0; k < N4; ++k) lds_or_u64(ga[k], my_bit);
+                if constexpr (NX > 0) {
+                    if (xn > 0u) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) lds_or_u64(xa[k] + gm_rel, my_bit);
+                    }
+                } else if constexpr (NC > 4)
                     for (uint32_t x = 0; x < xn; ++x) {
                         const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
@@ -405,27 +439,35 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
             }
             wave_order();
 #pragma unroll
-            for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ca[k] + gm_rel) & before;
+            for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ga[k]) & before;
             uint64_t gm_ext = 0;  // requests before this one that share any of the groups: holds for every further replica
             if constexpr (NC > 4) {
-                for (uint32_t x = 0; x < xn; ++x) {
-                    const Entry4 e = load_entries(x0 + x * 32u);
+                if constexpr (NX > 0) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
+                    for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(xa[k] + gm_rel);
+                } else {
+                    for (uint32_t x = 0; x < xn; ++x) {
+                        const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
+                    }
                 }
                 gm_ext = (gm_ext & before) | gm[0] | gm[1] | gm[2] | gm[3];
             }
             wave_order();
 #pragma unroll
-            for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ca[k] + gm_rel, 0);  // for the next block
-            if constexpr (NC > 4)
+            for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ga[k], 0);  // for the next block
+            if constexpr (NX > 0) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) lds_put<uint64_t>(xa[k] + gm_rel, 0);
+            } else if constexpr (NC > 4)
                 for (uint32_t x = 0; x < xn; ++x) {
                     const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
                     for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
                 }
             // ---- fetched ahead: the requests of the block after the next, the replicas of the next
-            nrep = load_rep(nxt.m);
+            nrep = load_rep((int)nxt.z);
             if constexpr (W == 64) {
                 nn = load_req(blk + 128u + (uint32_t)j);
             } else {
@@ -465,28 +507,32 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     Cand win = first_min(Cand{c[0], word[0], q.e[0].l, gm[0]}, Cand{c[1], word[1], q.e[1].l, gm[1]});
                     if constexpr (NC > 2)
                         win = first_min(win, first_min(Cand{c[2], word[2], q.e[2].l, gm[2]}, Cand{c[3], word[3], q.e[3].l, gm[3]}));
-                    if constexpr (NC > 4)
+                    if constexpr (NX > 0) {
+                        Cand y[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) y[k] = Cand{cx[k], xword[k], more.e[k].l, gm_ext};
+                        win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
+                    } else if constexpr (NC > 4)
                         for (uint32_t x = 0; x < xn; ++x) {
                             const Entry4 e = load_entries(x0 + x * 32u);
                             Cand y[4];
 #pragma unroll
                             for (int k = 0; k < 4; ++k) {
                                 const uint32_t at = entry_addr(e.e[k].d);
-                                y[k] = Cand{lds_get<double>(at), SMAX == 1 ? at : e.e[k].d, e.e[k].l, gm_ext};
+                                y[k] = Cand{lds_get<double>(at), e.e[k].d, e.e[k].l, gm_ext};
                             }
-                            win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
+                            Cand z = first_min(first_min(y[0], y[1]), first_min(y[2], y[3]));
+                            z.d = walk_word(z.d);
+                            win = first_min(win, z);
                         }
                     best = win.c;
                     chosen = win.d;
-                    // a clock that is infinite is never chosen (:590-598)
-                    const double limit = __hiloint2double(best < 1e100 ? __double2hiint(slo) : 0x7FF80000, __double2loint(slo));
                     const double l_last = (double)win.l;
                     // ---- walk the stages and decide (:605-613).  All requests read and walk the near stages from their group's first
                     // on and take the time after their last one (what lies behind a shallower group's slots does not matter).
                     double cv[D];
-                    const uint32_t last = SMAX == 1 ? win.d : entry_addr(win.d);
-                    const int sm1 = SMAX == 1 ? 0 : entry_stages_m1(win.d);
-                    const uint32_t gclk = last - (uint32_t)sm1 * 8u;
+                    const int sm1 = stages_m1(win.d);
+                    const uint32_t gclk = first_clock(win.d);
                     if constexpr (SMAX == 1) {
                         t = vmax(arr, best) + l_last;
                         cv[0] = t;
@@ -533,7 +579,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                         }
                     }
                     latency = (t + overhead) - arr;
-                    const uint64_t accs = ballot(latency <= limit);
+                    const uint64_t accs = ballot(latency <= slo) & ballot(best < 1e100);  // a clock that is infinite is never chosen (:590-598)
                     // ---- whose verdict is final
                     const uint64_t blockers = win.g & accs;
                     waits = blockers != 0ull;
@@ -575,6 +621,8 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     wave_order();
 #pragma unroll
                     for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
+#pragma unroll
+                    for (int k = 0; k < NX; ++k) cx[k] = lds_get<double>(xa[k]);
                 } while (waits);
             };
             if (in_mask(pend)) {
@@ -594,7 +642,8 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
             }
         };
         if constexpr (EXT) {
-            if (mores != 0ull) block(Int<5>{});
+            if (eights != 0ull) block(Int<9>{});
+            else if (mores != 0ull) block(Int<8>{});
             else if (fours != 0ull) block(Int<4>{});
             else block(Int<2>{});
         } else {
@@ -607,7 +656,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         const double took = good ? latency : 0.0;
         n_good += good ? 1 : 0;
         if constexpr (OUTPUTS) {
-            if (in_mask(found)) lds_add_u64((SMAX == 1 ? chosen : entry_addr(chosen)) + cnt_rel, good ? 0x100000001ull : 1ull);  // :611, :618
+            if (in_mask(found)) lds_add_u64(first_clock(chosen) + (uint32_t)stages_m1(chosen) * 8u + cnt_rel, good ? 0x100000001ull : 1ull);  // :611, :618
             if (good) lds_add_u32(mcnt + (uint32_t)m * 4u, 1u);
         }
         if constexpr (OUTPUTS)
@@ -615,8 +664,8 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                 fin_out[blk + (uint32_t)j] = good ? t + overhead : arr;
                 good_out[blk + (uint32_t)j] = good ? 1 : 0;
             }
-        if constexpr (W == 64) arrived_req(nn);
-        cur = nxt;
+        if constexpr (W == 64) arrived(nn);
+        cur = as_req(nxt);
         nxt = nn;
         q = nrep;
         look();
