@@ -11,7 +11,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <chrono>
-#include <cmath>
 #include <cstring>
 #include <functional>
 #include <limits>
@@ -234,30 +233,6 @@ int mmsim::compact_latency(const mmsim_tables *t, bool all_batch_sizes, CompactL
 }
 
 namespace {
-
-// How busy the streams keep the groups, about: requests of a second, times the time a group needs for one (the longest of
-// its stages, alone in its batch, over the models as often as they are asked for), over the groups of a placement.
-double offered_load(const mmsim_workload *const *wls, int32_t n_streams, const mmsim_tables *t, const RepLists &rl) {
-    double requests = 0.0, seconds = 0.0;
-    std::vector<double> weight(t->M, 0.0), busy(t->C, 0.0);
-    for (int s = 0; s < n_streams; ++s) {
-        seconds += wls[s]->span;
-        for (int32_t m = 0; m < t->M; ++m) {
-            weight[m] += (double)wls[s]->model_num_requests[m];
-            requests += (double)wls[s]->model_num_requests[m];
-        }
-    }
-    for (int32_t c = 0; c < t->C; ++c)
-        for (int32_t m = 0; m < t->M; ++m) {
-            float longest = 0.0f;
-            for (int k = 0; k < t->cfg_pp[c]; ++k) longest = std::max(longest, t->cfg_lat[(((size_t)m * t->C + c) * t->Smax + k) * t->NB]);
-            if (std::isfinite(longest)) busy[c] += weight[m] / requests * (double)longest;
-        }
-    double a_second = 0.0;  // requests that the groups of all placements take in a second
-    for (int32_t p = 0; p < rl.B; ++p)
-        for (int32_t g = 0; g < rl.num_groups[p]; ++g) a_second += 1.0 / std::max(1e-9, busy[rl.group_cfg[(size_t)p * rl.Gmax + g]]);
-    return a_second > 0.0 && seconds > 0.0 ? requests / seconds * rl.B / a_second : 0.0;
-}
 
 // Builds every device table of a batch from replica lists and launches nothing.
 int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
@@ -561,7 +536,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         int64_t requests = 0;
         for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
         const bool all_solo = can_solo && requests >= (int64_t)512 * n_seeds &&
-                              (sims <= at_once || (sims <= at_once * 64 / kSoloWavesPerCu && offered_load(wls, n_seeds, t, rl) >= 0.5));
+                              (sims <= at_once || (sims <= at_once * 64 / kSoloWavesPerCu && offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()) >= 0.5));
         if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
         } else if (all_solo) {

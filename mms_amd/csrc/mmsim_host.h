@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <exception>
 #include <map>
 #include <memory>
@@ -196,6 +197,33 @@ struct mmsim_workload {
     std::vector<int64_t> mq_off;
     DevBuf<MqEntry> mq;
 };
+
+// How busy the streams keep the groups, about: requests of a second, times the time a group needs for one (the longest of
+// its stages, alone in its batch, over the models as often as they are asked for), over the groups of a placement (of some
+// sixty that are looked at).
+inline double offered_load(const mmsim_workload *const *wls, int32_t n_streams, const mmsim_tables *t, int32_t B, int32_t Gmax,
+                           const int32_t *num_groups, const int32_t *group_cfg) {
+    double requests = 0.0, seconds = 0.0;
+    std::vector<double> weight(t->M, 0.0), busy(t->C, 0.0);
+    for (int s = 0; s < n_streams; ++s) {
+        seconds += wls[s]->span;
+        for (int32_t m = 0; m < t->M; ++m) {
+            weight[m] += (double)wls[s]->model_num_requests[m];
+            requests += (double)wls[s]->model_num_requests[m];
+        }
+    }
+    for (int32_t c = 0; c < t->C; ++c)
+        for (int32_t m = 0; m < t->M; ++m) {
+            float longest = 0.0f;
+            for (int k = 0; k < t->cfg_pp[c]; ++k) longest = std::max(longest, t->cfg_lat[(((size_t)m * t->C + c) * t->Smax + k) * t->NB]);
+            if (std::isfinite(longest)) busy[c] += weight[m] / requests * (double)longest;
+        }
+    double a_second = 0.0;  // requests that the groups of `looked` placements take in a second
+    const int32_t every = std::max(1, B / 64), looked = (B + every - 1) / every;
+    for (int32_t p = 0; p < B; p += every)
+        for (int32_t g = 0; g < num_groups[p]; ++g) a_second += 1.0 / std::max(1e-9, busy[group_cfg[(size_t)p * Gmax + g]]);
+    return a_second > 0.0 && seconds > 0.0 ? requests / seconds * looked / a_second : 0.0;
+}
 
 // Ordered replica lists per (placement, model): the rows of m_id2g_id.
 struct RepLists {

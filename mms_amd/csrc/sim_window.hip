@@ -205,8 +205,8 @@ struct Int {
 template <int W, int SMAX, bool OUTPUTS, bool EXT, bool POW2, bool UNIFORM>
 __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(const WindowArgs a) {
     constexpr int P = kWave / W;
-    const int lane = lane_id(), j = lane % W, sub = lane / W;
-    const int wv = (int)(threadIdx.x >> 6);
+    const int lane = lane_id(), j = lane % W, sub = W == 64 ? 0 : lane / W;
+    const int wv = SMAX >= 16 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
     // latency table for the per-stage latencies of the walk (general tables only), shared by the workgroup
     if (!UNIFORM && a.lat_lds_bytes > 0) {
         for (int i = (int)threadIdx.x; i < a.M * a.lat_row; i += (int)blockDim.x) lds_put<float>((uint32_t)i * 4u, a.lat[i]);
@@ -467,7 +467,6 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                     for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
                 }
             // ---- fetched ahead: the requests of the block after the next, the replicas of the next
-            nrep = load_rep((int)nxt.z);
             if constexpr (W == 64) {
                 nn = load_req(blk + 128u + (uint32_t)j);
             } else {
@@ -664,6 +663,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                 fin_out[blk + (uint32_t)j] = good ? t + overhead : arr;
                 good_out[blk + (uint32_t)j] = good ? 1 : 0;
             }
+        nrep = load_rep((int)nxt.z);
         if constexpr (W == 64) arrived(nn);
         cur = as_req(nxt);
         nxt = nn;

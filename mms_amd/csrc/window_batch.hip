@@ -264,8 +264,13 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
             // / 3.8 / 5.0, 8192: 4.5 / 4.2 / 4.4 / 5.7; eight-stage pipelines, 12288: 14.8 / 10.0 / 6.9 / 6.1; 32-stage ones 45 / 29
             // / 19 / 15.  A narrower wavefront needs more LDS, for its placements and for the requests on their way to them:
             // where it would take two rounds instead of one, up to twice as many wavefronts stay (5000 placements of 128
-            // models, 5.1 / 6.4).
-            const int64_t most = (a.smax_bucket == 1 ? 16 : mean > 7 ? 8 : 12) * cus;
+            // models, 5.1 / 6.4).  Streams that ask twice what the groups can do are mostly runs of rejects, which the widest
+            // blocks settle in the fewest steps: four to a SIMD there (4096 placements of groups of 1 to 16 stages, 64 / 32 lanes,
+            // load 0.4: 26.8 / 23.7, 3.4: 14.6 / 14.6, single devices or 16 stages: load 0.9 263 / 264, 3.5 144 / 157; four-stage
+            // pipelines 0.4: 18.9 / 18.1, 1.7: 13.7 / 14.4, 3.4: 9.4 / 10.4; streams of a few blocks take microseconds either way).
+            int64_t most = (a.smax_bucket == 1 ? 16 : mean > 7 ? 8 : 12) * cus;
+            if (most == 12 * cus && sims > most && sims <= 16 * cus && longest >= 1024 && offered_load(wls, n_seeds, t, B, Gmax, p->num_groups, p->group_cfg) >= 2.0)
+                most = 16 * cus;
             while (lanes > 8 && sims * lanes / kWave > most && fits(lanes / 2) &&
                    (sims <= at_once(lanes / 2) || sims * lanes / kWave > 2 * most || (depth > 10 && sims > at_once(lanes))))
                 lanes /= 2;

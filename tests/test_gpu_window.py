@@ -249,3 +249,24 @@ def test_which_batches_have_their_requests_side_by_side(stages, B, kernel):
     ref = oracle_batch(st, table, E.pack_placements(sols, table))
     for got in (out, once):
         assert np.array_equal(got["n_good"][0], ref["n_good"][of]) and np.array_equal(got["latency_sum"][0], ref["latency_sum"][of])
+
+
+@pytest.mark.parametrize("B,R,pace,lanes", [(3073, 1024, 0.2, 64), (3073, 1023, 0.2, 32), (3073, 1024, 9.0, 32), (4096, 1100, 0.2, 64), (4097, 1100, 0.2, 32)])
+def test_overloaded_streams_keep_the_widest_blocks(B, R, pace, lanes):
+    """Streams that ask more than twice what the groups can do: 64 requests side by side up to four wavefronts to a SIMD."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(4, (4,), True, 4, 2, 64, 3)
+    table = E.LatencyTable(profiles, [1])
+    st = _stream(4, R, 4, 2.0)
+    st.tstamps *= pace
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, 4)
+    of = np.arange(B) % len(sols)
+    batch = E.Batch(eng, [dw], table, E.pack_placements([sols[b] for b in of], table), 0)
+    assert batch.kernel_name().startswith(f"sim_window_kernel<{lanes},"), batch.kernel_name()
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    dw.close()
+    ref = oracle_batch(st, table, E.pack_placements(sols, table))
+    assert np.array_equal(out["n_good"][0], ref["n_good"][of]) and np.array_equal(out["latency_sum"][0], ref["latency_sum"][of])
