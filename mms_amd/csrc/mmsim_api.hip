@@ -524,19 +524,23 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
         const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(M, t->NB, heap_cap, Gmax) && rl.models_ascend();
-        // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them; beyond that,
-        // up to 64, if the groups are busy.  ms with octets / with these, 150000 requests, 96 models on 48 devices, all of them
-        // busy: 2048 simulations 54 / 39, 3072 132 / 46, 4096 133 / 52, 8192 161 / 90, 16384 200 / 157; 30000 requests, 48 models
-        // on 24 devices, half of them: 8192 61 / 40, 16384 73 / 67, 65536 216 / 235; 23108 requests, 5 models on 49 devices, a
-        // tenth, where nearly every request is a batch and the octets of a wavefront share the cost of their events: 4096 164 /
-        // 116, 8192 181 / 202.  Streams of a few hundred requests are over within a millisecond and keep fewer wavefronts (16384
-        // simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
+        // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them; beyond that
+        // up to 64 if the groups are busy half of the time, and any number if they have more to do than they can.  ms with
+        // octets / with these, 150000 requests, 96 models on 48 devices, load 2.7: 2048 simulations 54 / 39, 3072 132 / 46, 4096
+        // 133 / 52, 8192 161 / 90, 16384 200 / 157, 32768 411 / 298, and 12000 requests, 65536, load 1.4: 75 / 57; 30000
+        // requests, 48 models on 24 devices, load 0.7: 8192 61 / 40, 16384 73 / 67, 65536 216 / 235; 23108 requests, 5 models on
+        // 49 devices, load 0.1, where nearly every request is a batch and the octets of a wavefront share the cost of their
+        // events: 4096 164 / 116, 8192 181 / 202.  Streams of a few hundred requests are over within a millisecond and keep
+        // fewer wavefronts (16384 simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
         const int64_t cus = std::max(1, ctx->prop.multiProcessorCount), sims = (int64_t)B * b->out_seeds;
         const int64_t at_once = cus * std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         int64_t requests = 0;
         for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
-        const bool all_solo = can_solo && requests >= (int64_t)512 * n_seeds &&
-                              (sims <= at_once || (sims <= at_once * 64 / kSoloWavesPerCu && offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()) >= 0.5));
+        bool all_solo = can_solo && requests >= (int64_t)512 * n_seeds;
+        if (all_solo && sims > at_once) {
+            const double load = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data());
+            all_solo = load >= (sims <= at_once * 64 / kSoloWavesPerCu ? 0.5 : 1.0);
+        }
         if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
         } else if (all_solo) {

@@ -436,11 +436,11 @@ def test_models_of_one_simulation(eng, M):
     assert 0 < g0.sum() < R
 
 
-@pytest.mark.parametrize("B,n_streams,R,pace,solo", [(71, 29, 511, 3.0, False), (71, 29, 512, 3.0, True), (512, 32, 513, 3.0, True), (513, 32, 513, 3.0, False),
+@pytest.mark.parametrize("B,n_streams,R,pace,solo", [(71, 29, 511, 3.0, False), (71, 29, 512, 3.0, True), (512, 32, 513, 0.3, True), (513, 32, 513, 0.3, False), (513, 32, 513, 3.0, True),
                                                      (160, 32, 520, 0.01, True), (161, 32, 520, 0.01, False)])
 def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, pace, solo):
-    """Twenty simulations to a CU, or sixty-four if their groups are busy, have a wavefront each, unless their streams are
-    short: the oracle's counts and traces on both sides of each line."""
+    """Twenty simulations to a CU, sixty-four if their groups are busy half of the time or any number if they have more to do
+    than they can, have a wavefront each, unless their streams are short: the oracle's counts and traces on both sides of each line."""
     cfg = make_config(5, B)
     table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
     packed = E.pack_placements(cfg.placements, table)
