@@ -245,15 +245,15 @@ constexpr int64_t kMaxWindowSims = 12288;
 typedef void (*WindowKernel)(const WindowArgs);
 // The kernel for LANES requests side by side (64, 32, 16, 8), stage bucket smax and the rest of its template arguments.
 template <int LANES>
-WindowKernel window_kernel(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+WindowKernel window_kernel(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<64>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+WindowKernel window_kernel<64>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<32>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+WindowKernel window_kernel<32>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<16>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+WindowKernel window_kernel<16>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<8>(int smax, bool outputs, bool ext, bool pow2, bool uniform);
+WindowKernel window_kernel<8>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 std::string sim_window_kernel_name(const WindowArgs &args);
 
 // Arguments of the scalar-clock request loop (one placement, device pointers).

@@ -40,9 +40,12 @@
 // 4800 cycles a block, 40 % issuing, 32 % waiting to issue, 28 % for LDS.  (One request after the other, 64 placements to
 // a wavefront: 24 ms either way.)
 // Few instructions to a step count most where a wavefront is alone.  That a block's second four replicas are in registers like
-// the first, instead of being fetched for every step (only blocks with a ninth do that), and that the words that the walk
-// needs are ready for it took, 108000 requests: 700 placements of single-device groups, a model in 25 on more than four of them, 6.1
-// -> 5.3 ms, 1025 placements of groups up to 16 deep 15.5 -> 13.1 ms, 600 of four-stage pipelines 10.4 -> 9.65 ms.
+// the first, instead of being fetched for every step, and that the words that the walk needs are ready for it took, 108000
+// requests: 700 placements of single-device groups, a model in 25 on more than four of them, 6.1 -> 5.3 ms, 1025 placements of
+// groups up to 16 deep 15.5 -> 13.1 ms, 600 of four-stage pipelines 10.4 -> 9.65 ms.  Batches of up to eight wavefronts to a CU
+// whose models have more than eight replicas keep sixteen in registers (EXT 2; 150 to 180 of them) and fetch the others: 12000
+// requests, 6 models on 20 devices, up to 12 replicas, 1 / 64 / 700 / 1500 placements 2.7 / 3.3 / 3.9 / 4.4 -> 1.85 / 2.0 / 2.2 /
+// 3.1 ms; 12 models on 33 devices, up to 17, 5.7 / 5.9 / 7.1 / 7.6 -> 3.7 / 3.8 / 4.7 / 5.7 ms.
 //
 // LDS of one placement (byte offsets in WindowArgs, built by the wavefront itself from the packed placement):
 //   clk  [slots+SMAX] f64   stage clocks, a placement's groups laid end to end, and SMAX slots for what does not count
@@ -54,7 +57,7 @@
 //   gd   [Gmax] u32         entry word of every group
 //   mcnt [M] u32            accepted requests per model  (OUTPUTS)
 // Entry word: bits 0-14 LDS address / 8 of the group's last-stage clock, 15-19 stages - 1, 20-29 index of its
-// last-stage latency in the model's row of the latency table, 30 "there are more" (fourth entry), "more than eight" (third), 31 "no such replica":
+// last-stage latency in the model's row of the latency table, 30 "there are more" (fourth entry), "than eight" (third), "than sixteen" (second), 31 "no such replica":
 // the word then repeats the first replica's (which wins every tie against its copies) or, without any replica, the
 // placement's first slot.
 #include "mmsim_internal.h"
@@ -200,9 +203,9 @@ struct Int {
     static constexpr int value = I;
 };
 // W: requests (lanes) of one placement.  SMAX: most stages of a group (bucket).  OUTPUTS: anything beyond the scores
-// (a.flags says what).  EXT: some model has more than four replicas.  POW2: every group has 1, 2, 4, ... stages.
+// (a.flags says what).  EXT: 1, some model has more than four replicas; 2, and up to sixteen are kept in registers, not eight.  POW2: every group has 1, 2, 4, ... stages.
 // UNIFORM: one latency per (model, configuration).
-template <int W, int SMAX, bool OUTPUTS, bool EXT, bool POW2, bool UNIFORM>
+template <int W, int SMAX, bool OUTPUTS, int EXT, bool POW2, bool UNIFORM>
 __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(const WindowArgs a) {
     constexpr int P = kWave / W;
     const int lane = lane_id(), j = lane % W, sub = W == 64 ? 0 : lane / W;
@@ -275,7 +278,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         int n = 0;
         for (int w = 0; w < GW; ++w) n += __popc(lds_get<uint32_t>(mb + (uint32_t)w * 4u));
         uint32_t chunk0 = 0;
-        if constexpr (EXT) {
+        if constexpr (EXT > 0) {
             const uint32_t chunks = n > 4 ? (uint32_t)(n - 1) / 4u : 0u;
             if (chunks > 0) chunk0 = lds_fetch_add_u32(ext_used, chunks);
             lds_put<uint32_t>(xi + (uint32_t)m * 4u, chunk0 | chunks << 16);
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         int k = 0;
         auto put = [&](const Entry &e) {
             const uint32_t at = k < 4 ? rep + (uint32_t)(m * 4 + k) * 8u : ext + (chunk0 * 4u + (uint32_t)(k - 4)) * 8u;
-            lds_put<uint32_t>(at, (k == 3 && n > 4) || (k == 2 && n > 8) ? e.d | kEntryMore : e.d);
+            lds_put<uint32_t>(at, (k == 3 && n > 4) || (k == 2 && n > 8) || (k == 1 && n > 16) ? e.d | kEntryMore : e.d);
             lds_put<float>(at + 4u, e.l);
             ++k;
         };
@@ -341,21 +344,22 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     Entry4 q = load_rep(cur.m);
     // What a block is like: requests that can be served at all, that list several groups, more than two, more than
     // four; how deep their groups are.  Worked out a block ahead (a scalar that depends on vector compares is slow to come).
-    uint64_t pend, multis, fours, mores, eights, deep_a, deep_b;
+    uint64_t pend, multis, fours, mores, eights, sixteens, deep_a, deep_b;
     auto look = [&]() {
         pend = ballot(cur.m >= 0 && !entry_none(q.e[0].d));  // (past the end of the stream: m is -1)
         multis = ballot(!entry_none(q.e[1].d)) & pend;
         fours = ballot(!entry_none(q.e[2].d)) & pend;
-        if constexpr (EXT) {
+        if constexpr (EXT > 0) {
             mores = ballot((q.e[3].d & kEntryMore) != 0u) & pend;
             eights = ballot((q.e[2].d & kEntryMore) != 0u) & pend;
+            if constexpr (EXT > 1) sixteens = ballot((q.e[1].d & kEntryMore) != 0u) & pend;
         }
         if constexpr (SMAX > 1) {
             const int deep = max2(max2(entry_stages_m1(q.e[0].d), entry_stages_m1(q.e[1].d)),
                                   max2(entry_stages_m1(q.e[2].d), entry_stages_m1(q.e[3].d)));
             deep_a = ballot(deep >= (SMAX == 4 ? 2 : SMAX == 16 ? 8 : 16)) & pend;
             if constexpr (SMAX == 16) deep_b = ballot(deep >= 4) & pend;
-            if constexpr (EXT) {  // (the groups behind the fourth are not looked at: as deep as any of the batch)
+            if constexpr (EXT > 0) {  // (the groups behind the fourth are not looked at: as deep as any of the batch)
                 if (a.smax > (SMAX == 4 ? 2 : SMAX == 16 ? 8 : 16)) deep_a |= mores;
                 if (SMAX == 16 && a.smax > 4) deep_b |= mores;
             }
@@ -387,33 +391,40 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         u32x4 nn;
         double best = 0.0, t = 0.0, latency = 0.0;
         uint32_t chosen = SMAX > 1 && !UNIFORM ? clk >> 3 : clk;  // the chosen group's walk word
-        // The block, for requests that list at most NC groups (2, 4, 8, or 9: more than eight).
+        // The block, for requests that list at most NC groups (2, 4, 8, 16, or 0: any number).
         auto block = [&](auto NCv) {
-            constexpr int NC = decltype(NCv)::value, N4 = NC > 4 ? 4 : NC, NX = NC == 8 ? 4 : 0;
+            constexpr int NC = decltype(NCv)::value, N4 = NC == 2 ? 2 : 4;
+            // Further ones kept in registers.  (Not beside the fetched ones with 16 stages and counts: 133 registers instead of 126, three
+            // wavefronts to a SIMD instead of four.)
+            constexpr int NX = NC > 4 ? NC - 4 : NC == 0 ? (EXT > 1 ? 12 : SMAX < 16 ? 4 : 0) : 0;
+            constexpr bool MORE = NC != 2 && NC != 4, ANY = NC == 0;                // ANY: and others are fetched in every step
             double c[N4];
 #pragma unroll
             for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
             // ---- the masks of the block's requests.  (Copies of the first replica set its bit again: harmless.)
             uint64_t gm[N4];
             uint32_t x0 = 0, xn = 0;  // chunks of further replicas
-            if constexpr (NC > 4) {
+            if constexpr (MORE) {
                 const uint32_t v = lds_get<uint32_t>(xi + (uint32_t)(m < 0 ? 0 : m) * 4u);
                 x0 = ext + (v & 0xFFFFu) * 32u;
                 xn = in_mask(pend) ? v >> 16 : 0u;
             }
-            // up to eight: the second four like the first, in registers (of a request without: copies of its first, which
-            // never beat it)
-            Entry4 more = q;
-            uint32_t xa[4], xword[4];
-            double cx[4];
-            if constexpr (NX > 0) {
-                if (xn > 0u) more = load_entries(x0);
-                else more.e[1] = more.e[2] = more.e[3] = more.e[0];
+            // the further ones in registers, like the first four (of a request without: copies of its first, which never beat it)
+            constexpr int NA = NX > 0 ? NX : 1;
+            uint32_t xa[NA], xword[NA];
+            float xl[NA];
+            double cx[NA];
+#pragma unroll
+            for (int x = 0; x < NX / 4; ++x) {
+                Entry4 more;
+                if (xn > (uint32_t)x) more = load_entries(x0 + (uint32_t)x * 32u);
+                else more.e[0] = more.e[1] = more.e[2] = more.e[3] = q.e[0];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    xa[k] = entry_addr(more.e[k].d);
-                    xword[k] = walk_word(more.e[k].d);
-                    cx[k] = lds_get<double>(xa[k]);
+                    xa[4 * x + k] = entry_addr(more.e[k].d);
+                    xword[4 * x + k] = walk_word(more.e[k].d);
+                    xl[4 * x + k] = more.e[k].l;
+                    cx[4 * x + k] = lds_get<double>(xa[4 * x + k]);
                 }
             }
             uint32_t ga[N4];
@@ -426,12 +437,15 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
 #pragma unroll
                 for (int k = 0; k < N4; ++k) lds_or_u64(ga[k], my_bit);
                 if constexpr (NX > 0) {
-                    if (xn > 0u) {
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) lds_or_u64(xa[k] + gm_rel, my_bit);
-                    }
-                } else if constexpr (NC > 4)
-                    for (uint32_t x = 0; x < xn; ++x) {
+                    for (int x = 0; x < NX / 4; ++x)
+                        if (xn > (uint32_t)x) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) lds_or_u64(xa[4 * x + k] + gm_rel, my_bit);
+                        }
+                }
+                if constexpr (ANY)
+                    for (uint32_t x = NX / 4; x < xn; ++x) {
                         const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
                         for (int k = 0; k < 4; ++k) lds_or_u64(entry_addr(e.e[k].d) + gm_rel, my_bit);
@@ -441,12 +455,13 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
 #pragma unroll
             for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ga[k]) & before;
             uint64_t gm_ext = 0;  // requests before this one that share any of the groups: holds for every further replica
-            if constexpr (NC > 4) {
+            if constexpr (MORE) {
                 if constexpr (NX > 0) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(xa[k] + gm_rel);
-                } else {
-                    for (uint32_t x = 0; x < xn; ++x) {
+                    for (int k = 0; k < NX; ++k) gm_ext |= lds_get<uint64_t>(xa[k] + gm_rel);
+                }
+                if constexpr (ANY) {
+                    for (uint32_t x = NX / 4; x < xn; ++x) {
                         const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
                         for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
@@ -459,9 +474,10 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
             for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ga[k], 0);  // for the next block
             if constexpr (NX > 0) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) lds_put<uint64_t>(xa[k] + gm_rel, 0);
-            } else if constexpr (NC > 4)
-                for (uint32_t x = 0; x < xn; ++x) {
+                for (int k = 0; k < NX; ++k) lds_put<uint64_t>(xa[k] + gm_rel, 0);
+            }
+            if constexpr (ANY)
+                for (uint32_t x = NX / 4; x < xn; ++x) {
                     const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
                     for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
@@ -504,15 +520,19 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                 do {
                     // ---- choose the replica group: strictly smallest last-stage clock, first listed wins ties (:590-598)
                     Cand win = first_min(Cand{c[0], word[0], q.e[0].l, gm[0]}, Cand{c[1], word[1], q.e[1].l, gm[1]});
-                    if constexpr (NC > 2)
+                    if constexpr (NC != 2)
                         win = first_min(win, first_min(Cand{c[2], word[2], q.e[2].l, gm[2]}, Cand{c[3], word[3], q.e[3].l, gm[3]}));
                     if constexpr (NX > 0) {
-                        Cand y[4];
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) y[k] = Cand{cx[k], xword[k], more.e[k].l, gm_ext};
-                        win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
-                    } else if constexpr (NC > 4)
-                        for (uint32_t x = 0; x < xn; ++x) {
+                        for (int x = 0; x < NX; x += 4) {
+                            Cand y[4];
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) y[k] = Cand{cx[x + k], xword[x + k], xl[x + k], gm_ext};
+                            win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
+                        }
+                    }
+                    if constexpr (ANY)
+                        for (uint32_t x = NX / 4; x < xn; ++x) {
                             const Entry4 e = load_entries(x0 + x * 32u);
                             Cand y[4];
 #pragma unroll
@@ -640,8 +660,9 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
                 }
             }
         };
-        if constexpr (EXT) {
-            if (eights != 0ull) block(Int<9>{});
+        if constexpr (EXT > 0) {
+            if ((EXT > 1 ? sixteens : eights) != 0ull) block(Int<0>{});
+            else if (EXT > 1 && eights != 0ull) block(Int<(EXT > 1 ? 16 : 8)>{});
             else if (mores != 0ull) block(Int<8>{});
             else if (fours != 0ull) block(Int<4>{});
             else block(Int<2>{});
@@ -693,13 +714,17 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
 
 constexpr int W_ = MMSIM_WINDOW_LANES;  // the file is compiled once for each number of requests side by side
 
+template <int SMAX, bool OUTPUTS, bool POW2, bool UNIFORM>
+WindowKernel pick_ext(int ext) {
+    if (W_ == 64 && ext > 1) return sim_window_kernel<W_, SMAX, OUTPUTS, W_ == 64 ? 2 : 1, POW2, UNIFORM>;
+    return ext > 0 ? sim_window_kernel<W_, SMAX, OUTPUTS, 1, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, OUTPUTS, 0, POW2, UNIFORM>;
+}
 template <int SMAX, bool POW2, bool UNIFORM>
-WindowKernel pick_out(bool outputs, bool ext) {
-    if (outputs) return ext ? sim_window_kernel<W_, SMAX, true, true, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, true, false, POW2, UNIFORM>;
-    return ext ? sim_window_kernel<W_, SMAX, false, true, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, false, false, POW2, UNIFORM>;
+WindowKernel pick_out(bool outputs, int ext) {
+    return outputs ? pick_ext<SMAX, true, POW2, UNIFORM>(ext) : pick_ext<SMAX, false, POW2, UNIFORM>(ext);
 }
 template <int SMAX>
-WindowKernel pick_depths(bool outputs, bool ext, bool pow2, bool uniform) {
+WindowKernel pick_depths(bool outputs, int ext, bool pow2, bool uniform) {
     if (pow2) return uniform ? pick_out<SMAX, true, true>(outputs, ext) : pick_out<SMAX, true, false>(outputs, ext);
     return uniform ? pick_out<SMAX, false, true>(outputs, ext) : pick_out<SMAX, false, false>(outputs, ext);
 }
@@ -707,7 +732,7 @@ WindowKernel pick_depths(bool outputs, bool ext, bool pow2, bool uniform) {
 }  // namespace
 
 template <>
-WindowKernel window_kernel<MMSIM_WINDOW_LANES>(int smax, bool outputs, bool ext, bool pow2, bool uniform) {
+WindowKernel window_kernel<MMSIM_WINDOW_LANES>(int smax, bool outputs, int ext, bool pow2, bool uniform) {
     switch (smax) {
         case 1: return pick_out<1, true, true>(outputs, ext);  // one stage: its latency is the configuration's
         case 4: return pick_depths<4>(outputs, ext, pow2, uniform);

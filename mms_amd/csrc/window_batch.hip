@@ -29,7 +29,8 @@ bool has_outputs(uint32_t flags) {
 }
 
 hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_bytes, hipStream_t stream) {
-    const bool out = has_outputs(a.flags), ext = a.has_ext != 0, pow2 = a.pow2_depths != 0, uniform = a.uniform_stages != 0;
+    const int ext = a.has_ext;
+    const bool out = has_outputs(a.flags), pow2 = a.pow2_depths != 0, uniform = a.uniform_stages != 0;
     const WindowKernel kern = a.lanes == 64   ? window_kernel<64>(a.smax_bucket, out, ext, pow2, uniform)
                               : a.lanes == 32 ? window_kernel<32>(a.smax_bucket, out, ext, pow2, uniform)
                               : a.lanes == 16 ? window_kernel<16>(a.smax_bucket, out, ext, pow2, uniform)
@@ -369,7 +370,8 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     a.lanes = lanes;
     a.pow2_depths = shape.pow2 ? 1 : 0;
     a.uniform_stages = uniform ? 1 : 0;
-    a.has_ext = shape.ext_cap > 0 ? 1 : 0;
+    // (2: sixteen replicas in registers, which leaves two or three wavefronts to a SIMD: sim_window.hip has both sides)
+    a.has_ext = shape.ext_cap > 0 ? (lanes == kWave && shape.rmax > 8 && units <= 8 * cus ? 2 : 1) : 0;
     a.lat_lds_bytes = (int32_t)lat_lds;
     a.place_bytes = (int32_t)place;
     a.Rmax = b->Rmax;
@@ -391,7 +393,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
 
 std::string sim_window_kernel_name(const WindowArgs &a) {
     auto tf = [](bool v) { return v ? ", true" : ", false"; };
-    return "sim_window_kernel<" + std::to_string(a.lanes) + ", " + std::to_string(a.smax_bucket) + tf(has_outputs(a.flags)) + tf(a.has_ext != 0) +
+    return "sim_window_kernel<" + std::to_string(a.lanes) + ", " + std::to_string(a.smax_bucket) + tf(has_outputs(a.flags)) + ", " + std::to_string(a.has_ext) +
            tf(a.pow2_depths != 0) + tf(a.uniform_stages != 0) + ">";
 }
 

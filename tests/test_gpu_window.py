@@ -83,36 +83,39 @@ def test_requests_side_by_side(lanes, depths, uniform, groups, hosts):
 @pytest.mark.parametrize("lanes", [64, 32, 16, 8])
 @pytest.mark.parametrize("depths,uniform", [((1,), True), ((1, 2, 4), True), ((1, 3), False), ((2, 16), True)])
 def test_where_the_number_of_replicas_changes_the_kernels_path(lanes, depths, uniform):
-    """A block takes two, four, eight or any number of groups per request, by its most listed model: placements with 2 to 13
-    replicas of their most listed one, beside models with one, two or none."""
+    """A block takes two, four, eight, sixteen or any number of groups per request, by its most listed model: placements with 2
+    to 21 replicas of their most listed one, beside models with one, two or none; with more than eight wavefronts to a CU the
+    kernel that keeps eight of them in registers, not sixteen."""
     eng = E.Engine.default()
     rng = np.random.default_rng(lanes + len(depths))
-    counts = (2, 3, 4, 5, 7, 8, 9, 12, 13)
+    counts = (2, 3, 4, 5, 7, 8, 9, 12, 13, 16, 17, 20, 21)
     profiles, _ = _problem(5, depths, uniform, 5, 1, 1, 1)
     pcs = [ParallelConfig(1, 1, d) for d in depths]
     sols = []
     for n in counts:
-        hosts = [set() for _ in range(14)]
+        hosts = [set() for _ in range(22)]
         for m, k in ((0, n), (1, 1), (2, 2), (3, max(1, n - 4))):      # (model 4: nowhere)
-            for g in rng.permutation(14)[:k]:
+            for g in rng.permutation(22)[:k]:
                 hosts[g].add(m)
-        sols.append(ModelPlacement([pcs[int(rng.integers(len(pcs)))] for _ in hosts], [sorted(int(m) for m in h) for h in hosts]))
+        sols.append(ModelPlacement([pcs[min(int(rng.exponential(0.7)), len(pcs) - 1)] for _ in hosts], [sorted(int(m) for m in h) for h in hosts]))
     streams = [_stream(17 * lanes + k, R, 5, load) for k, (R, load) in enumerate(((lanes + 1, 4.0), (900, 2.0), (900, 9.0)))]
     table = E.LatencyTable(profiles)
     packed = E.pack_placements(sols, table)
     dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, 5) for s in streams]
-    for flags in (0, COUNTS):
-        batch = E.Batch(eng, dws, table, packed, flags, options=dict(window_lanes=lanes))
-        assert batch.kernel_name().startswith(f"sim_window_kernel<{lanes}, ")
+    for flags, times in ((0, 1), (COUNTS, 1), (0, 60), (COUNTS, 60)):
+        batch = E.Batch(eng, dws, table, E.pack_placements(sols * times, table), flags, options=dict(window_lanes=lanes))
+        name = batch.kernel_name()
+        assert name.startswith(f"sim_window_kernel<{lanes}, ") and name.split(", ")[3] == ("2" if lanes == 64 and times == 1 else "1")
         batch.run()
         batch.sync()
         out = batch.fetch()
         batch.close()
         for k, s in enumerate(streams):
             ref = oracle_batch(s, table, packed)
-            assert np.array_equal(out["n_good"][k], ref["n_good"]) and np.array_equal(out["latency_sum"][k], ref["latency_sum"])
-            for key in ("model_num_good", "group_num_requests", "group_num_good"):
-                assert not flags or np.array_equal(out[key][k], ref[key]), (k, key)
+            for t in {0, times - 1}:
+                mine = slice(t * len(sols), (t + 1) * len(sols))
+                for key in ("n_good", "latency_sum") + (("model_num_good", "group_num_requests", "group_num_good") if flags else ()):
+                    assert np.array_equal(out[key][k][mine], ref[key]), (k, t, key)
             assert k == 0 or 0 < ref["n_good"].min() and ref["n_good"].max() < len(s.tstamps)
     for dw in dws:
         dw.close()
