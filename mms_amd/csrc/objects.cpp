@@ -11,7 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <new>
+#include <exception>
 #include <vector>
 
 namespace {
@@ -117,7 +117,7 @@ PyObject *pack(PyObject *, PyObject *args) {
         Ref n(PyLong_FromLong(most)), a(bytes_of(groups)), c(bytes_of(group_cfg)), o(bytes_of(gm_off)), i(bytes_of(ids));
         if (!n.p || !a.p || !c.p || !o.p || !i.p) return nullptr;
         return PyTuple_Pack(5, n.p, a.p, c.p, o.p, i.p);
-    } catch (const std::bad_alloc &) {
+    } catch (const std::exception &) {  // (vectors throw nothing else than that there is no memory for them)
         return PyErr_NoMemory();
     }
 }
@@ -141,7 +141,7 @@ PyObject *count_models(PyObject *, PyObject *sols) {
             counts.push_back(n);
         }
         return bytes_of(counts);
-    } catch (const std::bad_alloc &) {
+    } catch (const std::exception &) {  // (vectors throw nothing else than that there is no memory for them)
         return PyErr_NoMemory();
     }
 }
@@ -174,7 +174,7 @@ PyObject *request_arrays(PyObject *, PyObject *args) {
         Ref a(bytes_of(ids)), b(bytes_of(slos));
         if (!a.p || !b.p) return nullptr;
         return PyTuple_Pack(2, a.p, b.p);
-    } catch (const std::bad_alloc &) {
+    } catch (const std::exception &) {  // (vectors throw nothing else than that there is no memory for them)
         return PyErr_NoMemory();
     }
 }
