@@ -1567,25 +1567,28 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
     }
     if (wr && b->Rmax > 0) {
         const size_t Rm = (size_t)b->Rmax;
-        std::vector<double> hf(Rm * row_w);
-        std::vector<uint8_t> hg(Rm * row_w);
+        // so many wavefronts' rows to a copy: one 64 wide, or up to 16 MB of those that are one wide
+        const int32_t at_once = row_w > 1 ? 1 : (int32_t)std::max<size_t>(1, std::min<size_t>((size_t)tiles, ((size_t)16 << 20) / (Rm * sizeof(double))));
+        std::vector<double> hf(Rm * row_w * at_once);
+        std::vector<uint8_t> hg(Rm * row_w * at_once);
         std::vector<int32_t> owner((size_t)tiles * row_w, -1);  // placement simulated on each lane
         for (int32_t p = 0; p < B; ++p) owner[b->pos[p]] = p;
         for (int s = 0; s < b->out_seeds; ++s)
-            for (int32_t tile = 0; tile < tiles; ++tile) {
-                const size_t wave = (size_t)s * tiles + tile;
-                HIP_TRY(hipMemcpy(hf.data(), b->finish.p + wave * Rm * row_w, sizeof(double) * Rm * row_w, hipMemcpyDeviceToHost));
-                HIP_TRY(hipMemcpy(hg.data(), b->good.p + wave * Rm * row_w, Rm * row_w, hipMemcpyDeviceToHost));
-                for (int l = 0; l < row_w; ++l) {
-                    const int32_t p = owner[(size_t)tile * row_w + l];
-                    if (p < 0) continue;
-                    const size_t Rs = (size_t)b->wl_R[(size_t)(b->paired ? b->stream_of[p] : s)];
-                    const size_t row = ((size_t)s * B + (size_t)p) * Rm;
-                    for (size_t i = 0; i < Rs; ++i) {
-                        out->finish[row + i] = hf[i * row_w + l];
-                        out->good[row + i] = hg[i * row_w + l];
+            for (int32_t tile0 = 0; tile0 < tiles; tile0 += at_once) {
+                const size_t wave = (size_t)s * tiles + tile0, n = Rm * row_w * (size_t)std::min(at_once, tiles - tile0);
+                HIP_TRY(hipMemcpy(hf.data(), b->finish.p + wave * Rm * row_w, sizeof(double) * n, hipMemcpyDeviceToHost));
+                HIP_TRY(hipMemcpy(hg.data(), b->good.p + wave * Rm * row_w, n, hipMemcpyDeviceToHost));
+                for (int32_t tile = tile0; tile < std::min(tiles, tile0 + at_once); ++tile)
+                    for (int l = 0; l < row_w; ++l) {
+                        const int32_t p = owner[(size_t)tile * row_w + l];
+                        if (p < 0) continue;
+                        const size_t Rs = (size_t)b->wl_R[(size_t)(b->paired ? b->stream_of[p] : s)];
+                        const size_t row = ((size_t)s * B + (size_t)p) * Rm, from = (size_t)(tile - tile0) * Rm * row_w + l;
+                        for (size_t i = 0; i < Rs; ++i) {
+                            out->finish[row + i] = hf[from + i * row_w];
+                            out->good[row + i] = hg[from + i * row_w];
+                        }
                     }
-                }
             }
     }
     if (any_bad && !out->status)
