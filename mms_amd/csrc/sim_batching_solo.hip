@@ -201,10 +201,8 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             for (int i = 0; i < MW; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
         }
     }
-    uint64_t hosting = 0;  // groups that host a model
-#pragma unroll
-    for (int i = 0; i < MW; ++i) hosting |= ballot(members[i] != 0ull);
-    const uint32_t group = lane < a.Gmax ? ginfo[lane] : 0u;  // lane g: descriptor of group g
+    const uint32_t group = lane < a.Gmax ? ginfo[lane] : kEmpty;  // lane g: descriptor of group g
+    const uint64_t groups = ballot((int32_t)group >= 0);  // (a group that lists no model may still be some model's replica)
     uint64_t waiting[MW] = {};  // models with waiting requests
     double ev_t = inf;          // lane e: event slot e
     uint32_t ev_d = 0;
@@ -530,7 +528,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             const double tf = lane_value(t, fl);
             const int mf = lane_value(m, fl);
             uint32_t dsel = lane_value(dj, first_of(selected >> fl) + fl);
-            if (ROWSLDS) dsel = lane_value(group, first_of(ballot((group & 0x1FFFu) == (dsel & 0x1FFFu)) & hosting));
+            if (ROWSLDS) dsel = lane_value(group, first_of(ballot((group & 0x1FFFu) == (dsel & 0x1FFFu)) & groups));
             bool ready = (idle >> fl & 0xFFull) != 0ull;
             if (rarely((special >> fl & 1ull) != 0ull)) {
                 double best = lane_value(mn, fl);

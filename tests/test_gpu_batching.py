@@ -65,6 +65,28 @@ def test_random_cases_match_oracle(eng):
             assert np.array_equal(a, b), seed
 
 
+def test_groups_that_list_no_model(eng):
+    """Which groups a model may use and which models a group may turn to are lists of their own: a group that lists no model
+    still runs the requests that arrive while it is idle."""
+    ran = 0
+    for seed in range(120):
+        nb = 1 + seed % 5
+        c = random_case(9_500_000 + seed, max_m=6, max_g=5, max_s=4, max_r=200, nb=nb, load=0.3 + 0.3 * (seed % 5), inf_slo=False)
+        c["g2m"][np.random.default_rng(seed).random(len(c["g2m"])) < 0.5] = -1
+        try:
+            f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
+                c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], BSS[:nb])
+        except AssertionError:      # requests that nobody turns to are left over at the end: the reference stops there
+            continue
+        fin, good, cnt = _single(eng, c, BSS[:nb])
+        assert np.array_equal(good, g0), seed
+        assert np.array_equal(fin.view(np.uint64), f0.view(np.uint64)), seed
+        for a, b in zip(cnt, c0):
+            assert np.array_equal(a, b), seed
+        ran += int(c0[2][c["g2m"][:, 0] < 0].sum() > 0)
+    assert ran > 20
+
+
 def test_batches_of_sixteen_and_more(eng):
     """Batches larger than the sixteen queue entries that an octet fetches at once: the arrival behind the batch
     and the members past the fetched ones come from memory.  (Seeds found by a randomized comparison.)"""
