@@ -2155,7 +2155,7 @@ int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8
             const int32_t m = g_id2m_id[(size_t)g * M + j];
             if (m < 0) break;
             if (m >= M) return fail(MMSIM_E_INVALID, "simulate_requests_mixed_batching: g_id2m_id names a model >= M");
-            rl.g2m_m.push_back(m);
+            if (rl.off[m + 1] > rl.off[m]) rl.g2m_m.push_back(m);  // (requests of a model without a group are never queued, :754-757)
         }
         rl.g2m_off[g + 1] = (int64_t)rl.g2m_m.size();
     }

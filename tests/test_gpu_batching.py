@@ -87,6 +87,26 @@ def test_groups_that_list_no_model(eng):
     assert ran > 20
 
 
+@pytest.mark.parametrize("lanes", [0, 8, 64])
+def test_groups_that_list_a_model_without_a_group(eng, opts, lanes):
+    """Requests of a model that may use no group are dropped as they arrive (controller.py:754-757), also if a group lists it."""
+    opts(batching_lanes=lanes)
+    ran = 0
+    for seed in range(60):
+        nb = 1 + seed % 5
+        c = random_case(9_600_000 + seed, max_m=6, max_g=5, max_s=4, max_r=200, nb=nb, load=0.3 + 0.6 * (seed % 9), inf_slo=False)
+        c["m2g"][np.random.default_rng(seed).random(len(c["m2g"])) < 0.4] = -1
+        f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
+            c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], BSS[:nb])
+        fin, good, cnt = _single(eng, c, BSS[:nb])
+        assert np.array_equal(good, g0), seed
+        assert np.array_equal(fin.view(np.uint64), f0.view(np.uint64)), seed
+        for a, b in zip(cnt, c0):
+            assert np.array_equal(a, b), seed
+        ran += int(np.isin(c["g2m"], np.flatnonzero(c["m2g"][:, 0] < 0)).any() and g0.any())
+    assert ran > 20
+
+
 def test_batches_of_sixteen_and_more(eng):
     """Batches larger than the sixteen queue entries that an octet fetches at once: the arrival behind the batch
     and the members past the fetched ones come from memory.  (Seeds found by a randomized comparison.)"""
