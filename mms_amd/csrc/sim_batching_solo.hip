@@ -220,6 +220,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     // and these clocks, kept as they change.  (Lanes without a replica: slot 0, not used.)
     uint32_t last = clk;
     double c_last = 0.0, c_first = 0.0;
+    uint64_t here = 0;  // octets that hold an arrival; none from when a simulation is given up
 
     auto set_waiting = [&](int m, bool on) {
 #pragma unroll
@@ -421,10 +422,11 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 group_good[g] += bs;
             }
             if (want_model && lane == 0) model_good[m] += bs;
-            if (rarely(used == slots)) {  // nothing more happens; the arrivals' loop looks at `dead` once a window
+            if (rarely(used == slots)) {  // given up: no event is due, no arrival left (`dead` is looked at once a window)
                 dead = MMSIM_E_OVERFLOW;
                 used = 0ull;
                 next_due = inf;
+                here = 0ull;
                 return;
             }
             const int slot = first_of(~used);
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         const bool valid = ((int32_t)dj >= 0) & (m >= 0);
         const uint64_t valids = ballot((int32_t)dj >= 0) & ballot(m >= 0), known = ballot(m >= 0);
         const uint64_t hosted = valids & kFirstOfOctets, longer = valids >> 7 & kFirstOfOctets;  // longer: the list may go on
-        const uint64_t here = ~0ull >> (64 - 8 * n);
+        here = ~0ull >> (64 - 8 * n);
         int cur = 0;             // arrivals before this one are settled
         uint64_t unseen = ~0ull;  // arrivals whose due events have not been seen to
         while (cur < n) {

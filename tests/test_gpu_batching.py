@@ -14,7 +14,7 @@ import pytest
 
 from mms_amd import _lib, engine as E
 from mms_amd.synthetic import make_config
-from oracle import oracle_c
+from oracle import oracle_c, oracle_py
 from randcase import random_case
 from helpers import oracle_batch
 
@@ -253,6 +253,47 @@ def test_a_simulation_that_runs_out_of_event_slots(eng, opts, lanes):
     dw.close()
     opts(batching_event_slots=0)
     _single(eng, c, BSS[:3])                 # and the context is fine afterwards
+
+
+def test_one_simulation_to_a_wavefront_that_runs_out_of_event_slots(eng, opts):
+    """A simulation that is given up does nothing more: what it has counted is what the reference has when its heap first holds
+    an entry more than there are slots."""
+    class Full(Exception):
+        pass
+
+    class Sim(oracle_py._BatchingSim):
+        def serve(self, t0, m, g):
+            super().serve(t0, m, g)
+            if len(self.events) > 8:
+                raise Full
+
+    opts(batching_event_slots=8)
+    cfg = make_config(5, 24)
+    table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
+    packed = E.pack_placements(cfg.placements, table)
+    st = cfg.stream(0)
+    n = 1500
+    dw = E.DeviceWorkload(eng, st.tstamps[:n], st.model_ids[:n], st.slos[:n], cfg.num_models)
+    batch = E.Batch(eng, [dw], table, packed, _lib.BATCHING | _lib.WANT_MODEL_COUNTS)
+    assert batch.kernel_name().startswith("sim_batching_solo")
+    batch.run()
+    batch.sync()
+    out = batch.fetch(allow_failed=True)
+    batch.close()
+    dw.close()
+    failed = 0
+    for b, pl in enumerate(cfg.placements):
+        sim = Sim(st.tstamps[:n], st.model_ids[:n], st.slos[:n],
+                  *oracle_py.build_tables(pl.group_configs, pl.group_models, cfg.profiles, cfg.batch_sizes), cfg.batch_sizes)
+        try:
+            sim.run()
+            status = 0
+        except Full:
+            status = _lib.E_OVERFLOW
+            failed += 1
+        assert out["status"][0, b] == status, b
+        assert out["n_good"][0, b] == sim.mgood.sum() and np.array_equal(out["model_num_good"][0, b], sim.mgood), b
+    assert failed > 4
 
 
 def test_groups_that_become_idle_at_the_same_instant(eng):
