@@ -380,6 +380,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     int blanes = kWave;  // batching simulator: lanes of a wavefront that simulate
     int tile_sims = kWave;  // simulations of a tile
     bool solo = false;      // batching simulator: a wavefront for each simulation
+    bool solo_masks = false;  // ... whose models that wait are bits of a mask
     int row = kWave;        // width of the rows of the device tables and results
     // Wavefronts per workgroup: no more than it takes to give every CU its share of the
     // batch (a small batch is spread over the CUs, one wavefront per workgroup), and
@@ -523,7 +524,8 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         if (heap_cap < heap_min) return fail(MMSIM_E_UNSUPPORTED, "batching simulator: per-wavefront state does not fit in LDS (too many models/stages/groups)");
         batching_bytes_for = bytes_for;
         tile_sims = blanes;
-        const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(M, t->NB, heap_cap, Gmax) && rl.models_ascend();
+        const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(t->NB, heap_cap, Gmax);
+        solo_masks = M <= kSoloMasks && rl.models_ascend();
         // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them; beyond that
         // up to 64 if the groups are busy half of the time, and any number if they have more to do than they can.  ms with
         // octets / with these, 150000 requests, 96 models on 48 devices, load 2.7: 2048 simulations 54 / 39, 3072 132 / 46, 4096
@@ -536,14 +538,19 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         const int64_t at_once = cus * std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         int64_t requests = 0;
         for (int s = 0; s < n_seeds; ++s) requests += wls[s]->R;
-        bool all_solo = can_solo && requests >= (int64_t)512 * n_seeds;
+        bool all_solo = can_solo && solo_masks && requests >= (int64_t)512 * n_seeds;
         if (all_solo && sims > at_once) {
             const double load = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data());
             all_solo = load >= (sims <= at_once * 64 / kSoloWavesPerCu ? 0.5 : 1.0);
         }
+        // More models than a mask has bits: up to eight simulations to a CU, whatever the streams (600 models on 24 devices, 15000
+        // requests, ms with octets / a wavefront each: 1000 simulations 42.8 / 10.4, with counts 63 / 14.3; 2048 53.7 / 11.3;
+        // 513 models, one simulation 18.0 / 8.4, 128 of them 23.7 / 10.3; 2000 models, 128 32.5 / 9.1; whole calls on 100 requests,
+        // 600 models, with counts: 256 simulations 5.5 / 5.4, 2000 53 / 37).  Beyond that nothing has been measured.
+        const int64_t few = cus * std::min<int64_t>(2 * kMaxWavesPerBlockBatching, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         if (B == 1 && blanes == 8 && o.batching_lanes == 0) {
             tile_sims = 1;  // (no more tiles than otherwise)
-        } else if (all_solo) {
+        } else if (all_solo || (can_solo && !solo_masks && sims <= few)) {
             tile_sims = 1;
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
@@ -957,7 +964,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     int batching_g2m_lds = 0;
     if (batching) {
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
-        const size_t g2m_b = solo ? 0 : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
+        const size_t g2m_b = solo ? (solo_masks ? 0 : ((size_t)members_max * 2 + 15) & ~(size_t)15) : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
         const size_t cap = (size_t)ctx->max_lds;
         // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
         const int tiles_here = std::max(1, b->tiles);
@@ -1203,7 +1210,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         q.g2m_in_lds = batching_g2m_lds;
         q.lane_stride = blanes;
         q.tile_sims = tile_sims;
-        q.solo = solo ? 1 : 0;
+        q.solo = !solo ? 0 : solo_masks ? 1 : 2;
         q.uniform_stages = uniform_stages ? 1 : 0;
         q.tile_seed = b->tile_seed.p;
         q.paired = b->paired ? 1 : 0;

@@ -186,7 +186,8 @@ struct BatchingArgs {
     int32_t g2m_in_lds;          // 1: each wavefront keeps its g2m_off / g2m_idx rows in LDS
     int32_t lane_stride;         // 64, 32, 16 or 8 (octets): lanes of a wavefront that simulate; pitch of the per-lane LDS arrays
     int32_t tile_sims;           // simulations of a tile: lane_stride, or fewer in an octet tile (1, 2 or 4)
-    int32_t solo;                // 1: tile_sims is 1 and the kernel for one simulation to a wavefront runs
+    int32_t solo;                // 1, 2: tile_sims is 1 and the kernel for one simulation to a wavefront runs (2: any number of
+                                 // models, in any order)
     int32_t uniform_stages;      // 1: a configuration's stages all have the same latencies and lat holds them once ([M][lat_row][NB], one row per configuration)
     const int32_t *tile_seed;    // as in MixedArgs
     int32_t paired;
@@ -296,8 +297,9 @@ constexpr int64_t kStatsScratchBytes = (int64_t)1 << 30;  // scratch rows of one
 
 hipError_t launch_sim_scalar(const ScalarArgs &args, hipStream_t stream, std::string *err);
 
-// One simulation to a wavefront (sim_batching_solo.hip), for tables, event slots and models that its lanes hold.
-constexpr bool batching_solo_fits(int M, int NB, int heap_cap, int Gmax) { return M <= 512 && NB <= 8 && heap_cap <= 64 && Gmax <= 64; }
+// One simulation to a wavefront (sim_batching_solo.hip), for tables and event slots that its lanes hold.
+constexpr bool batching_solo_fits(int NB, int heap_cap, int Gmax) { return NB <= 8 && heap_cap <= 64 && Gmax <= 64; }
+constexpr int kSoloMasks = 512;  // up to so many models, listed in ascending order, a bit each says whether they wait
 constexpr int kSoloRowsInLds = 128;  // up to so many models their replicas' descriptors are in LDS (halves: 8 x 2 bytes)
 constexpr size_t batching_solo_bytes(int nslots, int M) {  // LDS of a wavefront (three clocks more than there are)
     return (size_t)((nslots + 4) & ~1) * 8 + (size_t)M * (M <= kSoloRowsInLds ? 32 : 16);

@@ -7,7 +7,7 @@
 //   lane e  event slot e: time and group of a pending idle event (:728, :739-740).  The earliest is found by comparing
 //           all lanes with the earliest time, which is kept exact (one minimum over the wavefront when an event is
 //           taken, none when one is added).
-//   lane g  the models of group g, a bit per model.  Which models have waiting requests is a scalar mask, so whether
+//   lane g  the models of group g, a bit per model (up to 512 of them in ascending order).  Which models have waiting requests is a scalar mask, so whether
 //           a group that became idle has anything to do is one AND, and only when several of its models wait are
 //           the ranks of their heads looked at (:654-664).
 //   lane j  entry j of the queue a batch is taken from, sixteen of them, and latency column j (:666-704).
@@ -34,7 +34,8 @@
 // writes by one lane cost more than the chain); six wavefronts to a SIMD.
 //
 // LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
-// its head and of its next arrival in the stream's lists, rank of the head; up to 128 models also their replicas.
+// its head and of its next arrival in the stream's lists, rank of the head; up to 128 models also their replicas; without
+// masks the groups' lists of models, if they fit.
 #include "mmsim_internal.h"
 
 namespace mmsim {
@@ -146,7 +147,9 @@ __device__ __forceinline__ double wave_min(double v) {
 
 // LATLDS: the latency table is in LDS.  UNIF: every (model,
 // configuration) has the same latencies in all of its stages, held once.  OUTPUTS: anything beyond the scores (a.flags
-// says what).  MW: 64-bit words that hold a bit per model.
+// says what).  MW: 64-bit words that hold a bit per model; 0: any number of models, and groups that list them in any order.
+// Then who waits is read from the queues, and the group's list is gone through 64 entries at a time (LDS if it fits): the first of
+// the earliest heads by its place in the list.
 template <bool LATLDS, bool UNIF, bool OUTPUTS, int MW>
 __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching_solo_kernel(const BatchingArgs a) {
     const int lane = (int)(threadIdx.x & 63), oct = lane >> 3;
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const int64_t *__restrict__ mo = a.mq_off + (size_t)seed * (M + 1);
     const MqEntry *__restrict__ mq = a.mq + mo[0];
     const uint32_t *__restrict__ rows = reinterpret_cast<const uint32_t *>(a.rep8) + (size_t)tile * M * 8;
-    constexpr bool ROWSLDS = 64 * MW <= kSoloRowsInLds;
+    constexpr bool ROWSLDS = MW != 0 && 64 * MW <= kSoloRowsInLds;
     const uint32_t rows16 = queues + (uint32_t)M * 16u;  // [M][8] the descriptors' low halves, if they are in LDS
     const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra;
     const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1);
@@ -191,19 +194,27 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{0u, (uint32_t)(mo[m] - mo[0]), (uint32_t)(mo[m] - mo[0]), (uint32_t)a.mq[mo[m]].rank});
     if constexpr (ROWSLDS)
         for (int x = lane; x < M * 8; x += kWave) lds_put<uint16_t>(rows16 + (uint32_t)x * 2u, (uint16_t)((rows[x] & 0x1FFFu) | (rows[x] >> 16 & 0x8000u)));
-    uint64_t members[MW] = {};  // lane g: models of group g
+    constexpr int W = MW != 0 ? MW : 1;
+    uint64_t members[W] = {};  // lane g: models of group g
+    uint32_t list_begin = 0, list_end = 0;  // MW 0, lane g: their places in the lists
+    const uint16_t *__restrict__ lists = a.g2m_idx + (size_t)tile * a.members_max;
+    const uint32_t lists16 = clk + (uint32_t)batching_solo_bytes(a.nslots, M);
+    if (MW == 0 && a.g2m_in_lds)
+        for (int x = lane; x < a.members_max; x += kWave) lds_put<uint16_t>(lists16 + (uint32_t)x * 2u, lists[x]);
     if (lane < a.Gmax) {
         const uint16_t *first = a.g2m_off + (size_t)tile * (a.Gmax + 1) + lane;
-        const uint16_t *list = a.g2m_idx + (size_t)tile * a.members_max;
-        for (int x = first[0]; x < (int)first[1]; ++x) {
-            const int m = list[x];
+        list_begin = first[0];
+        list_end = first[1];
+        if constexpr (MW != 0)
+            for (uint32_t x = list_begin; x < list_end; ++x) {
+                const int m = lists[x];
 #pragma unroll
-            for (int i = 0; i < MW; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
-        }
+                for (int i = 0; i < W; ++i) members[i] |= m >> 6 == i ? 1ull << (m & 63) : 0ull;
+            }
     }
     const uint32_t group = lane < a.Gmax ? ginfo[lane] : kEmpty;  // lane g: descriptor of group g
     const uint64_t groups = ballot((int32_t)group >= 0);  // (a group that lists no model may still be some model's replica)
-    uint64_t waiting[MW] = {};  // models with waiting requests
+    uint64_t waiting[W] = {};  // models with waiting requests
     double ev_t = inf;          // lane e: event slot e
     uint32_t ev_d = 0;
     uint64_t used = 0;          // event slots that hold an event
@@ -233,7 +244,8 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 
     // the models m of these octets wait
     auto add_waiting = [&](int m, uint64_t lanes) {
-        if constexpr (MW <= 2) {
+        if constexpr (MW == 0) {
+        } else if constexpr (MW <= 2) {
             uint32_t bits[2 * MW];
 #pragma unroll
             for (int i = 0; i < 2 * MW; ++i) bits[i] = in_mask(lanes & ballot(m >> 5 == i)) ? 1u << (m & 31) : 0u;
@@ -246,9 +258,25 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     };
 
     // :654-664 -- among the models of group g with a waiting request, the one whose head arrived first; of several that
-    // arrived at the same time the first of the (ascending) list
+    // arrived at the same time the first of the list (which ascends, unless MW is 0)
     auto select_model = [&](uint32_t g) -> int {
-        uint64_t cand[MW];
+        if constexpr (MW == 0) {
+            const uint32_t end = lane_value(list_end, (int)g);
+            uint32_t best = 0xFFFFFFFFu;
+            int pick = -1;
+            for (uint32_t x = lane_value(list_begin, (int)g); x < end; x += kWave) {
+                const uint32_t at = x + (uint32_t)lane < end ? x + (uint32_t)lane : end - 1u;  // (the last one again: comes later)
+                const int m = a.g2m_in_lds ? lds_get<uint16_t>(lists16 + at * 2u) : lists[at];
+                const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
+                const uint32_t rank = queue.z != queue.y ? queue.w : 0xFFFFFFFFu, least = wave_min(rank);
+                if (least < best) {
+                    best = least;
+                    pick = lane_value(m, first_of(ballot(rank == least)));
+                }
+            }
+            return pick;
+        }
+        uint64_t cand[W];
         int n = 0, only = -1;
 #pragma unroll
         for (int i = 0; i < MW; ++i) {
@@ -257,7 +285,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             if (cand[i] != 0ull) only = 64 * i + first_of(cand[i]);
         }
         if (n <= 1) return only;
-        uint32_t rank[MW], least = 0xFFFFFFFFu;
+        uint32_t rank[W], least = 0xFFFFFFFFu;
 #pragma unroll
         for (int i = 0; i < MW; ++i) {
             rank[i] = 0xFFFFFFFFu;
@@ -363,6 +391,10 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             if (h == arr) {  // none of them (:709-713)
                 const int32_t next_rank = mq[(size_t)h].rank;
                 set_waiting(m, false);
+                if (MW == 0) {  // (select_model looks at it)
+                    lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, h);
+                    wave_order();
+                }
                 const int m_next = select_model(g);
                 lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, h);
                 lds_put<uint32_t>(queues + (uint32_t)m * 16u + 12u, (uint32_t)next_rank);
@@ -586,10 +618,11 @@ bool solo_outputs(const BatchingArgs &a) {
 
 hipError_t launch_sim_batching_solo(const BatchingArgs &args, int wpb, size_t lds_bytes, hipStream_t stream) {
     const bool ll = args.lat_lds_bytes > 0, unif = args.uniform_stages != 0, outputs = solo_outputs(args);
-    if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.tile_sims != 1 || !batching_solo_fits(args.M, args.NB, args.heap_cap, args.Gmax)) return hipErrorInvalidValue;
+    if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.tile_sims != 1 || !batching_solo_fits(args.NB, args.heap_cap, args.Gmax) || (args.solo == 1 && args.M > kSoloMasks)) return hipErrorInvalidValue;
     void (*kern)(const BatchingArgs) = nullptr;
 #define MMSIM_PICK3(L, U, O)                                       \
-    (args.M <= 64    ? sim_batching_solo_kernel<L, U, O, 1>          \
+    (args.solo == 2  ? sim_batching_solo_kernel<L, U, O, 0>          \
+     : args.M <= 64  ? sim_batching_solo_kernel<L, U, O, 1>          \
      : args.M <= 128 ? sim_batching_solo_kernel<L, U, O, 2>          \
      : args.M <= 256 ? sim_batching_solo_kernel<L, U, O, 4>          \
                      : sim_batching_solo_kernel<L, U, O, 8>)
@@ -616,7 +649,7 @@ hipError_t launch_sim_batching_solo(const BatchingArgs &args, int wpb, size_t ld
 
 std::string sim_batching_solo_kernel_name(const BatchingArgs &args) {
     return std::string("sim_batching_solo_kernel<") + (args.lat_lds_bytes > 0 ? "true, " : "false, ") +
-           (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.M <= 64 ? "1>" : args.M <= 128 ? "2>" : args.M <= 256 ? "4>" : "8>");
+           (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.solo == 2 ? "0>" : args.M <= 64 ? "1>" : args.M <= 128 ? "2>" : args.M <= 256 ? "4>" : "8>");
 }
 
 }  // namespace mmsim

@@ -519,6 +519,67 @@ def test_models_of_one_simulation(eng, M):
     assert 0 < g0.sum() < R
 
 
+@pytest.mark.parametrize("lds_tables", [0, 3])
+@pytest.mark.parametrize("M,listed", [(3, 3), (70, 63), (70, 64), (70, 65), (513, 129), (700, 700)])
+def test_models_listed_in_any_order(eng, opts, M, listed, lds_tables):
+    """Groups that list their models in any order, or more of them than a mask has bits: the first listed of several heads that arrived
+    at the same instant, in lists that end inside and at the end of 64 entries, from LDS and from memory."""
+    opts(batching_lds_tables=lds_tables)
+    rng = np.random.default_rng(1000 * M + listed)
+    G, R, sizes = 6, 1500, [1, 2, 4]
+    c = random_case(8_100_000 + M, max_m=1, max_g=1, max_r=1)       # (keys; every value is made here)
+    c["m2g"], c["g2m"] = np.full((M, G), -1, np.int32), np.full((G, M), -1, np.int32)
+    for g in range(G):
+        ms = rng.choice(M, listed, replace=False)
+        c["g2m"][g, :listed] = ms
+        for m in ms:
+            c["m2g"][m, (c["m2g"][m] >= 0).sum()] = g
+    c["num_stages"] = np.array([1, 2, 4, 7, 1, 3], np.int32)
+    c["lat"] = (rng.uniform(0.01, 0.05, (M, G, 7, 1)) * np.array([1.0, 1.3, 1.9])).astype(np.float32)
+    gaps = rng.exponential(0.03, R)
+    gaps[rng.random(R) < 0.8] = 0.0
+    c["tstamps"], c["slos"] = np.cumsum(gaps), rng.uniform(0.1, 2.0, R).astype(np.float32)
+    c["model_ids"] = rng.integers(0, M, R).astype(np.int32)
+    f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
+        c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], sizes)
+    fin, good, cnt = _single(eng, c, sizes)
+    assert np.array_equal(good, g0) and np.array_equal(fin.view(np.uint64), f0.view(np.uint64))
+    for a, b in zip(cnt, c0):
+        assert np.array_equal(a, b)
+    assert 0 < g0.sum() < R
+
+
+@pytest.mark.parametrize("M,instance", [(512, "8>"), (513, "0>"), (900, "0>")])
+def test_many_models_one_simulation_to_a_wavefront(eng, M, instance):
+    """Batches of more models than a mask has bits have a wavefront for each simulation too, while the chip has room for them."""
+    from mms_amd.profiling import ParallelConfig, synthetic_profile
+    from mms_amd.placement_policy import ModelPlacement
+    rng = np.random.default_rng(M)
+    G, B, sizes = 9, 70, [1, 2, 4, 8]
+    pcs = [ParallelConfig(1, 1, 1), ParallelConfig(1, 1, 2), ParallelConfig(1, 1, 4)]
+    profiles = [synthetic_profile(f"m{m}", float(rng.uniform(0.05, 0.3)), pcs, batch_sizes=sizes, batch_slope=0.2) for m in range(M)]
+    sols = [ModelPlacement([pcs[int(rng.integers(3))] for _ in range(G)],
+                           [sorted(rng.choice(M, int(rng.integers(1, 200)), replace=False).tolist()) for _ in range(G)]) for _ in range(B)]
+    table = E.LatencyTable(profiles, sizes)
+    packed = E.pack_placements(sols, table)
+    streams = [SimpleNamespace(tstamps=np.cumsum(rng.exponential(0.02, R) * (rng.random(R) < 0.5)), model_ids=rng.integers(0, M, R).astype(np.int32),
+                               slos=rng.uniform(0.2, 1.5, R).astype(np.float32)) for R in (5000, 4999)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    batch = E.Batch(eng, dws, table, packed, _lib.BATCHING | _lib.WANT_MODEL_COUNTS)
+    assert batch.kernel_name().startswith("sim_batching_solo") and batch.kernel_name().endswith(instance)
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    for k in (0, 1):
+        ref = oracle_batch(streams[k], table, packed, batching=True)
+        assert np.array_equal(out["n_good"][k], ref["n_good"]) and np.array_equal(out["model_num_good"][k], ref["model_num_good"])
+        assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
+        assert 0 < ref["n_good"].sum() < B * len(streams[k].tstamps)
+    for dw in dws:
+        dw.close()
+
+
 @pytest.mark.parametrize("B,n_streams,R,pace,solo", [(71, 29, 511, 3.0, False), (71, 29, 512, 3.0, True), (512, 32, 513, 0.3, True), (513, 32, 513, 0.3, False), (513, 32, 513, 3.0, True),
                                                      (160, 32, 520, 0.01, True), (161, 32, 520, 0.01, False)])
 def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, pace, solo):
