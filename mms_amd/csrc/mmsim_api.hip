@@ -526,14 +526,26 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         tile_sims = blanes;
         const bool can_solo = blanes == 8 && o.batching_lanes == 0 && batching_solo_fits(t->NB, heap_cap, Gmax);
         solo_masks = M <= kSoloMasks && rl.models_ascend();
-        // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them; beyond that
-        // up to 64 if the groups are busy half of the time, and any number if they have more to do than they can.  ms with
-        // octets / with these, 150000 requests, 96 models on 48 devices, load 2.7: 2048 simulations 54 / 39, 3072 132 / 46, 4096
-        // 133 / 52, 8192 161 / 90, 16384 200 / 157, 32768 411 / 298, and 12000 requests, 65536, load 1.4: 75 / 57; 30000
-        // requests, 48 models on 24 devices, load 0.7: 8192 61 / 40, 16384 73 / 67, 65536 216 / 235; 23108 requests, 5 models on
-        // 49 devices, load 0.1, where nearly every request is a batch and the octets of a wavefront share the cost of their
-        // events: 4096 164 / 116, 8192 181 / 202.  Streams of a few hundred requests are over within a millisecond and keep
-        // fewer wavefronts (16384 simulations of 200 requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
+        // A wavefront for each simulation (sim_batching_solo.hip) while a CU takes them all at once, 20 of them.  Beyond that they
+        // share the CU's issue, and what one costs goes with how many of its requests start a batch: the fewer, the busier the
+        // groups and the fewer replicas there are to find an idle one among.  Eight to a wavefront take about as long whether 20
+        // or 64 of them are on a CU.  Where both are level, in simulations to a CU (4000 to 6000 requests, CV 4, twelve problems of 5 to
+        // 64 models on 16 to 64 devices):
+        //     replicas   1.2   2.0   2.3   4.6   4.8   7.4   7.5   9.6    12    15
+        //     load 0.1    52    47                                               28
+        //     load 0.2    57    52    54    47    39    38    30    28    29    28
+        //     load 0.5    65    60    62    57    47    43    37    34    31    29
+        //     load 0.8    70    65    64    62    55    46    43    38    32    30
+        // which 76 + 10 ln(load) - 3.5 replicas follows, as does "at least 24".  Of the 419 batches measured for it and 240 others (CV 1
+        // and 8, 2000 and 20000 requests) the rule takes 1.01 and 1.02 times as long as the better choice would, the line at half a
+        // load that was here before 1.09 and 1.08 (2.1 at most: 24 to a CU at load 0.4, 14.7 against 6.9 ms).  Below a tenth nothing
+        // was measured; octets stay.
+        // Beyond 64 octets take several rounds, and the wavefronts, too, only add up: any number of them if the groups have more
+        // to do than they can (ms with octets / with these, 65536 simulations of 4000 requests at load 1, 1.2 replicas 34.5 / 28.6
+        // and 36.3 / 27.2, 2.3 replicas 31.6 / 28.3, but 4.6 replicas 30.1 / 37.3, 7.4 replicas 41.0 / 60.6; at load 5 21.2 / 14.4,
+        // 22.0 / 13.4, 20.0 / 14.9, 19.9 / 20.9, 30.8 / 44.3).
+        // Streams of a few hundred requests are over within a millisecond and keep fewer wavefronts (16384 simulations of 200
+        // requests: 0.40 / 0.42, of 1000: 1.28 / 1.05).
         const int64_t cus = std::max(1, ctx->prop.multiProcessorCount), sims = (int64_t)B * b->out_seeds;
         const int64_t at_once = cus * std::min<int64_t>(kSoloWavesPerCu, (int64_t)((size_t)ctx->max_lds / batching_solo_bytes(nslots, M)));
         int64_t requests = 0;
@@ -541,7 +553,9 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         bool all_solo = can_solo && solo_masks && requests >= (int64_t)512 * n_seeds;
         if (all_solo && sims > at_once) {
             const double load = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data());
-            all_solo = load >= (sims <= at_once * 64 / kSoloWavesPerCu ? 0.5 : 1.0);
+            const double replicas = replicas_of_a_request(wls, n_seeds, rl), per_cu = (double)sims / (double)at_once * kSoloWavesPerCu;
+            const double level = std::min(64.0, std::max(24.0, 76.0 + 10.0 * std::log(std::max(load, 0.1)) - 3.5 * replicas));
+            all_solo = (load >= 0.1 && per_cu <= level) || (load >= 1.0 && replicas <= 3.0);
         }
         // More models than a mask has bits: up to eight simulations to a CU, whatever the streams (600 models on 24 devices, 15000
         // requests, ms with octets / a wavefront each: 1000 simulations 42.8 / 10.4, with counts 63 / 14.3; 2048 53.7 / 11.3;

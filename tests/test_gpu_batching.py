@@ -583,8 +583,8 @@ def test_many_models_one_simulation_to_a_wavefront(eng, M, instance):
 @pytest.mark.parametrize("B,n_streams,R,pace,solo", [(71, 29, 511, 3.0, False), (71, 29, 512, 3.0, True), (512, 32, 513, 0.3, True), (513, 32, 513, 0.3, False), (513, 32, 513, 3.0, True),
                                                      (160, 32, 520, 0.01, True), (161, 32, 520, 0.01, False)])
 def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, pace, solo):
-    """Twenty simulations to a CU, sixty-four if their groups are busy half of the time or any number if they have more to do
-    than they can, have a wavefront each, unless their streams are short: the oracle's counts and traces on both sides of each line."""
+    """Twenty simulations to a CU, sixty-four of this problem if its groups are busy half of the time or any number if they have more
+    to do than they can, have a wavefront each, unless their streams are short: the oracle's counts and traces on both sides of each line."""
     cfg = make_config(5, B)
     table = E.LatencyTable(cfg.profiles, cfg.batch_sizes)
     packed = E.pack_placements(cfg.placements, table)
@@ -607,6 +607,37 @@ def test_a_wavefront_for_each_of_many_simulations(eng, B, n_streams, R, pace, so
                 _check(out, ref, k, per_request=bool(flags & _lib.WANT_PER_REQUEST))
             assert np.array_equal(out["n_good"][k], ref["n_good"]) and np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0)
             assert 0 < ref["n_good"].sum() < B * R
+    for dw in dws:
+        dw.close()
+
+
+@pytest.mark.parametrize("M,G,k,load,B,solo", [(16, 8, 2, 0.2, 384, True), (16, 8, 2, 0.2, 480, False), (8, 10, 8, 0.5, 240, True), (8, 10, 8, 0.5, 288, False),
+                                               (16, 8, 2, 2.0, 520, True), (8, 10, 8, 2.0, 520, False)])
+def test_a_wavefront_for_each_by_load_and_replicas(eng, M, G, k, load, B, solo):
+    """From 24 to 64 simulations to a CU, and beyond, how busy the groups are and how many replicas a request may choose from decide whether
+    each has a wavefront (32 streams; 256 CUs): the oracle's results on both sides."""
+    from mms_amd.profiling import ParallelConfig, synthetic_profile
+    from mms_amd.placement_policy import ModelPlacement
+    rng = np.random.default_rng(B)
+    R, n_streams, sizes = 512, 32, [1, 2, 4]
+    profiles = [synthetic_profile(f"m{m}", 0.1, [ParallelConfig(1, 1, 1)], batch_sizes=sizes, batch_slope=0.2) for m in range(M)]
+    sols = [ModelPlacement([ParallelConfig(1, 1, 1)] * G, [sorted(((np.arange(k) + g * k) % M).tolist()) for g in rng.permutation(G)]) for _ in range(B)]
+    table = E.LatencyTable(profiles, sizes)
+    packed = E.pack_placements(sols, table)
+    streams = [SimpleNamespace(tstamps=np.cumsum(rng.exponential(0.1 / G / load, R)), model_ids=rng.integers(0, M, R).astype(np.int32),
+                               slos=np.full(R, 0.3, np.float32)) for _ in range(n_streams)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    batch = E.Batch(eng, dws, table, packed, _lib.BATCHING | _lib.WANT_MODEL_COUNTS)
+    name = batch.kernel_name()
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    assert name.startswith("sim_batching_solo" if solo else "sim_batching_kernel")
+    for s in (0, n_streams - 1):
+        ref = oracle_batch(streams[s], table, packed, batching=True)
+        assert np.array_equal(out["n_good"][s], ref["n_good"]) and np.array_equal(out["model_num_good"][s], ref["model_num_good"])
+        assert np.allclose(out["latency_sum"][s], ref["latency_sum"], rtol=1e-12, atol=0)
     for dw in dws:
         dw.close()
 
