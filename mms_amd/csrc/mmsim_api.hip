@@ -483,7 +483,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
                 if (wave_bytes <= (size_t)ctx->max_lds) break;
             }
         };
-        // Rows of the device tables and of the counts are 64 wide whatever a tile holds; the microsecond or two of a
+        // Rows of the device tables and of the counts are 64 wide whatever an octet tile holds; the microsecond or two of a
         // request's time that narrow tiles gain makes up for a few kilobytes of them.  The per-request outputs and the
         // tables of a call without allocations stay dense.
         auto affordable = [&](int sims) {
@@ -569,8 +569,9 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         } else if (blanes == 8 && o.batching_lanes == 0) {
             // Fewer simulations to an octet tile while all wavefronts are still on the chip at once: between two
             // arrivals the octets of a wavefront have their events one after the other (10000 requests, 96 models on 48
-            // devices, ms at 8 / 4 / 2 / 1 simulations, a single one in the kernel that looks at eight arrivals at once: 1024
-            // placements 16.6 / 13.8 / 11.4 / 7.4, 4096: 17.3 / 14.8 / 12.7 / 16.0 (two rounds), 8192: 17.7 / 15.8 / 25).
+            // devices, ms at 8 / 4 / 2 simulations: 1024 placements 16.6 / 13.8 / 11.4, 4096: 17.3 / 14.8 / 12.7, 8192: 17.7 / 15.8 /
+            // 25, two rounds).  One to a tile: short streams, and what sim_batching_solo.hip does not take (more than eight
+            // batch sizes or 64 event slots).
             const size_t least = bytes_for(8, std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7)));  // (event slots are trimmed below)
             const int64_t per_cu = std::max<int64_t>(1, std::max(std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / least)),
                                                                  2 * std::min<int64_t>(kMaxWavesPerBlockBatching, (int64_t)(ctx->max_lds / 2 / least))));
@@ -814,7 +815,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     }
     // ---- replica lists.  Plain simulator: descriptors, the first 8 as [tiles][M][2][64] x (4 x u32),
     //      the rest [tiles][M][RX][64] x u32, missing entries empty.  Batching simulator: group
-    //      indices, first 8 packed [tiles][M][64] x u64, the rest [tiles][M][RX][64] x u8, missing
+    //      indices, first 8 packed [tiles][M][64] x u64, the rest [tiles][M][RX][row] x u8, missing
     //      entries name the empty descriptor row Gmax.
     const int RX = std::max(rmax_all - kPackedReplicas, 0);
     const uint64_t none8 = 0x0101010101010101ull * (uint64_t)Gmax;
@@ -1545,7 +1546,7 @@ int mmsim_batch_fetch(mmsim_batch *b, mmsim_result *out) try {
             if (!st_host.empty() && st_host[src] != 0) any_bad = st_host[src];
             if (!ops.empty()) out->fp_ops[(size_t)s * B + p] = ops[src];
         }
-    // device rows are [wave][x][64] with wave = seed*tiles + tile; lane l of a seed is placement l
+    // device rows are [wave][x][row] with wave = seed*tiles + tile; pos[p] = tile*row + lane says where placement p is
     auto unpack_i32 = [&](const DevBuf<int32_t> &dev, int32_t width, int32_t *dst) -> int {
         std::vector<int32_t> h(dev.n);
         HIP_TRY(hipMemcpy(h.data(), dev.p, dev.bytes(), hipMemcpyDeviceToHost));

@@ -166,24 +166,25 @@ constexpr int kSchedLdsBytes = 1024;  // LDS reserved for its schedule state
 // Arguments of the batching simulation kernel.  Replica lists and group
 // descriptors are shared with the plain kernel; on top come, per seed, the
 // arrivals regrouped by model (a model's FIFO is always a window of that list)
-// and, per lane, the models of each group.
+// and, per simulation, the models of each group.  Rows of its tables and results are `row` wide: 64, or 1 where every
+// simulation has a wavefront (solo).
 struct BatchingArgs {
     const Req *streams;          // all seeds' requests, back to back
     const int64_t *stream_off;   // [n_seeds+1]
     const int64_t *mq_off;       // [n_seeds][M+1] offsets into mq of the arrivals of each model
     const MqEntry *mq;           // model-ordered arrivals of all seeds, plus kMqPadding zeroed entries at the end
-    const uint64_t *rep8;        // as in MixedArgs; octet tiles: descriptors, [tiles][M][8 * tile_sims] u32
-    const uint8_t *repx;
-    const uint32_t *ginfo;       // [tiles][Gmax+1][64]
-    const uint16_t *g2m_off;     // [tiles][Gmax+1][64] start of each group's model list
-    const uint16_t *g2m_idx;     // [tiles][members_max][64] model ids, ascending per group
+    const uint64_t *rep8;        // [tiles][M][64] the first eight replicas, a byte each; octet tiles: descriptors, [tiles][M][8 * tile_sims] u32
+    const uint8_t *repx;         // [tiles][M][rep_extra][row] the others
+    const uint32_t *ginfo;       // [tiles][Gmax+1][row]
+    const uint16_t *g2m_off;     // [tiles][Gmax+1][row] start of each group's model list
+    const uint16_t *g2m_idx;     // [tiles][members_max][row] model ids, in the order they are looked at (solo 1: ascending per group)
     const float *lat;            // [M][lat_row][NB]
     const int32_t *batch_sizes;  // [NB]
     int32_t M, lat_row, NB, rep_extra, members_max, heap_cap;
     int32_t n_seeds, B, tiles, nslots, Gmax;
     int32_t wave_lds_bytes;
     int32_t lat_lds_bytes;       // > 0: the workgroup keeps a copy of lat in LDS (that many bytes, 16-aligned)
-    int32_t g2m_in_lds;          // 1: each wavefront keeps its g2m_off / g2m_idx rows in LDS
+    int32_t g2m_in_lds;          // 1: each wavefront keeps its g2m_off / g2m_idx rows in LDS (solo 2: g2m_idx)
     int32_t lane_stride;         // 64, 32, 16 or 8 (octets): lanes of a wavefront that simulate; pitch of the per-lane LDS arrays
     int32_t tile_sims;           // simulations of a tile: lane_stride, or fewer in an octet tile (1, 2 or 4)
     int32_t solo;                // 1, 2: tile_sims is 1 and the kernel for one simulation to a wavefront runs (2: any number of
@@ -195,14 +196,14 @@ struct BatchingArgs {
     double fixed_overhead;
     uint32_t flags;
     // outputs
-    int32_t *n_good;             // [n_seeds][tiles*64]
-    double *lat_sum;             // [n_seeds][tiles*64]
-    int32_t *status;             // [n_seeds][tiles*64] 0 or MMSIM_E_OVERFLOW
-    int32_t *model_good;         // [waves][M][64]
-    int32_t *group_req;          // [waves][Gmax][64]
-    int32_t *group_good;         // [waves][Gmax][64]
-    double *finish;              // [waves][Rmax][64]
-    uint8_t *good;               // [waves][Rmax][64]
+    int32_t *n_good;             // [n_seeds][tiles*row]
+    double *lat_sum;             // [n_seeds][tiles*row]
+    int32_t *status;             // [n_seeds][tiles*row] 0, MMSIM_E_OVERFLOW or MMSIM_E_UNSUPPORTED
+    int32_t *model_good;         // [waves][M][row]
+    int32_t *group_req;          // [waves][Gmax][row]
+    int32_t *group_good;         // [waves][Gmax][row]
+    double *finish;              // [waves][Rmax][row]
+    uint8_t *good;               // [waves][Rmax][row]
 };
 // Arguments of the plain simulator's kernel for small and middle-sized batches (sim_window.hip): the lanes of a
 // wavefront hold requests of 64 / lanes placements.

@@ -7,9 +7,9 @@
 //   lane e  event slot e: time and group of a pending idle event (:728, :739-740).  The earliest is found by comparing
 //           all lanes with the earliest time, which is kept exact (one minimum over the wavefront when an event is
 //           taken, none when one is added).
-//   lane g  the models of group g, a bit per model (up to 512 of them in ascending order).  Which models have waiting requests is a scalar mask, so whether
-//           a group that became idle has anything to do is one AND, and only when several of its models wait are
-//           the ranks of their heads looked at (:654-664).
+//   lane g  the models of group g, a bit per model (up to 512 of them in ascending order; other batches keep lists).  Which
+//           models have waiting requests is a scalar mask, so whether a group that became idle has anything to do is one
+//           AND, and only when several of its models wait are the ranks of their heads looked at (:654-664).
 //   lane j  entry j of the queue a batch is taken from, sixteen of them, and latency column j (:666-704).
 //
 // Latency sums are kept by place in the queue, as the octets there keep them, so that they are equal bit for bit.

@@ -35,9 +35,9 @@
 // What bounds it: a lone wavefront per SIMD is one dependent chain per step, LDS read of the replicas' clocks ->
 // tournament -> walk -> ballot -> commit; when several share a SIMD, instruction issue.  Per placement all state is a
 // few KB of LDS and nothing in a step touches global memory; requests are fetched two blocks ahead, replica entries
-// one block ahead.  Measured, 120280 requests on single-device groups, 64 side by side: 256 placements 2.9 ms, 3590 cycles a
-// block, 53 % of them issuing (418 instructions) and 46 % waiting; 4096 placements, four wavefronts to a SIMD, 5.6 ms,
-// 4800 cycles a block, 40 % issuing, 32 % waiting to issue, 28 % for LDS.  (One request after the other, 64 placements to
+// one block ahead.  Measured, 120280 requests on single-device groups, 64 side by side: 256 placements 2.57 ms, 2902 cycles a
+// block, 64 % of them issuing (275 vector, 98 scalar, 35 LDS instructions) and 36 % waiting; 4096 placements, four wavefronts
+// to a SIMD, 5.32 ms, 4464 cycles a block, 42 % issuing, 33 % waiting to issue, 25 % for LDS.  (One request after the other, 64 placements to
 // a wavefront: 24 ms either way.)
 // Few instructions to a step count most where a wavefront is alone.  That a block's second four replicas are in registers like
 // the first, instead of being fetched for every step, and that the words that the walk needs are ready for it took, 108000
