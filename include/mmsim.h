@@ -374,7 +374,9 @@ int mmsim_eval_batch(mmsim_ctx *ctx, const mmsim_workload *const *workloads, int
  * finish [R] and good [R] are written for every request; the four count
  * arrays are zeroed and filled.  Layouts:
  *   m_id2g_id     [M][G]  replica groups of each model, -1 terminated
- *   g_id2m_id     [G][M]  models of each group, -1 terminated (batching only)
+ *   g_id2m_id     [G][M]  models of each group, -1 terminated (batching only); MMSIM_E_INVALID if requests are left
+ *                         waiting because no group lists their model (the reference asserts that none are,
+ *                         controller.py:789-790)
  *   num_stages    [G]
  *   stage_latency [M][G][Smax]        (plain)   float32
  *                 [M][G][Smax][NB]    (batching)

@@ -2213,6 +2213,13 @@ int mmsim_simulate_requests_mixed_batching(mmsim_ctx *ctx, double *finish, uint8
         mmsim_batch_destroy(b);
         if (rc != MMSIM_E_OVERFLOW) break;
     }
+    // Every queued request is dropped or served by one group, unless no group lists its model: the reference asserts that
+    // no queue holds any at the end (:789-790).
+    int64_t queued = 0, settled = 0;
+    for (int32_t m = 0; m < M; ++m) queued += model_num_requests[m];
+    for (int32_t g = 0; g < G; ++g) settled += group_num_requests[g];
+    if (rc == MMSIM_OK && queued != settled)
+        return fail(MMSIM_E_INVALID, "simulate_requests_mixed_batching: requests are left waiting that no group turns to (g_id2m_id lists too few models)");
     return rc;
 } catch (...) {
     return caught();

@@ -67,8 +67,8 @@ def test_random_cases_match_oracle(eng):
 
 def test_groups_that_list_no_model(eng):
     """Which groups a model may use and which models a group may turn to are lists of their own: a group that lists no model
-    still runs the requests that arrive while it is idle."""
-    ran = 0
+    still runs the requests that arrive while it is idle.  Requests that no group turns to are an error."""
+    ran = left = 0
     for seed in range(120):
         nb = 1 + seed % 5
         c = random_case(9_500_000 + seed, max_m=6, max_g=5, max_s=4, max_r=200, nb=nb, load=0.3 + 0.3 * (seed % 5), inf_slo=False)
@@ -77,6 +77,10 @@ def test_groups_that_list_no_model(eng):
             f0, g0, c0, _ = oracle_c.simulate_requests_mixed_batching(
                 c["tstamps"], c["model_ids"], c["slos"], c["m2g"], c["g2m"], c["num_stages"], c["lat"], BSS[:nb])
         except AssertionError:      # requests that nobody turns to are left over at the end: the reference stops there
+            with pytest.raises(_lib.MmsimError) as err:
+                _single(eng, c, BSS[:nb])
+            assert err.value.code == _lib.E_INVALID
+            left += 1
             continue
         fin, good, cnt = _single(eng, c, BSS[:nb])
         assert np.array_equal(good, g0), seed
@@ -84,7 +88,7 @@ def test_groups_that_list_no_model(eng):
         for a, b in zip(cnt, c0):
             assert np.array_equal(a, b), seed
         ran += int(c0[2][c["g2m"][:, 0] < 0].sum() > 0)
-    assert ran > 20
+    assert ran > 20 and left > 10
 
 
 @pytest.mark.parametrize("lanes", [0, 8, 64])
@@ -490,7 +494,7 @@ def test_one_simulation_to_a_wavefront(eng, sizes, groups):
 
 @pytest.mark.parametrize("M", [1, 64, 65, 128, 129, 256, 257, 512, 513])
 def test_models_of_one_simulation(eng, M):
-    """The models that wait are bits of one, two, four or eight words (more models: the kernel of wider tiles): the oracle's flags
+    """The models that wait are bits of one, two, four or eight words (more models: read from the queues): the oracle's flags
     and finish times where a word ends, with heads that arrived at the same instant in different words."""
     rng = np.random.default_rng(M)
     G, R, sizes = 5, 1200, [1, 2, 4]
