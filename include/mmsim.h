@@ -100,8 +100,11 @@ typedef struct {
     int32_t segment_requests;     /* requests per turn of an item in the scheduled launch; 0: 16384             */
     int32_t sched_spin_limit;     /* looks in a row after which a wavefront that finds only busy items leaves;
                                      -1: 20000                                                                  */
-    int32_t skip_ahead;           /* loop over runs: 0 = simulate every request; -1 / 1: requests that every lane
-                                     of a wavefront must reject are not simulated                              */
+    int32_t skip_ahead;           /* loop over runs: 0 = simulate every request; 1 = requests that every lane
+                                     of a wavefront must reject are not simulated; 2 = every lane goes through the
+                                     stream at its own pace and passes over what it must reject (scores, groups of
+                                     several stages with one latency per (model, configuration); otherwise as 1);
+                                     -1: 2 where the groups have much more to do than they can, else 1         */
     int32_t xcd_map;              /* chunked loop: 0 = seeds innermost in the workgroup numbering; -1 / 1: all
                                      seeds of a tile group on one XCD                                           */
     int32_t batching_lanes;       /* batching simulator: 8, 16, 32 or 64 simulations per wavefront; 0: the widest

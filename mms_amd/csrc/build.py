@@ -22,7 +22,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 # instances are many; four translation units build in parallel).
 UNITS = {"mmsim_api": ("mmsim_api.hip", []), "window_batch": ("window_batch.hip", []),
          **{f"sim_window_{w}": ("sim_window.hip", [f"-DMMSIM_WINDOW_LANES={w}"]) for w in (64, 32, 16, 8)},
-         "sim_mixed": ("sim_mixed.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_batching_solo": ("sim_batching_solo.hip", []),
+         "sim_mixed": ("sim_mixed.hip", []), "sim_lanes": ("sim_lanes.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_batching_solo": ("sim_batching_solo.hip", []),
          "sim_scalar": ("sim_scalar.hip", []),
          "stats": ("stats.hip", [])}
 
@@ -48,8 +48,11 @@ FLAGS = [
 # Requests side by side (20000 requests; 1025 four-stage pipelines / 4096 of them / 1025 and 4096 mixed groups / 4096 single
 # devices): default 2.91 / 4.36 / 2.95 / 4.84 / 2.17 ms, with max-ilp 2.69 / 4.23 / 2.86 / 4.79 / 2.17, with the aligned
 # blocks as well 2.70 / 4.13 / 2.90 / 4.71 / 2.16, with these alone no change; iterative-ilp fails on it.
+# Lanes at their own pace (configuration 4): default 223.8 ms, iterative-ilp with the aligned blocks 218, iterative-minreg 216.7, these
+# alone 214.5, max-ilp with them 211.4.
 SOURCE_FLAGS = {"sim_window.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
+                "sim_lanes.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_batching_solo.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"],
                 "sim_batching.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-mllvm", "-align-all-nofallthru-blocks=6"]}
 

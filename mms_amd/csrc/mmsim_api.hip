@@ -55,7 +55,7 @@ int check_options(const mmsim_options *o) {
     if (o->struct_size != (int32_t)sizeof(mmsim_options))
         return fail(MMSIM_E_INVALID, "options: struct_size is not sizeof(mmsim_options); start from mmsim_options_default");
     auto tri = [](int32_t v) { return v >= -1 && v <= 1; };
-    if (!tri(o->request_loop) || !tri(o->counts_in_lds) || !tri(o->tile_order_by_slots) || !tri(o->skip_ahead) || !tri(o->xcd_map))
+    if (!tri(o->request_loop) || !tri(o->counts_in_lds) || !tri(o->tile_order_by_slots) || !(tri(o->skip_ahead) || o->skip_ahead == 2) || !tri(o->xcd_map))
         return fail(MMSIM_E_INVALID, "options: a -1 / 0 / 1 switch has another value");
     if (o->waves_per_cu < 0 || o->waves_per_cu > kMaxWavesPerBlock) return fail(MMSIM_E_INVALID, "options: waves_per_cu outside 0..8");
     if (o->sched_groups < 0 || o->segment_requests < 0 || o->sched_spin_limit < -1 || o->batching_event_slots < 0 ||
@@ -234,7 +234,70 @@ int mmsim::compact_latency(const mmsim_tables *t, bool all_batch_sizes, CompactL
 
 namespace {
 
-// Builds every device table of a batch from replica lists and launches nothing.
+// What the lanes at their own pace read besides the tables of the loop over runs: the runs of every block of the streams,
+// and the entries with latencies.
+int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mmsim_tables *t, const std::vector<float> &lat) {
+    MixedArgs &a = b->args;
+    hipStream_t st = b->ctx->stream;
+    std::vector<int64_t> base((size_t)b->n_seeds), first;
+    std::vector<int32_t> of;
+    for (int32_t s = 0; s < b->n_seeds; ++s) {
+        base[(size_t)s] = (int64_t)of.size();
+        for (int64_t r = 0; r < soff[(size_t)s + 1] - soff[(size_t)s]; r += a.run_block) {
+            of.push_back(s);
+            first.push_back(r);
+        }
+    }
+    const size_t blocks = of.size();
+    if (blocks > 0x7FFFFFFFu) return fail(MMSIM_E_UNSUPPORTED, "option segment_requests is too small for these streams");
+    DevBuf<int32_t> d_of;
+    DevBuf<int64_t> d_first;
+    HIP_TRY(d_of.alloc(blocks));
+    HIP_TRY(d_first.alloc(blocks));
+    HIP_TRY(b->run_base.alloc(base.size()));
+    HIP_TRY(b->run_off.alloc(blocks + 1));
+    HIP_TRY(hipMemcpyAsync(b->run_base.p, base.data(), sizeof(int64_t) * base.size(), hipMemcpyHostToDevice, st));
+    std::vector<uint32_t> off(blocks + 1, 0);
+    if (blocks > 0) {
+        HIP_TRY(hipMemcpyAsync(d_of.p, of.data(), sizeof(int32_t) * blocks, hipMemcpyHostToDevice, st));
+        HIP_TRY(hipMemcpyAsync(d_first.p, first.data(), sizeof(int64_t) * blocks, hipMemcpyHostToDevice, st));
+        HIP_TRY(launch_list_runs(b->streams.p, b->stream_off.p, d_of.p, d_first.p, (int32_t)blocks, a.run_block, nullptr, nullptr, nullptr, b->run_off.p + 1, st));
+        HIP_TRY(hipMemcpyAsync(off.data() + 1, b->run_off.p + 1, sizeof(uint32_t) * blocks, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+    }
+    uint64_t runs = 0;
+    for (size_t k = 0; k < blocks; ++k) {
+        runs += off[k + 1];
+        off[k + 1] = (uint32_t)runs;
+    }
+    if (runs > 0xFFFFFFFFull) return fail(MMSIM_E_UNSUPPORTED, "too many requests in one batch");
+    HIP_TRY(hipMemcpyAsync(b->run_off.p, off.data(), sizeof(uint32_t) * off.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(b->run_list.alloc((size_t)runs + 1));
+    HIP_TRY(b->run_times.alloc((size_t)b->Rtotal));
+    if (runs > 0)
+        HIP_TRY(launch_list_runs(b->streams.p, b->stream_off.p, d_of.p, d_first.p, (int32_t)blocks, a.run_block, b->run_off.p, b->run_list.p, b->run_times.p, nullptr, st));
+    HIP_TRY(b->rep16.alloc((size_t)b->tiles * b->M * 2 * kWave));
+    HIP_TRY(launch_entries(a, b->rep16.p, st));
+    std::vector<uint2> stage(lat.size(), make_uint2(0x7F800000u, 0u));
+    for (int32_t m = 0; m < b->M; ++m)
+        for (int32_t c = 0; c < t->C; ++c) {
+            const size_t at = (size_t)m * a.lat_row + c;
+            std::memcpy(&stage[at].x, &lat[at], sizeof(float));
+            stage[at].y = (uint32_t)t->cfg_pp[c] - 1u;
+        }
+    HIP_TRY(b->stage.alloc(stage.size()));
+    HIP_TRY(hipMemcpyAsync(b->stage.p, stage.data(), sizeof(uint2) * stage.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    a.run_base = b->run_base.p;
+    a.run_off = b->run_off.p;
+    a.run_list = b->run_list.p;
+    a.run_times = b->run_times.p;
+    a.rep16 = b->rep16.p;
+    a.stage = b->stage.p;
+    return MMSIM_OK;
+}
+
+// Builds every device table of a batch from replica lists.
 int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
                 const RepLists &rl, uint32_t flags, mmsim_batch **out, const int32_t *stream_of = nullptr,
                 const mmsim_options *options = nullptr) {
@@ -367,6 +430,31 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         // (with one latency per (model, configuration) the loop over runs keeps a model's row of the table in a
         // register, one entry per lane, and no table in LDS)
         if (uniform_stages && lat_row > kWave) runs = false;
+    }
+    // Lanes at their own pace (sim_lanes.hip): scores of groups of several stages on streams of which two thirds of the requests repeat the
+    // model of the one before, where the groups have so much more to do than they can that a placement accepts few requests.  A
+    // lane takes a step for each that it accepts and one for each run that it ends rejecting; in the loop over runs a wavefront takes one for each
+    // request that any of its lanes accepts, however few these are.  What is accepted goes with the load and with how many
+    // replicas a request may choose from.  Against the better one of the other two loops, 131072 simulations of 10000 requests
+    // (32768 of 30000: about 0.15 more), by load: 1.2 replicas (groups of 2 to 16 devices) 0.25 1.09, 0.7 0.95, 1.6 0.86, 5 0.60; 0.6 replicas 0.8 0.90 to 0.95, 6 0.60;
+    // 0.26 replicas 0.4 0.63 to 0.68; four-stage pipelines, 1.95 replicas 1.2 1.28, 3 1.0 (with CV 4 2.3 1.15), 0.75 replicas 0.4 1.06, 1.2 0.92;
+    // groups of 1 to 8 devices, 2.3 replicas 1.2 1.25, 3 0.97 (CV 4 2.3 1.23), 1.0 replicas 1.2 1.07 to 1.19, 3.4 0.83.  Single devices need
+    // no walk, which is what the steps save: at load 8 and 1 replica 0.9, with 1.5 1.0 and more; they keep the other loops.
+    bool own_pace = false;
+    if (!batching && uniform_stages && lat_row <= kWave && b->smax_bucket > 1 && M <= 65535 && !g_arena && o.request_loop != 0 &&
+        (o.skip_ahead < 0 || o.skip_ahead == 2) &&
+        !(flags & (MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST | MMSIM_WANT_OP_COUNT))) {
+        int64_t rep = 0, tot = 0;
+        for (int s = 0; s < n_seeds; ++s) {
+            rep += wls[s]->repeats;
+            tot += wls[s]->R;
+        }
+        own_pace = o.skip_ahead == 2;
+        if (!own_pace && 3 * rep > 2 * tot && tot >= (int64_t)kRunBlock * n_seeds) {  // (shorter streams do not pay for the further tables)
+            const double replicas = replicas_of_a_request(wls, n_seeds, rl);
+            own_pace = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()) >= 2.2 * replicas * replicas;
+        }
+        if (own_pace) runs = true;
     }
 
     phase("latency table, loop choice");
@@ -673,6 +761,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     //      take the items in turns, a segment of the stream at a time, always the item that is furthest behind, so
     //      that all items of a workgroup finish together however many regions there are.
     std::vector<int32_t> plan;
+    int32_t run_block = 0;
     if (!batching && runs) {
         // Rows the walk of a tile can read past the tile's clock slots (power-of-two walk: every walking lane reads
         // as many rows as the deepest walking lane, from its own group's first slot on).  They are part of the
@@ -738,6 +827,10 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         if (o.waves_per_cu > 0) max_regions = std::min(kMaxWavesPerBlock, o.waves_per_cu);
         int64_t seg_requests = 16384;
         if (o.segment_requests > 0) seg_requests = std::max<int64_t>(kWave, (int64_t)o.segment_requests & ~(int64_t)(kWave - 1));
+        if (own_pace) {  // a segment is a whole number of blocks
+            run_block = (int32_t)std::min<int64_t>(kRunBlock, seg_requests);
+            seg_requests = std::min<int64_t>((seg_requests + run_block - 1) / run_block * run_block, 0x7FFFFFC0 / run_block * run_block);
+        }
         std::vector<int32_t> wg_off(groups + 1, 0), part_off((size_t)groups * kMaxWavesPerBlock, -1), part_bytes((size_t)groups * kMaxWavesPerBlock, 0);
         bool shared = false;  // some workgroup has more items than regions: streams are cut into segments
         size_t lds_used = 0;
@@ -769,7 +862,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         }
         int64_t rmin = b->wl_R.empty() ? 0 : b->wl_R[0];
         for (int s2 = 0; s2 < n_seeds; ++s2) rmin = std::min(rmin, b->wl_R[(size_t)s2]);
-        if (!shared) seg_requests = 0x7FFFFFC0;  // every item has a wavefront of its own: one segment
+        if (!shared) seg_requests = own_pace ? 0x7FFFFFC0 / run_block * run_block : 0x7FFFFFC0;  // every item has a wavefront of its own: one segment
         int32_t max_nseg = 1;
         const size_t total = (size_t)wg_off[groups];
         plan.assign((size_t)(groups + 1) + 5 * total + 2 * (size_t)groups * kMaxWavesPerBlock, 0);
@@ -1196,6 +1289,17 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     a.finish = b->finish.p;
     a.good = b->good.p;
     a.fp_ops = b->fp_ops.p;
+    a.run_block = run_block;
+    if (own_pace) {
+        const int rc = prepare_own_pace(b.get(), soff, t, lat);
+        if (rc == MMSIM_E_NOMEM) {  // (the loop over runs does without the further tables)
+            (void)hipGetLastError();
+            a.run_block = 0;
+        } else if (rc != MMSIM_OK) {
+            return rc;
+        }
+        phase("runs of the streams, entries");
+    }
     if (batching) {
         BatchingArgs &q = b->bargs;
         q.streams = b->streams.p;
@@ -1476,7 +1580,8 @@ int mmsim_batch_run(mmsim_batch *b) try {
     if (b->flags & MMSIM_BATCHING) {
         if (launch_sim_batching(b->bargs, b->waves_per_block, b->lds_bytes, ctx->stream, &err) != hipSuccess) return fail(MMSIM_E_HIP, err);
     } else {
-        if (launch_sim_mixed(b->args, b->smax_bucket, b->waves_per_block, b->lds_bytes, ctx->stream, &err) != hipSuccess)
+        if ((b->args.run_block > 0 ? launch_sim_lanes : launch_sim_mixed)(b->args, b->smax_bucket, b->waves_per_block, b->lds_bytes, ctx->stream,
+                                                                         &err) != hipSuccess)
             return fail(MMSIM_E_HIP, err);
     }
     HIP_TRY(hipEventRecord(b->ev_stop, ctx->stream));
@@ -1751,9 +1856,9 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {
     out->slots = b->nslots;
     out->lds_bytes = (int32_t)b->lds_bytes;
     out->requests_total = b->Rtotal;
-    out->table_bytes = b->window ? (int64_t)b->win_in.bytes() : (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() +
+    out->table_bytes = b->window ? (int64_t)b->win_in.bytes() : (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep16.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() +
                                  b->rmax.bytes() + b->lat.bytes() + b->lat_nb.bytes());
-    out->stream_bytes = b->window ? b->Rtotal * (int64_t)sizeof(Req) : (int64_t)b->streams.bytes();
+    out->stream_bytes = b->window ? b->Rtotal * (int64_t)sizeof(Req) : (int64_t)(b->streams.bytes() + b->run_list.bytes() + b->run_times.bytes());
     out->workgroups = b->sched_groups;
     out->segments = b->max_nseg;
     out->launches = 1;
@@ -1769,6 +1874,7 @@ int mmsim_batch_kernel_name(const mmsim_batch *b, char *buf, size_t size) try {
     if (!b || !buf || size == 0) return fail(MMSIM_E_INVALID, "batch_kernel_name: null pointer or empty buffer");
     const std::string name = (b->flags & MMSIM_BATCHING) ? sim_batching_kernel_name(b->bargs)
                              : b->window                   ? sim_window_kernel_name(b->wargs)
+                                                           : b->args.run_block > 0       ? sim_lanes_kernel_name(b->args, b->smax_bucket)
                                                            : sim_mixed_kernel_name(b->args, b->smax_bucket);
     std::snprintf(buf, size, "%s", name.c_str());
     return MMSIM_OK;

@@ -281,6 +281,12 @@ struct mmsim_batch {
     int32_t sched_groups = 0, sched_waves = 0, seg_requests = 0, max_nseg = 1;
     DevBuf<int32_t> plan;      // wg_off | item_tile | item_seed | item_nslots | item_bytes | item_nseg | part_off | part_bytes
     DevBuf<double> state;
+    // ... with lanes at their own pace
+    DevBuf<int64_t> run_base;
+    DevBuf<uint32_t> run_off;
+    DevBuf<Run> run_list;
+    DevBuf<double> run_times;
+    DevBuf<uint2> rep16, stage;
 
     DevBuf<Req> streams;
     DevBuf<int64_t> stream_off;

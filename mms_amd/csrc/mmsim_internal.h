@@ -88,6 +88,18 @@ constexpr int kPackedReplicas = 8;
 constexpr int kWave = 64;
 constexpr int kStageBytes = kWave * (int)sizeof(Req);  // one staged block of requests
 
+// Requests of a block of a stream that follow one another and have one model and one SLO (sim_lanes.hip).
+struct __attribute__((aligned(32))) Run {
+    double t0;        // arrival of the first
+    float latest;     // latest arrival, rounded up
+    float slo;
+    uint32_t places;  // byte offsets in the block's arrivals: of its second request | behind its last << 16
+    uint32_t models;  // its model | the next run's << 16
+    uint32_t pad[2];
+};
+static_assert(sizeof(Run) == 32, "Run must be 32 bytes");
+constexpr int kRunBlock = 4096;  // most requests of a block (8 bytes of each in 16 bits)
+
 // Arguments of the plain (non-batching) simulation kernel.
 struct MixedArgs {
     const Req *streams;          // all seeds' requests, back to back
@@ -147,6 +159,14 @@ struct MixedArgs {
     int32_t runs;                // 1: the request loop walks runs of equal models (streams whose requests mostly repeat the
                                  // model of the one before); 0: fixed chunks of four requests
     int32_t skip_ahead;          // 1: requests that every lane must reject are found a block at a time and not simulated (scores only)
+    // Lanes at their own pace (sim_lanes.hip)
+    int32_t run_block;           // requests of a block, of which a segment has a whole number; 0: another kernel
+    const int64_t *run_base;     // [n_seeds] a stream's first block
+    const uint32_t *run_off;     // [blocks + 1] a block's first run
+    const Run *run_list;
+    const double *run_times;     // arrivals of all streams, back to back
+    const uint2 *rep16;          // [tiles][M][2][64] entries of the first 8 replicas, four to a word
+    const uint2 *stage;          // [M][lat_row] {last-stage latency, stages - 1} of a configuration
     int32_t xcd_map;             // 1: all seeds of a tile group on one XCD (see sim_mixed.hip); 0: seeds innermost
 };
 
@@ -315,6 +335,14 @@ hipError_t launch_sim_batching(const BatchingArgs &args, int waves_per_block, si
 hipError_t launch_sim_mixed(const MixedArgs &args, int smax_bucket, int waves_per_block, size_t lds_bytes,
                             hipStream_t stream, std::string *err);
 std::string sim_mixed_kernel_name(const MixedArgs &args, int smax_bucket);
+// The same with lanes at their own pace, and what it reads: rep16 from rep32 and repx32; the runs of every block of
+// the streams (runs null: how many each block has).
+hipError_t launch_sim_lanes(const MixedArgs &args, int smax_bucket, int waves_per_block, size_t lds_bytes, hipStream_t stream,
+                            std::string *err);
+std::string sim_lanes_kernel_name(const MixedArgs &args, int smax_bucket);
+hipError_t launch_entries(const MixedArgs &args, uint2 *rep16, hipStream_t stream);
+hipError_t launch_list_runs(const Req *streams, const int64_t *stream_off, const int32_t *block_stream, const int64_t *block_first,
+                            int32_t blocks, int32_t run_block, const uint32_t *off, Run *runs, double *times, uint32_t *counts, hipStream_t stream);
 std::string sim_batching_kernel_name(const BatchingArgs &args);
 // Smallest compiled stage bucket >= value, or -1.
 int smax_bucket_for(int smax);

@@ -81,6 +81,7 @@
 // blockIdx.x = tile_group * n_seeds + seed.
 
 #include "mmsim_internal.h"
+#include "sched.h"
 #include "walk_asm.inc"
 
 namespace mmsim {
@@ -209,14 +210,6 @@ __device__ __forceinline__ uint32_t pick_desc(const uint4 &a, const uint4 &b) {
     return b.w;
 }
 
-// Schedule state of one workgroup (in LDS behind the latency table): one word per item, twice the segment
-// the item is at, plus one while a wavefront is simulating that segment.  A wavefront takes an item by
-// compare-and-swap on its word and hands it back with a plain atomic store, so there is no lock to hold.
-struct SchedLds {
-    uint32_t item[kMaxGroupItems];
-};
-static_assert(sizeof(SchedLds) <= kSchedLdsBytes, "schedule state outgrew its LDS reservation");
-
 // SMAX: most stages of a group (bucket).  LATLDS: the latency table is kept in LDS.  UNIFORM: one
 // latency per (model, configuration).  POW2: every group has 1, 2, 4, 8 or 16 stages.  OUT: what the
 // request loop produces beyond goodput and latency sum (a.flags says which of it): 0 nothing, 1
@@ -305,50 +298,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_mixed_kernel(con
   for (int spins = 0;;) {  // SCHED: one turn per (item, segment) this wavefront is given; otherwise a single turn
     int seg = 0, item_k = 0;
     if constexpr (SCHED) {
-        // Take the item of this workgroup that is furthest behind among those that fit this wavefront's LDS
-        // region and that nobody is simulating right now (ties: the largest, so that the large regions serve
-        // the large items).  One lane looks and claims the item with a compare-and-swap; if another
-        // wavefront was faster it looks again.
-        int got = -1;  // -1: nothing left for this wavefront, -2: what is left is being simulated by others right now
-        if (lane == 0) {
-            for (int tries = 0; tries < 64; ++tries) {
-                int best = -1, best_bytes = -1;
-                uint32_t best_word = 0xFFFFFFFFu;
-                bool pending = false;
-                for (int k = 0; k < n_items; ++k) {
-                    const uint32_t w = __hip_atomic_load(&sched->item[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    const int sg = (int)(w >> 1), nsg = a.item_nseg[item0 + k];
-                    const int bytes = a.item_bytes[item0 + k];
-                    if (sg >= nsg || bytes > part_bytes) continue;
-                    if (w & 1u) {  // worth waiting for only if a segment follows the one being simulated
-                        if (sg + 1 < nsg) pending = true;
-                        continue;
-                    }
-                    if (w < best_word || (w == best_word && bytes > best_bytes)) {
-                        best = k;
-                        best_word = w;
-                        best_bytes = bytes;
-                    }
-                }
-                if (best < 0) {
-                    got = pending ? -2 : -1;
-                    break;
-                }
-                uint32_t expect = best_word;
-                if (__hip_atomic_compare_exchange_strong(&sched->item[best], &expect, best_word | 1u, __ATOMIC_ACQUIRE,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
-                    got = best;
-                    break;
-                }
-                got = -2;  // lost the race for that item: look again (or, after many losses, sleep first)
-            }
-        }
-        got = uniform(got);
+        const int got = sched_claim(sched, a, item0, n_items, part_bytes, lane);
         if (got == -1) break;
         if (got == -2) {
-            // Everything left for this wavefront is in another wavefront's hands.  Wait a little for a segment to
-            // end; a wavefront that has waited long leaves: no item depends on it (an item is either being
-            // simulated or was just handed back by a wavefront that is about to look for work itself).
             __builtin_amdgcn_s_sleep(127);
             if (++spins > a.sched_spin_limit) break;
             continue;
@@ -357,8 +309,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_mixed_kernel(con
         item_k = got;
         tile = a.item_tile[item0 + item_k];
         seed = a.item_seed[item0 + item_k];
-        seg = uniform((int)(__hip_atomic_load(&sched->item[item_k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> 1));
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // the state another wavefront parked for this item
+        seg = sched_segment(sched, item_k);
         for (int i = lane; i < a.M; i += kWave) rmax_lds[i] = a.rmax[(size_t)tile * a.M + i];
     }
     const int nslots = SCHED ? a.item_nslots[item0 + item_k] : a.nslots;
@@ -985,12 +936,7 @@ asm volatile(NAME##_TEXT                                                        
         }
     }
     if constexpr (SCHED) {
-        // hand the item back: its parked state must be visible to whichever wavefront takes its next segment
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        if (lane == 0) {
-            __hip_atomic_store(&sched->item[item_k], (uint32_t)(seg + 1) << 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (last_seg) atomicAdd(a.error + 1, 1);  // items completed: the host checks that none is missing
-        }
+        sched_hand_back(sched, a, item_k, seg, last_seg, lane);
     } else {
         break;
     }
