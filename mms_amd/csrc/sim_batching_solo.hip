@@ -33,8 +33,13 @@
 // arrivals touched a window ahead; the batch's times worked out beside the look at its deadline (14.2 -> 14.6, 90 -> 97 ms: its
 // writes by one lane cost more than the chain); six wavefronts to a SIMD.
 //
+// Counts of groups are in the lanes' registers and counts of models beside the queues until the end: added to global memory where
+// a batch is run, each was a load that the batch waited for (128 placements 21.8 -> 16.6 ms with both, scores 14.9; one
+// placement with all outputs 18.0 -> 14.5 ms).  Tried, no gain: the next sixteen entries of every queue in LDS, fetched when the batch before
+// them was run (14.8 -> 15.0 ms: the wait for entries of a queue is not what a lone wavefront's time goes to).
+//
 // LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
-// its head and of its next arrival in the stream's lists, rank of the head; up to 128 models also their replicas; without
+// its head and of its next arrival in the stream's lists, rank of the head, requests accepted; up to 128 models also their replicas; without
 // masks the groups' lists of models, if they fit.
 #include "mmsim_internal.h"
 
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const bool want_group = OUTPUTS && (a.flags & MMSIM_WANT_GROUP_COUNTS) != 0;
     const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
     const uint32_t clk = (uint32_t)a.lat_lds_bytes + (uint32_t)wv * (uint32_t)a.wave_lds_bytes;
-    const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {-, head, behind the last arrival so far: places in the stream's lists; rank of the head}
+    const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {requests accepted, head, behind the last arrival so far: places in the stream's lists; rank of the head}
 
     const int wave = a.paired ? tile : seed * a.tiles + tile;  // where this (tile, stream) pair's results go
     const int64_t off = a.stream_off[seed], R = a.stream_off[seed + 1] - off;
@@ -181,8 +186,6 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     const uint32_t rows16 = queues + (uint32_t)M * 16u;  // [M][8] the descriptors' low halves, if they are in LDS
     const uint8_t *__restrict__ more_replicas = a.repx + (size_t)tile * M * a.rep_extra;
     const uint32_t *__restrict__ ginfo = a.ginfo + (size_t)tile * (a.Gmax + 1);
-    int32_t *model_good = a.model_good + (size_t)wave * M;
-    int32_t *group_req = a.group_req + (size_t)wave * a.Gmax, *group_good = a.group_good + (size_t)wave * a.Gmax;
     double *fin_out = a.finish + (size_t)wave * a.Rmax;
     uint8_t *good_out = a.good + (size_t)wave * a.Rmax;
     const double overhead = a.fixed_overhead, inf = __builtin_inf();
@@ -220,6 +223,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     uint64_t used = 0;          // event slots that hold an event
     const uint64_t slots = ~0ull >> (64 - a.heap_cap);
     double next_due = inf;      // the earliest event's time
+    int32_t requests_of_group = 0, good_of_group = 0;  // lane g (a count in global memory would be waited for in every batch)
     int32_t n_good = 0;
     double lat_sum = 0.0;       // of the batch members this lane accounts for
     int dead = 0;
@@ -373,7 +377,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                     fin_out[idx] = hv.x;
                     good_out[idx] = 0;
                 }
-                if (want_group && lane == 0) group_req[g] += k;
+                if (want_group) requests_of_group += lane == (int)g ? k : 0;
                 return k;
             };
             auto waiting_heads = [&]() -> int { return (int)(arr - h) < 8 ? (int)(arr - h) : 8; };
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 kfirst = first_that_can(avail);
             }
             if (h == arr) {  // none of them (:709-713)
-                const int32_t next_rank = mq[(size_t)h].rank;
+                const int32_t next_rank = lane_value(rank, avail);  // (behind those of the entries fetched last that were looked at)
                 set_waiting(m, false);
                 if (MW == 0) {  // (select_model looks at it)
                     lds_put<uint32_t>(queues + (uint32_t)m * 16u + 4u, h);
@@ -449,11 +453,13 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 }
             }
             n_good += bs;
-            if (want_group && lane == 0) {
-                group_req[g] += bs;
-                group_good[g] += bs;
+            if (want_group) {
+                requests_of_group += lane == (int)g ? bs : 0;
+                good_of_group += lane == (int)g ? bs : 0;
             }
-            if (want_model && lane == 0) model_good[m] += bs;
+            if (want_model && lane == 0)
+                __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u), (uint32_t)bs,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             if (rarely(used == slots)) {  // given up: no event is due, no arrival left (`dead` is looked at once a window)
                 dead = MMSIM_E_OVERFLOW;
                 used = 0ull;
@@ -607,6 +613,14 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         a.n_good[out] = n_good;
         a.lat_sum[out] = lat_sum;
         a.status[out] = dead;
+    }
+    if (want_group && lane < a.Gmax) {
+        a.group_req[(size_t)wave * a.Gmax + lane] = requests_of_group;
+        a.group_good[(size_t)wave * a.Gmax + lane] = good_of_group;
+    }
+    if (want_model) {
+        wave_order();
+        for (int m = lane; m < M; m += kWave) a.model_good[(size_t)wave * M + m] = lds_get<int32_t>(queues + (uint32_t)m * 16u);
     }
 }
 
