@@ -450,7 +450,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
             tot += wls[s]->R;
         }
         own_pace = o.skip_ahead == 2;
-        if (!own_pace && 3 * rep > 2 * tot && tot >= (int64_t)kRunBlock * n_seeds) {  // (shorter streams do not pay for the further tables)
+        if (!own_pace && 3 * rep > 2 * tot && tot >= (int64_t)4096 * n_seeds) {  // (shorter streams do not pay for the further tables)
             const double replicas = replicas_of_a_request(wls, n_seeds, rl);
             own_pace = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()) >= 2.2 * replicas * replicas;
         }

@@ -93,12 +93,12 @@ struct __attribute__((aligned(32))) Run {
     double t0;        // arrival of the first
     float latest;     // latest arrival, rounded up
     float slo;
-    uint32_t places;  // byte offsets in the block's arrivals: of its second request | behind its last << 16
+    uint32_t places;  // byte offsets in the block's arrivals: of its first request | of its last << 16
     uint32_t models;  // its model | the next run's << 16
     uint32_t pad[2];
 };
 static_assert(sizeof(Run) == 32, "Run must be 32 bytes");
-constexpr int kRunBlock = 4096;  // most requests of a block (8 bytes of each in 16 bits)
+constexpr int kRunBlock = 8192;  // most requests of a block (offsets of 8 bytes to a request in 16 bits)
 
 // Arguments of the plain (non-batching) simulation kernel.
 struct MixedArgs {

@@ -23,17 +23,19 @@
 //
 // The stream is cut into blocks (MixedArgs::run_block requests); the lanes of a wavefront finish a block before any of
 // them starts the next, so that what they read stays together (without the cut they drift apart by a tenth of the stream;
-// blocks of 4096 cost 3 % more steps, of 1024 12 %).  The runs of a block are listed ahead (list_runs_kernel).  A lane has the
+// blocks of 8192 cost 1.5 % more steps, of 4096 3 %, of 1024 12 %).  The runs of a block are listed ahead (list_runs_kernel).  A lane has the
 // run that it is at in registers, with up to eight replicas; the next one that it hosts, whose latencies are on their way; and the
 // run after that, which is on its way with its entries.  The arrival of the next request of its run is fetched a step ahead.
 // Everything is asked for at the end of a step and looked at at the end of the next one; a step waits for nothing but LDS.
 //
 // What bounds it (configuration 4, 131072 simulations, two wavefronts to a SIMD): a step is about 285 instructions, 165 of them vector
 // instructions, in 2200 cycles; 55 % of a wavefront's cycles issue, 32 % wait (LDS, and memory where an XCD's L2 misses), 14 % wait for the SIMD.
-// 506 ms with all lanes at the same request (102 instructions and 978 cycles for each of the stream's), 211 ms here.  On the way:
+// 506 ms with all lanes at the same request (102 instructions and 978 cycles for each of the stream's), 208 ms here.  On the way:
 // entries and latencies as 8 bytes a replica, 2 KB to a row, 338 ms; without the copies for which the compiler waits at the end of a step 261
 // (rows of all tiles of an XCD 8.4 MB, 20 % of its L2 requests miss); entries of 16 bits, 512 bytes to a row, and the latencies from a table 226
-// (misses 3 %); blocks on 64-byte boundaries and max-ilp scheduling 211.
+// (misses 3 %); branch targets on 64-byte boundaries and max-ilp scheduling 212; blocks of 8192 instead of 4096 requests 208.  A wavefront that has a CU to
+// itself takes 178 ms for the stream: what is left is the length of one wavefront's step.  Without effect: tiles composed by the steps that their lanes
+// take, items dealt by what they cost, a higher issue priority for the large items' wavefronts (all within 0.5 %).
 //
 // LDS, the schedule of items and segments and the clocks' layout are those of the loop over runs in sim_mixed.hip.
 #include "mmsim_internal.h"
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(64) void list_runs_kernel(const Req *streams, const
                 }
             float bound = (float)latest;
             if ((double)bound < latest) bound = nextafterf(bound, __builtin_inff());
-            Run out{r.t, bound, r.slo, (i + 1) * 8 | end * 8 << 16, (uint32_t)r.m | next << 16, {0u, 0u}};
+            Run out{r.t, bound, r.slo, i * 8 | (end - 1) * 8 << 16, (uint32_t)r.m | next << 16, {0u, 0u}};
             runs[off[blockIdx.x] + listed + (uint32_t)__popcll(lanes & ((1ull << lane) - 1ull))] = out;
         }
         listed += (uint32_t)__popcll(lanes);
@@ -231,7 +233,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
             uint64_t act = 0;                 // lanes that have one
             uint64_t last = 0;                // ... and are at its last request
             uint64_t more4 = 0, more8 = 0;    // ... whose model has more than four (eight) replicas
-            uint32_t next = 0, end = 0, model = 0;  // next: byte offset of the arrival of its next request
+            uint32_t at = 0, end = 0, model = 0;  // byte offsets of the arrivals of its present and of its last request
             double t = 0.0, t_next = 0.0;
             float latest = 0.0f, slo = 0.0f;
             uint32_t ca[kPackedReplicas] = {}, word[kPackedReplicas] = {};  // LDS address of the last-stage clock; the same with stages - 1 from bit 20 on
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                 const uint64_t rejects = ballot((double)latest <= win.c) & ballot(c_fin - (double)latest > slo_d) & act & ~acc;
                 const uint64_t fin = (last & act) | rejects;
                 act &= ~fin;
-                next += in_mask(act) ? 8u : 0u;
+                at += in_mask(act) ? 8u : 0u;
                 t = in_mask(act) ? t_next : t;
                 // ---- lanes without a run take the next one, if all of it is here
                 const uint64_t take = full & ~lacks & ~act;
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                     t = b_t0;
                     latest = __int_as_float(__double2loint(b_limits));
                     slo = __int_as_float(__double2hiint(b_limits));
-                    next = (uint32_t)__double2loint(b_where) & 0xFFFFu;
+                    at = (uint32_t)__double2loint(b_where) & 0xFFFFu;
                     end = (uint32_t)__double2loint(b_where) >> 16;
                     model = (uint32_t)__double2hiint(b_where) & 0xFFFFu;
 #pragma unroll
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                     asked |= ask1;
                     lacks &= ~ask2;
                 }
-                last = ballot(next >= end);
+                last = ballot(at >= end);
                 // ---- where it was taken the one after it moves up, if the lane hosts its model; if it does not, it is passed over
                 full &= ~take;
                 const uint64_t hosted = ballot((ahead_entries.x & kEntryNone) == 0);
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                 // ---- what the next step reads is asked for.  (Behind everything that was: a load that something waits for has all those
                 // before it to wait for as well.)
                 const uint32_t b_model = (uint32_t)__double2hiint(b_where) & 0xFFFFu;
-                if (in_mask(act & ~last)) t_next = load_f64(times + next);
+                if (in_mask(act & ~last)) t_next = load_f64(times + at + 8);
                 if (in_mask(up)) {
                     const uint32_t w0 = (uint32_t)__double2loint(b_entries), w1 = (uint32_t)__double2hiint(b_entries);
                     bs[0] = load_stage(w0, 0, b_model);
@@ -412,10 +414,10 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                 asked &= ~up;
                 if (in_mask(on)) {
                     ++ia;
-                    const unsigned char *at = runs + ia * (uint32_t)sizeof(Run);
+                    const unsigned char *run = runs + ia * (uint32_t)sizeof(Run);
                     ahead_entries = load_entries(next_model, 0);
-                    ahead = load4(at);  // (the list has a run more than there are)
-                    ahead2 = load2(at + 16);
+                    ahead = load4(run);  // (the list has a run more than there are)
+                    ahead2 = load2(run + 16);
                 }
                 valid &= ~(on & ballot(ia >= n_runs));
                 if ((act | full | valid) == 0) break;

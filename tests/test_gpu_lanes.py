@@ -1,5 +1,5 @@
 """The plain simulator with lanes at their own pace (sim_lanes.hip) against the CPU oracle, bit for bit, at the sizes where it can
-go wrong: streams that end inside a block of 4096 requests or a segment, runs cut by a model, an SLO, a block or a request of no
+go wrong: streams that end inside a block of 8192 requests or a segment, runs cut by a model, an SLO, a block or a request of no
 model, arrivals out of order, models with none, one to four, five to eight and more replicas, depths that are powers of two and others,
 infinite latencies and odd SLOs, items that take turns, placements with a stream of their own."""
 from types import SimpleNamespace
@@ -56,7 +56,7 @@ def _check(eng, streams, profiles, sols, M, options, expect="sim_lanes_kernel<")
 def test_lanes_at_their_own_pace(depths, groups, hosts, options):
     eng = E.Engine.default()
     M = 5 if groups > 6 else 9
-    streams = [_bursts(k, R, M, 1.0 + k) for k, R in enumerate((0, 1, 63, 65, 4095, 4097, 9000))]
+    streams = [_bursts(k, R, M, 1.0 + k) for k, R in enumerate((0, 1, 63, 65, 8191, 8193, 17000))]
     for B in (1, 64, 131):
         profiles, sols = _problem(B + sum(depths), depths, True, M, groups, B, hosts)
         _check(eng, streams, profiles, sols, M, dict(OWN, **options))
@@ -90,7 +90,7 @@ def test_arrivals_out_of_order_and_runs_of_one_model():
     mixed = _bursts(1, 5000, M, 8.0)
     rng = np.random.default_rng(2)
     shuffled = SimpleNamespace(tstamps=mixed.tstamps + rng.choice([0.0, 3.0], 5000) * (rng.random(5000) < 0.2), model_ids=mixed.model_ids, slos=mixed.slos)
-    one = _bursts(3, 9000, M, 4.0, odd_slos=False)
+    one = _bursts(3, 17000, M, 4.0, odd_slos=False)
     one.model_ids[:] = 2
     one.slos[:] = 0.4
     nobody = _bursts(4, 4200, M, 4.0)
@@ -102,7 +102,7 @@ def test_a_stream_for_every_placement():
     eng = E.Engine.default()
     M = 7
     profiles, sols = _problem(21, (1, 2, 4, 8), True, M, 6, 200, 3)
-    streams = [_bursts(40 + k, R, M, 6.0) for k, R in enumerate((5000, 4096, 0, 700))]
+    streams = [_bursts(40 + k, R, M, 6.0) for k, R in enumerate((9000, 8192, 0, 700))]
     table = E.LatencyTable(profiles, [1])
     packed = E.pack_placements(sols, table)
     dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
@@ -122,4 +122,4 @@ def test_load_decides(depths, load, expect):
     eng = E.Engine.default()
     M = 20
     profiles, sols = _problem(31, depths, True, M, 4, 70, 2)
-    _check(eng, [_bursts(50, 4200, M, load)], profiles, sols, M, dict(window_lanes=-1), expect)
+    _check(eng, [_bursts(50, 8200, M, load)], profiles, sols, M, dict(window_lanes=-1), expect)
