@@ -34,8 +34,10 @@
 // entries and latencies as 8 bytes a replica, 2 KB to a row, 338 ms; without the copies for which the compiler waits at the end of a step 261
 // (rows of all tiles of an XCD 8.4 MB, 20 % of its L2 requests miss); entries of 16 bits, 512 bytes to a row, and the latencies from a table 226
 // (misses 3 %); branch targets on 64-byte boundaries and max-ilp scheduling 212; blocks of 8192 instead of 4096 requests 208.  A wavefront that has a CU to
-// itself takes 178 ms for the stream: what is left is the length of one wavefront's step.  Without effect: tiles composed by the steps that their lanes
-// take, items dealt by what they cost, a higher issue priority for the large items' wavefronts (all within 0.5 %).
+// itself takes 178 ms for the stream: what is left is the length of one wavefront's step.  All items are on the
+// chip from the start, so the time is that of the slowest: half of them end 33 ms before it.  Without effect: tiles composed by the steps that
+// their lanes take, items dealt by what they cost, a higher issue priority for the large items' wavefronts, a run of a model with one replica
+// left in the step that accepts the last of it (4 % fewer steps; -3.6 to +1.9 % over 18 batches, 0.5 % here): all within 0.5 %.
 //
 // LDS, the schedule of items and segments and the clocks' layout are those of the loop over runs in sim_mixed.hip.
 #include "mmsim_internal.h"
