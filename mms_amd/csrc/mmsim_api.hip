@@ -1292,9 +1292,15 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     a.run_block = run_block;
     if (own_pace) {
         const int rc = prepare_own_pace(b.get(), soff, t, lat);
-        if (rc == MMSIM_E_NOMEM) {  // (the loop over runs does without the further tables)
+        if (rc == MMSIM_E_NOMEM || rc == MMSIM_E_UNSUPPORTED) {  // the loop over runs does without the further tables
             (void)hipGetLastError();
             a.run_block = 0;
+            b->run_base.release();
+            b->run_off.release();
+            b->run_list.release();
+            b->run_times.release();
+            b->rep16.release();
+            b->stage.release();
         } else if (rc != MMSIM_OK) {
             return rc;
         }
