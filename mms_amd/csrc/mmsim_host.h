@@ -192,6 +192,7 @@ struct mmsim_workload {
     std::vector<int32_t> model_num_requests;  // requests per model id (placement independent)
     double span = 0.0;                        // from the first arrival to the last
     int64_t repeats = 0;                      // requests with the model of the request before
+    int64_t run_repeats = 0;                  // ... and with its SLO (bit for bit)
     // arrivals regrouped by model (batching simulator): offsets per model, then per arrival
     // its time, its deadline time + (double)slo and its index in the stream
     std::vector<int64_t> mq_off;

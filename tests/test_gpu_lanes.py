@@ -123,3 +123,16 @@ def test_load_decides(depths, load, expect):
     M = 20
     profiles, sols = _problem(31, depths, True, M, 4, 70, 2)
     _check(eng, [_bursts(50, 8200, M, load)], profiles, sols, M, dict(window_lanes=-1), expect)
+
+
+@pytest.mark.parametrize("change,expect", [(0.0, "sim_lanes_kernel<4, true>"), (0.04, "sim_lanes_kernel<4, true>"), (0.4, "sim_mixed_kernel<4,"),
+                                           (1.0, "sim_mixed_kernel<4,")])
+def test_runs_of_one_slo_decide(change, expect):
+    """A run ends where the SLO changes: bursts of a model whose requests have SLOs of their own are runs of one request each."""
+    eng = E.Engine.default()
+    M = 20
+    profiles, sols = _problem(31, (2, 4), True, M, 4, 70, 2)
+    st = _bursts(50, 8200, M, 300.0, odd_slos=False)
+    new = np.random.default_rng(4).random(8200) < change
+    st.slos[new] = np.linspace(0.2, 0.9, int(new.sum()), dtype=np.float32)
+    _check(eng, [st], profiles, sols, M, dict(window_lanes=-1), expect)
