@@ -104,7 +104,8 @@ typedef struct {
                                      of a wavefront must reject are not simulated; 2 = every lane goes through the
                                      stream at its own pace and passes over what it must reject (scores, groups of
                                      several stages with one latency per (model, configuration); otherwise as 1);
-                                     -1: 2 where the groups have much more to do than they can, else 1         */
+                                     -1: 2 on streams of long runs (one model, one SLO) where the groups have
+                                     much more to do than they can and a request few replicas, else 1          */
     int32_t xcd_map;              /* chunked loop: 0 = seeds innermost in the workgroup numbering; -1 / 1: all
                                      seeds of a tile group on one XCD                                           */
     int32_t batching_lanes;       /* batching simulator: 8, 16, 32 or 64 simulations per wavefront; 0: the widest

@@ -19,11 +19,11 @@ pytestmark = pytest.mark.gpu
 OWN = dict(skip_ahead=2, window_lanes=-1)
 
 
-def _bursts(seed, R, M, load, odd_slos=True):
+def _bursts(seed, R, M, load, odd_slos=True, ends=0.12):
     """Runs of 1 to some 30 requests of a model, its SLO mostly the same over a run."""
     rng = np.random.default_rng(seed)
     n = R + 1
-    lengths = rng.geometric(0.12, n)
+    lengths = rng.geometric(ends, n)
     ids = np.repeat(rng.integers(-1, M, n), lengths)[:R].astype(np.int32)
     slos = np.repeat(rng.uniform(0.1, 0.9, n), lengths)[:R].astype(np.float32)
     if odd_slos:
@@ -136,3 +136,15 @@ def test_runs_of_one_slo_decide(change, expect):
     new = np.random.default_rng(4).random(8200) < change
     st.slos[new] = np.linspace(0.2, 0.9, int(new.sum()), dtype=np.float32)
     _check(eng, [st], profiles, sols, M, dict(window_lanes=-1), expect)
+
+
+@pytest.mark.parametrize("models,hosts,load,ends,expect", [(20, 2, 300.0, 0.12, "sim_lanes_kernel<4, true>"), (3, 3, 3000.0, 0.12, "sim_mixed_kernel<4,"),
+                                                         (20, 0, 300.0, 0.12, "sim_mixed_kernel<4,"), (20, 2, 300.0, 0.04, "sim_mixed_kernel<4,")])
+def test_what_the_loops_have_to_do_decides(models, hosts, load, ends, expect):
+    """Requests with many replicas, with none, and bursts of more than twenty requests on shallow groups keep the loop over runs, however
+    large the load."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(31, (2, 4), True, models, 12 if hosts == 3 else 4, 70, hosts)
+    if hosts == 3:
+        sols = [ModelPlacement(s.group_configs, [[0, 1, 2]] * len(s.group_models)) for s in sols]
+    _check(eng, [_bursts(50, 8200, models, load, odd_slos=False, ends=ends)], profiles, sols, models, dict(window_lanes=-1), expect)
