@@ -88,7 +88,8 @@ typedef struct {
     int32_t struct_size;          /* sizeof(mmsim_options), set by mmsim_options_default                      */
     int32_t request_loop;         /* plain simulator: 1 = loop over runs of equal models (scheduled launch),
                                      0 = chunks of four requests; -1: runs when at least four in five requests
-                                     of the batch's streams repeat the model of the request before.  A latency
+                                     of the batch's streams repeat the model of the request before, else chunks,
+                                     unless skip_ahead has the lanes at their own pace.  A latency
                                      table with one latency per (model, configuration) and more than 63
                                      configurations takes the chunks whatever this says                        */
     int32_t waves_per_cu;         /* 1..8: most wavefronts per workgroup of the plain simulator; 0: as many as fit */
@@ -97,15 +98,17 @@ typedef struct {
     int32_t tile_order_by_slots;  /* loop over runs: 0 = tiles composed by pipeline depth only; -1 / 1: by clock
                                      slots as well                                                              */
     int32_t sched_groups;         /* workgroups of the scheduled launch; 0: one per CU                          */
-    int32_t segment_requests;     /* requests per turn of an item in the scheduled launch; 0: 16384             */
+    int32_t segment_requests;     /* requests per turn of an item in the scheduled launch; 0: 16384.  With lanes at
+                                     their own pace more than 8192 are taken up to a multiple of 8192          */
     int32_t sched_spin_limit;     /* looks in a row after which a wavefront that finds only busy items leaves;
                                      -1: 20000                                                                  */
     int32_t skip_ahead;           /* loop over runs: 0 = simulate every request; 1 = requests that every lane
                                      of a wavefront must reject are not simulated; 2 = every lane goes through the
                                      stream at its own pace and passes over what it must reject (scores, groups of
-                                     several stages with one latency per (model, configuration); otherwise as 1);
-                                     -1: 2 on streams of long runs (one model, one SLO) where the groups have
-                                     much more to do than they can and a request few replicas, else 1          */
+                                     several stages with one latency per (model, configuration), request_loop not
+                                     0; otherwise as 1); -1: with request_loop -1, 2 on streams of long runs (one
+                                     model, one SLO) where the groups have much more to do than they can and a
+                                     request few replicas, else 1                                              */
     int32_t xcd_map;              /* chunked loop: 0 = seeds innermost in the workgroup numbering; -1 / 1: all
                                      seeds of a tile group on one XCD                                           */
     int32_t batching_lanes;       /* batching simulator: 8, 16, 32 or 64 simulations per wavefront; 0: the widest

@@ -471,7 +471,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     }
     bool own_pace = false;  // lanes at their own pace (sim_lanes.hip): scores of groups of several stages
     if (!batching && uniform_stages && lat_row <= kWave && b->smax_bucket > 1 && M <= 65535 && !g_arena && o.request_loop != 0 &&
-        (o.skip_ahead < 0 || o.skip_ahead == 2) &&
+        (o.skip_ahead == 2 || (o.skip_ahead < 0 && o.request_loop < 0)) &&
         !(flags & (MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST | MMSIM_WANT_OP_COUNT))) {
         own_pace = o.skip_ahead == 2 || own_pace_pays(wls, n_seeds, t, rl, b->smax_bucket);
         if (own_pace) runs = true;

@@ -148,3 +148,13 @@ def test_what_the_loops_have_to_do_decides(models, hosts, load, ends, expect):
     if hosts == 3:
         sols = [ModelPlacement(s.group_configs, [[0, 1, 2]] * len(s.group_models)) for s in sols]
     _check(eng, [_bursts(50, 8200, models, load, odd_slos=False, ends=ends)], profiles, sols, models, dict(window_lanes=-1), expect)
+
+
+@pytest.mark.parametrize("options,expect", [(dict(request_loop=1), "sim_mixed_kernel<4, true, true, true, 0, true>"),
+                                            (dict(request_loop=0), "sim_mixed_kernel<4, true, true, true, 0, false>"),
+                                            (dict(request_loop=1, skip_ahead=2), "sim_lanes_kernel<4, true>"),
+                                            (dict(request_loop=0, skip_ahead=2), "sim_mixed_kernel<4, true, true, true, 0, false>")])
+def test_a_loop_that_is_asked_for_is_taken(options, expect):
+    eng = E.Engine.default()
+    profiles, sols = _problem(31, (2, 4), True, 20, 4, 70, 2)
+    _check(eng, [_bursts(50, 8200, 20, 300.0)], profiles, sols, 20, dict(window_lanes=-1, **options), expect)
