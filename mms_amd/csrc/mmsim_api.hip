@@ -249,7 +249,8 @@ int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mms
         }
     }
     const size_t blocks = of.size();
-    if (blocks > 0x7FFFFFFFu) return fail(MMSIM_E_UNSUPPORTED, "option segment_requests is too small for these streams");
+    // (a launch has fewer than 2^32 threads, and both kernels below a wavefront for each of these)
+    if (blocks > 0x3FFFFFFu || (int64_t)b->tiles * b->M > 0x3FFFFFF) return fail(MMSIM_E_UNSUPPORTED, "too many blocks or rows in one batch");
     DevBuf<int32_t> d_of;
     DevBuf<int64_t> d_first;
     HIP_TRY(d_of.alloc(blocks));
@@ -335,11 +336,13 @@ bool own_pace_pays(const mmsim_workload *const *wls, int32_t n_seeds, const mmsi
     return (1.0 + 0.7 * r.mean) * (2.5 * q + v) <= 1.85 * (1.0 - std::exp(-3.2 * q) + u);
 }
 
-// Builds every device table of a batch from replica lists.
-int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
-                const RepLists &rl, uint32_t flags, mmsim_batch **out, const int32_t *stream_of = nullptr,
-                const mmsim_options *options = nullptr) {
-    const mmsim_options &o = options ? *options : ctx->opt;
+// Builds every device table of a batch from replica lists.  own_pace: whether lanes at their own pace may be chosen;
+// afterwards, whether they were.
+int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
+                     const RepLists &rl, uint32_t flags, mmsim_batch **out, const int32_t *stream_of, const mmsim_options &o,
+                     bool *own_pace_chosen) {
+    const bool may_own_pace = *own_pace_chosen;
+    *own_pace_chosen = false;
     // MMSIM_TIMING=1 prints the host time of each phase of the packing (diagnostics)
     const bool timing = std::getenv("MMSIM_TIMING") != nullptr;
     auto t_last = std::chrono::steady_clock::now();
@@ -470,11 +473,12 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
         if (uniform_stages && lat_row > kWave) runs = false;
     }
     bool own_pace = false;  // lanes at their own pace (sim_lanes.hip): scores of groups of several stages
-    if (!batching && uniform_stages && lat_row <= kWave && b->smax_bucket > 1 && M <= 65535 && !g_arena && o.request_loop != 0 &&
+    if (may_own_pace && !batching && uniform_stages && lat_row <= kWave && b->smax_bucket > 1 && M <= 65535 && !g_arena && o.request_loop != 0 &&
         (o.skip_ahead == 2 || (o.skip_ahead < 0 && o.request_loop < 0)) &&
         !(flags & (MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST | MMSIM_WANT_OP_COUNT))) {
         own_pace = o.skip_ahead == 2 || own_pace_pays(wls, n_seeds, t, rl, b->smax_bucket);
         if (own_pace) runs = true;
+        *own_pace_chosen = own_pace;
     }
 
     phase("latency table, loop choice");
@@ -1312,18 +1316,7 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     a.run_block = run_block;
     if (own_pace) {
         const int rc = prepare_own_pace(b.get(), soff, t, lat);
-        if (rc == MMSIM_E_NOMEM || rc == MMSIM_E_UNSUPPORTED) {  // the loop over runs does without the further tables
-            (void)hipGetLastError();
-            a.run_block = 0;
-            b->run_base.release();
-            b->run_off.release();
-            b->run_list.release();
-            b->run_times.release();
-            b->rep16.release();
-            b->stage.release();
-        } else if (rc != MMSIM_OK) {
-            return rc;
-        }
+        if (rc != MMSIM_OK) return rc;
         phase("runs of the streams, entries");
     }
     if (batching) {
@@ -1374,6 +1367,21 @@ int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seed
     phase("schedule tables, kernel args");
     *out = b.release();
     return MMSIM_OK;
+}
+
+// The same, whatever the lanes at their own pace cannot have: the schedule takes only so many (tile, stream) pairs and
+// segments, which the chunked loop does not need, and the further tables may find no memory or be too long.  Such a batch is
+// built again for the loop that is chosen without them.
+int build_batch(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
+                const RepLists &rl, uint32_t flags, mmsim_batch **out, const int32_t *stream_of = nullptr,
+                const mmsim_options *options = nullptr) {
+    const mmsim_options &o = options ? *options : ctx->opt;
+    bool own_pace = true;
+    const int rc = build_batch_with(ctx, wls, n_seeds, t, rl, flags, out, stream_of, o, &own_pace);
+    if (rc == MMSIM_OK || rc == MMSIM_E_HIP || !own_pace) return rc;
+    (void)hipGetLastError();
+    own_pace = false;
+    return build_batch_with(ctx, wls, n_seeds, t, rl, flags, out, stream_of, o, &own_pace);
 }
 
 // A batch from placements as the caller gave them, for whichever kernel suits it.  events: the batch will be timed

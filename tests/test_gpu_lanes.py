@@ -158,3 +158,38 @@ def test_a_loop_that_is_asked_for_is_taken(options, expect):
     eng = E.Engine.default()
     profiles, sols = _problem(31, (2, 4), True, 20, 4, 70, 2)
     _check(eng, [_bursts(50, 8200, 20, 300.0)], profiles, sols, 20, dict(window_lanes=-1, **options), expect)
+
+
+@pytest.mark.parametrize("what", ["items", "segments", "runs"])
+def test_what_the_schedule_or_the_list_of_runs_cannot_hold_takes_the_loop_it_had(what):
+    """Two in three requests repeat model and SLO, four in five do not: the loop without lanes at their own pace is the chunked one,
+    which takes any number of (tile, stream) pairs, ignores the segments, and needs no list of runs (with 2^32 of them, refused
+    after they were counted)."""
+    eng = E.Engine.default()
+    M = 20
+    profiles, sols = _problem(31, (2, 4), True, M, 4, 70, 2)
+    R, copies, options = {"items": (4100, 140, dict(sched_groups=1)),
+                          "segments": (60010 * 64, 1, dict(sched_groups=1, waves_per_cu=1, segment_requests=64)),
+                          "runs": (1 << 24, 257, dict(skip_ahead=2))}[what]
+    st = _bursts(50, R, M, 300.0, odd_slos=False, ends=0.28)
+    if what == "runs":      # every request a run of its own
+        st.model_ids = (np.arange(R) % M).astype(np.int32)
+    table = E.LatencyTable(profiles, [1])
+    packed = E.pack_placements(sols, table)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, M)
+    chunked = "sim_mixed_kernel<4, true, true, true, 0, false>"
+    if what != "runs":      # (the streams alone are for lanes at their own pace)
+        batch = E.Batch(eng, [dw], table, packed, 0, options=dict(window_lanes=-1))
+        assert batch.kernel_name() == "sim_lanes_kernel<4, true>"
+        batch.close()
+    batch = E.Batch(eng, [dw] * copies, table, packed, 0, options=dict(window_lanes=-1, **options))
+    assert batch.kernel_name() == chunked, batch.kernel_name()
+    if what == "items":
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        ref = oracle_batch(st, table, packed)
+        for k in range(copies):
+            assert_batch_matches(out, ref, k, packed[0], where=f"stream {k}")
+    batch.close()
+    dw.close()
