@@ -253,12 +253,14 @@ int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mms
     if (blocks > 0x3FFFFFFu || (int64_t)b->tiles * b->M > 0x3FFFFFF) return fail(MMSIM_E_UNSUPPORTED, "too many blocks or rows in one batch");
     DevBuf<int32_t> d_of;
     DevBuf<int64_t> d_first;
+    std::vector<uint32_t> off(blocks + 1, 0);
+    std::vector<uint2> stage(lat.size(), make_uint2(0x7F800000u, 0u));
+    StreamWait copies(st);
     HIP_TRY(d_of.alloc(blocks));
     HIP_TRY(d_first.alloc(blocks));
     HIP_TRY(b->run_base.alloc(base.size()));
     HIP_TRY(b->run_off.alloc(blocks + 1));
     HIP_TRY(hipMemcpyAsync(b->run_base.p, base.data(), sizeof(int64_t) * base.size(), hipMemcpyHostToDevice, st));
-    std::vector<uint32_t> off(blocks + 1, 0);
     if (blocks > 0) {
         HIP_TRY(hipMemcpyAsync(d_of.p, of.data(), sizeof(int32_t) * blocks, hipMemcpyHostToDevice, st));
         HIP_TRY(hipMemcpyAsync(d_first.p, first.data(), sizeof(int64_t) * blocks, hipMemcpyHostToDevice, st));
@@ -279,7 +281,6 @@ int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mms
         HIP_TRY(launch_list_runs(b->streams.p, b->stream_off.p, d_of.p, d_first.p, (int32_t)blocks, a.run_block, b->run_off.p, b->run_list.p, b->run_times.p, nullptr, st));
     HIP_TRY(b->rep16.alloc((size_t)b->tiles * b->M * 2 * kWave));
     HIP_TRY(launch_entries(a, b->rep16.p, st));
-    std::vector<uint2> stage(lat.size(), make_uint2(0x7F800000u, 0u));
     for (int32_t m = 0; m < b->M; ++m)
         for (int32_t c = 0; c < t->C; ++c) {
             const size_t at = (size_t)m * a.lat_row + c;
@@ -288,7 +289,7 @@ int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mms
         }
     HIP_TRY(b->stage.alloc(stage.size()));
     HIP_TRY(hipMemcpyAsync(b->stage.p, stage.data(), sizeof(uint2) * stage.size(), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(copies.now());
     a.run_base = b->run_base.p;
     a.run_off = b->run_off.p;
     a.run_list = b->run_list.p;
@@ -1148,6 +1149,8 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
     b->Rtotal = soff[n_seeds];
 
     hipStream_t st = ctx->stream;
+    std::vector<int64_t> mqo(batching ? (size_t)n_seeds * (M + 1) : 0);
+    StreamWait copies(st);  // (of the vectors above)
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(b->streams.alloc((size_t)b->Rtotal));
     for (int s = 0; s < n_seeds; ++s)
@@ -1182,7 +1185,6 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
     HIP_TRY(hipMemcpyAsync(b->lat.p, lat.data(), sizeof(float) * lat.size(), hipMemcpyHostToDevice, st));
 
     if (batching) {
-        std::vector<int64_t> mqo((size_t)n_seeds * (M + 1));
         int64_t total = 0;
         for (int s = 0; s < n_seeds; ++s) {
             for (int32_t m = 0; m <= M; ++m) mqo[(size_t)s * (M + 1) + m] = total + wls[s]->mq_off[m];
@@ -1244,7 +1246,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
         HIP_TRY(hipEventCreate(&b->ev_start));
         HIP_TRY(hipEventCreate(&b->ev_stop));
     }
-    HIP_TRY(hipStreamSynchronize(st));  // host staging vectors go out of scope below
+    HIP_TRY(copies.now());
 
     phase("streams + uploads");
     // ---- loop over runs: the schedule's tables, and room to park clocks between segments
@@ -1561,11 +1563,12 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
     HIP_TRY(w->reqs->alloc((size_t)R));
     HIP_TRY(w->mq.alloc(known));
     if (R > 0) {
+        StreamWait copies(ctx->stream);
         HIP_TRY(hipMemcpyAsync(w->reqs->p, host.data(), sizeof(Req) * (size_t)R, hipMemcpyHostToDevice, ctx->stream));
         if (known > 0) {
             HIP_TRY(hipMemcpyAsync(w->mq.p, mq.data(), sizeof(MqEntry) * known, hipMemcpyHostToDevice, ctx->stream));
         }
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        HIP_TRY(copies.now());
     }
     *out = w.release();
     return MMSIM_OK;
@@ -1822,9 +1825,12 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
     if (d_i32.n < (size_t)n_sims + 2 * cells) HIP_TRY(d_i32.alloc((size_t)n_sims + 2 * cells));
     if (d_f64.n < 7 * cells) HIP_TRY(d_f64.alloc(7 * cells));
     if (d_scratch.n < (size_t)rows * (size_t)pitch) HIP_TRY(d_scratch.alloc((size_t)rows * (size_t)pitch));
+    std::vector<int32_t> h_i32(2 * cells);
+    std::vector<double> h_f64(7 * cells);
+    std::vector<int64_t> up;  // one upload: mq_off | lo | hi | sim_base
+    StreamWait copies(st);
     HIP_TRY(hipMemcpyAsync(d_mq.p, mq.data(), sizeof(mq[0]) * mq.size(), hipMemcpyHostToDevice, st));
     int64_t *i64 = d_i64.p;
-    std::vector<int64_t> up;  // one upload: mq_off | lo | hi | sim_base (alive until the stream is waited for below)
     up.reserve(mqo.size() + 2 * lo.size() + sim_base.size());
     up.insert(up.end(), mqo.begin(), mqo.end());
     up.insert(up.end(), lo.begin(), lo.end());
@@ -1857,11 +1863,9 @@ int mmsim_batch_model_stats(mmsim_batch *b, const mmsim_workload *const *workloa
         if (e != hipSuccess) return fail(MMSIM_E_HIP, err.empty() ? std::string("model_stats launch: ") + hipGetErrorString(e) : err);
     }
     // two copies back (the integer results, the double results), then into the caller's arrays
-    std::vector<int32_t> h_i32(2 * cells);
-    std::vector<double> h_f64(7 * cells);
     HIP_TRY(hipMemcpyAsync(h_i32.data(), f.model_req, sizeof(int32_t) * 2 * cells, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(h_f64.data(), d, sizeof(double) * 7 * cells, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(copies.now());
     std::memcpy(out->model_num_requests, h_i32.data(), sizeof(int32_t) * cells);
     std::memcpy(out->model_num_good, h_i32.data() + cells, sizeof(int32_t) * cells);
     double *const o64[7] = {out->first_start, out->last_start, out->latency_sum, out->latency_mean,
@@ -2231,6 +2235,8 @@ int mmsim_simulate_requests(mmsim_ctx *ctx, double *finish, uint8_t *good, const
     HIP_TRY(d_max.alloc(MG));
     HIP_TRY(d_sum.alloc(MG));
     HIP_TRY(d_cnt.alloc(2 * (size_t)M + 2 * (size_t)G));
+    std::vector<int32_t> cnt(2 * (size_t)M + 2 * (size_t)G);
+    StreamWait copies(st);
     HIP_TRY(hipMemcpyAsync(d_t.p, tstamps, sizeof(double) * R, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(d_m.p, model_ids, sizeof(int32_t) * R, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(d_slo.p, slos, sizeof(float) * R, hipMemcpyHostToDevice, st));
@@ -2259,9 +2265,8 @@ int mmsim_simulate_requests(mmsim_ctx *ctx, double *finish, uint8_t *good, const
     if (launch_sim_scalar(a, st, &err) != hipSuccess) return fail(MMSIM_E_HIP, err);
     HIP_TRY(hipMemcpyAsync(finish, d_fin.p, sizeof(double) * R, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(good, d_good.p, R, hipMemcpyDeviceToHost, st));
-    std::vector<int32_t> cnt(2 * (size_t)M + 2 * (size_t)G);
     HIP_TRY(hipMemcpyAsync(cnt.data(), d_cnt.p, d_cnt.bytes(), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(copies.now());
     std::memcpy(model_num_requests, cnt.data(), sizeof(int32_t) * (size_t)M);
     std::memcpy(model_num_good_requests, cnt.data() + M, sizeof(int32_t) * (size_t)M);
     std::memcpy(group_num_requests, cnt.data() + 2 * (size_t)M, sizeof(int32_t) * (size_t)G);

@@ -44,6 +44,23 @@ inline int hip_fail(hipError_t e, const char *what) {
         if (e__ != hipSuccess) return hip_fail(e__, #expr); \
     } while (0)
 
+// Copies on a stream read and write host memory until the stream has been waited for.  Declared behind that memory, this
+// waits for them on every way out of a function.
+struct StreamWait {
+    hipStream_t stream;
+    bool pending = true;
+    explicit StreamWait(hipStream_t st) : stream(st) {}
+    StreamWait(const StreamWait &) = delete;
+    StreamWait &operator=(const StreamWait &) = delete;
+    hipError_t now() {
+        pending = false;
+        return hipStreamSynchronize(stream);
+    }
+    ~StreamWait() {
+        if (pending) (void)hipStreamSynchronize(stream);
+    }
+};
+
 // Device memory for a batch comes either from hipMalloc or, while g_arena is set (mmsim_eval_batch_static), from
 // a bump allocator over the library's static device scratch: such buffers are never freed one by one.
 struct Arena {

@@ -421,12 +421,13 @@ int fetch_window(mmsim_batch *b, mmsim_result *out) {
         HIP_TRY(stage.ensure(b->win_finish));
     }
     unsigned char *host = b->in_scratch ? plain.data() : stage.p;
+    StreamWait copies(st);
     HIP_TRY(hipMemcpyAsync(host, b->win_out.p, b->win_finish, hipMemcpyDeviceToHost, st));
     if (wr && Rm > 0) {
         HIP_TRY(hipMemcpyAsync(out->finish, b->win_out.p + b->win_finish, sizeof(double) * L * Rm, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipMemcpyAsync(out->good, b->win_out.p + b->win_good, L * Rm, hipMemcpyDeviceToHost, st));
     }
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(copies.now());
     const int32_t *ng = reinterpret_cast<const int32_t *>(host);
     for (size_t l = 0; l < L; ++l) out->n_good[l] = ng[l];
     std::memcpy(out->latency_sum, host + b->win_lat_sum, sizeof(double) * L);
