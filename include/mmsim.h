@@ -351,8 +351,8 @@ typedef struct {
     int32_t lanes, waves, n_seeds, B;
     int32_t smax_bucket, max_replicas, slots, lds_bytes;
     int64_t requests_total;   /* sum of stream lengths over seeds                     */
-    int64_t table_bytes;      /* device bytes of the packed placement tables          */
-    int64_t stream_bytes;     /* device bytes of the request streams                  */
+    int64_t table_bytes;      /* bytes of the packed placement tables that the kernel reads */
+    int64_t stream_bytes;     /* bytes of the request streams as the kernel reads them      */
     int32_t workgroups;       /* scheduled launch (bursty streams): workgroups, each owning a set of
                                  (64 placements, stream) items; 0 for the other launches            */
     int32_t segments;         /* pieces a stream is cut into so that a workgroup's items take turns  */

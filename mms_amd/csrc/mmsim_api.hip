@@ -1897,9 +1897,18 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {
     out->slots = b->nslots;
     out->lds_bytes = (int32_t)b->lds_bytes;
     out->requests_total = b->Rtotal;
-    out->table_bytes = b->window ? (int64_t)b->win_in.bytes() : (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep16.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() +
-                                 b->rmax.bytes() + b->lat.bytes() + b->lat_nb.bytes());
-    out->stream_bytes = b->window ? b->Rtotal * (int64_t)sizeof(Req) : (int64_t)(b->streams.bytes() + b->run_list.bytes() + b->run_times.bytes());
+    // what the kernel reads: lanes at their own pace have the streams and the first eight replicas in tables of their own
+    if (b->window) {
+        out->table_bytes = (int64_t)b->win_in.bytes();
+        out->stream_bytes = b->Rtotal * (int64_t)sizeof(Req);
+    } else if (b->args.run_block > 0) {
+        out->table_bytes = (int64_t)(b->rep16.bytes() + b->stage.bytes() + (b->args.rep_extra > 0 ? b->repx32.bytes() + b->lat.bytes() : 0));
+        out->stream_bytes = (int64_t)(b->run_list.bytes() + b->run_times.bytes() + b->run_off.bytes() + b->run_base.bytes());
+    } else {
+        out->table_bytes = (int64_t)(b->rep32.bytes() + b->repx32.bytes() + b->rep8.bytes() + b->repx.bytes() + b->ginfo.bytes() + b->rmax.bytes() +
+                                     b->lat.bytes() + b->lat_nb.bytes());
+        out->stream_bytes = (int64_t)b->streams.bytes();
+    }
     out->workgroups = b->sched_groups;
     out->segments = b->max_nseg;
     out->launches = 1;

@@ -193,3 +193,21 @@ def test_what_the_schedule_or_the_list_of_runs_cannot_hold_takes_the_loop_it_had
             assert_batch_matches(out, ref, k, packed[0], where=f"stream {k}")
     batch.close()
     dw.close()
+
+
+def test_reported_bytes_are_those_that_the_kernel_reads():
+    eng = E.Engine.default()
+    M, R = 20, 20000
+    profiles, sols = _problem(31, (2, 4), True, M, 4, 70, 2)
+    table = E.LatencyTable(profiles, [1])
+    st = _bursts(50, R, M, 300.0, odd_slos=False)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, M)
+    batch = E.Batch(eng, [dw], table, E.pack_placements(sols, table), 0, options=OWN)
+    starts = np.ones(R, bool)       # of the runs: a change of model or SLO, or of the block of 8192 requests
+    starts[1:] = (st.model_ids[1:] != st.model_ids[:-1]) | (st.slos[1:] != st.slos[:-1]) | (np.arange(1, R) % 8192 == 0)
+    runs = int((starts & (st.model_ids >= 0)).sum())
+    info = batch.info()
+    assert info["stream_bytes"] == 32 * (runs + 1) + 8 * R + 4 * (3 + 1) + 8      # runs (a spare one), arrivals, first run of a block, first block
+    assert info["table_bytes"] == 2 * M * 2 * 64 * 8 + 8 * M * (len(table.arrays()[1]) + 1)      # entries, latencies of the configurations
+    batch.close()
+    dw.close()
