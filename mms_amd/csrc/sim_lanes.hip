@@ -15,8 +15,7 @@
 // "All that is left": a lane's clocks change only when it accepts, so while it rejects it keeps its choice, a last-stage clock c
 // and a latency l, and a later request at t <= c is rejected if fl(fl(fl(c + l) + overhead) - t) > slo, as the walk's
 // finish time is never below that (t >= arrival at every stage and rounding is monotone).  The left side falls with t,
-// so the latest arrival of the run decides for the rest of it.  On configuration 4 a lane takes 0.17 steps per request of the stream, the slowest
-// lane of a wavefront 0.19.
+// so the latest arrival of the run decides for the rest of it.  On configuration 4 a wavefront takes about 0.18 steps per request of its stream.
 //
 // Every lane makes the decisions of the serial loop in the serial loop's order, with the same fp64 operations: results
 // equal it bit for bit.
@@ -26,10 +25,11 @@
 // blocks of 8192 cost 1.5 % more steps, of 4096 3 %, of 1024 12 %).  The runs of a block are listed ahead (list_runs_kernel).  A lane has the
 // run that it is at in registers, with up to eight replicas; the next one that it hosts, whose latencies are on their way; and the
 // run after that, which is on its way with its entries.  The arrival of the next request of its run is fetched a step ahead.
-// Everything is asked for at the end of a step and looked at at the end of the next one; a step waits for nothing but LDS.
+// Everything is asked for at the end of a step and looked at at the end of the next one: where it comes from L2, a step waits for nothing but
+// LDS.  Only replicas beyond the eighth are read where they are looked at, each in two dependent loads.
 //
-// What bounds it (configuration 4, 131072 simulations, two wavefronts to a SIMD): a step is about 285 instructions, 165 of them vector
-// instructions, in 2200 cycles; 55 % of a wavefront's cycles issue, 32 % wait (LDS, and memory where an XCD's L2 misses), 14 % wait for the SIMD.
+// What bounds it (configuration 4, 131072 simulations, two wavefronts to a SIMD): a step is about 290 instructions, 160 of them vector
+// instructions, in 2300 cycles; 56 % of a wavefront's cycles issue, 30 % wait (LDS, and memory where an XCD's L2 misses), the rest wait for the SIMD.
 // 506 ms with all lanes at the same request (102 instructions and 978 cycles for each of the stream's), 208 ms here.  On the way:
 // entries and latencies as 8 bytes a replica, 2 KB to a row, 338 ms; without the copies for which the compiler waits at the end of a step 261
 // (rows of all tiles of an XCD 8.4 MB, 20 % of its L2 requests miss); entries of 16 bits, 512 bytes to a row, and the latencies from a table 226
@@ -280,8 +280,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void sim_lanes_kernel(con
                 if (__builtin_expect((more4 & act) != 0, 0)) {
                     const Cand x = scan(std::integral_constant<int, 4>{});
                     if (in_mask(more4)) win = first_min(win, x);
-                    if (__builtin_expect((more8 & act) != 0, 0))
-                        if (in_mask(more8)) {
+                    const uint64_t beyond = more8 & more4;  // (more8 keeps a lane's bit until it takes a run of more than four again)
+                    if (__builtin_expect((beyond & act) != 0, 0))
+                        if (in_mask(beyond)) {
                             const uint32_t *row = repx_tile + (size_t)model * a.rep_extra * kWave;
                             for (int j = 0; j < a.rep_extra; ++j) {
                                 const uint32_t d = row[(size_t)j * kWave];
