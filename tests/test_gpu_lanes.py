@@ -211,3 +211,24 @@ def test_reported_bytes_are_those_that_the_kernel_reads():
     assert info["table_bytes"] == 2 * M * 2 * 64 * 8 + 8 * M * (len(table.arrays()[1]) + 1)      # entries, latencies of the configurations
     batch.close()
     dw.close()
+
+
+@pytest.mark.parametrize("segment,segments", [(0, 3), (12288, 3), (8192, 6), (8256, 3), (4096, 11)])
+@pytest.mark.parametrize("waves", [1, 2])
+def test_items_that_take_turns_go_on_where_they_were(segment, segments, waves):
+    """Segments of several blocks, the default one among them: a parked item goes on at the block that its segment starts with, its
+    clocks and sums as they were.  Segments are whole numbers of blocks of 8192 requests, or one block if they are shorter."""
+    eng = E.Engine.default()
+    M = 6
+    profiles, sols = _problem(41, (1, 2, 4, 8), True, M, 7, 131, 3)
+    streams = [_bursts(60 + k, R, M, 3.0 + 3 * k) for k, R in enumerate((40961, 33001, 8191))]
+    options = dict(OWN, sched_groups=1, waves_per_cu=waves, segment_requests=segment)
+    table = E.LatencyTable(profiles, [1])
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    batch = E.Batch(eng, dws, table, E.pack_placements(sols, table), 0, options=options)
+    info = batch.info()
+    assert (info["segments"], info["workgroups"]) == (segments, 1), info
+    batch.close()
+    for dw in dws:
+        dw.close()
+    _check(eng, streams, profiles, sols, M, options)
