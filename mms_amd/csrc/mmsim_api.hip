@@ -1515,19 +1515,27 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
     w->model_num_requests.assign(M, 0);
     std::vector<Req> host((size_t)R);
     bool sorted = true;
+    int64_t repeats = 0, run_repeats = 0;
+    int32_t model = M;  // of the request before, and its SLO
+    uint32_t slo = 0;
     for (int64_t i = 0; i < R; ++i) {
         if (model_ids[i] >= M) return fail(MMSIM_E_INVALID, "workload_create: model id >= M");
         if (tstamps[i] != tstamps[i]) return fail(MMSIM_E_INVALID, "workload_create: arrival time is NaN");
+        const int32_t m = model_ids[i] < 0 ? -1 : model_ids[i];
+        uint32_t slo_bits;
+        std::memcpy(&slo_bits, &slos[i], sizeof(slo_bits));
         host[i].t = tstamps[i];
-        host[i].m = model_ids[i] < 0 ? -1 : model_ids[i];
+        host[i].m = m;
         host[i].slo = slos[i];
-        if (model_ids[i] >= 0) w->model_num_requests[model_ids[i]] += 1;
-        if (i > 0 && host[i].m == host[i - 1].m) {
-            w->repeats += 1;
-            w->run_repeats += std::memcmp(&host[i].slo, &host[i - 1].slo, sizeof(float)) == 0;
-        }
+        if (m >= 0) w->model_num_requests[m] += 1;
+        repeats += m == model;
+        run_repeats += (int)(m == model) & (int)(slo_bits == slo);  // (no branch: bursts make it a coin toss)
+        model = m;
+        slo = slo_bits;
         if (i > 0 && tstamps[i] < tstamps[i - 1]) sorted = false;
     }
+    w->repeats = repeats;
+    w->run_repeats = run_repeats;
     if (R > 0) w->span = std::max(0.0, tstamps[R - 1] - tstamps[0]);
     w->mq_off.assign((size_t)M + 1, 0);
     for (int32_t m = 0; m < M; ++m) w->mq_off[m + 1] = w->mq_off[m] + w->model_num_requests[m];
