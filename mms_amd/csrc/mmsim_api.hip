@@ -303,23 +303,23 @@ int prepare_own_pace(mmsim_batch *b, const std::vector<int64_t> &soff, const mms
 //
 // A lane takes a step for each request that it accepts and one for each run (model and SLO) that it ends rejecting, and a
 // wavefront waits for its slowest lane; in the loop over runs a wavefront takes a step for each request that any of its lanes
-// accepts and one for each run of a model, and passes over the rest.  With q the requests that a placement accepts, u the runs
-// of a model and v those of a model and an SLO, of a request of the stream, and r the replicas that it may choose from, the one
-// takes about (2.5 q + v) (1 + 0.7 r) where the other takes 1 - exp(-3.2 q) + u; q is taken as 1.5 of the share that is hosted
-// at all over 1 + load.  On 1154 random batches (six layouts of groups of 1 to 32 stages, 12 to 200 models, 16384 to 131072
-// simulations of 5000 to 60000 requests, CV 4 to 12, load 0.1 to 2000, a new SLO inside a burst for up to 30 % of the requests)
-// the rule takes 329, at 0.38 to 1.19 times the better one of the other loops, 0.67 in the mean and more than 1.02 on seven.
-// What it leaves of those with load >= 2.2 r^2 is at 1.16 in the mean and up to 6.3:
-//   a new SLO inside a burst, where nine in ten requests repeat the model of the one before: for none / 10 / 20 / 40 % / all of
-//     them 0.52 / 0.75 / 1.01 / 1.49 / 2.95 (groups of 2 to 16 devices, load 8) and 0.77 / 0.77 / 0.89 / 1.15 / 1.91 (four-stage
-//     pipelines, load 2);
-//   many replicas or a very large load, where nearly nothing is accepted and the loop over runs passes over whole blocks: 0.95
-//     replicas at load 8 / 84 / 840 0.51 / 0.73 / 1.00, 1.5 at 45 / 450 0.78 / 1.11, 2.3 at 7 / 70 / 700 0.73 / 1.13 / 1.76, 4.2
-//     at 42 / 83 / 420 1.31 / 1.45 / 1.77, 8 at 420 2.5;
-//   bursts of more than twenty requests, where the lanes of a wavefront differ most, with walks of up to four stages (up to
-//     1.53) or in streams of a few hundred runs (up to 1.33).
-// Single devices need no walk, which is what the steps save: at load 8 and 1 replica 0.9, with 1.5 1.0 and more; they keep the
-// other loops.
+// accepts, however few these are, and passes over what all of them reject.  So the first is the faster one where the groups
+// have so much more to do than they can that a placement accepts few requests, and yet not so much more that a wavefront
+// accepts few.  Measured against the better one of the other loops on 1414 random batches (six layouts of groups of 1 to 32
+// stages, 12 to 200 models, 16384 to 131072 simulations of 5000 to 200000 requests, CV 4 to 12, load 0.1 to 2000, a new SLO inside
+// a burst for up to 30 % of the requests): the rule takes 414, at 0.38 to 1.24 times the other, 0.68 in the mean, more than
+// 1.02 on 16.  Of the 864 with two thirds of the requests repeating the model of the one before and load >= 2.2 r^2 (r: replicas that
+// a request may choose from) it leaves 450, at 1.14 in the mean and up to 6.3 times:
+//   new SLOs inside bursts: where nine in ten requests repeat the model, for none / 10 / 20 / 40 % / all of the requests 0.52 /
+//     0.75 / 1.01 / 1.49 / 2.95 (groups of 2 to 16 devices, load 8) and 0.77 / 0.77 / 0.89 / 1.15 / 1.91 (four-stage pipelines,
+//     load 2);
+//   large loads and many replicas, which add to a lane's step only: 0.95 replicas at load 8 / 84 / 840 0.51 / 0.73 / 1.00, 1.5 at
+//     45 / 450 0.78 / 1.11, 2.3 at 7 / 70 / 700 0.73 / 1.13 / 1.76, 4.2 at 42 / 83 / 420 1.31 / 1.45 / 1.77, 8 at 420 2.5;
+//   bursts of more than twenty requests, where the lanes of a wavefront differ most, with walks of up to four stages (0.65 to
+//     1.53) or in streams of a few hundred runs (0.36 to 1.33).
+// Less load, by load: 1.2 replicas (groups of 2 to 16 devices) 0.25 1.09, 0.7 0.95; four-stage pipelines, 1.95 replicas 1.2 1.28, 3
+// 1.0; groups of 1 to 8 devices, 2.3 replicas 1.2 1.25, 3 0.97.  Single devices need no walk, which is what the steps save: at
+// load 8 and 1 replica 0.9, with 1.5 1.0 and more; they keep the other loops.
 bool own_pace_pays(const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t, const RepLists &rl, int smax_bucket) {
     int64_t model = 0, run = 0, all = 0;
     for (int s = 0; s < n_seeds; ++s) {
@@ -328,13 +328,11 @@ bool own_pace_pays(const mmsim_workload *const *wls, int32_t n_seeds, const mmsi
         all += wls[s]->R;
     }
     if (all < (int64_t)4096 * n_seeds) return false;  // (shorter streams do not pay for the further tables)
-    if (3 * run <= 2 * all || all - run > 2 * (all - model)) return false;
+    if (3 * run <= 2 * all || 5 * (all - run) > 8 * (all - model)) return false;
     if (20 * (all - model) < all && (smax_bucket <= 4 || all - model < (int64_t)600 * n_seeds)) return false;
-    const RequestReplicas r = replicas_of_a_request(wls, n_seeds, rl);
+    const double r = replicas_of_a_request(wls, n_seeds, rl);
     const double load = offered_load(wls, n_seeds, t, rl.B, rl.Gmax, rl.num_groups.data(), rl.group_cfg.data());
-    if (r.hosted <= 0.0 || !(load >= 2.2 * r.mean * r.mean)) return false;
-    const double q = std::min(r.hosted, 1.5 * r.hosted / (1.0 + load)), u = (double)(all - model) / (double)all, v = (double)(all - run) / (double)all;
-    return (1.0 + 0.7 * r.mean) * (2.5 * q + v) <= 1.85 * (1.0 - std::exp(-3.2 * q) + u);
+    return r > 0.0 && load >= 2.2 * r * r && load * r * r * r * r <= 100.0;
 }
 
 // Builds every device table of a batch from replica lists.  own_pace: whether lanes at their own pace may be chosen;
@@ -666,7 +664,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
         bool all_solo = can_solo && solo_masks && requests >= (int64_t)512 * n_seeds;
         if (all_solo && sims > at_once) {
             const double load = offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data());
-            const double replicas = replicas_of_a_request(wls, n_seeds, rl).mean, per_cu = (double)sims / (double)at_once * kSoloWavesPerCu;
+            const double replicas = replicas_of_a_request(wls, n_seeds, rl), per_cu = (double)sims / (double)at_once * kSoloWavesPerCu;
             const double level = std::min(64.0, std::max(24.0, 76.0 + 10.0 * std::log(std::max(load, 0.1)) - 3.5 * replicas));
             all_solo = (load >= 0.1 && per_cu <= level) || (load >= 1.0 && replicas <= 3.0);
         }

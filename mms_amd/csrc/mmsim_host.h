@@ -262,26 +262,17 @@ struct RepLists {
     }
 };
 
-// Replicas that a request may choose from, on average, and the share of the requests that have any (over the placements
-// that offered_load looks at).
-struct RequestReplicas {
-    double mean = 0.0, hosted = 0.0;
-};
-inline RequestReplicas replicas_of_a_request(const mmsim_workload *const *wls, int32_t n_streams, const RepLists &rl) {
-    double requests = 0.0, replicas = 0.0, hosted = 0.0;
+// Replicas that a request may choose from, on average (over the placements that offered_load looks at).
+inline double replicas_of_a_request(const mmsim_workload *const *wls, int32_t n_streams, const RepLists &rl) {
+    double requests = 0.0, replicas = 0.0;
     const int32_t every = std::max(1, rl.B / 64), looked = (rl.B + every - 1) / every;
     for (int s = 0; s < n_streams; ++s)
         for (int32_t m = 0; m < rl.M; ++m) {
             const double n = (double)wls[s]->model_num_requests[m];
             requests += n;
-            for (int32_t p = 0; p < rl.B; p += every) {
-                const int64_t here = rl.off[(size_t)p * rl.M + m + 1] - rl.off[(size_t)p * rl.M + m];
-                replicas += n * (double)here;
-                hosted += here > 0 ? n : 0.0;
-            }
+            for (int32_t p = 0; p < rl.B; p += every) replicas += n * (double)(rl.off[(size_t)p * rl.M + m + 1] - rl.off[(size_t)p * rl.M + m]);
         }
-    if (requests <= 0.0) return {};
-    return {replicas / requests / looked, hosted / requests / looked};
+    return requests > 0.0 ? replicas / requests / looked : 0.0;
 }
 
 struct mmsim_batch {

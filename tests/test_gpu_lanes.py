@@ -125,7 +125,7 @@ def test_load_decides(depths, load, expect):
     _check(eng, [_bursts(50, 8200, M, load)], profiles, sols, M, dict(window_lanes=-1), expect)
 
 
-@pytest.mark.parametrize("change,expect", [(0.0, "sim_lanes_kernel<4, true>"), (0.04, "sim_lanes_kernel<4, true>"), (0.4, "sim_mixed_kernel<4,"),
+@pytest.mark.parametrize("change,expect", [(0.0, "sim_lanes_kernel<4, true>"), (0.02, "sim_lanes_kernel<4, true>"), (0.4, "sim_mixed_kernel<4,"),
                                            (1.0, "sim_mixed_kernel<4,")])
 def test_runs_of_one_slo_decide(change, expect):
     """A run ends where the SLO changes: bursts of a model whose requests have SLOs of their own are runs of one request each."""
@@ -140,7 +140,7 @@ def test_runs_of_one_slo_decide(change, expect):
 
 @pytest.mark.parametrize("models,hosts,load,ends,expect", [(20, 2, 300.0, 0.12, "sim_lanes_kernel<4, true>"), (3, 3, 3000.0, 0.12, "sim_mixed_kernel<4,"),
                                                          (20, 0, 300.0, 0.12, "sim_mixed_kernel<4,"), (20, 2, 300.0, 0.04, "sim_mixed_kernel<4,")])
-def test_what_the_loops_have_to_do_decides(models, hosts, load, ends, expect):
+def test_replicas_and_bursts_decide(models, hosts, load, ends, expect):
     """Requests with many replicas, with none, and bursts of more than twenty requests on shallow groups keep the loop over runs, however
     large the load."""
     eng = E.Engine.default()
