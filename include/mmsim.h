@@ -99,7 +99,10 @@ typedef struct {
                                      slots as well                                                              */
     int32_t sched_groups;         /* workgroups of the scheduled launch; 0: one per CU                          */
     int32_t segment_requests;     /* requests per turn of an item in the scheduled launch; 0: 16384.  With lanes at
-                                     their own pace more than 8192 are taken up to a multiple of 8192          */
+                                     their own pace more than 8192 are taken up to a multiple of 8192.  With
+                                     window_lanes 64: a simulation is cut into runs of so many requests (512 at
+                                     least, 64 runs at most) that are simulated at the same time; 0: not cut,
+                                     and with window_lanes 0 as many as the chip has room for                  */
     int32_t sched_spin_limit;     /* looks in a row after which a wavefront that finds only busy items leaves;
                                      -1: 20000                                                                  */
     int32_t skip_ahead;           /* loop over runs: 0 = simulate every request; 1 = requests that every lane

@@ -19,8 +19,9 @@ OBJECTS = os.path.join(PKG, "_objects.so")   # Python extension: objects.cpp
 OBJ_DIR = os.path.join(HERE, "build")
 
 # object name -> source, flags of its own.  sim_window.hip is compiled once per number of requests side by side (its
-# instances are many; four translation units build in parallel).
+# instances are many; they build in parallel), and once more for simulations that are cut into runs.
 UNITS = {"mmsim_api": ("mmsim_api.hip", []), "window_batch": ("window_batch.hip", []),
+         "sim_window_runs": ("sim_window.hip", ["-DMMSIM_WINDOW_LANES=64", "-DMMSIM_WINDOW_SPANS"]),
          **{f"sim_window_{w}": ("sim_window.hip", [f"-DMMSIM_WINDOW_LANES={w}"]) for w in (64, 32, 16, 8)},
          "sim_mixed": ("sim_mixed.hip", []), "sim_lanes": ("sim_lanes.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_batching_solo": ("sim_batching_solo.hip", []),
          "sim_scalar": ("sim_scalar.hip", []),

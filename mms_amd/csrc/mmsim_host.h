@@ -189,6 +189,7 @@ void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
 
 struct mmsim_ctx {
     Staging staging;
+    mmsim::DevBuf<uint8_t> runs;           // of simulations that are cut into runs (window_batch.hip): no launch needs another's
     int device = 0;
     hipStream_t stream = nullptr;
     hipDeviceProp_t prop{};
@@ -343,7 +344,7 @@ struct mmsim_batch {
     // Requests side by side (window_batch.hip): all inputs in one buffer, all outputs in another
     bool window = false;
     WindowArgs wargs{};
-    DevBuf<uint8_t> win_in, win_out;
+    DevBuf<uint8_t> win_in, win_out, win_runs;
     std::vector<std::shared_ptr<DevBuf<Req>>> win_streams;
     size_t win_lat_sum = 0, win_model = 0, win_group = 0, win_finish = 0, win_good = 0;  // offsets in win_out (n_good: 0)
 

@@ -248,6 +248,16 @@ struct WindowArgs {
     int64_t Rmax;
     double fixed_overhead;
     uint32_t flags;
+    // simulations cut into runs (sim_window.hip), blocks of 64 requests
+    int32_t spans;                   // runs of a simulation; 1: not cut
+    int32_t span_blocks, ext_blocks; // blocks of a span, and how many a run goes on behind its own
+    int32_t marks, state_words;      // most marks of a span, 64-bit words of a state
+    int64_t run_cap, true_cap;       // values of a run: 64 * (span_blocks + ext_blocks), and of a whole stream
+    uint32_t *span_sync;             // [L][spans + 1] marks that every run has published, and how many runs have ended: 0 before a launch and after
+    uint64_t *mark_state;            // [L][spans][marks][state_words]
+    uint64_t *end_state;             // [L][spans][state_words + kEndWords]
+    double *run_vals;                // [L][true_cap + (spans - 1) * run_cap] latencies of the requests of a run (finish times, if wanted)
+    uint32_t *pieces;                // [L][2 * kMaxSpans][4] blocks [first, end) of the stream are run [2]'s; the last word: how many pieces
     // outputs, laid out as the caller's: simulation = seed * B + placement
     int32_t *n_good;
     double *lat_sum;
@@ -260,22 +270,31 @@ struct WindowArgs {
 // placements that share the wavefront.
 __host__ __device__ constexpr int window_ring_bytes(int lanes) { return lanes == kWave ? 0 : 2 * kWave * (int)sizeof(Req); }
 constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
+constexpr int kEndWords = 2;        // of end_state: end block, link
+constexpr int kSumWaves = 4;        // wavefronts of a workgroup that puts a simulation's runs together, if per-request outputs are wanted
+constexpr int kMaxSpans = 64;       // most runs of a simulation (their records are a lane's each)
+constexpr int kMaxRuns = 4096;      // most runs of a launch, if its simulations are cut
+// Where the k-th mark of a span is, in blocks from its beginning: 4, 8, 12, 16, 24, 32, 48, 64, 96, ...
+__host__ __device__ constexpr int span_mark(int k) { return k < 4 ? 4 * (k + 1) : ((k & 1) != 0 ? 32 : 24) << ((k - 4) / 2); }
 // More simulations than this put 64 placements to a wavefront, whatever they are (20000 requests, best number of lanes against
 // that: 16384 single devices 6.8 against 6.5 ms, two-stage pipelines 8.9 / 8.9, four-stage ones 7.9 / 7.8; 24576: 10.4 / 7.0,
 // 13.8 / 9.4, 12.5 / 8.2; build_window says when fewer do).
 constexpr int64_t kMaxWindowSims = 12288;
 typedef void (*WindowKernel)(const WindowArgs);
 // The kernel for LANES requests side by side (64, 32, 16, 8), stage bucket smax and the rest of its template arguments.
-template <int LANES>
+template <int LANES, bool SPANS>
 WindowKernel window_kernel(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<64>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+WindowKernel window_kernel<64, true>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<32>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+WindowKernel window_kernel<64, false>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<16>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+WindowKernel window_kernel<32, false>(int smax, bool outputs, int ext, bool pow2, bool uniform);
 template <>
-WindowKernel window_kernel<8>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+WindowKernel window_kernel<16, false>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+template <>
+WindowKernel window_kernel<8, false>(int smax, bool outputs, int ext, bool pow2, bool uniform);
+WindowKernel window_sum();
 std::string sim_window_kernel_name(const WindowArgs &args);
 
 // Arguments of the scalar-clock request loop (one placement, device pointers).

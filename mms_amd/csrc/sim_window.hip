@@ -47,6 +47,24 @@
 // requests, 6 models on 20 devices, up to 12 replicas, 1 / 64 / 700 / 1500 placements 2.7 / 3.3 / 3.9 / 4.4 -> 1.85 / 2.0 / 2.2 /
 // 3.1 ms; 12 models on 33 devices, up to 17, 5.7 / 5.9 / 7.1 / 7.6 -> 3.7 / 3.8 / 4.7 / 5.7 ms.
 //
+// Few simulations of long streams leave most of the chip idle, and a simulation is one chain of blocks.  It is cut into spans then
+// (SPANS): a run, a wavefront of its own, starts at the beginning of every span with all clocks at zero, as if nothing had come before.
+// That is wrong at first.  But what a simulation does next depends on its clocks alone, and clocks forget: a group that was
+// idle finishes its next request at a time that does not depend on what it did before, and one that rejected until it had caught up
+// agrees soon after.  So a run goes on behind its span and compares its clocks with those that the next run had at the same places
+// (marks: it left them in memory on its way).  Where all clocks are equal, bit for bit, both runs do the same for ever, and the one
+// that started further on has done it already: the run ends.  The first run is what the simulation does; where it ended
+// the run that it met takes over, and so on: the results are the serial loop's.  A run that meets nobody within half a span (48 blocks
+// at least) is given up; the wavefront that ends last follows the runs, takes up again one that was given up where
+// it is needed, and the first run never gives up: runs that never agree cost what they take from the first one, not the result.
+// Counts are differences between a run's end and the mark at which it was taken over; latencies are kept per request and added in their
+// order by a second kernel (LatencySum).  Runs agree after 200 to 2000 requests of bursty streams (of 108000 requests at 0.6 accepted, 32 models
+// on 32 single devices: 1000 in the median, 4000 at most of 180; eight four-stage pipelines: 400, 430), or never: steady overload, or groups
+// that are all idle most of the time, whose requests go round in the order the groups were used.
+// Kernels, 108000 requests: 700 placements of single devices, four runs each, 5.2 -> 2.9 + 0.2 ms (three wavefronts to a SIMD take 1.9 times
+// as long as one: issue); 600 of four-stage pipelines, five, 9.6 -> 3.4 + 0.3; 1025 up to 16 deep, three, 13.1 -> 8.4 + 0.3; one placement, 30000
+// requests, 24 runs, 1.85 -> 0.21 + 0.10 ms.  Where no runs agree: five placements, 82000 requests, 64 runs, 2.71 -> 2.84 ms.
+//
 // LDS of one placement (byte offsets in WindowArgs, built by the wavefront itself from the packed placement):
 //   clk  [slots+SMAX] f64   stage clocks, a placement's groups laid end to end, and SMAX slots for what does not count
 //   gm   [slots+SMAX] u64   mask of the block's requests that list the group whose last slot this is
@@ -178,6 +196,88 @@ __device__ __forceinline__ double ordered_sum(double s, double x, uint64_t lanes
 #undef MMSIM_ADD16
 #undef MMSIM_ADD1
 
+// x of this lane + x of all others, in lane 63
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double plus_moved(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double sum_of_lanes(double v) {
+    v = plus_moved<0x111 /* row_shr:1 */, 0xF>(v);
+    v = plus_moved<0x112, 0xF>(v);
+    v = plus_moved<0x114, 0xF>(v);
+    v = plus_moved<0x118, 0xF>(v);
+    v = plus_moved<0x142 /* row_bcast:15 */, 0xA>(v);
+    v = plus_moved<0x143 /* row_bcast:31 */, 0xC>(v);
+    return __hiloint2double(lane_value(__double2hiint(v), 63), lane_value(__double2loint(v), 63));
+}
+
+// The sum S of the accepted requests' latencies, added up in the order of their arrival: what S + x1 + x2 + ... gives with a
+// rounding behind every addition, without the chain of additions.  While S stays in [2^k, 2^(k+1)) it is a multiple of
+// u = 2^(k-52), and an addition adds x rounded to a multiple of u, r(x), whatever S is: unless x is half-way between two of them, where
+// S/u must come out even.  (That is common: times are multiples of 2^-43 or so.)  Whether S/u is odd before a request is how many odd
+// r(x) there were since the last half-way one, behind which it is even.  So the r(x) of 64 requests are found side by side, and
+// several blocks are added exactly, in any order.  Blocks that take S to 2^(k+1) or beyond (then their sum does as well, however it is
+// rounded), or have a negative x, go through ordered_sum one by one: S doubles a dozen times in a stream.
+struct LatencySum {
+    double s, base, half;  // base: 2^k, half: u / 2
+    int odd;               // whether s / u is odd, or s and what was taken since
+    __device__ __forceinline__ explicit LatencySum(double v) { set(v); }
+    __device__ __forceinline__ void set(double v) {
+        s = v;
+        odd = __double2loint(v) & 1;
+        const int hi = __double2hiint(v) & 0x7FF00000;
+        base = __hiloint2double(hi, 0);
+        half = __hiloint2double(hi > (53 << 20) ? hi - (53 << 20) : 0, 0);
+    }
+    // What the lanes add for their x.
+    __device__ __forceinline__ double take(double x) {
+        const double up = base + x, r = up - base, off = x - r;
+        const bool half_way = __builtin_fabs(off) == half;
+        const uint64_t ties = ballot(half_way), odds = ballot((__double2loint(up) & 1) != 0);  // (half-way ones came out even)
+        // whether S / u is odd behind these requests: as many odd ones from the last half-way one on
+        auto odd_behind = [&](uint64_t lanes) {
+            const uint64_t t = ties & lanes;
+            const uint64_t since = odds & lanes & (t != 0ull ? ~0ull << (63 - __builtin_clzll(t | 1ull)) : ~0ull);
+            return (__popcll(since) ^ (t != 0ull ? 0 : odd)) & 1;
+        };
+        const double added = half_way && odd_behind((1ull << lane_id()) - 1ull) != 0 ? x + off : r;
+        odd = odd_behind(~0ull);
+        return added;
+    }
+    // Adds N blocks' latencies, 0 where a request is not accepted; false, and nothing is done: not together.
+    template <int N>
+    __device__ __forceinline__ bool add(const double (&x)[N]) {
+        const int odd_before = odd;
+        double lanes = 0.0;
+        bool negative = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            lanes += take(x[i]);
+            negative = negative || x[i] < 0.0;
+        }
+        const double sum = sum_of_lanes(lanes);
+        if (!(sum <= 2.0 * base - s) || ballot(negative) != 0ull) {
+            odd = odd_before;
+            return false;
+        }
+        set(s + sum);
+        return true;
+    }
+    __device__ __forceinline__ void add_block(double x) {
+        const double one[1] = {x};
+        const uint64_t some = ballot(x != 0.0);
+        if (some != 0ull && !add(one)) set(ordered_sum<kWave>(s, x, some));
+    }
+};
+
+// What wavefronts of different workgroups tell one another while the kernel runs: stores and loads that all of the device sees.
+__device__ __forceinline__ void tell(uint64_t *p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void tell(uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ uint64_t told(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ uint32_t told(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 struct Entry {  // a replica, as rep and ext hold it
     uint32_t d;
     float l;
@@ -202,23 +302,102 @@ template <int I>
 struct Int {
     static constexpr int value = I;
 };
+// The arguments as they lie in memory, for what is done rarely: asked for there, and not kept in scalar registers, which the loop over blocks
+// has none to spare of (71 of its instructions, of 930 a block, moved them to and fro).
+typedef const __attribute__((address_space(4))) WindowArgs ColdArgs;
+__device__ __forceinline__ ColdArgs *cold_args() {
+    ColdArgs *p = (ColdArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// Where a run's latencies are (finish times, if wanted), by place in the stream: those of runs that are taken up again in an array of
+// the whole stream.  (Run 0 adds up its own and writes its outputs.)
+__device__ __forceinline__ double *values_of(ColdArgs *q, int sim, int r) {
+    double *v = q->run_vals + (size_t)sim * (size_t)(q->true_cap + (q->spans - 1) * q->run_cap);
+    return r == 0 ? v : v + q->true_cap + (r - 1) * q->run_cap - (int64_t)r * q->span_blocks * kWave;
+}
+
+struct Runs {  // what a run goes by (scalars; blocks of 64 requests)
+    int own;         // the run, or -1: one that is taken up again
+    int in, mark;    // the span of the next mark, and which of that span's it is
+    uint32_t since;  // where the run left its own span
+    uint32_t next;   // block before which something happens
+    bool looked;     // another run's mark: what to compare with is on its way (asked for a block ahead)
+    bool met;        // the run of span `in` at that mark
+
+    // known to be what the simulation does: the first run, or one taken up again
+    __device__ __forceinline__ bool true_one() const { return own <= 0; }
+    __device__ __forceinline__ uint32_t limit(ColdArgs *a) const {
+        return true_one() ? 0xFFFFFFFFu : (uint32_t)((own + 1) * a->span_blocks + a->ext_blocks);
+    }
+    __device__ __forceinline__ void start(ColdArgs *a, int span) {
+        own = in = span;
+        mark = 0;
+        looked = met = false;
+        since = (uint32_t)((own + 1) * a->span_blocks);
+        next = (uint32_t)(own * a->span_blocks + span_mark(0));  // (within the span: it has more than eight blocks)
+    }
+    __device__ __forceinline__ void resume(ColdArgs *a, uint32_t at) {
+        own = -1;
+        in = (int)(at / (uint32_t)a->span_blocks);
+        mark = -1;
+        met = false;
+        since = at;
+        go_on(a, at);
+    }
+    // From block `at` to the next mark: of its own span all, of others those that are further by an eighth of how far the run has come on
+    // its own (a run that meets nobody looks fifty times or so, not at every mark of the stream).
+    __device__ __forceinline__ void go_on(ColdArgs *a, uint32_t at) {
+        const int span = a->span_blocks;
+        const uint32_t least = at < since ? 0u : at + 2u + (at - since) / 8u;
+        uint32_t m;
+        do {
+            mark += 1;
+            if (span_mark(mark) >= span) {
+                in += 1;
+                mark = 0;
+            }
+            m = (uint32_t)(in * span + span_mark(mark));
+        } while (m < least);
+        looked = false;
+        next = in != own ? m - 1u : m;
+        next = next < limit(a) ? next : limit(a);
+    }
+};
+
+// Wavefronts of a SIMD that the registers have to leave room for, with simulations cut into runs.
+constexpr int least_waves(int smax, bool outputs, int ext) {
+    return ext > 1 || (smax == 32 && (outputs || ext > 0)) ? 2 : outputs || smax == 32 || (smax == 16 && ext > 0) ? 3 : 4;
+}
+
 // W: requests (lanes) of one placement.  SMAX: most stages of a group (bucket).  OUTPUTS: anything beyond the scores
 // (a.flags says what).  EXT: 1, some model has more than four replicas; 2, and up to sixteen are kept in registers, not eight.  POW2: every group has 1, 2, 4, ... stages.
 // UNIFORM: one latency per (model, configuration).
-template <int W, int SMAX, bool OUTPUTS, int EXT, bool POW2, bool UNIFORM>
-__global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(const WindowArgs a) {
+// SPANS: a simulation is cut into a.spans runs (W == 64).
+template <int W, int SMAX, bool OUTPUTS, int EXT, bool POW2, bool UNIFORM, bool SPANS>
+__global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, OUTPUTS, EXT) : 1) void sim_window_kernel(const WindowArgs a) {
     constexpr int P = kWave / W;
     const int lane = lane_id(), j = lane % W, sub = W == 64 ? 0 : lane / W;
-    const int wv = SMAX >= 16 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
+    const int wv = SMAX >= 16 || SPANS ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
     // latency table for the per-stage latencies of the walk (general tables only), shared by the workgroup
     if (!UNIFORM && a.lat_lds_bytes > 0) {
         for (int i = (int)threadIdx.x; i < a.M * a.lat_row; i += (int)blockDim.x) lds_put<float>((uint32_t)i * 4u, a.lat[i]);
         __syncthreads();
     }
-    const int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;  // (seed, tile of P placements)
+    int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;  // (seed, tile of P placements)
+    int own = 0;                                                  // the run
+    if constexpr (SPANS) {
+        // First runs first, each workgroup's on another SIMD than those of the workgroups that share its CU.
+        const int waves = (int)(blockDim.x >> 6), sims = a.tiles * a.out_seeds;
+        const int at = __builtin_amdgcn_readfirstlane((wv + (int)(blockIdx.x >> 8)) % waves) * (int)gridDim.x + (int)blockIdx.x;
+        own = __builtin_amdgcn_readfirstlane(at / sims);
+        if (own >= a.spans) return;
+        unit = at - own * sims;
+    }
     if (unit >= (int64_t)a.tiles * a.out_seeds) return;
-    const int seed_row = (int)(unit / a.tiles);
-    const int b = (int)(unit % a.tiles) * P + sub;
+    const int seed_row = SPANS ? __builtin_amdgcn_readfirstlane((int)unit / a.tiles) : (int)(unit / a.tiles);
+    const int b = SPANS ? (int)unit - seed_row * a.tiles : (int)(unit % a.tiles) * P + sub;
     const bool mine = b < a.B;
     // (with a stream of its own for every placement there is one placement to a wavefront: the host sees to that)
     const int seed = a.stream_of ? lane_value(a.stream_of[mine ? b : 0], 0) : seed_row;
@@ -322,26 +501,11 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     // Requests come 64 at a time, one to a lane.  W == 64: that is a block, fetched two blocks ahead.  Otherwise the
     // chunks pass through LDS, which deals them to the placements' lanes; the chunk after the one a block is of is in
     // LDS as well, and the one after that on its way.
-    u32x4 far = load_req((uint32_t)lane);
+    u32x4 far, nxt;
     Req cur;
-    u32x4 nxt;
     auto store_ring = [&](uint32_t chunk) { lds_put<u32x4>(ring + (chunk & 1u) * 1024u + (uint32_t)lane * 16u, far); };
     auto load_ring = [&](uint32_t i) -> u32x4 { return lds_get<u32x4>(ring + (i & 127u) * 16u); };
-    if constexpr (W == 64) {
-        nxt = load_req(64u + (uint32_t)lane);
-        arrived(far);  // (here, or the first step of every block waits for what is on its way then)
-        arrived(nxt);
-        cur = as_req(far);
-    } else {
-        store_ring(0u);
-        far = load_req(64u + (uint32_t)lane);
-        store_ring(1u);
-        far = load_req(128u + (uint32_t)lane);
-        wave_order();
-        cur = as_req(load_ring((uint32_t)j));
-        nxt = load_ring((uint32_t)(W + j));
-    }
-    Entry4 q = load_rep(cur.m);
+    Entry4 q;
     // What a block is like: requests that can be served at all, that list several groups, more than two, more than
     // four; how deep their groups are.  Worked out a block ahead (a scalar that depends on vector compares is slow to come).
     uint64_t pend, multis, fours, mores, eights, sixteens, deep_a, deep_b;
@@ -365,7 +529,25 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
             }
         }
     };
-    look();
+    auto start_at = [&](uint32_t first) {  // (a multiple of 64)
+        far = load_req(first + (uint32_t)lane);
+        if constexpr (W == 64) {
+            nxt = load_req(first + 64u + (uint32_t)lane);
+            arrived(far);  // (here, or the first step of every block waits for what is on its way then)
+            arrived(nxt);
+            cur = as_req(far);
+        } else {
+            store_ring(0u);
+            far = load_req(64u + (uint32_t)lane);
+            store_ring(1u);
+            far = load_req(128u + (uint32_t)lane);
+            wave_order();
+            cur = as_req(load_ring((uint32_t)j));
+            nxt = load_ring((uint32_t)(W + j));
+        }
+        q = load_rep(cur.m);
+        look();
+    };
 
     // What a step needs of an entry word, ready for it: the address of the group's first clock and, from bit 18 on, stages - 1;
     // of a single stage the address, of several latencies the word itself.
@@ -378,326 +560,492 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
         return SMAX == 1 ? w : w & 0x3FFFFu;
     };
     auto stages_m1 = [](uint32_t w) -> int { return SMAX == 1 ? 0 : UNIFORM ? (int)(w >> 18) : entry_stages_m1(w); };
-    for (uint32_t blk = 0; blk < R; blk += W) {
-        const int m = cur.m;
-        const double arr = cur.t, slo = (double)cur.slo;
-        uint32_t ca[4], word[4];  // what the tournament carries of an entry word
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ca[k] = entry_addr(q.e[k].d);
-            word[k] = walk_word(q.e[k].d);
+    // ---- SPANS: this wavefront's run, and the simulation's others
+    const int sim = (int)unit;
+    Runs runs;
+    if constexpr (SPANS) {
+        runs.start(cold_args(), own);
+    }
+    auto marked = [&](int r, int i) {
+        ColdArgs *q = cold_args();
+        return q->mark_state + (((size_t)sim * q->spans + r) * q->marks + i) * (size_t)q->state_words;
+    };
+    auto ended = [&](int r) {
+        ColdArgs *q = cold_args();
+        return q->end_state + ((size_t)sim * q->spans + r) * (size_t)(q->state_words + kEndWords);
+    };
+    // state: accepted requests, clocks; counts of the slots and of the models
+    auto for_state = [&](auto f) {
+        const int nslots = cold_args()->nslots;
+        for (int k = j; k < nslots; k += W) f(1 + k, clk + (uint32_t)k * 8u, false);
+        if constexpr (OUTPUTS) {
+            for (int k = j; k < nslots; k += W) f(1 + nslots + k, clk + (uint32_t)k * 8u + cnt_rel, false);
+            for (int m = j; m < M; m += W) f(1 + 2 * nslots + m, mcnt + (uint32_t)m * 4u, true);
         }
-        Entry4 nrep;
-        u32x4 nn;
-        double best = 0.0, t = 0.0, latency = 0.0;
-        uint32_t chosen = SMAX > 1 && !UNIFORM ? clk >> 3 : clk;  // the chosen group's walk word
-        // The block, for requests that list at most NC groups (2, 4, 8, 16, or 0: any number).
-        auto block = [&](auto NCv) {
-            constexpr int NC = decltype(NCv)::value, N4 = NC == 2 ? 2 : 4;
-            // Further ones kept in registers.  (Not beside the fetched ones with 16 stages and counts: 133 registers instead of 126, three
-            // wavefronts to a SIMD instead of four.)
-            constexpr int NX = NC > 4 ? NC - 4 : NC == 0 ? (EXT > 1 ? 12 : SMAX < 16 ? 4 : 0) : 0;
-            constexpr bool MORE = NC != 2 && NC != 4, ANY = NC == 0;                // ANY: and others are fetched in every step
-            double c[N4];
-#pragma unroll
-            for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
-            // ---- the masks of the block's requests.  (Copies of the first replica set its bit again: harmless.)
-            uint64_t gm[N4];
-            uint32_t x0 = 0, xn = 0;  // chunks of further replicas
-            if constexpr (MORE) {
-                const uint32_t v = lds_get<uint32_t>(xi + (uint32_t)(m < 0 ? 0 : m) * 4u);
-                x0 = ext + (v & 0xFFFFu) * 32u;
-                xn = in_mask(pend) ? v >> 16 : 0u;
+    };
+    auto get_word = [&](uint32_t at, bool half) -> uint64_t { return half ? (uint64_t)lds_get<uint32_t>(at) : lds_get<uint64_t>(at); };
+    // Something happens before block `at`: a mark of this run, one of a later run or the block ahead of it, the end of the run (true).
+    auto published = [&](int r) {
+        ColdArgs *q = cold_args();
+        return q->span_sync + (size_t)sim * (q->spans + 1) + r;
+    };
+    uint64_t peeked = 0;
+    auto event = [&](uint32_t at) -> bool {
+        ColdArgs *q = cold_args();
+        if (at >= runs.limit(q)) return true;
+        uint64_t *st = marked(runs.in, runs.mark);
+        if (runs.in == runs.own) {
+            if (lane == 0) tell(st, (uint64_t)(uint32_t)n_good);
+            for_state([&](int w, uint32_t addr, bool half) { tell(st + w, get_word(addr, half)); });
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (stores of device scope have been carried out then)
+            if (lane == 0) tell(published(runs.in), (uint32_t)runs.mark + 1u);
+        } else if (!runs.looked) {
+            if (__builtin_amdgcn_readfirstlane(told(published(runs.in))) > (uint32_t)runs.mark) {
+                asm volatile("" ::: "memory");
+                peeked = told(st + 1 + (lane < q->nslots ? lane : 0));
+                runs.looked = true;
+                runs.next = at + 1u;
+                return false;
             }
-            // the further ones in registers, like the first four (of a request without: copies of its first, which never beat it)
-            constexpr int NA = NX > 0 ? NX : 1;
-            uint32_t xa[NA], xword[NA];
-            float xl[NA];
-            double cx[NA];
+        } else {
+            bool same = lane >= q->nslots || peeked == lds_get<uint64_t>(clk + (uint32_t)lane * 8u);
+            if (ballot(!same) == 0ull) {
+                for (int k = j + W; k < q->nslots; k += W) same = same && told(st + 1 + k) == lds_get<uint64_t>(clk + (uint32_t)k * 8u);
+                runs.met = ballot(!same) == 0ull;
+                if (runs.met) return true;
+            }
+        }
+        runs.go_on(q, at);
+        return false;
+    };
+    auto q_pieces = [&](int of) { return cold_args()->pieces + (size_t)of * (8 * kMaxSpans); };
+    auto piece = [&](uint32_t at, uint32_t first, uint32_t end, int src) {
+        uint32_t *w = q_pieces(sim) + at * 4u;
+        w[0] = first;
+        w[1] = end;
+        w[2] = (uint32_t)src;
+    };
+    uint32_t from = SPANS ? (uint32_t)own * (uint32_t)a.span_blocks * 64u : 0u, blk = from;
+    double *run_vals = SPANS ? values_of(cold_args(), sim, own) : nullptr;  // by place in the stream
+    uint32_t num_pieces = 0;
+    bool last = false;  // this wavefront puts the simulation together
+    for (;;) {
+        if (from < R) start_at(from);
+        for (blk = from; blk < R; blk += W) {
+            if constexpr (SPANS)
+                if (blk / 64u == runs.next && event(blk / 64u)) break;
+            const int m = cur.m;
+            const double arr = cur.t, slo = (double)cur.slo;
+            uint32_t ca[4], word[4];  // what the tournament carries of an entry word
 #pragma unroll
-            for (int x = 0; x < NX / 4; ++x) {
-                Entry4 more;
-                if (xn > (uint32_t)x) more = load_entries(x0 + (uint32_t)x * 32u);
-                else more.e[0] = more.e[1] = more.e[2] = more.e[3] = q.e[0];
+            for (int k = 0; k < 4; ++k) {
+                ca[k] = entry_addr(q.e[k].d);
+                word[k] = walk_word(q.e[k].d);
+            }
+            Entry4 nrep;
+            u32x4 nn;
+            double best = 0.0, t = 0.0, latency = 0.0;
+            uint32_t chosen = SMAX > 1 && !UNIFORM ? clk >> 3 : clk;  // the chosen group's walk word
+            // The block, for requests that list at most NC groups (2, 4, 8, 16, or 0: any number).
+            auto block = [&](auto NCv) {
+                constexpr int NC = decltype(NCv)::value, N4 = NC == 2 ? 2 : 4;
+                // Further ones kept in registers.  (Not beside the fetched ones with 16 stages and counts: 133 registers instead of 126, three
+                // wavefronts to a SIMD instead of four.)
+                constexpr int NX = NC > 4 ? NC - 4 : NC == 0 ? (EXT > 1 ? 12 : SMAX < 16 ? 4 : 0) : 0;
+                constexpr bool MORE = NC != 2 && NC != 4, ANY = NC == 0;                // ANY: and others are fetched in every step
+                double c[N4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    xa[4 * x + k] = entry_addr(more.e[k].d);
-                    xword[4 * x + k] = walk_word(more.e[k].d);
-                    xl[4 * x + k] = more.e[k].l;
-                    cx[4 * x + k] = lds_get<double>(xa[4 * x + k]);
+                for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
+                // ---- the masks of the block's requests.  (Copies of the first replica set its bit again: harmless.)
+                uint64_t gm[N4];
+                uint32_t x0 = 0, xn = 0;  // chunks of further replicas
+                if constexpr (MORE) {
+                    const uint32_t v = lds_get<uint32_t>(xi + (uint32_t)(m < 0 ? 0 : m) * 4u);
+                    x0 = ext + (v & 0xFFFFu) * 32u;
+                    xn = in_mask(pend) ? v >> 16 : 0u;
                 }
-            }
-            uint32_t ga[N4];
+                // the further ones in registers, like the first four (of a request without: copies of its first, which never beat it)
+                constexpr int NA = NX > 0 ? NX : 1;
+                uint32_t xa[NA], xword[NA];
+                float xl[NA];
+                double cx[NA];
 #pragma unroll
-            for (int k = 0; k < N4; ++k) {
-                ga[k] = ca[k] + gm_rel;
-                pin(ga[k]);
-            }
-            if (in_mask(pend)) {
+                for (int x = 0; x < NX / 4; ++x) {
+                    Entry4 more;
+                    if (xn > (uint32_t)x) more = load_entries(x0 + (uint32_t)x * 32u);
+                    else more.e[0] = more.e[1] = more.e[2] = more.e[3] = q.e[0];
 #pragma unroll
-                for (int k = 0; k < N4; ++k) lds_or_u64(ga[k], my_bit);
+                    for (int k = 0; k < 4; ++k) {
+                        xa[4 * x + k] = entry_addr(more.e[k].d);
+                        xword[4 * x + k] = walk_word(more.e[k].d);
+                        xl[4 * x + k] = more.e[k].l;
+                        cx[4 * x + k] = lds_get<double>(xa[4 * x + k]);
+                    }
+                }
+                uint32_t ga[N4];
+#pragma unroll
+                for (int k = 0; k < N4; ++k) {
+                    ga[k] = ca[k] + gm_rel;
+                    pin(ga[k]);
+                }
+                if (in_mask(pend)) {
+#pragma unroll
+                    for (int k = 0; k < N4; ++k) lds_or_u64(ga[k], my_bit);
+                    if constexpr (NX > 0) {
+#pragma unroll
+                        for (int x = 0; x < NX / 4; ++x)
+                            if (xn > (uint32_t)x) {
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) lds_or_u64(xa[4 * x + k] + gm_rel, my_bit);
+                            }
+                    }
+                    if constexpr (ANY)
+                        for (uint32_t x = NX / 4; x < xn; ++x) {
+                            const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) lds_or_u64(entry_addr(e.e[k].d) + gm_rel, my_bit);
+                        }
+                }
+                wave_order();
+#pragma unroll
+                for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ga[k]) & before;
+                uint64_t gm_ext = 0;  // requests before this one that share any of the groups: holds for every further replica
+                if constexpr (MORE) {
+                    if constexpr (NX > 0) {
+#pragma unroll
+                        for (int k = 0; k < NX; ++k) gm_ext |= lds_get<uint64_t>(xa[k] + gm_rel);
+                    }
+                    if constexpr (ANY) {
+                        for (uint32_t x = NX / 4; x < xn; ++x) {
+                            const Entry4 e = load_entries(x0 + x * 32u);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
+                        }
+                    }
+                    gm_ext = (gm_ext & before) | gm[0] | gm[1] | gm[2] | gm[3];
+                }
+                wave_order();
+#pragma unroll
+                for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ga[k], 0);  // for the next block
                 if constexpr (NX > 0) {
 #pragma unroll
-                    for (int x = 0; x < NX / 4; ++x)
-                        if (xn > (uint32_t)x) {
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) lds_or_u64(xa[4 * x + k] + gm_rel, my_bit);
-                        }
+                    for (int k = 0; k < NX; ++k) lds_put<uint64_t>(xa[k] + gm_rel, 0);
                 }
                 if constexpr (ANY)
                     for (uint32_t x = NX / 4; x < xn; ++x) {
                         const Entry4 e = load_entries(x0 + x * 32u);
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) lds_or_u64(entry_addr(e.e[k].d) + gm_rel, my_bit);
+                        for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
                     }
-            }
-            wave_order();
-#pragma unroll
-            for (int k = 0; k < N4; ++k) gm[k] = lds_get<uint64_t>(ga[k]) & before;
-            uint64_t gm_ext = 0;  // requests before this one that share any of the groups: holds for every further replica
-            if constexpr (MORE) {
-                if constexpr (NX > 0) {
-#pragma unroll
-                    for (int k = 0; k < NX; ++k) gm_ext |= lds_get<uint64_t>(xa[k] + gm_rel);
-                }
-                if constexpr (ANY) {
-                    for (uint32_t x = NX / 4; x < xn; ++x) {
-                        const Entry4 e = load_entries(x0 + x * 32u);
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) gm_ext |= lds_get<uint64_t>(entry_addr(e.e[k].d) + gm_rel);
+                // ---- fetched ahead: the requests of the block after the next, the replicas of the next
+                if constexpr (W == 64) {
+                    nn = load_req(blk + 128u + (uint32_t)j);
+                } else {
+                    if ((blk & 63u) == 0u && blk != 0u) {  // a chunk begins: the one after it takes the place of the one before
+                        store_ring(blk / 64u + 1u);
+                        far = load_req(blk + 128u + (uint32_t)lane);
+                        wave_order();
                     }
+                    nn = load_ring(blk + 2u * W + (uint32_t)j);
                 }
-                gm_ext = (gm_ext & before) | gm[0] | gm[1] | gm[2] | gm[3];
-            }
-            wave_order();
+                wave_order();
+                // ---- the steps.  Each lane stays in the loop until its verdict is final and leaves with what it found.
+                // D: most stages of a group.
+                auto steps = [&](auto Dv) {
+                    constexpr int D = decltype(Dv)::value;
+                    // The stages behind the first NEAR are read, walked and written by the lanes that chose a group with
+                    // so many, in a branch that most steps skip.  A wavefront on its own (W == 64) takes up to eight
+                    // without a branch, as the stages are a shorter chain than the branch; wavefronts that share a
+                    // SIMD (W < 64) gain from four stages on, as they share its issue slots.  20000 requests, against
+                    // all stages in every lane: 4096 placements of groups up to 16 deep 6.44 -> 5.11 ms, up to 8 deep
+                    // 5.02 -> 4.81 ms; 1025 placements, W == 64, up to 16 deep 3.60 -> 3.20 ms (2.88 -> 2.98 ms up to 8
+                    // deep, where only the registers of the unused deep path differ).
+                    constexpr int NEAR = W == 64 ? 8 : 4;
+                    struct Cand {
+                        double c;
+                        uint32_t d;
+                        float l;
+                        uint64_t g;
+                    };
+                    auto first_min = [](const Cand &x, const Cand &y) {
+                        const bool right = y.c < x.c;
+                        return Cand{vmin(x.c, y.c), right ? y.d : x.d, right ? y.l : x.l, right ? y.g : x.g};
+                    };
+                    bool waits;
+                    do {
+                        // ---- choose the replica group: strictly smallest last-stage clock, first listed wins ties (:590-598)
+                        Cand win = first_min(Cand{c[0], word[0], q.e[0].l, gm[0]}, Cand{c[1], word[1], q.e[1].l, gm[1]});
+                        if constexpr (NC != 2)
+                            win = first_min(win, first_min(Cand{c[2], word[2], q.e[2].l, gm[2]}, Cand{c[3], word[3], q.e[3].l, gm[3]}));
+                        if constexpr (NX > 0) {
 #pragma unroll
-            for (int k = 0; k < N4; ++k) lds_put<uint64_t>(ga[k], 0);  // for the next block
-            if constexpr (NX > 0) {
+                            for (int x = 0; x < NX; x += 4) {
+                                Cand y[4];
 #pragma unroll
-                for (int k = 0; k < NX; ++k) lds_put<uint64_t>(xa[k] + gm_rel, 0);
-            }
-            if constexpr (ANY)
-                for (uint32_t x = NX / 4; x < xn; ++x) {
-                    const Entry4 e = load_entries(x0 + x * 32u);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) lds_put<uint64_t>(entry_addr(e.e[k].d) + gm_rel, 0);
-                }
-            // ---- fetched ahead: the requests of the block after the next, the replicas of the next
-            if constexpr (W == 64) {
-                nn = load_req(blk + 128u + (uint32_t)j);
-            } else {
-                if ((blk & 63u) == 0u && blk != 0u) {  // a chunk begins: the one after it takes the place of the one before
-                    store_ring(blk / 64u + 1u);
-                    far = load_req(blk + 128u + (uint32_t)lane);
-                    wave_order();
-                }
-                nn = load_ring(blk + 2u * W + (uint32_t)j);
-            }
-            wave_order();
-            // ---- the steps.  Each lane stays in the loop until its verdict is final and leaves with what it found.
-            // D: most stages of a group.
-            auto steps = [&](auto Dv) {
-                constexpr int D = decltype(Dv)::value;
-                // The stages behind the first NEAR are read, walked and written by the lanes that chose a group with
-                // so many, in a branch that most steps skip.  A wavefront on its own (W == 64) takes up to eight
-                // without a branch, as the stages are a shorter chain than the branch; wavefronts that share a
-                // SIMD (W < 64) gain from four stages on, as they share its issue slots.  20000 requests, against
-                // all stages in every lane: 4096 placements of groups up to 16 deep 6.44 -> 5.11 ms, up to 8 deep
-                // 5.02 -> 4.81 ms; 1025 placements, W == 64, up to 16 deep 3.60 -> 3.20 ms (2.88 -> 2.98 ms up to 8
-                // deep, where only the registers of the unused deep path differ).
-                constexpr int NEAR = W == 64 ? 8 : 4;
-                struct Cand {
-                    double c;
-                    uint32_t d;
-                    float l;
-                    uint64_t g;
-                };
-                auto first_min = [](const Cand &x, const Cand &y) {
-                    const bool right = y.c < x.c;
-                    return Cand{vmin(x.c, y.c), right ? y.d : x.d, right ? y.l : x.l, right ? y.g : x.g};
-                };
-                bool waits;
-                do {
-                    // ---- choose the replica group: strictly smallest last-stage clock, first listed wins ties (:590-598)
-                    Cand win = first_min(Cand{c[0], word[0], q.e[0].l, gm[0]}, Cand{c[1], word[1], q.e[1].l, gm[1]});
-                    if constexpr (NC != 2)
-                        win = first_min(win, first_min(Cand{c[2], word[2], q.e[2].l, gm[2]}, Cand{c[3], word[3], q.e[3].l, gm[3]}));
-                    if constexpr (NX > 0) {
-#pragma unroll
-                        for (int x = 0; x < NX; x += 4) {
-                            Cand y[4];
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) y[k] = Cand{cx[x + k], xword[x + k], xl[x + k], gm_ext};
-                            win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
-                        }
-                    }
-                    if constexpr (ANY)
-                        for (uint32_t x = NX / 4; x < xn; ++x) {
-                            const Entry4 e = load_entries(x0 + x * 32u);
-                            Cand y[4];
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const uint32_t at = entry_addr(e.e[k].d);
-                                y[k] = Cand{lds_get<double>(at), e.e[k].d, e.e[k].l, gm_ext};
+                                for (int k = 0; k < 4; ++k) y[k] = Cand{cx[x + k], xword[x + k], xl[x + k], gm_ext};
+                                win = first_min(win, first_min(first_min(y[0], y[1]), first_min(y[2], y[3])));
                             }
-                            Cand z = first_min(first_min(y[0], y[1]), first_min(y[2], y[3]));
-                            z.d = walk_word(z.d);
-                            win = first_min(win, z);
                         }
-                    best = win.c;
-                    chosen = win.d;
-                    const double l_last = (double)win.l;
-                    // ---- walk the stages and decide (:605-613).  All requests read and walk the near stages from their group's first
-                    // on and take the time after their last one (what lies behind a shallower group's slots does not matter).
-                    double cv[D];
-                    const int sm1 = stages_m1(win.d);
-                    const uint32_t gclk = first_clock(win.d);
-                    if constexpr (SMAX == 1) {
-                        t = vmax(arr, best) + l_last;
-                        cv[0] = t;
-                    } else {
-                        const uint32_t lrow = (uint32_t)m * (uint32_t)a.lat_row + entry_lat(win.d) - (uint32_t)sm1;
-                        float l[UNIFORM ? 1 : D];
-                        auto read = [&](int k) {
-                            cv[k] = lds_get<double>(gclk + (uint32_t)k * 8u);
-                            if constexpr (!UNIFORM)
-                                l[k] = a.lat_lds_bytes > 0 ? lds_get<float>((lrow + (uint32_t)k) * 4u) : a.lat[lrow + (uint32_t)k];
-                        };
-                        auto pass = [&](int k) {
-                            cv[k] = vmax(k == 0 ? arr : cv[k > 0 ? k - 1 : 0], cv[k]) + (UNIFORM ? l_last : (double)l[UNIFORM ? 0 : k]);
-                            if (k == 0)
-                                t = cv[0];
-                            else if (!POW2 || (k & (k + 1)) == 0)
-                                t = sm1 >= k ? cv[k] : t;
-                        };
+                        if constexpr (ANY)
+                            for (uint32_t x = NX / 4; x < xn; ++x) {
+                                const Entry4 e = load_entries(x0 + x * 32u);
+                                Cand y[4];
 #pragma unroll
-                        for (int k = 0; k < (D < 8 ? D : 8); ++k) read(k);
+                                for (int k = 0; k < 4; ++k) {
+                                    const uint32_t at = entry_addr(e.e[k].d);
+                                    y[k] = Cand{lds_get<double>(at), e.e[k].d, e.e[k].l, gm_ext};
+                                }
+                                Cand z = first_min(first_min(y[0], y[1]), first_min(y[2], y[3]));
+                                z.d = walk_word(z.d);
+                                win = first_min(win, z);
+                            }
+                        best = win.c;
+                        chosen = win.d;
+                        const double l_last = (double)win.l;
+                        // ---- walk the stages and decide (:605-613).  All requests read and walk the near stages from their group's first
+                        // on and take the time after their last one (what lies behind a shallower group's slots does not matter).
+                        double cv[D];
+                        const int sm1 = stages_m1(win.d);
+                        const uint32_t gclk = first_clock(win.d);
+                        if constexpr (SMAX == 1) {
+                            t = vmax(arr, best) + l_last;
+                            cv[0] = t;
+                        } else {
+                            const uint32_t lrow = (uint32_t)m * (uint32_t)a.lat_row + entry_lat(win.d) - (uint32_t)sm1;
+                            float l[UNIFORM ? 1 : D];
+                            auto read = [&](int k) {
+                                cv[k] = lds_get<double>(gclk + (uint32_t)k * 8u);
+                                if constexpr (!UNIFORM)
+                                    l[k] = a.lat_lds_bytes > 0 ? lds_get<float>((lrow + (uint32_t)k) * 4u) : a.lat[lrow + (uint32_t)k];
+                            };
+                            auto pass = [&](int k) {
+                                cv[k] = vmax(k == 0 ? arr : cv[k > 0 ? k - 1 : 0], cv[k]) + (UNIFORM ? l_last : (double)l[UNIFORM ? 0 : k]);
+                                if (k == 0)
+                                    t = cv[0];
+                                else if (!POW2 || (k & (k + 1)) == 0)
+                                    t = sm1 >= k ? cv[k] : t;
+                            };
 #pragma unroll
-                        for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) pass(k);
-                        if constexpr (D > NEAR) {
-                            if (sm1 >= NEAR) {
+                            for (int k = 0; k < (D < 8 ? D : 8); ++k) read(k);
 #pragma unroll
-                                for (int k = NEAR; k < (D < 8 ? D : 8); ++k) pass(k);
-                                if constexpr (D > 8) {
-                                    if (sm1 >= 8) {
+                            for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) pass(k);
+                            if constexpr (D > NEAR) {
+                                if (sm1 >= NEAR) {
 #pragma unroll
-                                        for (int k = 8; k < (D < 16 ? D : 16); ++k) read(k);
+                                    for (int k = NEAR; k < (D < 8 ? D : 8); ++k) pass(k);
+                                    if constexpr (D > 8) {
+                                        if (sm1 >= 8) {
 #pragma unroll
-                                        for (int k = 8; k < (D < 16 ? D : 16); ++k) pass(k);
-                                        if constexpr (D > 16) {
-                                            if (sm1 >= 16) {
+                                            for (int k = 8; k < (D < 16 ? D : 16); ++k) read(k);
 #pragma unroll
-                                                for (int k = 16; k < D; ++k) read(k);
+                                            for (int k = 8; k < (D < 16 ? D : 16); ++k) pass(k);
+                                            if constexpr (D > 16) {
+                                                if (sm1 >= 16) {
 #pragma unroll
-                                                for (int k = 16; k < D; ++k) pass(k);
+                                                    for (int k = 16; k < D; ++k) read(k);
+#pragma unroll
+                                                    for (int k = 16; k < D; ++k) pass(k);
+                                                }
                                             }
                                         }
                                     }
                                 }
                             }
                         }
-                    }
-                    latency = (t + overhead) - arr;
-                    const uint64_t accs = ballot(latency <= slo) & ballot(best < 1e100);  // a clock that is infinite is never chosen (:590-598)
-                    // ---- whose verdict is final
-                    const uint64_t blockers = win.g & accs;
-                    waits = blockers != 0ull;
-                    uint64_t waiting = ballot(waits);
-                    // requests that wait, are not accepted so far and list several groups: they hold up others too
-                    for (uint64_t open = waiting & multis & ~accs; __builtin_expect(open != 0ull, 0);) {
-                        waits = (win.g & (accs | waiting)) != 0ull;
-                        const uint64_t w2 = ballot(waits);
-                        open = w2 & ~waiting & multis & ~accs;
-                        waiting = w2;
-                    }
-                    // accepted and final: the clocks (:614-619).  Everybody writes the near stages, the others where it does
-                    // not matter.
-                    uint32_t to = in_mask(accs) ? gclk : spare;
-                    pin(to);
-                    to = waits ? spare : to;
-                    pin(to);
-                    auto commit = [&](int k) {
-                        if (k > 0 && (!POW2 || (k & (k - 1)) == 0)) {
-                            to = sm1 >= k ? to : spare;
-                            pin(to);
+                        latency = (t + overhead) - arr;
+                        const uint64_t accs = ballot(latency <= slo) & ballot(best < 1e100);  // a clock that is infinite is never chosen (:590-598)
+                        // ---- whose verdict is final
+                        const uint64_t blockers = win.g & accs;
+                        waits = blockers != 0ull;
+                        uint64_t waiting = ballot(waits);
+                        // requests that wait, are not accepted so far and list several groups: they hold up others too
+                        for (uint64_t open = waiting & multis & ~accs; __builtin_expect(open != 0ull, 0);) {
+                            waits = (win.g & (accs | waiting)) != 0ull;
+                            const uint64_t w2 = ballot(waits);
+                            open = w2 & ~waiting & multis & ~accs;
+                            waiting = w2;
                         }
-                        lds_put<double>(to + (uint32_t)k * 8u, cv[k]);
-                    };
+                        // accepted and final: the clocks (:614-619).  Everybody writes the near stages, the others where it does
+                        // not matter.
+                        uint32_t to = in_mask(accs) ? gclk : spare;
+                        pin(to);
+                        to = waits ? spare : to;
+                        pin(to);
+                        auto commit = [&](int k) {
+                            if (k > 0 && (!POW2 || (k & (k - 1)) == 0)) {
+                                to = sm1 >= k ? to : spare;
+                                pin(to);
+                            }
+                            lds_put<double>(to + (uint32_t)k * 8u, cv[k]);
+                        };
 #pragma unroll
-                    for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) commit(k);
-                    if constexpr (D > NEAR) {
-                        if (to == gclk && sm1 >= NEAR) {
+                        for (int k = 0; k < (D < NEAR ? D : NEAR); ++k) commit(k);
+                        if constexpr (D > NEAR) {
+                            if (to == gclk && sm1 >= NEAR) {
 #pragma unroll
-                            for (int k = NEAR; k < (D < 8 ? D : 8); ++k) commit(k);
-                            if constexpr (D > 8) {
-                                if (sm1 >= 8) {
+                                for (int k = NEAR; k < (D < 8 ? D : 8); ++k) commit(k);
+                                if constexpr (D > 8) {
+                                    if (sm1 >= 8) {
 #pragma unroll
-                                    for (int k = 8; k < D; ++k) commit(k);
+                                        for (int k = 8; k < D; ++k) commit(k);
+                                    }
                                 }
                             }
                         }
+                        wave_order();
+#pragma unroll
+                        for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
+#pragma unroll
+                        for (int k = 0; k < NX; ++k) cx[k] = lds_get<double>(xa[k]);
+                    } while (waits);
+                };
+                if (in_mask(pend)) {
+                    if constexpr (SMAX == 1) {
+                        steps(Int<1>{});
+                    } else if constexpr (SMAX == 4) {
+                        if (deep_a == 0ull) steps(Int<2>{});
+                        else steps(Int<4>{});
+                    } else if constexpr (SMAX == 16) {
+                        if (deep_a != 0ull) steps(Int<16>{});
+                        else if (deep_b != 0ull) steps(Int<8>{});
+                        else steps(Int<4>{});
+                    } else {
+                        if (deep_a == 0ull) steps(Int<16>{});
+                        else steps(Int<32>{});
                     }
-                    wave_order();
-#pragma unroll
-                    for (int k = 0; k < N4; ++k) c[k] = lds_get<double>(ca[k]);
-#pragma unroll
-                    for (int k = 0; k < NX; ++k) cx[k] = lds_get<double>(xa[k]);
-                } while (waits);
-            };
-            if (in_mask(pend)) {
-                if constexpr (SMAX == 1) {
-                    steps(Int<1>{});
-                } else if constexpr (SMAX == 4) {
-                    if (deep_a == 0ull) steps(Int<2>{});
-                    else steps(Int<4>{});
-                } else if constexpr (SMAX == 16) {
-                    if (deep_a != 0ull) steps(Int<16>{});
-                    else if (deep_b != 0ull) steps(Int<8>{});
-                    else steps(Int<4>{});
-                } else {
-                    if (deep_a == 0ull) steps(Int<16>{});
-                    else steps(Int<32>{});
                 }
+            };
+            if constexpr (EXT > 0) {
+                if ((EXT > 1 ? sixteens : eights) != 0ull) block(Int<0>{});
+                else if (EXT > 1 && eights != 0ull) block(Int<(EXT > 1 ? 16 : 8)>{});
+                else if (mores != 0ull) block(Int<8>{});
+                else if (fours != 0ull) block(Int<4>{});
+                else block(Int<2>{});
+            } else {
+                if (fours != 0ull) block(Int<4>{});
+                else block(Int<2>{});
             }
-        };
-        if constexpr (EXT > 0) {
-            if ((EXT > 1 ? sixteens : eights) != 0ull) block(Int<0>{});
-            else if (EXT > 1 && eights != 0ull) block(Int<(EXT > 1 ? 16 : 8)>{});
-            else if (mores != 0ull) block(Int<8>{});
-            else if (fours != 0ull) block(Int<4>{});
-            else block(Int<2>{});
+            wave_order();
+            const uint64_t found = ballot(best < 1e100) & pend, accepted = ballot(latency <= slo) & found;
+            const bool good = in_mask(accepted);
+            const double took = good ? latency : 0.0;
+            n_good += SPANS ? __popcll(accepted) : good ? 1 : 0;
+            if constexpr (OUTPUTS) {
+                if (in_mask(found)) lds_add_u64(first_clock(chosen) + (uint32_t)stages_m1(chosen) * 8u + cnt_rel, good ? 0x100000001ull : 1ull);  // :611, :618
+                if (good) lds_add_u32(mcnt + (uint32_t)m * 4u, 1u);
+            }
+            if constexpr (OUTPUTS)
+                if (want_req && mine && blk + (uint32_t)j < R && (!SPANS || runs.own == 0)) {
+                    fin_out[blk + (uint32_t)j] = good ? t + overhead : arr;
+                    good_out[blk + (uint32_t)j] = good ? 1 : 0;
+                }
+            nrep = load_rep((int)nxt.z);
+            if constexpr (W == 64) arrived(nn);
+            cur = as_req(nxt);
+            nxt = nn;
+            q = nrep;
+            look();
+            if (SPANS && runs.own != 0) run_vals[blk + (uint32_t)j] = OUTPUTS && want_req ? (good ? t + overhead : __builtin_nan("")) : took;
+            else if (accepted != 0ull) lat_sum = ordered_sum<W>(lat_sum, took, accepted);
+        }
+        if constexpr (!SPANS) break;
+        // ---- the end of a run
+        ColdArgs *q = cold_args();
+        int first = 0, first_mark = -1;
+        if (!last) {
+            uint64_t *e = ended(own);
+            for_state([&](int w, uint32_t addr, bool half) { e[w] = get_word(addr, half); });
+            if (lane == 0) {
+                if (own == 0) q->lat_sum[sim] = lat_sum;
+                e[0] = (uint64_t)(uint32_t)n_good;
+                e[q->state_words] = (uint64_t)(blk < R ? blk / 64u : (R + 63u) / 64u);
+                e[q->state_words + 1] = runs.met ? (uint64_t)(uint32_t)runs.in | (uint64_t)(uint32_t)runs.mark << 32 : ~0ull;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            uint32_t before_me = 0;
+            if (lane == 0)
+                before_me = __hip_atomic_fetch_add(q->span_sync + (size_t)sim * (q->spans + 1) + q->spans, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_amdgcn_readfirstlane(before_me) + 1u != (uint32_t)q->spans) return;
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            // All runs have ended: this wavefront follows them from the first on.
+            last = true;
+            for (int k = j; k <= q->spans; k += W) tell(q->span_sync + (size_t)sim * (q->spans + 1) + k, 0u);  // for the next launch
+            n_good = 0;
+            if constexpr (OUTPUTS) {
+                for (int k = j; k < q->nslots; k += W) lds_put<uint64_t>(clk + (uint32_t)k * 8u + cnt_rel, 0ull);
+                for (int m = j; m < M; m += W) lds_put<uint32_t>(mcnt + (uint32_t)m * 4u, 0u);
+            }
         } else {
-            if (fours != 0ull) block(Int<4>{});
-            else block(Int<2>{});
+            if (lane == 0) piece(num_pieces, from / 64u, blk < R ? blk / 64u : (R + 63u) / 64u, 0);
+            num_pieces += 1;
+            if (!runs.met) break;
+            first = runs.in;
+            first_mark = runs.mark;
         }
-        wave_order();
-        const uint64_t found = ballot(best < 1e100) & pend, accepted = ballot(latency <= slo) & found;
-        const bool good = in_mask(accepted);
-        const double took = good ? latency : 0.0;
-        n_good += good ? 1 : 0;
+        // Lane k: where run k ended, which it met and at which mark, and at which mark it is taken over (-1: from its beginning).
+        int ends = 0, met = -1, met_mark = 0, taken_at = first_mark;
+        uint32_t count = 0;
+        if (lane < q->spans) {
+            const uint64_t *e = ended(lane);
+            count = (uint32_t)e[0];
+            ends = (int)(uint32_t)e[q->state_words];
+            met = (int)(uint32_t)e[q->state_words + 1];
+            met_mark = (int)(uint32_t)(e[q->state_words + 1] >> 32);
+        }
+        uint64_t followed = 0;
+        int tail = first;
+        for (;;) {
+            followed |= 1ull << tail;
+            const int to = lane_value(met, tail);
+            if (to < 0) break;
+            if (lane == to) taken_at = lane_value(met_mark, tail);
+            tail = to;
+        }
+        if (!in_mask(followed)) count = 0;
+        else if (taken_at >= 0) count -= (uint32_t)marked(lane, taken_at)[0];
+        for (int d = 1; d < kWave; d *= 2) count += (uint32_t)shfl_xor<kWave>((int)count, d);
+        n_good += __builtin_amdgcn_readfirstlane((int)count);
         if constexpr (OUTPUTS) {
-            if (in_mask(found)) lds_add_u64(first_clock(chosen) + (uint32_t)stages_m1(chosen) * 8u + cnt_rel, good ? 0x100000001ull : 1ull);  // :611, :618
-            if (good) lds_add_u32(mcnt + (uint32_t)m * 4u, 1u);
-        }
-        if constexpr (OUTPUTS)
-            if (want_req && mine && blk + (uint32_t)j < R) {
-                fin_out[blk + (uint32_t)j] = good ? t + overhead : arr;
-                good_out[blk + (uint32_t)j] = good ? 1 : 0;
+            auto counts = [&](int w) -> uint64_t {
+                uint64_t v = 0;
+#pragma unroll 2
+                for (uint64_t left = followed; left != 0ull; left &= left - 1ull) {
+                    const int r = __builtin_ctzll(left), m = lane_value(taken_at, r);
+                    v += ended(r)[w] - (m < 0 ? 0ull : marked(r, m)[w]);
+                }
+                return v;
+            };
+            for (int k = j; k < q->nslots; k += W) {
+                const uint32_t at = clk + (uint32_t)k * 8u + cnt_rel;
+                lds_put<uint64_t>(at, lds_get<uint64_t>(at) + counts(1 + q->nslots + k));
             }
-        nrep = load_rep((int)nxt.z);
-        if constexpr (W == 64) arrived(nn);
-        cur = as_req(nxt);
-        nxt = nn;
-        q = nrep;
-        look();
-        if (accepted != 0ull) lat_sum = ordered_sum<W>(lat_sum, took, accepted);
+            for (int m = j; m < M; m += W) {
+                const uint32_t at = mcnt + (uint32_t)m * 4u;
+                lds_put<uint32_t>(at, lds_get<uint32_t>(at) + (uint32_t)counts(1 + 2 * q->nslots + m));
+            }
+        }
+        if (in_mask(followed))
+            piece(num_pieces + (uint32_t)__popcll(followed & ((1ull << lane) - 1ull)), (uint32_t)(lane * q->span_blocks + (taken_at < 0 ? 0 : span_mark(taken_at))),
+                  (uint32_t)ends, lane);
+        num_pieces += (uint32_t)__popcll(followed);
+        const uint32_t end = (uint32_t)lane_value(ends, tail);
+        if ((uint64_t)end * 64u >= R) break;
+        // The last of them was given up: on from there.
+        const uint32_t resume = end;
+        for (int k = j; k < q->nslots; k += W) lds_put<uint64_t>(clk + (uint32_t)k * 8u, ended(tail)[1 + k]);
+        wave_order();
+        runs.resume(q, resume);
+        from = resume * 64u;
+        run_vals = values_of(q, sim, 0);
     }
 
-    for (int d = 1; d < W; d *= 2) n_good += shfl_xor<W>(n_good, d);
+    if constexpr (!SPANS)
+        for (int d = 1; d < W; d *= 2) n_good += shfl_xor<W>(n_good, d);
     if (!mine) return;
     if (j == 0) {
         a.n_good[row] = n_good;
-        a.lat_sum[row] = lat_sum;
+        if constexpr (SPANS) q_pieces(sim)[8 * kMaxSpans - 1] = num_pieces;
+        else a.lat_sum[row] = lat_sum;
     }
     if constexpr (OUTPUTS) {
         if (a.flags & MMSIM_WANT_MODEL_COUNTS)
@@ -712,12 +1060,100 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave) void sim_window_kernel(cons
     }
 }
 
+#ifdef MMSIM_WINDOW_SPANS
+// What the runs of a simulation come to: a wavefront adds up the latencies of the pieces that are followed, in order; with
+// per-request outputs the others of the workgroup write these.
+__global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const WindowArgs a) {
+    constexpr int N = 16;
+    __shared__ uint32_t pieces[8 * kMaxSpans];
+    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), sim = (int)blockIdx.x;
+    const int worker = wv + (int)blockIdx.y * kSumWaves;  // 0: the sum, others: outputs
+    ColdArgs *q = cold_args();
+    for (int k = (int)threadIdx.x; k < 8 * kMaxSpans; k += (int)blockDim.x) pieces[k] = a.pieces[(size_t)sim * (8 * kMaxSpans) + k];
+    __syncthreads();
+    const int num = __builtin_amdgcn_readfirstlane((int)pieces[8 * kMaxSpans - 1]);
+    const bool want_req = (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
+    const int seed = __builtin_amdgcn_readfirstlane(a.stream_of ? a.stream_of[sim] : sim / a.tiles);
+    const Req *__restrict__ reqs = a.stream_ptr[seed];
+    const uint32_t R = (uint32_t)a.stream_len[seed], blocks = (R + 63u) / 64u;
+    double *fin_out = a.finish + (size_t)sim * (size_t)a.Rmax;
+    uint8_t *good_out = a.good + (size_t)sim * (size_t)a.Rmax;
+    if (num < 2) return;
+    const uint32_t begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)pieces[1]);  // where the first run ends
+    int p = 0;
+    uint32_t p_end = begin;
+    const double *v = nullptr;
+    auto load = [&](uint32_t first, double *x, double *arr) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint32_t at = first + i < blocks ? first + i : blocks - 1;
+            while (at >= p_end && p + 1 < num) {
+                ++p;
+                p_end = (uint32_t)__builtin_amdgcn_readfirstlane((int)pieces[4 * p + 1]);
+                v = values_of(q, sim, __builtin_amdgcn_readfirstlane((int)pieces[4 * p + 2]));
+            }
+            const uint32_t pos = at * (uint32_t)kWave + (uint32_t)lane;
+            x[i] = v[pos];
+            if (want_req) arr[i] = as_req(load_global(reqs + (pos < R ? pos : R - 1u))).t;
+        }
+    };
+    // latencies, 0 of what is not accepted or past the end
+    auto latencies = [&](uint32_t first, double *x, const double *arr) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (want_req) x[i] = x[i] == x[i] ? x[i] - arr[i] : 0.0;
+            if ((first + i) * (uint32_t)kWave + (uint32_t)lane >= R) x[i] = 0.0;
+        }
+    };
+    if (worker > 0) {
+        const int workers = (int)(gridDim.y * (blockDim.x >> 6)) - 1;
+        for (uint32_t at = begin + (uint32_t)(worker - 1) * N; at < blocks; at += (uint32_t)workers * N) {
+            double x[N], arr[N];
+            load(at, x, arr);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const uint32_t pos = (at + i) * (uint32_t)kWave + (uint32_t)lane;
+                if (at + i >= blocks || pos >= R) continue;
+                const bool good = x[i] == x[i];
+                fin_out[pos] = good ? x[i] : arr[i];
+                good_out[pos] = good ? 1 : 0;
+            }
+        }
+        return;
+    }
+    LatencySum sum(a.lat_sum[sim]);
+    double x[N], y[N], arr[N];
+    load(begin, y, arr);
+    for (uint32_t at = begin; at < blocks; at += N) {
+        latencies(at, y, arr);
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i] = y[i];
+        if (at + N < blocks) load(at + N, y, arr);
+        if (!sum.add(x)) {
+#pragma unroll 1
+            for (int i = 0; i < N; ++i) {
+                double w = x[0];
+#pragma unroll
+                for (int k = 1; k < N; ++k) w = i == k ? x[k] : w;
+                sum.add_block(w);
+            }
+        }
+    }
+    if (lane == 0) a.lat_sum[sim] = sum.s;
+}
+#endif
+
 constexpr int W_ = MMSIM_WINDOW_LANES;  // the file is compiled once for each number of requests side by side
+#ifdef MMSIM_WINDOW_SPANS
+constexpr bool kSpans = true;           // and for simulations cut into runs
+#else
+constexpr bool kSpans = false;
+#endif
 
 template <int SMAX, bool OUTPUTS, bool POW2, bool UNIFORM>
 WindowKernel pick_ext(int ext) {
-    if (W_ == 64 && ext > 1) return sim_window_kernel<W_, SMAX, OUTPUTS, W_ == 64 ? 2 : 1, POW2, UNIFORM>;
-    return ext > 0 ? sim_window_kernel<W_, SMAX, OUTPUTS, 1, POW2, UNIFORM> : sim_window_kernel<W_, SMAX, OUTPUTS, 0, POW2, UNIFORM>;
+    if (W_ == 64 && ext > 1) return sim_window_kernel<W_, SMAX, OUTPUTS, W_ == 64 ? 2 : 1, POW2, UNIFORM, kSpans>;
+    return ext > 0 ? sim_window_kernel<W_, SMAX, OUTPUTS, 1, POW2, UNIFORM, kSpans> : sim_window_kernel<W_, SMAX, OUTPUTS, 0, POW2, UNIFORM, kSpans>;
 }
 template <int SMAX, bool POW2, bool UNIFORM>
 WindowKernel pick_out(bool outputs, int ext) {
@@ -731,8 +1167,12 @@ WindowKernel pick_depths(bool outputs, int ext, bool pow2, bool uniform) {
 
 }  // namespace
 
+#ifdef MMSIM_WINDOW_SPANS
+WindowKernel window_sum() { return window_sum_kernel; }
+#endif
+
 template <>
-WindowKernel window_kernel<MMSIM_WINDOW_LANES>(int smax, bool outputs, int ext, bool pow2, bool uniform) {
+WindowKernel window_kernel<MMSIM_WINDOW_LANES, kSpans>(int smax, bool outputs, int ext, bool pow2, bool uniform) {
     switch (smax) {
         case 1: return pick_out<1, true, true>(outputs, ext);  // one stage: its latency is the configuration's
         case 4: return pick_depths<4>(outputs, ext, pow2, uniform);

@@ -31,10 +31,11 @@ bool has_outputs(uint32_t flags) {
 hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_bytes, hipStream_t stream) {
     const int ext = a.has_ext;
     const bool out = has_outputs(a.flags), pow2 = a.pow2_depths != 0, uniform = a.uniform_stages != 0;
-    const WindowKernel kern = a.lanes == 64   ? window_kernel<64>(a.smax_bucket, out, ext, pow2, uniform)
-                              : a.lanes == 32 ? window_kernel<32>(a.smax_bucket, out, ext, pow2, uniform)
-                              : a.lanes == 16 ? window_kernel<16>(a.smax_bucket, out, ext, pow2, uniform)
-                                              : window_kernel<8>(a.smax_bucket, out, ext, pow2, uniform);
+    const WindowKernel kern = a.spans > 1     ? window_kernel<64, true>(a.smax_bucket, out, ext, pow2, uniform)
+                              : a.lanes == 64 ? window_kernel<64, false>(a.smax_bucket, out, ext, pow2, uniform)
+                              : a.lanes == 32 ? window_kernel<32, false>(a.smax_bucket, out, ext, pow2, uniform)
+                              : a.lanes == 16 ? window_kernel<16, false>(a.smax_bucket, out, ext, pow2, uniform)
+                                              : window_kernel<8, false>(a.smax_bucket, out, ext, pow2, uniform);
     if (!kern || waves_per_block < 1 || waves_per_block > kMaxWindowWaves) return hipErrorInvalidValue;
     // The kernel takes LDS addresses as numbers from 0 on: its dynamic LDS starts there as long as nothing static lies
     // before it.
@@ -46,9 +47,14 @@ hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_by
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         if (e != hipSuccess) return e;
     }
-    const int64_t units = (int64_t)a.tiles * a.out_seeds;
+    const int64_t units = (int64_t)a.tiles * a.out_seeds * a.spans;
     hipLaunchKernelGGL(kern, dim3((unsigned)((units + waves_per_block - 1) / waves_per_block)), dim3((unsigned)waves_per_block * kWave),
                        lds_bytes, stream, a);
+    const bool per_request = (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
+    if (a.spans > 1)
+        hipLaunchKernelGGL(window_sum(), dim3((unsigned)(a.tiles * a.out_seeds), per_request && a.tiles * a.out_seeds <= 32 ? 8 : 1),
+                           dim3(kWave * (per_request ? kSumWaves : 1)), 0,
+                           stream, a);
     return hipGetLastError();
 }
 
@@ -59,6 +65,11 @@ struct Shape {
 };
 
 }  // namespace
+
+// Blocks of a span, and what a run may go on behind its span, at least, how many bytes the runs of a launch may take, and how many a context
+// keeps for the next call (a gigabyte costs 0.3 ms to allocate and free).
+constexpr int32_t kLeastSpan = 20, kLeastExt = 48;
+constexpr size_t kMostRunBytes = (size_t)16 << 30, kMostRunsKept = (size_t)2 << 30;
 
 int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
                  const mmsim_placements *p, const int32_t *stream_of, uint32_t flags, const mmsim_options &o, bool events,
@@ -117,6 +128,9 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     const size_t at_ng = in.take((size_t)B), at_cfg = in.take((size_t)B * Gmax), at_off = in.take(sizeof(uint32_t) * ((size_t)B + 1));
     const size_t at_ent = in.take(sizeof(uint32_t) * (size_t)replicas), at_pp = in.take((size_t)C), at_loff = in.take(sizeof(uint16_t) * (size_t)C);
     const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
+    const int64_t blocks = (longest + kWave - 1) / kWave;
+    const bool may_cut = !g_arena && (o.window_lanes > 0 ? o.segment_requests > 0 : blocks >= 6 * kLeastSpan);
+    const size_t at_sync = in.take(may_cut ? sizeof(uint32_t) * (size_t)(sims + std::min<int64_t>(kMaxRuns, sims * kMaxSpans)) : 0);
     HIP_TRY(hipSetDevice(ctx->device));
     std::vector<unsigned char> plain;  // (read until the wait below)
     if (g_arena)
@@ -280,8 +294,58 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     if (stream_of) lanes = kWave;  // (the placements of a wavefront share a stream)
     while (lanes < kWave && !fits(lanes)) lanes *= 2;
     if (!fits(lanes)) return kOther;
-    const int per_wave = kWave / lanes, waves = waves_for(lanes);
+    const int per_wave = kWave / lanes;
     const int64_t tiles = (B + per_wave - 1) / per_wave, units = tiles * out_seeds;
+
+    // ---- runs
+    a.state_words = 1 + shape.nslots + (counts ? shape.nslots + M : 0);
+    Layout runs;
+    size_t at_ends = 0, at_pieces = 0, at_vals = 0;
+    auto cut = [&](int64_t spans) {
+        a.span_blocks = (int32_t)std::max<int64_t>((blocks + spans - 1) / spans, 1);
+        a.spans = (int32_t)std::max<int64_t>((blocks + a.span_blocks - 1) / a.span_blocks, 1);
+        a.ext_blocks = std::max(a.span_blocks / 2, kLeastExt);
+        a.run_cap = (int64_t)kWave * (a.span_blocks + a.ext_blocks);
+        a.true_cap = (int64_t)kWave * blocks;
+        for (a.marks = 0; span_mark(a.marks) < a.span_blocks;) ++a.marks;
+        const size_t n = a.spans > 1 ? (size_t)(units * a.spans) : 0;
+        runs = Layout{};
+        runs.take(8 * n * (size_t)a.marks * (size_t)a.state_words);
+        at_ends = runs.take(8 * n * (size_t)(a.state_words + kEndWords));
+        at_pieces = runs.take(4 * (n > 0 ? (size_t)units : 0) * 8 * kMaxSpans);
+        at_vals = runs.take(n > 0 ? 8 * (size_t)units * (size_t)(a.true_cap + (a.spans - 1) * a.run_cap) : 0);
+    };
+    // sixteen replicas in registers, which leaves two or three wavefronts to a SIMD: sim_window.hip has both sides
+    const bool sixteen = lanes == kWave && shape.rmax > 8 && units <= 8 * cus;
+    int64_t spans = 1;
+    if (lanes == kWave && may_cut) {
+        // As many runs as leave three wavefronts to a SIMD (a few more than that wait for their turn; 2.9 ms of kernel with two
+        // to a SIMD, 700 placements and 108000 requests, are 4.3, and four do not fit with counts: 6.0), of 20 blocks at least (30000 requests of one placement: 16 and 24
+        // are level, 8 a third slower, as runs are given up).  Streams of less than 384 blocks have them while every run has a SIMD to itself: where runs
+        // do not agree the first one shares issue with the others for a span and a half (393 placements, 5844 requests: 2.0 ms not cut, 2.6
+        // with four runs); below 120 blocks there is little to gain (5757 requests 155 us, with a second kernel 190).
+        const int64_t per_cu = blocks < 384 ? 4 : sixteen || a.smax_bucket == 32 ? 8 : 12;
+        spans = std::min((per_cu * cus + cus / 2) / units, blocks / kLeastSpan);
+        if (o.window_lanes > 0) spans = blocks / std::max<int64_t>(8, o.segment_requests / kWave);
+    }
+    cut(std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / units))));
+    DevBuf<uint8_t> own_runs;  // of a batch that is kept; a call that runs its batch once borrows the context's
+    DevBuf<uint8_t> &run_memory = events ? own_runs : ctx->runs;
+    if (a.spans > 1 && (runs.used > kMostRunBytes || (run_memory.n < runs.used && run_memory.alloc(runs.used) != hipSuccess))) {
+        (void)hipGetLastError();
+        run_memory.release();
+        cut(1);
+    }
+    spans = a.spans;
+    if (spans > 1) {
+        a.mark_state = reinterpret_cast<uint64_t *>(run_memory.p);
+        a.end_state = reinterpret_cast<uint64_t *>(run_memory.p + at_ends);
+        a.pieces = reinterpret_cast<uint32_t *>(run_memory.p + at_pieces);
+        a.run_vals = reinterpret_cast<double *>(run_memory.p + at_vals);
+    }
+    const int64_t wave_units = units * spans;
+    int waves = spans > 1 ? (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (wave_units + cus - 1) / cus)) : waves_for(lanes);
+    while (spans > 1 && waves > 1 && lat_lds + wave_lds(lanes) * (size_t)waves > lds) --waves;
 
     std::unique_ptr<mmsim_batch> b(new (std::nothrow) mmsim_batch);
     if (!b) return fail(MMSIM_E_NOMEM, "host allocation failed");
@@ -296,7 +360,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     b->paired = stream_of != nullptr;
     b->out_seeds = out_seeds;
     b->tiles = (int32_t)tiles;
-    b->waves = (int32_t)units;
+    b->waves = (int32_t)wave_units;
     b->smax_bucket = a.smax_bucket;
     b->rmax_all = shape.rmax;
     b->nslots = shape.nslots;
@@ -321,6 +385,8 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         reinterpret_cast<uint16_t *>(host + at_loff)[c] = (uint16_t)cl.off[c];
     }
     std::memcpy(host + at_lat, cl.lat.data(), sizeof(float) * cl.lat.size());
+
+    std::memset(host + at_sync, 0, spans > 1 ? sizeof(uint32_t) * (size_t)(units * (spans + 1)) : 0);
 
     // ---- outputs: one buffer, laid out as the caller's arrays
     Layout res;
@@ -348,7 +414,8 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         HIP_TRY(hipStreamSynchronize(ctx->stream));  // a batch that is kept: the staging memory serves other calls before its run
         if (!g_arena) ctx->staging.trim();
     }
-    const uint8_t *d = b->win_in.p;
+    uint8_t *d = b->win_in.p;
+    a.span_sync = reinterpret_cast<uint32_t *>(d + at_sync);
     a.stream_ptr = reinterpret_cast<const Req *const *>(d + at_ptr);
     a.stream_len = reinterpret_cast<const int64_t *>(d + at_len);
     a.stream_of = stream_of ? reinterpret_cast<const int32_t *>(d + at_so) : nullptr;
@@ -370,8 +437,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     a.lanes = lanes;
     a.pow2_depths = shape.pow2 ? 1 : 0;
     a.uniform_stages = uniform ? 1 : 0;
-    // (2: sixteen replicas in registers, which leaves two or three wavefronts to a SIMD: sim_window.hip has both sides)
-    a.has_ext = shape.ext_cap > 0 ? (lanes == kWave && shape.rmax > 8 && units <= 8 * cus ? 2 : 1) : 0;
+    a.has_ext = shape.ext_cap > 0 ? (sixteen ? 2 : 1) : 0;
     a.lat_lds_bytes = (int32_t)lat_lds;
     a.place_bytes = (int32_t)place;
     a.Rmax = b->Rmax;
@@ -386,6 +452,11 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     a.finish = reinterpret_cast<double *>(r + b->win_finish);
     a.good = r + b->win_good;
     b->wargs = a;
+    if (events && spans > 1) {
+        b->win_runs.p = own_runs.p;
+        b->win_runs.n = own_runs.n;
+        own_runs.owned = false;
+    }
     unless_made.staging = nullptr;
     *out = b.release();
     return MMSIM_OK;
@@ -394,7 +465,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
 std::string sim_window_kernel_name(const WindowArgs &a) {
     auto tf = [](bool v) { return v ? ", true" : ", false"; };
     return "sim_window_kernel<" + std::to_string(a.lanes) + ", " + std::to_string(a.smax_bucket) + tf(has_outputs(a.flags)) + ", " + std::to_string(a.has_ext) +
-           tf(a.pow2_depths != 0) + tf(a.uniform_stages != 0) + ">";
+           tf(a.pow2_depths != 0) + tf(a.uniform_stages != 0) + (a.spans > 1 ? ", true>" : ">");
 }
 
 int run_window(mmsim_batch *b) {
@@ -443,6 +514,7 @@ int fetch_window(mmsim_batch *b, mmsim_result *out) {
         std::memcpy(out->group_num_good, host + b->win_group + sizeof(int32_t) * L * G, sizeof(int32_t) * L * G);
     }
     if (!b->in_scratch) stage.trim();
+    if (b->ctx->runs.n > kMostRunsKept) b->ctx->runs.release();
     return MMSIM_OK;
 }
 

@@ -1,0 +1,78 @@
+"""Simulations cut into runs that are simulated at the same time (sim_window.hip) against the CPU oracle, bit for bit: streams
+with pauses, in which neighbouring runs come to agree, streams that overload the groups all along, where none do and the first
+run goes through the whole stream, and streams of both, where runs are given up and taken up again; streams that end inside a
+span, at its edge and before it; all outputs."""
+import numpy as np
+import pytest
+
+from mms_amd import _lib, engine as E
+from helpers import assert_batch_matches, oracle_batch
+from test_gpu_window import COUNTS, _problem, _stream
+
+pytestmark = pytest.mark.gpu
+
+
+def _with_pauses(seed, R, M, load, every, pause=4.0, quiet_until=1.0):
+    """Pauses once in ``every`` requests, in the first ``quiet_until`` of the stream."""
+    st = _stream(seed, R, M, load)
+    rng = np.random.default_rng(seed + 1)
+    gaps = np.diff(st.tstamps, prepend=0.0)
+    gaps[(rng.random(R) < 1.0 / every) & (np.arange(R) < quiet_until * R)] += pause
+    st.tstamps = np.cumsum(gaps)
+    st.slos[np.isinf(st.slos) & (rng.random(R) < 0.97)] = 0.7      # (few: a clock that never comes down again never agrees)
+    return st
+
+
+@pytest.mark.parametrize("depths,uniform,groups,hosts,M", [((1,), True, 6, 4, 9), ((1,), True, 40, 5, 5), ((1, 2, 4), True, 5, 4, 9),
+                                                           ((1, 3, 4), False, 9, 5, 5), ((1, 2, 4, 8, 16), True, 7, 4, 9), ((8, 32), True, 6, 4, 9)])
+@pytest.mark.parametrize("span", [512, 1024])
+def test_runs_of_one_simulation(depths, uniform, groups, hosts, M, span):
+    eng = E.Engine.default()
+    streams = [_with_pauses(1, 7 * span + 333, M, 0.6, 150), _with_pauses(2, 8 * span, M, 4.0, 10 ** 9), _with_pauses(3, 7 * span + 1, M, 2.0, 200, quiet_until=0.6),
+               _with_pauses(4, 3 * span, M, 1.0, 100), _with_pauses(5, 1, M, 1.0, 100), _with_pauses(6, 0, M, 1.0, 100)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    for B, flags in ((1, COUNTS | _lib.WANT_PER_REQUEST), (5, COUNTS), (40, 0)):
+        profiles, sols = _problem(B + sum(depths), depths, uniform, M, groups, B, hosts)
+        table = E.LatencyTable(profiles, [1])
+        packed = E.pack_placements(sols, table)
+        batch = E.Batch(eng, dws, table, packed, flags, options=dict(window_lanes=64, segment_requests=span))
+        assert batch.kernel_name().count(",") == 6            # (the last one: cut into runs)
+        for _ in range(3):                                 # further runs start from scratch again
+            batch.run()
+            batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k, st in enumerate(streams):
+            ref = oracle_batch(st, table, packed, want_per_request=bool(flags & _lib.WANT_PER_REQUEST))
+            if flags & _lib.WANT_PER_REQUEST:
+                R = len(st.tstamps)
+                assert np.array_equal(out["good"][k][:, :R], ref["good"]) and np.array_equal(out["finish"][k][:, :R], ref["finish"])
+            assert_batch_matches(out, ref, k, packed[0], where=f"B={B}, stream {k}")
+    for dw in dws:
+        dw.close()
+
+
+def test_where_simulations_are_cut_by_themselves():
+    """Few simulations of long streams, plain and paired; a latency sum that doubles many times, with half-way roundings."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(3, (1, 2, 4), True, 9, 6, 12, 4)
+    table = E.LatencyTable(profiles, [1])
+    packed = E.pack_placements(sols, table)
+    streams = [_with_pauses(11, 40000, 9, 0.8, 120), _with_pauses(12, 21000, 9, 0.8, 10 ** 9)]
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, 9) for s in streams]
+    refs = [oracle_batch(s, table, packed) for s in streams]
+    for flags in (0, COUNTS):
+        batch = E.Batch(eng, dws, table, packed, flags)
+        assert batch.kernel_name().count(",") == 6            # (the last one: cut into runs)
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k in range(2):
+            assert_batch_matches(out, refs[k], k, packed[0], where=f"flags {flags}, stream {k}")
+    of = np.arange(len(sols)) % 2
+    got = E.eval_pairs(eng, dws, table, packed, of, COUNTS)
+    for key in ("n_good", "latency_sum", "model_num_good", "group_num_requests", "group_num_good"):
+        assert np.array_equal(got[key], np.where((of == 0).reshape((-1,) + (1,) * (refs[0][key].ndim - 1)), refs[0][key], refs[1][key])), key
+    for dw in dws:
+        dw.close()
