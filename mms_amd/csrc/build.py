@@ -24,6 +24,7 @@ UNITS = {"mmsim_api": ("mmsim_api.hip", []), "window_batch": ("window_batch.hip"
          "sim_window_runs": ("sim_window.hip", ["-DMMSIM_WINDOW_LANES=64", "-DMMSIM_WINDOW_SPANS"]),
          **{f"sim_window_{w}": ("sim_window.hip", [f"-DMMSIM_WINDOW_LANES={w}"]) for w in (64, 32, 16, 8)},
          "sim_mixed": ("sim_mixed.hip", []), "sim_lanes": ("sim_lanes.hip", []), "sim_batching": ("sim_batching.hip", []), "sim_batching_solo": ("sim_batching_solo.hip", []),
+         "sim_batching_runs": ("sim_batching_solo.hip", ["-DMMSIM_SOLO_RUNS"]),
          "sim_scalar": ("sim_scalar.hip", []),
          "stats": ("stats.hip", [])}
 

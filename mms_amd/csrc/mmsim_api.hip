@@ -1092,16 +1092,30 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
     //      workgroup (up to one per SIMD) come first: the loops are bound by latency, so a CU with an
     //      idle SIMD loses more than one that reads these tables through the caches.
     size_t batching_lat_lds = 0;
-    int batching_g2m_lds = 0;
+    int batching_g2m_lds = 0, runs_of = 1;  // runs_of: a simulation's
+    int64_t span_blocks = 1;
     if (batching) {
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
         const size_t g2m_b = solo ? (solo_masks ? 0 : ((size_t)members_max * 2 + 15) & ~(size_t)15) : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
         const size_t cap = (size_t)ctx->max_lds;
-        // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
-        const int tiles_here = std::max(1, b->tiles);
         const int64_t cus = std::max(1, ctx->prop.multiProcessorCount);
+        // A wavefront for each simulation, on few of them: cut into runs that are simulated at the same time, three wavefronts to a SIMD.
+        if (solo && solo_masks && !(flags & MMSIM_WANT_PER_REQUEST) && !g_arena) {
+            int64_t longest = 0;
+            for (int s = 0; s < n_seeds; ++s) longest = std::max(longest, wls[s]->R);
+            const int64_t blocks = (longest + kWave - 1) / kWave;
+            const int64_t spans = o.segment_requests > 0 ? blocks / std::max<int64_t>(8, o.segment_requests / kWave)
+                                  : blocks >= 6 * kLeastSpan ? std::min((12 * cus + cus / 2) / b->waves, blocks / kLeastSpan)
+                                                             : 1;
+            runs_of = (int)std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / b->waves)));
+            span_blocks = std::max<int64_t>((blocks + runs_of - 1) / runs_of, 1);
+            runs_of = (int)std::max<int64_t>((blocks + span_blocks - 1) / span_blocks, 1);
+        }
+        const int64_t wavefronts = (int64_t)b->waves * runs_of;
+        // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
+        const int tiles_here = (int)(runs_of > 1 ? wavefronts : std::max(1, b->tiles));
         const int most_shares = solo ? kSoloWavesPerCu / kMaxWavesPerBlockBatching : 2;  // workgroups to a CU
-        const int wanted = (int)std::min<int64_t>(most_shares * kMaxWavesPerBlockBatching, std::max<int64_t>(1, ((int64_t)b->waves + cus - 1) / cus));
+        const int wanted = (int)std::min<int64_t>(most_shares * kMaxWavesPerBlockBatching, std::max<int64_t>(1, (wavefronts + cus - 1) / cus));
         // Fewer event slots (down to G+8) are accepted when that puts more wavefronts on a CU.
         const int wpb_max = kMaxWavesPerBlockBatching;
         const int heap_try_min = solo ? heap_cap : std::min(heap_cap, std::max(heap_min, (Gmax + 8 + 7) & ~7));  // (its event slots are registers)
@@ -1132,7 +1146,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
         wave_bytes = solo ? batching_solo_bytes(nslots, M) : batching_bytes_for(blanes, heap_cap);
         wpb = std::max(1, best_w);
         if (batching_g2m_lds) wave_bytes += g2m_b;
-        b->waves_per_block = std::min(wpb, b->tiles);
+        b->waves_per_block = std::min(wpb, tiles_here);
         b->wave_bytes = wave_bytes;
         b->lds_bytes = batching_lat_lds + (size_t)b->waves_per_block * wave_bytes;
     }
@@ -1349,6 +1363,21 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
         q.lane_stride = blanes;
         q.tile_sims = tile_sims;
         q.solo = !solo ? 0 : solo_masks ? 1 : 2;
+        q.spans = runs_of;
+        if (runs_of > 1) {
+            const size_t L = (size_t)b->waves, n = L * (size_t)runs_of;
+            q.span_blocks = (int32_t)span_blocks;
+            q.ext_blocks = std::max(q.span_blocks / 2, kLeastExt);
+            for (q.marks = 0; span_mark(q.marks) < q.span_blocks;) ++q.marks;
+            q.state_words = 2 + nslots + M + 4 * kWave + M;
+            const size_t marks = 8 * n * (size_t)q.marks * (size_t)q.state_words, ends = 8 * n * (size_t)(q.state_words + kEndWords),
+                         sync = 4 * L * (size_t)(runs_of + 1);
+            HIP_TRY(b->run_memory.alloc(marks + ends + sync));
+            HIP_TRY(hipMemsetAsync(b->run_memory.p + marks + ends, 0, sync, st));
+            q.mark_state = reinterpret_cast<uint64_t *>(b->run_memory.p);
+            q.end_state = reinterpret_cast<uint64_t *>(b->run_memory.p + marks);
+            q.span_sync = reinterpret_cast<uint32_t *>(b->run_memory.p + marks + ends);
+        }
         q.uniform_stages = uniform_stages ? 1 : 0;
         q.tile_seed = b->tile_seed.p;
         q.paired = b->paired ? 1 : 0;

@@ -345,6 +345,7 @@ struct mmsim_batch {
     bool window = false;
     WindowArgs wargs{};
     DevBuf<uint8_t> win_in, win_out, win_runs;
+    DevBuf<uint8_t> run_memory;  // batching simulator: of simulations cut into runs
     std::vector<std::shared_ptr<DevBuf<Req>>> win_streams;
     size_t win_lat_sum = 0, win_model = 0, win_group = 0, win_finish = 0, win_good = 0;  // offsets in win_out (n_good: 0)
 

@@ -215,6 +215,10 @@ struct BatchingArgs {
     int64_t Rmax;
     double fixed_overhead;
     uint32_t flags;
+    // simulations cut into runs (solo), as in WindowArgs
+    int32_t spans, span_blocks, ext_blocks, marks, state_words;
+    uint32_t *span_sync;
+    uint64_t *mark_state, *end_state;
     // outputs
     int32_t *n_good;             // [n_seeds][tiles*row]
     double *lat_sum;             // [n_seeds][tiles*row]
@@ -273,6 +277,7 @@ constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
 constexpr int kEndWords = 2;        // of end_state: end block, link
 constexpr int kSumWaves = 4;        // wavefronts of a workgroup that puts a simulation's runs together, if per-request outputs are wanted
 constexpr int kMaxSpans = 64;       // most runs of a simulation (their records are a lane's each)
+constexpr int32_t kLeastSpan = 20, kLeastExt = 48;  // blocks of a span, and what a run may go on behind its span, at least
 constexpr int kMaxRuns = 4096;      // most runs of a launch, if its simulations are cut
 // Where the k-th mark of a span is, in blocks from its beginning: 4, 8, 12, 16, 24, 32, 48, 64, 96, ...
 __host__ __device__ constexpr int span_mark(int k) { return k < 4 ? 4 * (k + 1) : ((k & 1) != 0 ? 32 : 24) << ((k - 4) / 2); }
@@ -345,7 +350,12 @@ constexpr size_t batching_solo_bytes(int nslots, int M) {  // LDS of a wavefront
     return (size_t)((nslots + 4) & ~1) * 8 + (size_t)M * (M <= kSoloRowsInLds ? 32 : 16);
 }
 constexpr int kSoloWavesPerCu = 20;  // that share a CU: five to a SIMD, by their registers
+template <bool RUNS>
 hipError_t launch_sim_batching_solo(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream);
+template <>
+hipError_t launch_sim_batching_solo<false>(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream);
+template <>
+hipError_t launch_sim_batching_solo<true>(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream);
 std::string sim_batching_solo_kernel_name(const BatchingArgs &args);
 hipError_t launch_sim_batching(const BatchingArgs &args, int waves_per_block, size_t lds_bytes, hipStream_t stream,
                                std::string *err);

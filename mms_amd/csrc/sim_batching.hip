@@ -1039,7 +1039,7 @@ hipError_t launch_sim_batching(const BatchingArgs &args, int wpb, size_t lds_byt
     if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.NB > kMaxLatencyColumns || (args.heap_cap & 7) != 0) {
         e = hipErrorInvalidValue;
     } else if (args.solo) {
-        e = launch_sim_batching_solo(args, wpb, lds_bytes, stream);
+        e = args.spans > 1 ? launch_sim_batching_solo<true>(args, wpb, lds_bytes, stream) : launch_sim_batching_solo<false>(args, wpb, lds_bytes, stream);
     } else {
         const bool ll = args.lat_lds_bytes > 0, gl = args.g2m_in_lds != 0;
         const bool oct = args.lane_stride == 8, unif = args.uniform_stages != 0;

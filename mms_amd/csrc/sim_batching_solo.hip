@@ -38,10 +38,16 @@
 // placement with all outputs 18.0 -> 14.5 ms).  Tried, no gain: the next sixteen entries of every queue in LDS, fetched when the batch before
 // them was run (14.8 -> 15.0 ms: the wait for entries of a queue is not what a lone wavefront's time goes to).
 //
+// Few simulations of long streams without per-request outputs are cut into runs (SPANS), as sim_window.hip cuts its own: a run starts a span
+// with idle clocks and empty queues, and ends where its clocks, the queues of the models that some group lists and its idle events equal those that
+// the next run had there.  30000 requests, 128 placements, runs agree after 192 requests in the median, 704 at most of 24: 24 runs
+// each, calls 14.3 -> 2.03 ms; 105000 requests of 10 models on 30 single devices, 309 placements, of which some never agree, 126 -> 101 ms.
+//
 // LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
 // its head and of its next arrival in the stream's lists, rank of the head, requests accepted; up to 128 models also their replicas; without
 // masks the groups' lists of models, if they fit.
 #include "mmsim_internal.h"
+#include "runs.h"
 
 namespace mmsim {
 namespace {
@@ -155,24 +161,33 @@ __device__ __forceinline__ double wave_min(double v) {
 // says what).  MW: 64-bit words that hold a bit per model; 0: any number of models, and groups that list them in any order.
 // Then who waits is read from the queues, and the group's list is gone through 64 entries at a time (LDS if it fits): the first of
 // the earliest heads by its place in the list.
-template <bool LATLDS, bool UNIF, bool OUTPUTS, int MW>
+// SPANS: a simulation is cut into a.spans runs (MW not 0, no per-request outputs).
+template <bool LATLDS, bool UNIF, bool OUTPUTS, int MW, bool SPANS>
 __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching_solo_kernel(const BatchingArgs a) {
     const int lane = (int)(threadIdx.x & 63), oct = lane >> 3;
     const int wv = uni((int)(threadIdx.x >> 6));
     const unsigned grid_seeds = a.paired ? 1u : (unsigned)a.n_seeds;
-    const int tile = (int)(blockIdx.x / grid_seeds) * (int)(blockDim.x >> 6) + wv;
+    int tile = (int)(blockIdx.x / grid_seeds) * (int)(blockDim.x >> 6) + wv, seed_row = (int)(blockIdx.x % grid_seeds);
+    int own = 0;  // the run
+    if constexpr (SPANS) {  // (first runs first)
+        const int at = (int)blockIdx.x * (int)(blockDim.x >> 6) + wv, sims = a.tiles * (int)grid_seeds;
+        own = uni(at / sims);
+        const int sim = at - own * sims;
+        seed_row = uni(sim / a.tiles);
+        tile = sim - seed_row * a.tiles;
+    }
     const int M = a.M, NB = a.NB;
     if (LATLDS) {
         const int n = M * a.lat_row * NB;
         for (int i = (int)threadIdx.x; i < n; i += (int)blockDim.x) lds_put<float>((uint32_t)i * 4u, a.lat[i]);
         __syncthreads();
     }
-    if (tile >= a.tiles) return;
+    if (tile >= a.tiles || (SPANS && own >= a.spans)) return;
     // paired batches: the tile's own stream; otherwise every tile on every stream
-    const int seed = a.paired ? a.tile_seed[tile] : (int)(blockIdx.x % grid_seeds);
+    const int seed = a.paired ? a.tile_seed[tile] : seed_row;
     const bool want_model = OUTPUTS && (a.flags & MMSIM_WANT_MODEL_COUNTS) != 0;
     const bool want_group = OUTPUTS && (a.flags & MMSIM_WANT_GROUP_COUNTS) != 0;
-    const bool want_req = OUTPUTS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
+    const bool want_req = OUTPUTS && !SPANS && (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
     const uint32_t clk = (uint32_t)a.lat_lds_bytes + (uint32_t)wv * (uint32_t)a.wave_lds_bytes;
     const uint32_t queues = clk + (uint32_t)((a.nslots + 4) & ~1) * 8u;  // [M] {requests accepted, head, behind the last arrival so far: places in the stream's lists; rank of the head}
 
@@ -193,8 +208,17 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
 
     // ---- state
     for (int s = lane; s < a.nslots; s += kWave) lds_put<double>(clk + (uint32_t)s * 8u, 0.0);
-    for (int m = lane; m < M; m += kWave)
-        lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{0u, (uint32_t)(mo[m] - mo[0]), (uint32_t)(mo[m] - mo[0]), (uint32_t)a.mq[mo[m]].rank});
+    const int64_t start = SPANS ? (int64_t)own * a.span_blocks * kWave : 0;
+    for (int m = lane; m < M; m += kWave) {
+        uint32_t at = (uint32_t)(mo[m] - mo[0]);
+        if (SPANS && own > 0)  // the model's first arrival in the span
+            for (uint32_t end = (uint32_t)(mo[m + 1] - mo[0]); at < end;) {
+                const uint32_t mid = (at + end) >> 1;
+                if (mq[mid].idx < start) at = mid + 1;
+                else end = mid;
+            }
+        lds_put<u32x4>(queues + (uint32_t)m * 16u, u32x4{0u, at, at, (uint32_t)mq[at].rank});
+    }
     if constexpr (ROWSLDS)
         for (int x = lane; x < M * 8; x += kWave) lds_put<uint16_t>(rows16 + (uint32_t)x * 2u, (uint16_t)((rows[x] & 0x1FFFu) | (rows[x] >> 16 & 0x8000u)));
     constexpr int W = MW != 0 ? MW : 1;
@@ -502,109 +526,297 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         return rows[at];
     };
     auto time_of = [&](const Req &r, int l) -> double { return __hiloint2double(__shfl(__double2hiint(r.t), l), __shfl(__double2loint(r.t), l)); };
-    Req block = fetch_block(0), block_next = fetch_block(kWave);
+    Req block, block_next;
     // of the next window, and the models of the one after it
-    int m1 = __shfl(block.m, oct), m2 = __shfl(block.m, 8 + oct);
-    uint32_t d1 = row_word(m1);
-    double t1 = time_of(block, oct);
-    for (int64_t w0 = 0; w0 < R && !dead; w0 += 8) {
-        const int from = (int)(w0 & 63) + oct;  // the lane that holds this octet's request
-        const int n = R - w0 < 8 ? (int)(R - w0) : 8;
-        const int m = m1;
-        const uint32_t dj = d1;
-        const double t = t1;
-        last = clk + desc_last_slot(dj) * 8u;
-        c_last = lds_get<double>(last);
-        c_first = lds_get<double>(last - desc_stages_m1(dj) * 8u);
-        if ((w0 & 63) == 56) {
-            block = block_next;
-            block_next = fetch_block(w0 + 8 + kWave);
+    int m1, m2;
+    uint32_t d1;
+    double t1;
+    auto start_at = [&](int64_t w) {  // (a multiple of 64)
+        block = fetch_block(w);
+        block_next = fetch_block(w + kWave);
+        m1 = __shfl(block.m, oct);
+        m2 = __shfl(block.m, 8 + oct);
+        d1 = row_word(m1);
+        t1 = time_of(block, oct);
+    };
+
+    // ---- SPANS: this wavefront's run and the simulation's others.  What they agree in: clocks, queues of the models that some group lists
+    // (what no group turns to waits for ever), and the idle events, in whichever slots.
+    typedef const __attribute__((address_space(4))) BatchingArgs ColdArgs;
+    Runs runs;
+    uint64_t hosted_models[W] = {};
+    uint64_t peeked = 0;
+    if constexpr (SPANS) {
+        runs.start(cold_args<BatchingArgs>(), own);
+        for (int g = 0; g < a.Gmax; ++g)
+#pragma unroll
+            for (int i = 0; i < W; ++i) hosted_models[i] |= lane_value(members[i], g);
+    }
+    // A state, 64-bit words: accepted requests, event slots in use, clocks, queues {head, behind the last arrival}; a lane each: time and
+    // group of the events, latency sums; with counts groups {requests, accepted} (lanes) and models
+    auto marked = [&](int r, int i) {
+        ColdArgs *q = cold_args<BatchingArgs>();
+        return q->mark_state + (((size_t)wave * q->spans + r) * q->marks + i) * (size_t)q->state_words;
+    };
+    auto ended = [&](int r) {
+        ColdArgs *q = cold_args<BatchingArgs>();
+        return q->end_state + ((size_t)wave * q->spans + r) * (size_t)(q->state_words + kEndWords);
+    };
+    auto published = [&](int r) {
+        ColdArgs *q = cold_args<BatchingArgs>();
+        return q->span_sync + (size_t)wave * (q->spans + 1) + r;
+    };
+    const int at_queues = 2 + a.nslots, at_lanes = at_queues + M;  // where the queues and the lanes' words begin
+    auto save = [&](uint64_t *st) {
+        if (lane == 0) {
+            tell(st, (uint64_t)(uint32_t)n_good);
+            tell(st + 1, used);
         }
-        m1 = m2;
-        d1 = row_word(m1);  // (past the end of the stream: -1)
-        t1 = time_of(block, (from + 8) & 63);
-        m2 = __shfl((w0 & 63) == 48 ? block_next.m : block.m, (from + 16) & 63);
-        const bool valid = ((int32_t)dj >= 0) & (m >= 0);
-        const uint64_t valids = ballot((int32_t)dj >= 0) & ballot(m >= 0), known = ballot(m >= 0);
-        const uint64_t hosted = valids & kFirstOfOctets, longer = valids >> 7 & kFirstOfOctets;  // longer: the list may go on
-        here = ~0ull >> (64 - 8 * n);
-        int cur = 0;             // arrivals before this one are settled
-        uint64_t unseen = ~0ull;  // arrivals whose due events have not been seen to
-        while (cur < n) {
-            uint64_t due = ballot(next_due <= t) & unseen;
-            if ((due >> (cur * 8) & 1ull) != 0ull) {  // events first (:739-744)
-                due_events(lane_value(t, cur * 8));
-                unseen = ~0xFFull << (cur * 8);
-                due = ballot(next_due <= t) & unseen;
+        for (int k = lane; k < a.nslots; k += kWave) tell(st + 2 + k, lds_get<uint64_t>(clk + (uint32_t)k * 8u));
+        for (int m = lane; m < M; m += kWave) {
+            const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
+            tell(st + at_queues + m, (uint64_t)queue.z << 32 | queue.y);
+            if (OUTPUTS) tell(st + at_lanes + 4 * kWave + m, (uint64_t)queue.x);
+        }
+        uint64_t *mine = st + at_lanes + lane;
+        tell(mine, (uint64_t)__double_as_longlong(ev_t));
+        tell(mine + kWave, (uint64_t)ev_d);
+        tell(mine + 2 * kWave, (uint64_t)__double_as_longlong(lat_sum));
+        if (OUTPUTS) tell(mine + 3 * kWave, (uint64_t)(uint32_t)good_of_group << 32 | (uint32_t)requests_of_group);
+    };
+    auto agree = [&](const uint64_t *st) -> bool {
+        const uint64_t their_used = (uint64_t)uni((uint32_t)(told(st + 1) >> 32)) << 32 | uni((uint32_t)told(st + 1));
+        if (__builtin_popcountll(their_used) != __builtin_popcountll(used)) return false;
+        bool same = true;
+        for (int k = lane; k < a.nslots; k += kWave) same = same && told(st + 2 + k) == lds_get<uint64_t>(clk + (uint32_t)k * 8u);
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            const int m = 64 * i + lane;
+            if (in_mask(hosted_models[i]) && m < M) {
+                const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
+                same = same && told(st + at_queues + m) == ((uint64_t)queue.z << 32 | queue.y);
             }
-            const double mn = oct_min(valid ? c_last : inf);
-            const uint64_t found = ballot(mn < 1e100);
-            // the first listed of those with the smallest last-stage clock
-            const uint64_t selected = first_of_octets(ballot(c_last == mn) & valids);
-            const uint64_t idle = selected & found & ballot(t >= c_first), special = hosted & (~found | longer);
-            const uint64_t left = here & ~0ull << (cur * 8), happens = left & (due | idle | special);
-            // those before the first at which something happens join their queues, and that one unless it has events first
-            uint64_t joining = left;
-            int f = n;
-            if (happens != 0ull) {
-                f = first_of(happens) >> 3;
-                joining &= (((due >> (f * 8) & 1ull) != 0ull ? 1ull : 0x100ull) << (f * 8)) - 1ull;
+        }
+        if (ballot(!same) != 0ull) return false;
+        const double their_t = __longlong_as_double((long long)told(st + at_lanes + lane));
+        const uint32_t their_d = (uint32_t)told(st + at_lanes + kWave + lane);
+        for (uint64_t left = used; left != 0ull; left &= left - 1) {  // as often there as here
+            const double t = lane_value(ev_t, first_of(left));
+            const uint32_t d = lane_value(ev_d, first_of(left));
+            if (__builtin_popcountll(ballot(ev_t == t) & ballot(ev_d == d) & used) != __builtin_popcountll(ballot(their_t == t) & ballot(their_d == d) & their_used))
+                return false;
+        }
+        return true;
+    };
+    // Something happens before block `at`: a mark of this run, one of a later run or the block ahead of it, the end of the run (true).
+    auto event = [&](uint32_t at) -> bool {
+        ColdArgs *q = cold_args<BatchingArgs>();
+        if (at >= runs.limit(q)) return true;
+        uint64_t *st = marked(runs.in, runs.mark);
+        if (runs.in == runs.own) {
+            save(st);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (stores of device scope have been carried out then)
+            if (lane == 0) tell(published(runs.in), (uint32_t)runs.mark + 1u);
+        } else if (!runs.looked) {
+            if (uni(told(published(runs.in))) > (uint32_t)runs.mark) {
+                asm volatile("" ::: "memory");
+                peeked = told(st + 2 + (lane < a.nslots ? lane : 0));
+                runs.looked = true;
+                runs.next = at + 1u;
+                return false;
             }
-            if (in_mask(joining & known & kFirstOfOctets))
-                __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u + 8u), 1u,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            if (want_req && in_mask(joining & kFirstOfOctets & ~hosted)) {
-                fin_out[w0 + oct] = t;
-                good_out[w0 + oct] = 0;
-            }
-            wave_order();
-            add_waiting(m, joining & known);
-            cur = f;
-            if (happens == 0ull) break;
-            const int fl = f * 8;
-            if ((due >> fl & 1ull) != 0ull) continue;
-            // its group turns to the arrival if it is idle (:746-778)
-            cur = f + 1;
-            const double tf = lane_value(t, fl);
-            const int mf = lane_value(m, fl);
-            uint32_t dsel = lane_value(dj, first_of(selected >> fl) + fl);
-            if (ROWSLDS) dsel = lane_value(group, first_of(ballot((group & 0x1FFFu) == (dsel & 0x1FFFu)) & groups));
-            bool ready = (idle >> fl & 0xFFull) != 0ull;
-            if (rarely((special >> fl & 1ull) != 0ull)) {
-                double best = lane_value(mn, fl);
-                if (!(best < 1e100)) {
-                    best = 1e100;
-                    dsel = kEmpty;
-                    ready = false;
-                }
-                if ((longer >> fl & 1ull) != 0ull)
-                    for (int x = 0; x < a.rep_extra; ++x) {
-                        const uint32_t g = more_replicas[(size_t)mf * a.rep_extra + x];
-                        if (g == (uint32_t)a.Gmax) break;
-                        const uint32_t d2 = ginfo[g];
-                        const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
-                        if (c2 < best) {
-                            best = c2;
-                            dsel = d2;
-                            ready = tf >= uni(lds_get<double>(clk + (desc_last_slot(d2) - desc_stages_m1(d2)) * 8u));
-                        }
-                    }
-                dsel = uni(dsel);
-                if (rarely(dsel == kEmpty)) {  // every replica's clock is infinite (sim_batching.hip says when)
-                    dead = MMSIM_E_UNSUPPORTED;
-                    used = 0ull;
+        } else if (ballot(lane < a.nslots && peeked != lds_get<uint64_t>(clk + (uint32_t)lane * 8u)) == 0ull) {
+            runs.met = agree(st);
+            if (runs.met) return true;
+        }
+        runs.go_on(q, at);
+        return false;
+    };
+    int64_t from_w = start, w0 = start;
+    bool last_one = false;  // this wavefront puts the simulation together
+    for (;;) {
+        bool cut = false;
+        if (from_w < R) start_at(from_w);
+        for (w0 = from_w; w0 < R && !dead; w0 += 8) {
+            if constexpr (SPANS)
+                if ((w0 & 63) == 0 && (uint32_t)(w0 >> 6) == runs.next && event((uint32_t)(w0 >> 6))) {
+                    cut = true;
                     break;
                 }
+            const int from = (int)(w0 & 63) + oct;  // the lane that holds this octet's request
+            const int n = R - w0 < 8 ? (int)(R - w0) : 8;
+            const int m = m1;
+            const uint32_t dj = d1;
+            const double t = t1;
+            last = clk + desc_last_slot(dj) * 8u;
+            c_last = lds_get<double>(last);
+            c_first = lds_get<double>(last - desc_stages_m1(dj) * 8u);
+            if ((w0 & 63) == 56) {
+                block = block_next;
+                block_next = fetch_block(w0 + 8 + kWave);
             }
-            if (ready) handle(tf, mf, dsel);
+            m1 = m2;
+            d1 = row_word(m1);  // (past the end of the stream: -1)
+            t1 = time_of(block, (from + 8) & 63);
+            m2 = __shfl((w0 & 63) == 48 ? block_next.m : block.m, (from + 16) & 63);
+            const bool valid = ((int32_t)dj >= 0) & (m >= 0);
+            const uint64_t valids = ballot((int32_t)dj >= 0) & ballot(m >= 0), known = ballot(m >= 0);
+            const uint64_t hosted = valids & kFirstOfOctets, longer = valids >> 7 & kFirstOfOctets;  // longer: the list may go on
+            here = ~0ull >> (64 - 8 * n);
+            int cur = 0;             // arrivals before this one are settled
+            uint64_t unseen = ~0ull;  // arrivals whose due events have not been seen to
+            while (cur < n) {
+                uint64_t due = ballot(next_due <= t) & unseen;
+                if ((due >> (cur * 8) & 1ull) != 0ull) {  // events first (:739-744)
+                    due_events(lane_value(t, cur * 8));
+                    unseen = ~0xFFull << (cur * 8);
+                    due = ballot(next_due <= t) & unseen;
+                }
+                const double mn = oct_min(valid ? c_last : inf);
+                const uint64_t found = ballot(mn < 1e100);
+                // the first listed of those with the smallest last-stage clock
+                const uint64_t selected = first_of_octets(ballot(c_last == mn) & valids);
+                const uint64_t idle = selected & found & ballot(t >= c_first), special = hosted & (~found | longer);
+                const uint64_t left = here & ~0ull << (cur * 8), happens = left & (due | idle | special);
+                // those before the first at which something happens join their queues, and that one unless it has events first
+                uint64_t joining = left;
+                int f = n;
+                if (happens != 0ull) {
+                    f = first_of(happens) >> 3;
+                    joining &= (((due >> (f * 8) & 1ull) != 0ull ? 1ull : 0x100ull) << (f * 8)) - 1ull;
+                }
+                if (in_mask(joining & known & kFirstOfOctets))
+                    __hip_atomic_fetch_add(reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(queues + (uint32_t)m * 16u + 8u), 1u,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                if (want_req && in_mask(joining & kFirstOfOctets & ~hosted)) {
+                    fin_out[w0 + oct] = t;
+                    good_out[w0 + oct] = 0;
+                }
+                wave_order();
+                add_waiting(m, joining & known);
+                cur = f;
+                if (happens == 0ull) break;
+                const int fl = f * 8;
+                if ((due >> fl & 1ull) != 0ull) continue;
+                // its group turns to the arrival if it is idle (:746-778)
+                cur = f + 1;
+                const double tf = lane_value(t, fl);
+                const int mf = lane_value(m, fl);
+                uint32_t dsel = lane_value(dj, first_of(selected >> fl) + fl);
+                if (ROWSLDS) dsel = lane_value(group, first_of(ballot((group & 0x1FFFu) == (dsel & 0x1FFFu)) & groups));
+                bool ready = (idle >> fl & 0xFFull) != 0ull;
+                if (rarely((special >> fl & 1ull) != 0ull)) {
+                    double best = lane_value(mn, fl);
+                    if (!(best < 1e100)) {
+                        best = 1e100;
+                        dsel = kEmpty;
+                        ready = false;
+                    }
+                    if ((longer >> fl & 1ull) != 0ull)
+                        for (int x = 0; x < a.rep_extra; ++x) {
+                            const uint32_t g = more_replicas[(size_t)mf * a.rep_extra + x];
+                            if (g == (uint32_t)a.Gmax) break;
+                            const uint32_t d2 = ginfo[g];
+                            const double c2 = uni(lds_get<double>(clk + desc_last_slot(d2) * 8u));
+                            if (c2 < best) {
+                                best = c2;
+                                dsel = d2;
+                                ready = tf >= uni(lds_get<double>(clk + (desc_last_slot(d2) - desc_stages_m1(d2)) * 8u));
+                            }
+                        }
+                    dsel = uni(dsel);
+                    if (rarely(dsel == kEmpty)) {  // every replica's clock is infinite (sim_batching.hip says when)
+                        dead = MMSIM_E_UNSUPPORTED;
+                        used = 0ull;
+                        break;
+                    }
+                }
+                if (ready) handle(tf, mf, dsel);
+            }
         }
-    }
-    // ---- drain (:781-787)
-    while (used != 0ull && !dead) {
-        const double T = next_due;
-        const uint32_t d = take_event(T);
-        const int m = select_model(desc_group(d));
-        if (m >= 0) handle(T, m, d);
+        // ---- drain (:781-787)
+        while (used != 0ull && !dead && !cut) {
+            const double T = next_due;
+            const uint32_t d = take_event(T);
+            const int m = select_model(desc_group(d));
+            if (m >= 0) handle(T, m, d);
+        }
+        if constexpr (!SPANS) break;
+        // ---- the end of a run
+        ColdArgs *q = cold_args<BatchingArgs>();
+        int first = 0, first_mark = -1;
+        if (!last_one) {
+            uint64_t *e = ended(own);
+            save(e);
+            if (lane == 0) {
+                tell(e + q->state_words, (uint64_t)(uint32_t)dead << 32 | (cut ? (uint32_t)(w0 >> 6) : 0xFFFFFFFFu));
+                tell(e + q->state_words + 1, runs.met ? (uint64_t)(uint32_t)runs.in | (uint64_t)(uint32_t)runs.mark << 32 : ~0ull);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            uint32_t before_me = 0;
+            if (lane == 0) before_me = __hip_atomic_fetch_add(published(q->spans), 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            if (uni(before_me) + 1u != (uint32_t)q->spans) return;
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            // All runs have ended: this wavefront follows them from the first on.
+            last_one = true;
+            for (int k = lane; k <= q->spans; k += kWave) tell(published(k), 0u);  // for the next launch
+            n_good = requests_of_group = good_of_group = 0;
+            lat_sum = 0.0;
+            for (int m = lane; m < M; m += kWave) lds_put<uint32_t>(queues + (uint32_t)m * 16u, 0u);
+        } else {
+            if (!runs.met) break;
+            first = runs.in;
+            first_mark = runs.mark;
+        }
+        const uint64_t *e = nullptr;
+        for (int r = first, mark = first_mark;;) {  // run r from that mark of its (-1: from its beginning) to its end
+            e = ended(r);
+            const uint64_t *b = marked(r, mark < 0 ? 0 : mark);
+            const bool whole = mark < 0;
+            n_good += (int32_t)uni((uint32_t)(e[0] - (whole ? 0ull : b[0])));
+            const int l = at_lanes + 2 * kWave + lane;
+            lat_sum += __longlong_as_double((long long)e[l]) - (whole ? 0.0 : __longlong_as_double((long long)b[l]));
+            if constexpr (OUTPUTS) {
+                const uint64_t v = e[l + kWave] - (whole ? 0ull : b[l + kWave]);
+                requests_of_group += (int32_t)(uint32_t)v;
+                good_of_group += (int32_t)(v >> 32);
+                for (int m = lane; m < M; m += kWave) {
+                    const int w = at_lanes + 4 * kWave + m;
+                    const uint32_t at = queues + (uint32_t)m * 16u;
+                    lds_put<uint32_t>(at, lds_get<uint32_t>(at) + (uint32_t)(e[w] - (whole ? 0ull : b[w])));
+                }
+            }
+            const uint64_t to = e[q->state_words + 1];
+            if (to == ~0ull) break;
+            r = uni((int)(uint32_t)to);
+            mark = uni((int)(uint32_t)(to >> 32));
+        }
+        const uint32_t end = uni((uint32_t)e[q->state_words]);
+        dead = uni((int)(uint32_t)(e[q->state_words] >> 32));
+        if (dead != 0 || end == 0xFFFFFFFFu) break;
+        // The last of them was given up: on from there.
+        for (int k = lane; k < a.nslots; k += kWave) lds_put<uint64_t>(clk + (uint32_t)k * 8u, e[2 + k]);
+        for (int i = 0; i < W; ++i) {
+            const int m = 64 * i + lane;
+            uint64_t queue = 0;
+            if (m < M) {
+                queue = e[at_queues + m];
+                const uint32_t at = queues + (uint32_t)m * 16u, head = (uint32_t)queue;
+                lds_put<uint32_t>(at + 4u, head);
+                lds_put<uint32_t>(at + 8u, (uint32_t)(queue >> 32));
+                lds_put<uint32_t>(at + 12u, (uint32_t)mq[head].rank);
+            }
+            const uint64_t some = ballot((uint32_t)queue != (uint32_t)(queue >> 32));
+#pragma unroll
+            for (int k = 0; k < W; ++k) waiting[k] = k == i ? some : waiting[k];
+        }
+        ev_t = __longlong_as_double((long long)e[at_lanes + lane]);
+        ev_d = (uint32_t)e[at_lanes + kWave + lane];
+        used = (uint64_t)uni((uint32_t)(e[1] >> 32)) << 32 | uni((uint32_t)e[1]);
+        next_due = wave_min(ev_t);
+        wave_order();
+        runs.resume(q, end);
+        from_w = (int64_t)end * kWave;
     }
 
     for (int k = 1; k < 8; k *= 2) lat_sum += __hiloint2double(__shfl_xor(__double2hiint(lat_sum), k), __shfl_xor(__double2loint(lat_sum), k));
@@ -624,22 +836,32 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     }
 }
 
+#ifdef MMSIM_SOLO_RUNS
+constexpr bool kRuns = true;  // the file is compiled once more for simulations cut into runs
+#else
+constexpr bool kRuns = false;
+#endif
+template <bool LATLDS, bool UNIF, bool OUTPUTS, int MW>
+constexpr auto solo_kernel = sim_batching_solo_kernel<LATLDS, UNIF, OUTPUTS, kRuns && MW == 0 ? 1 : MW, kRuns>;
+
 bool solo_outputs(const BatchingArgs &a) {
     return (a.flags & (MMSIM_WANT_MODEL_COUNTS | MMSIM_WANT_GROUP_COUNTS | MMSIM_WANT_PER_REQUEST)) != 0;
 }
 
 }  // namespace
 
-hipError_t launch_sim_batching_solo(const BatchingArgs &args, int wpb, size_t lds_bytes, hipStream_t stream) {
+template <>
+hipError_t launch_sim_batching_solo<kRuns>(const BatchingArgs &args, int wpb, size_t lds_bytes, hipStream_t stream) {
     const bool ll = args.lat_lds_bytes > 0, unif = args.uniform_stages != 0, outputs = solo_outputs(args);
     if (wpb < 1 || wpb > kMaxWavesPerBlockBatching || args.tile_sims != 1 || !batching_solo_fits(args.NB, args.heap_cap, args.Gmax) || (args.solo == 1 && args.M > kSoloMasks)) return hipErrorInvalidValue;
+    if (kRuns && (args.solo != 1 || (args.flags & MMSIM_WANT_PER_REQUEST))) return hipErrorInvalidValue;
     void (*kern)(const BatchingArgs) = nullptr;
 #define MMSIM_PICK3(L, U, O)                                       \
-    (args.solo == 2  ? sim_batching_solo_kernel<L, U, O, 0>          \
-     : args.M <= 64  ? sim_batching_solo_kernel<L, U, O, 1>          \
-     : args.M <= 128 ? sim_batching_solo_kernel<L, U, O, 2>          \
-     : args.M <= 256 ? sim_batching_solo_kernel<L, U, O, 4>          \
-                     : sim_batching_solo_kernel<L, U, O, 8>)
+    (args.solo == 2  ? solo_kernel<L, U, O, 0>          \
+     : args.M <= 64  ? solo_kernel<L, U, O, 1>          \
+     : args.M <= 128 ? solo_kernel<L, U, O, 2>          \
+     : args.M <= 256 ? solo_kernel<L, U, O, 4>          \
+                     : solo_kernel<L, U, O, 8>)
 #define MMSIM_PICK2(L, U) (outputs ? MMSIM_PICK3(L, U, true) : MMSIM_PICK3(L, U, false))
 #define MMSIM_PICK(L) (unif ? MMSIM_PICK2(L, true) : MMSIM_PICK2(L, false))
     kern = ll ? MMSIM_PICK(true) : MMSIM_PICK(false);
@@ -656,14 +878,17 @@ hipError_t launch_sim_batching_solo(const BatchingArgs &args, int wpb, size_t ld
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         if (e != hipSuccess) return e;
     }
-    const unsigned tile_groups = (unsigned)((args.tiles + wpb - 1) / wpb);
-    hipLaunchKernelGGL(kern, dim3(tile_groups * (unsigned)(args.paired ? 1 : args.n_seeds)), dim3(wpb * kWave), lds_bytes, stream, args);
+    const unsigned seeds = (unsigned)(args.paired ? 1 : args.n_seeds);
+    const unsigned groups = kRuns ? (unsigned)(((int64_t)args.tiles * seeds * args.spans + wpb - 1) / wpb) : (unsigned)((args.tiles + wpb - 1) / wpb) * seeds;
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(wpb * kWave), lds_bytes, stream, args);
     return hipGetLastError();
 }
 
+#ifndef MMSIM_SOLO_RUNS
 std::string sim_batching_solo_kernel_name(const BatchingArgs &args) {
     return std::string("sim_batching_solo_kernel<") + (args.lat_lds_bytes > 0 ? "true, " : "false, ") +
            (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.solo == 2 ? "0>" : args.M <= 64 ? "1>" : args.M <= 128 ? "2>" : args.M <= 256 ? "4>" : "8>");
 }
+#endif
 
 }  // namespace mmsim

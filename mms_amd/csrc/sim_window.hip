@@ -79,6 +79,7 @@
 // the word then repeats the first replica's (which wins every tie against its copies) or, without any replica, the
 // placement's first slot.
 #include "mmsim_internal.h"
+#include "runs.h"
 
 namespace mmsim {
 namespace {
@@ -272,12 +273,6 @@ struct LatencySum {
     }
 };
 
-// What wavefronts of different workgroups tell one another while the kernel runs: stores and loads that all of the device sees.
-__device__ __forceinline__ void tell(uint64_t *p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ void tell(uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ uint64_t told(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ uint32_t told(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
 struct Entry {  // a replica, as rep and ext hold it
     uint32_t d;
     float l;
@@ -302,69 +297,13 @@ template <int I>
 struct Int {
     static constexpr int value = I;
 };
-// The arguments as they lie in memory, for what is done rarely: asked for there, and not kept in scalar registers, which the loop over blocks
-// has none to spare of (71 of its instructions, of 930 a block, moved them to and fro).
-typedef const __attribute__((address_space(4))) WindowArgs ColdArgs;
-__device__ __forceinline__ ColdArgs *cold_args() {
-    ColdArgs *p = (ColdArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
 // Where a run's latencies are (finish times, if wanted), by place in the stream: those of runs that are taken up again in an array of
 // the whole stream.  (Run 0 adds up its own and writes its outputs.)
+typedef const __attribute__((address_space(4))) WindowArgs ColdArgs;
 __device__ __forceinline__ double *values_of(ColdArgs *q, int sim, int r) {
     double *v = q->run_vals + (size_t)sim * (size_t)(q->true_cap + (q->spans - 1) * q->run_cap);
     return r == 0 ? v : v + q->true_cap + (r - 1) * q->run_cap - (int64_t)r * q->span_blocks * kWave;
 }
-
-struct Runs {  // what a run goes by (scalars; blocks of 64 requests)
-    int own;         // the run, or -1: one that is taken up again
-    int in, mark;    // the span of the next mark, and which of that span's it is
-    uint32_t since;  // where the run left its own span
-    uint32_t next;   // block before which something happens
-    bool looked;     // another run's mark: what to compare with is on its way (asked for a block ahead)
-    bool met;        // the run of span `in` at that mark
-
-    // known to be what the simulation does: the first run, or one taken up again
-    __device__ __forceinline__ bool true_one() const { return own <= 0; }
-    __device__ __forceinline__ uint32_t limit(ColdArgs *a) const {
-        return true_one() ? 0xFFFFFFFFu : (uint32_t)((own + 1) * a->span_blocks + a->ext_blocks);
-    }
-    __device__ __forceinline__ void start(ColdArgs *a, int span) {
-        own = in = span;
-        mark = 0;
-        looked = met = false;
-        since = (uint32_t)((own + 1) * a->span_blocks);
-        next = (uint32_t)(own * a->span_blocks + span_mark(0));  // (within the span: it has more than eight blocks)
-    }
-    __device__ __forceinline__ void resume(ColdArgs *a, uint32_t at) {
-        own = -1;
-        in = (int)(at / (uint32_t)a->span_blocks);
-        mark = -1;
-        met = false;
-        since = at;
-        go_on(a, at);
-    }
-    // From block `at` to the next mark: of its own span all, of others those that are further by an eighth of how far the run has come on
-    // its own (a run that meets nobody looks fifty times or so, not at every mark of the stream).
-    __device__ __forceinline__ void go_on(ColdArgs *a, uint32_t at) {
-        const int span = a->span_blocks;
-        const uint32_t least = at < since ? 0u : at + 2u + (at - since) / 8u;
-        uint32_t m;
-        do {
-            mark += 1;
-            if (span_mark(mark) >= span) {
-                in += 1;
-                mark = 0;
-            }
-            m = (uint32_t)(in * span + span_mark(mark));
-        } while (m < least);
-        looked = false;
-        next = in != own ? m - 1u : m;
-        next = next < limit(a) ? next : limit(a);
-    }
-};
 
 // Wavefronts of a SIMD that the registers have to leave room for, with simulations cut into runs.
 constexpr int least_waves(int smax, bool outputs, int ext) {
@@ -564,19 +503,19 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
     const int sim = (int)unit;
     Runs runs;
     if constexpr (SPANS) {
-        runs.start(cold_args(), own);
+        runs.start(cold_args<WindowArgs>(), own);
     }
     auto marked = [&](int r, int i) {
-        ColdArgs *q = cold_args();
+        ColdArgs *q = cold_args<WindowArgs>();
         return q->mark_state + (((size_t)sim * q->spans + r) * q->marks + i) * (size_t)q->state_words;
     };
     auto ended = [&](int r) {
-        ColdArgs *q = cold_args();
+        ColdArgs *q = cold_args<WindowArgs>();
         return q->end_state + ((size_t)sim * q->spans + r) * (size_t)(q->state_words + kEndWords);
     };
     // state: accepted requests, clocks; counts of the slots and of the models
     auto for_state = [&](auto f) {
-        const int nslots = cold_args()->nslots;
+        const int nslots = cold_args<WindowArgs>()->nslots;
         for (int k = j; k < nslots; k += W) f(1 + k, clk + (uint32_t)k * 8u, false);
         if constexpr (OUTPUTS) {
             for (int k = j; k < nslots; k += W) f(1 + nslots + k, clk + (uint32_t)k * 8u + cnt_rel, false);
@@ -586,12 +525,12 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
     auto get_word = [&](uint32_t at, bool half) -> uint64_t { return half ? (uint64_t)lds_get<uint32_t>(at) : lds_get<uint64_t>(at); };
     // Something happens before block `at`: a mark of this run, one of a later run or the block ahead of it, the end of the run (true).
     auto published = [&](int r) {
-        ColdArgs *q = cold_args();
+        ColdArgs *q = cold_args<WindowArgs>();
         return q->span_sync + (size_t)sim * (q->spans + 1) + r;
     };
     uint64_t peeked = 0;
     auto event = [&](uint32_t at) -> bool {
-        ColdArgs *q = cold_args();
+        ColdArgs *q = cold_args<WindowArgs>();
         if (at >= runs.limit(q)) return true;
         uint64_t *st = marked(runs.in, runs.mark);
         if (runs.in == runs.own) {
@@ -618,7 +557,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         runs.go_on(q, at);
         return false;
     };
-    auto q_pieces = [&](int of) { return cold_args()->pieces + (size_t)of * (8 * kMaxSpans); };
+    auto q_pieces = [&](int of) { return cold_args<WindowArgs>()->pieces + (size_t)of * (8 * kMaxSpans); };
     auto piece = [&](uint32_t at, uint32_t first, uint32_t end, int src) {
         uint32_t *w = q_pieces(sim) + at * 4u;
         w[0] = first;
@@ -626,7 +565,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         w[2] = (uint32_t)src;
     };
     uint32_t from = SPANS ? (uint32_t)own * (uint32_t)a.span_blocks * 64u : 0u, blk = from;
-    double *run_vals = SPANS ? values_of(cold_args(), sim, own) : nullptr;  // by place in the stream
+    double *run_vals = SPANS ? values_of(cold_args<WindowArgs>(), sim, own) : nullptr;  // by place in the stream
     uint32_t num_pieces = 0;
     bool last = false;  // this wavefront puts the simulation together
     for (;;) {
@@ -950,7 +889,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         }
         if constexpr (!SPANS) break;
         // ---- the end of a run
-        ColdArgs *q = cold_args();
+        ColdArgs *q = cold_args<WindowArgs>();
         int first = 0, first_mark = -1;
         if (!last) {
             uint64_t *e = ended(own);
@@ -1068,7 +1007,7 @@ __global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const Wind
     __shared__ uint32_t pieces[8 * kMaxSpans];
     const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), sim = (int)blockIdx.x;
     const int worker = wv + (int)blockIdx.y * kSumWaves;  // 0: the sum, others: outputs
-    ColdArgs *q = cold_args();
+    ColdArgs *q = cold_args<WindowArgs>();
     for (int k = (int)threadIdx.x; k < 8 * kMaxSpans; k += (int)blockDim.x) pieces[k] = a.pieces[(size_t)sim * (8 * kMaxSpans) + k];
     __syncthreads();
     const int num = __builtin_amdgcn_readfirstlane((int)pieces[8 * kMaxSpans - 1]);

@@ -66,9 +66,8 @@ struct Shape {
 
 }  // namespace
 
-// Blocks of a span, and what a run may go on behind its span, at least, how many bytes the runs of a launch may take, and how many a context
-// keeps for the next call (a gigabyte costs 0.3 ms to allocate and free).
-constexpr int32_t kLeastSpan = 20, kLeastExt = 48;
+// How many bytes the runs of a launch may take, and how many a context keeps for the next call (a gigabyte costs 0.3 ms to
+// allocate and free).
 constexpr size_t kMostRunBytes = (size_t)16 << 30, kMostRunsKept = (size_t)2 << 30;
 
 int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
