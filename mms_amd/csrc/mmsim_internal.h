@@ -275,7 +275,7 @@ struct WindowArgs {
 __host__ __device__ constexpr int window_ring_bytes(int lanes) { return lanes == kWave ? 0 : 2 * kWave * (int)sizeof(Req); }
 constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
 constexpr int kEndWords = 2;        // of end_state: end block, link
-constexpr int kSumWaves = 4;        // wavefronts of a workgroup that puts a simulation's runs together, if per-request outputs are wanted
+constexpr int kSumWaves = 4;        // wavefronts that put a simulation's runs together
 constexpr int kMaxSpans = 64;       // most runs of a simulation (their records are a lane's each)
 constexpr int32_t kLeastSpan = 20, kLeastExt = 48;  // blocks of a span, and what a run may go on behind its span, at least
 constexpr int kMaxRuns = 4096;      // most runs of a launch, if its simulations are cut

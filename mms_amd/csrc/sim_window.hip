@@ -224,6 +224,7 @@ __device__ __forceinline__ double sum_of_lanes(double v) {
 struct LatencySum {
     double s, base, half;  // base: 2^k, half: u / 2
     int odd;               // whether s / u is odd, or s and what was taken since
+    double first_tie = 0.0;
     __device__ __forceinline__ explicit LatencySum(double v) { set(v); }
     __device__ __forceinline__ void set(double v) {
         s = v;
@@ -237,39 +238,55 @@ struct LatencySum {
         const double up = base + x, r = up - base, off = x - r;
         const bool half_way = __builtin_fabs(off) == half;
         const uint64_t ties = ballot(half_way), odds = ballot((__double2loint(up) & 1) != 0);  // (half-way ones came out even)
-        // whether S / u is odd behind these requests: as many odd ones from the last half-way one on
-        auto odd_behind = [&](uint64_t lanes) {
-            const uint64_t t = ties & lanes;
-            const uint64_t since = odds & lanes & (t != 0ull ? ~0ull << (63 - __builtin_clzll(t | 1ull)) : ~0ull);
-            return (__popcll(since) ^ (t != 0ull ? 0 : odd)) & 1;
-        };
-        const double added = half_way && odd_behind((1ull << lane_id()) - 1ull) != 0 ? x + off : r;
-        odd = odd_behind(~0ull);
-        return added;
+        // Whether S / u is odd before a half-way request: as many odd ones came since the half-way one before it, or since the
+        // beginning and S / u was odd then.  since: whether the number of odd ones up to that one was odd, carried through the
+        // requests between them by an addition.
+        const uint64_t odd_below = ballot((__builtin_amdgcn_mbcnt_hi((uint32_t)(odds >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)odds, 0u)) & 1u) != 0u);
+        const uint64_t at_ties = odd_below & ties;
+        uint64_t since;
+        const bool out1 = __builtin_add_overflow(~ties, at_ties << 1, &since), out2 = __builtin_add_overflow(since, (uint64_t)odd, &since);
+        const uint64_t others = (odd_below ^ since) & ties;
+        odd = (__builtin_popcountll(odds) ^ (out1 || out2 ? 1 : 0) ^ (int)(at_ties >> 63)) & 1;
+        if (first_tie == 0.0 && ties != 0ull) {
+            const int l = __builtin_ctzll(ties);
+            first_tie = 2.0 * __hiloint2double(lane_value(__double2hiint(off), l), lane_value(__double2loint(off), l));
+            if ((others >> l & 1ull) != 0ull) first_tie = -first_tie;
+        }
+        const bool other = in_mask(others);
+        return other ? x + off : r;
     }
-    // Adds N blocks' latencies, 0 where a request is not accepted; false, and nothing is done: not together.
+    // What N blocks' latencies add to a sum in [2^k, 2^(k+1)), if it is even, and how much more if it is odd: only the first
+    // half-way one comes out differently then.  negative: they must be added one by one.
     template <int N>
-    __device__ __forceinline__ bool add(const double (&x)[N]) {
-        const int odd_before = odd;
+    __device__ __forceinline__ void look(const double (&x)[N], double *added, double *more_if_odd, bool *negative) const {
+        LatencySum even = *this;
+        even.odd = 0;
+        even.first_tie = 0.0;
         double lanes = 0.0;
-        bool negative = false;
+        bool neg = false;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            lanes += take(x[i]);
-            negative = negative || x[i] < 0.0;
+            lanes += even.take(x[i]);
+            neg = neg || x[i] < 0.0;
         }
-        const double sum = sum_of_lanes(lanes);
-        if (!(sum <= 2.0 * base - s) || ballot(negative) != 0ull) {
-            odd = odd_before;
-            return false;
-        }
+        *added = sum_of_lanes(lanes);
+        *more_if_odd = even.first_tie;
+        *negative = ballot(neg) != 0ull;
+    }
+    // Adds what look() found, unless the sum leaves [2^k, 2^(k+1)).
+    __device__ __forceinline__ bool add(double added, double more_if_odd, bool negative) {
+        const double sum = added + (odd != 0 ? more_if_odd : 0.0);
+        if (negative || !(sum <= 2.0 * base - s)) return false;
         set(s + sum);
         return true;
     }
     __device__ __forceinline__ void add_block(double x) {
         const double one[1] = {x};
         const uint64_t some = ballot(x != 0.0);
-        if (some != 0ull && !add(one)) set(ordered_sum<kWave>(s, x, some));
+        double added, more;
+        bool negative;
+        look(one, &added, &more, &negative);
+        if (some != 0ull && !add(added, more, negative)) set(ordered_sum<kWave>(s, x, some));
     }
 };
 
@@ -1000,13 +1017,17 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
 }
 
 #ifdef MMSIM_WINDOW_SPANS
-// What the runs of a simulation come to: a wavefront adds up the latencies of the pieces that are followed, in order; with
-// per-request outputs the others of the workgroup write these.
+// What the runs of a simulation come to: a workgroup adds up the latencies of the pieces that are followed, in their order, and writes
+// the per-request outputs.  Sixteen blocks to a wavefront and round: all look at theirs side by side, for the sum as it is at the
+// beginning of the round, and add in turn; one that takes the sum across a power of two is looked at again, block by block.
+// One wavefront to a placement and lanes that worked out 64-bit masks each, against this: 700 placements of 108000 requests, three quarters of them
+// here, 0.23 -> 0.22 ms (450 MB of latencies; a copy reads them in 0.1), 600 placements 0.34 -> 0.24, five of 82000 0.20 -> 0.12, one of 30000 with outputs 0.10 -> 0.08.
 __global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const WindowArgs a) {
     constexpr int N = 16;
     __shared__ uint32_t pieces[8 * kMaxSpans];
-    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), sim = (int)blockIdx.x;
-    const int worker = wv + (int)blockIdx.y * kSumWaves;  // 0: the sum, others: outputs
+    __shared__ double added[kSumWaves], more_if_odd[kSumWaves], exact;
+    __shared__ int negative[kSumWaves];
+    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = (int)(blockDim.x >> 6), sim = (int)blockIdx.x;
     ColdArgs *q = cold_args<WindowArgs>();
     for (int k = (int)threadIdx.x; k < 8 * kMaxSpans; k += (int)blockDim.x) pieces[k] = a.pieces[(size_t)sim * (8 * kMaxSpans) + k];
     __syncthreads();
@@ -1017,7 +1038,7 @@ __global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const Wind
     const uint32_t R = (uint32_t)a.stream_len[seed], blocks = (R + 63u) / 64u;
     double *fin_out = a.finish + (size_t)sim * (size_t)a.Rmax;
     uint8_t *good_out = a.good + (size_t)sim * (size_t)a.Rmax;
-    if (num < 2) return;
+    if (num < 2) return;  // (the first run went through the whole stream)
     const uint32_t begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)pieces[1]);  // where the first run ends
     int p = 0;
     uint32_t p_end = begin;
@@ -1036,49 +1057,59 @@ __global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const Wind
             if (want_req) arr[i] = as_req(load_global(reqs + (pos < R ? pos : R - 1u))).t;
         }
     };
-    // latencies, 0 of what is not accepted or past the end
-    auto latencies = [&](uint32_t first, double *x, const double *arr) {
+    LatencySum sum(a.lat_sum[sim]);  // (the same in all wavefronts)
+    double x[N], y[N], arr[N];
+    const uint32_t round = (uint32_t)(waves * N);
+    uint32_t mine = begin + (uint32_t)(wv * N);
+    load(mine, y, arr);
+    for (uint32_t at = begin; at < blocks; at += round, mine += round) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            if (want_req) x[i] = x[i] == x[i] ? x[i] - arr[i] : 0.0;
-            if ((first + i) * (uint32_t)kWave + (uint32_t)lane >= R) x[i] = 0.0;
-        }
-    };
-    if (worker > 0) {
-        const int workers = (int)(gridDim.y * (blockDim.x >> 6)) - 1;
-        for (uint32_t at = begin + (uint32_t)(worker - 1) * N; at < blocks; at += (uint32_t)workers * N) {
-            double x[N], arr[N];
-            load(at, x, arr);
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const uint32_t pos = (at + i) * (uint32_t)kWave + (uint32_t)lane;
-                if (at + i >= blocks || pos >= R) continue;
+            const uint32_t pos = (mine + i) * (uint32_t)kWave + (uint32_t)lane;
+            const bool in = mine + i < blocks && pos < R;
+            x[i] = y[i];
+            if (want_req) {  // finish times, NaN of the requests that are not accepted
                 const bool good = x[i] == x[i];
-                fin_out[pos] = good ? x[i] : arr[i];
-                good_out[pos] = good ? 1 : 0;
+                if (in) {
+                    fin_out[pos] = good ? x[i] : arr[i];
+                    good_out[pos] = good ? 1 : 0;
+                }
+                x[i] = good ? x[i] - arr[i] : 0.0;
             }
+            if (!in) x[i] = 0.0;
         }
-        return;
-    }
-    LatencySum sum(a.lat_sum[sim]);
-    double x[N], y[N], arr[N];
-    load(begin, y, arr);
-    for (uint32_t at = begin; at < blocks; at += N) {
-        latencies(at, y, arr);
-#pragma unroll
-        for (int i = 0; i < N; ++i) x[i] = y[i];
-        if (at + N < blocks) load(at + N, y, arr);
-        if (!sum.add(x)) {
+        if (mine + round < blocks) load(mine + round, y, arr);
+        double mine_added, mine_more;
+        bool mine_negative;
+        sum.look(x, &mine_added, &mine_more, &mine_negative);
+        if (lane == 0) {
+            added[wv] = mine_added;
+            more_if_odd[wv] = mine_more;
+            negative[wv] = mine_negative ? 1 : 0;
+        }
+        __syncthreads();
+        const double base = sum.base;  // what they were looked at for
+        for (int k = 0; k < waves; ++k) {
+            if (sum.base == base && sum.add(added[k], more_if_odd[k], negative[k] != 0)) continue;
+            if (wv == k) {
+                sum.look(x, &mine_added, &mine_more, &mine_negative);
+                if (!sum.add(mine_added, mine_more, mine_negative))
 #pragma unroll 1
-            for (int i = 0; i < N; ++i) {
-                double w = x[0];
+                for (int i = 0; i < N; ++i) {
+                    double w = x[0];
 #pragma unroll
-                for (int k = 1; k < N; ++k) w = i == k ? x[k] : w;
-                sum.add_block(w);
+                    for (int l = 1; l < N; ++l) w = i == l ? x[l] : w;
+                    sum.add_block(w);
+                }
+                if (lane == 0) exact = sum.s;
             }
+            __syncthreads();
+            sum.set(exact);
+            __syncthreads();
         }
+        __syncthreads();
     }
-    if (lane == 0) a.lat_sum[sim] = sum.s;
+    if (threadIdx.x == 0) a.lat_sum[sim] = sum.s;
 }
 #endif
 

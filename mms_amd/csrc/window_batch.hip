@@ -50,11 +50,8 @@ hipError_t launch_window(const WindowArgs &a, int waves_per_block, size_t lds_by
     const int64_t units = (int64_t)a.tiles * a.out_seeds * a.spans;
     hipLaunchKernelGGL(kern, dim3((unsigned)((units + waves_per_block - 1) / waves_per_block)), dim3((unsigned)waves_per_block * kWave),
                        lds_bytes, stream, a);
-    const bool per_request = (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
     if (a.spans > 1)
-        hipLaunchKernelGGL(window_sum(), dim3((unsigned)(a.tiles * a.out_seeds), per_request && a.tiles * a.out_seeds <= 32 ? 8 : 1),
-                           dim3(kWave * (per_request ? kSumWaves : 1)), 0,
-                           stream, a);
+        hipLaunchKernelGGL(window_sum(), dim3((unsigned)(a.tiles * a.out_seeds)), dim3(kWave * kSumWaves), 0, stream, a);
     return hipGetLastError();
 }
 
