@@ -1561,6 +1561,7 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
         slo = slo_bits;
         if (i > 0 && tstamps[i] < tstamps[i - 1]) sorted = false;
     }
+    w->sorted = sorted;
     w->repeats = repeats;
     w->run_repeats = run_repeats;
     if (R > 0) w->span = std::max(0.0, tstamps[R - 1] - tstamps[0]);

@@ -209,6 +209,7 @@ struct mmsim_workload {
     std::shared_ptr<DevBuf<Req>> reqs = std::make_shared<DevBuf<Req>>();  // shared with batches that read it in place
     std::vector<int32_t> model_num_requests;  // requests per model id (placement independent)
     double span = 0.0;                        // from the first arrival to the last
+    bool sorted = true;                       // arrivals ascend
     int64_t repeats = 0;                      // requests with the model of the request before
     int64_t run_repeats = 0;                  // ... and with its SLO (bit for bit)
     // arrivals regrouped by model (batching simulator): offsets per model, then per arrival

@@ -256,6 +256,7 @@ struct WindowArgs {
     int32_t spans;                   // runs of a simulation; 1: not cut
     int32_t span_blocks, ext_blocks; // blocks of a span, and how many a run goes on behind its own
     int32_t marks, state_words;      // most marks of a span, 64-bit words of a state
+    int32_t alike;                   // clocks that differ before the next arrival may count as equal: arrivals ascend, no latency is negative, up to 64 groups
     int64_t run_cap, true_cap;       // values of a run: 64 * (span_blocks + ext_blocks), and of a whole stream
     uint32_t *span_sync;             // [L][spans + 1] marks that every run has published, and how many runs have ended: 0 before a launch and after
     uint64_t *mark_state;            // [L][spans][marks][state_words]

@@ -52,7 +52,7 @@
 // That is wrong at first.  But what a simulation does next depends on its clocks alone, and clocks forget: a group that was
 // idle finishes its next request at a time that does not depend on what it did before, and one that rejected until it had caught up
 // agrees soon after.  So a run goes on behind its span and compares its clocks with those that the next run had at the same places
-// (marks: it left them in memory on its way).  Where all clocks are equal, bit for bit, both runs do the same for ever, and the one
+// (marks: it left them in memory on its way).  Where all clocks are equal, bit for bit, or differ in ways that no request can see (event), both runs do the same for ever, and the one
 // that started further on has done it already: the run ends.  The first run is what the simulation does; where it ended
 // the run that it met takes over, and so on: the results are the serial loop's.  A run that meets nobody within half a span (48 blocks
 // at least) is given up; the wavefront that ends last follows the runs, takes up again one that was given up where
@@ -139,6 +139,7 @@ __device__ __forceinline__ int shfl_last(int v) { return __shfl(v, W - 1, W); }
 template <int W>
 __device__ __forceinline__ int shfl_xor(int v, int d) { return __shfl_xor(v, d, W); }
 __device__ __forceinline__ int lane_value(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ double lane_value(double v, int l) { return __hiloint2double(lane_value(__double2hiint(v), l), lane_value(__double2loint(v), l)); }
 
 // S + x of lane 0 of the W lanes, + x of lane 1, ...: one addition after the other, as the serial loop adds.  In and
 // out S is the same in all W lanes.  v_fmac_f64 with a DPP operand that a lane of the row broadcasts computes
@@ -564,9 +565,26 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
                 return false;
             }
         } else {
-            bool same = lane >= q->nslots || peeked == lds_get<uint64_t>(clk + (uint32_t)lane * 8u);
+            // Equal clocks, or alike: what differs lies before the next arrival in both (limit; never, if a.alike is 0), so no walk sees it,
+            // and the groups' last clocks are in the same order, so every choice is the same.  That lasts: a clock that is written comes out the same in
+            // both, and not before that arrival.
+            const double limit = q->alike != 0 ? lane_value(cur.t, 0) : -1.0;
+            bool differ = false, same = true;
+            auto compare = [&](uint64_t theirs, uint32_t addr) {
+                const uint64_t mine = lds_get<uint64_t>(addr);
+                const bool other = theirs != mine;
+                differ = differ || other;
+                same = same && (!other || (__longlong_as_double((long long)theirs) < limit && __longlong_as_double((long long)mine) < limit));
+            };
+            if (lane < q->nslots) compare(peeked, clk + (uint32_t)lane * 8u);
             if (ballot(!same) == 0ull) {
-                for (int k = j + W; k < q->nslots; k += W) same = same && told(st + 1 + k) == lds_get<uint64_t>(clk + (uint32_t)k * 8u);
+                for (int k = j + W; k < q->nslots; k += W) compare(told(st + 1 + k), clk + (uint32_t)k * 8u);
+                if (ballot(differ) != 0ull && ballot(!same) == 0ull) {
+                    uint32_t slot = 0;  // lane g: the last one of group g (of others the first group's)
+                    if (q->Gmax > 0) slot = (entry_addr(lds_get<uint32_t>(gd + (uint32_t)(lane < ng ? lane : 0) * 4u)) - clk) >> 3;
+                    const double mine = lds_get<double>(clk + slot * 8u), theirs = __longlong_as_double((long long)told(st + 1 + slot));
+                    for (int g = 0; g < ng; ++g) same = same && (mine < lane_value(mine, g)) == (theirs < lane_value(theirs, g));
+                }
                 runs.met = ballot(!same) == 0ull;
                 if (runs.met) return true;
             }

@@ -333,6 +333,11 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         cut(1);
     }
     spans = a.spans;
+    a.alike = Gmax <= kWave ? 1 : 0;
+    for (int s = 0; s < n_seeds; ++s)
+        if (!wls[s]->sorted) a.alike = 0;
+    for (const float l : cl.lat)
+        if (!(l >= 0.0f)) a.alike = 0;
     if (spans > 1) {
         a.mark_state = reinterpret_cast<uint64_t *>(run_memory.p);
         a.end_state = reinterpret_cast<uint64_t *>(run_memory.p + at_ends);

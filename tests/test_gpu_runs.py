@@ -116,3 +116,33 @@ def test_runs_of_the_batching_simulator(depths, uniform, groups, hosts, M, span)
                 assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0), (B, k)
     for dw in dws:
         dw.close()
+
+
+def test_clocks_that_no_request_can_tell_apart():
+    """Groups that nobody asks for during a span (their clocks stay as they were, or at zero), in the same order and not, and an
+    arrival that is earlier than the one before it, which takes the shortcut away."""
+    eng = E.Engine.default()
+    M, span, R = 8, 512, 6 * 512
+    for uneven in (False, True):
+        rng = np.random.default_rng(5)
+        profiles, _ = _problem(5, (1, 2), True, M, 1, 1, 1)
+        pcs = sorted({pc for p in profiles for pc in p.para_dict}, key=lambda c: c.pp)
+        sols = [_problem(60 + k, (1, 2), True, M, 9, 1, 3)[1][0] for k in range(24)]
+        # a phase for the first half of the models, one for the second, and so on; pauses within
+        st = _with_pauses(21, R, M, 0.5, 40, pause=2.0)
+        phase = np.arange(R) // 700 % 2
+        st.model_ids = (rng.integers(0, M // 2, R) + phase * (M // 2)).astype(np.int32)
+        st.slos = np.where(np.isfinite(st.slos), st.slos, np.float32(0.5))
+        if uneven:
+            st.tstamps[2000:] -= 3.0
+        table = E.LatencyTable(profiles, [1])
+        packed = E.pack_placements(sols, table)
+        dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, M)
+        batch = E.Batch(eng, [dw], table, packed, COUNTS, options=dict(window_lanes=64, segment_requests=span))
+        assert batch.kernel_name().count(",") == 6 and pcs
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        batch.close()
+        assert_batch_matches(out, oracle_batch(st, table, packed), 0, packed[0], where=f"uneven {uneven}")
+        dw.close()
