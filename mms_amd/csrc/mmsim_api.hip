@@ -1370,6 +1370,11 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
             q.ext_blocks = std::max(q.span_blocks / 2, kLeastExt);
             for (q.marks = 0; span_mark(q.marks) < q.span_blocks;) ++q.marks;
             q.state_words = 2 + nslots + M + 4 * kWave + M;
+            q.alike = t->fixed_overhead >= 0.0 ? 1 : 0;
+            for (int s = 0; s < n_seeds; ++s)
+                if (!wls[s]->sorted) q.alike = 0;
+            for (const float l : lat_nb)
+                if (!(l >= 0.0f)) q.alike = 0;
             const size_t marks = 8 * n * (size_t)q.marks * (size_t)q.state_words, ends = 8 * n * (size_t)(q.state_words + kEndWords),
                          sync = 4 * L * (size_t)(runs_of + 1);
             HIP_TRY(b->run_memory.alloc(marks + ends + sync));

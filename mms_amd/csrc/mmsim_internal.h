@@ -216,7 +216,7 @@ struct BatchingArgs {
     double fixed_overhead;
     uint32_t flags;
     // simulations cut into runs (solo), as in WindowArgs
-    int32_t spans, span_blocks, ext_blocks, marks, state_words;
+    int32_t spans, span_blocks, ext_blocks, marks, state_words, alike;
     uint32_t *span_sync;
     uint64_t *mark_state, *end_state;
     // outputs

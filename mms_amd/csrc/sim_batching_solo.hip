@@ -40,7 +40,7 @@
 //
 // Few simulations of long streams without per-request outputs are cut into runs (SPANS), as sim_window.hip cuts its own: a run starts a span
 // with idle clocks and empty queues, and ends where its clocks, the queues of the models that some group lists and its idle events equal those that
-// the next run had there.  30000 requests, 128 placements, runs agree after 192 requests in the median, 704 at most of 24: 24 runs
+// the next run had there (or its clocks differ where nothing looks any more).  30000 requests, 128 placements, runs agree after 192 requests in the median, 704 at most of 24: 24 runs
 // each, calls 14.3 -> 2.03 ms; 105000 requests of 10 models on 30 single devices, 309 placements, of which some never agree, 126 -> 101 ms.
 //
 // LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
@@ -584,11 +584,19 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         tell(mine + 2 * kWave, (uint64_t)__double_as_longlong(lat_sum));
         if (OUTPUTS) tell(mine + 3 * kWave, (uint64_t)(uint32_t)good_of_group << 32 | (uint32_t)requests_of_group);
     };
-    auto agree = [&](const uint64_t *st) -> bool {
+    // Clocks that are equal, or that differ before anything that happens from here on (sim_window.hip): arrivals and idle events.
+    auto alike = [](uint64_t x, uint64_t y, double before) -> bool {
+        return x == y || (__longlong_as_double((long long)x) < before && __longlong_as_double((long long)y) < before);
+    };
+    auto agree = [&](const uint64_t *st, double unseen) -> bool {
         const uint64_t their_used = (uint64_t)uni((uint32_t)(told(st + 1) >> 32)) << 32 | uni((uint32_t)told(st + 1));
         if (__builtin_popcountll(their_used) != __builtin_popcountll(used)) return false;
-        bool same = true;
-        for (int k = lane; k < a.nslots; k += kWave) same = same && told(st + 2 + k) == lds_get<uint64_t>(clk + (uint32_t)k * 8u);
+        bool same = true, differ = false;
+        for (int k = lane; k < a.nslots; k += kWave) {
+            const uint64_t theirs = told(st + 2 + k), mine = lds_get<uint64_t>(clk + (uint32_t)k * 8u);
+            differ = differ || theirs != mine;
+            same = same && alike(theirs, mine, unseen);
+        }
 #pragma unroll
         for (int i = 0; i < W; ++i) {
             const int m = 64 * i + lane;
@@ -598,6 +606,13 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             }
         }
         if (ballot(!same) != 0ull) return false;
+        if (ballot(differ) != 0ull) {  // the groups' last clocks in the same order
+            const uint32_t slot = in_mask(groups) ? desc_last_slot(group) : 0u;
+            const double mine = lds_get<double>(clk + slot * 8u), theirs = __longlong_as_double((long long)told(st + 2 + slot));
+            for (uint64_t left = groups; left != 0ull; left &= left - 1)
+                same = same && (mine < lane_value(mine, first_of(left))) == (theirs < lane_value(theirs, first_of(left)));
+            if ((ballot(!same) & groups) != 0ull) return false;
+        }
         const double their_t = __longlong_as_double((long long)told(st + at_lanes + lane));
         const uint32_t their_d = (uint32_t)told(st + at_lanes + kWave + lane);
         for (uint64_t left = used; left != 0ull; left &= left - 1) {  // as often there as here
@@ -625,9 +640,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
                 runs.next = at + 1u;
                 return false;
             }
-        } else if (ballot(lane < a.nslots && peeked != lds_get<uint64_t>(clk + (uint32_t)lane * 8u)) == 0ull) {
-            runs.met = agree(st);
-            if (runs.met) return true;
+        } else {
+            const double next = lane_value(t1, 0), unseen = q->alike == 0 ? -1.0 : next_due < next ? next_due : next;
+            if (ballot(lane < a.nslots && !alike(peeked, lds_get<uint64_t>(clk + (uint32_t)lane * 8u), unseen)) == 0ull) {
+                runs.met = agree(st, unseen);
+                if (runs.met) return true;
+            }
         }
         runs.go_on(q, at);
         return false;
