@@ -1369,7 +1369,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
             q.span_blocks = (int32_t)span_blocks;
             q.ext_blocks = std::max(q.span_blocks / 2, kLeastExt);
             for (q.marks = 0; span_mark(q.marks) < q.span_blocks;) ++q.marks;
-            q.state_words = 2 + nslots + M + 4 * kWave + M;
+            q.state_words = 2 + nslots + M + 5 * kWave + M;
             q.alike = t->fixed_overhead >= 0.0 ? 1 : 0;
             for (int s = 0; s < n_seeds; ++s)
                 if (!wls[s]->sorted) q.alike = 0;

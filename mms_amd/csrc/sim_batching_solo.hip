@@ -249,7 +249,17 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     double next_due = inf;      // the earliest event's time
     int32_t requests_of_group = 0, good_of_group = 0;  // lane g (a count in global memory would be waited for in every batch)
     int32_t n_good = 0;
-    double lat_sum = 0.0;       // of the batch members this lane accounts for
+    // Of the batch members this lane accounts for.  SPANS: and what its roundings left out (Knuth's two-sum).  Where one run takes over from
+    // another depends on which marks were there in time: with 106 bits the sum of all of them is the same wherever that was.
+    double lat_sum = 0.0, lat_rest = 0.0;
+    auto add_latency = [&](double x) {
+        const double sum = lat_sum + x;
+        if constexpr (SPANS) {
+            const double of_x = sum - lat_sum;
+            lat_rest += (lat_sum - (sum - of_x)) + (x - of_x);
+        }
+        lat_sum = sum;
+    };
     int dead = 0;
     const int cand = a.batch_sizes[lane < NB ? lane : NB - 1], cand_col = ilog2i(cand);  // lane q: batch size q and its latency column
     const bool sizes_pow2 = ballot(lane < NB && cand != 1 << lane) == 0ull;
@@ -460,10 +470,10 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             wave_order();
             if (left == arr) set_waiting(m, false);
             // (sums by place in the queue, see above)
-            if (lane >= kfirst && lane < kfirst + bs && lane < 8) lat_sum += t - hv.x;
+            if (lane >= kfirst && lane < kfirst + bs && lane < 8) add_latency(t - hv.x);
             for (int k = 8; rarely(k < kb); ++k) {
                 const double at = k < 16 ? lane_value(hv.x, k) : mq[(size_t)first + (uint32_t)(k - kfirst)].t;
-                if (lane == 0) lat_sum += t - at;
+                if (lane == 0) add_latency(t - at);
             }
             if (want_req) {
                 if (lane >= kfirst && lane < kb && lane < 16) {
@@ -553,7 +563,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             for (int i = 0; i < W; ++i) hosted_models[i] |= lane_value(members[i], g);
     }
     // A state, 64-bit words: accepted requests, event slots in use, clocks, queues {head, behind the last arrival}; a lane each: time and
-    // group of the events, latency sums; with counts groups {requests, accepted} (lanes) and models
+    // group of the events, latency sums and what they left out; with counts groups {requests, accepted} (lanes) and models
     auto marked = [&](int r, int i) {
         ColdArgs *q = cold_args<BatchingArgs>();
         return q->mark_state + (((size_t)wave * q->spans + r) * q->marks + i) * (size_t)q->state_words;
@@ -576,13 +586,14 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         for (int m = lane; m < M; m += kWave) {
             const u32x4 queue = lds_get<u32x4>(queues + (uint32_t)m * 16u);
             tell(st + at_queues + m, (uint64_t)queue.z << 32 | queue.y);
-            if (OUTPUTS) tell(st + at_lanes + 4 * kWave + m, (uint64_t)queue.x);
+            if (OUTPUTS) tell(st + at_lanes + 5 * kWave + m, (uint64_t)queue.x);
         }
         uint64_t *mine = st + at_lanes + lane;
         tell(mine, (uint64_t)__double_as_longlong(ev_t));
         tell(mine + kWave, (uint64_t)ev_d);
         tell(mine + 2 * kWave, (uint64_t)__double_as_longlong(lat_sum));
-        if (OUTPUTS) tell(mine + 3 * kWave, (uint64_t)(uint32_t)good_of_group << 32 | (uint32_t)requests_of_group);
+        tell(mine + 3 * kWave, (uint64_t)__double_as_longlong(lat_rest));
+        if (OUTPUTS) tell(mine + 4 * kWave, (uint64_t)(uint32_t)good_of_group << 32 | (uint32_t)requests_of_group);
     };
     // Clocks that are equal, or that differ before anything that happens from here on (sim_window.hip): arrivals and idle events.
     auto alike = [](uint64_t x, uint64_t y, double before) -> bool {
@@ -779,7 +790,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             last_one = true;
             for (int k = lane; k <= q->spans; k += kWave) tell(published(k), 0u);  // for the next launch
             n_good = requests_of_group = good_of_group = 0;
-            lat_sum = 0.0;
+            lat_sum = lat_rest = 0.0;
             for (int m = lane; m < M; m += kWave) lds_put<uint32_t>(queues + (uint32_t)m * 16u, 0u);
         } else {
             if (!runs.met) break;
@@ -793,13 +804,17 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             const bool whole = mark < 0;
             n_good += (int32_t)uni((uint32_t)(e[0] - (whole ? 0ull : b[0])));
             const int l = at_lanes + 2 * kWave + lane;
-            lat_sum += __longlong_as_double((long long)e[l]) - (whole ? 0.0 : __longlong_as_double((long long)b[l]));
+            // (A sum that was infinite at the mark: so was a clock, and whoever came to agree with it has an infinite sum as well.)
+            const double sum_before = whole ? 0.0 : __longlong_as_double((long long)b[l]);
+            add_latency(__longlong_as_double((long long)e[l]));
+            if (sum_before < inf) add_latency(-sum_before);
+            lat_rest += __longlong_as_double((long long)e[l + kWave]) - (whole ? 0.0 : __longlong_as_double((long long)b[l + kWave]));
             if constexpr (OUTPUTS) {
-                const uint64_t v = e[l + kWave] - (whole ? 0ull : b[l + kWave]);
+                const uint64_t v = e[l + 2 * kWave] - (whole ? 0ull : b[l + 2 * kWave]);
                 requests_of_group += (int32_t)(uint32_t)v;
                 good_of_group += (int32_t)(v >> 32);
                 for (int m = lane; m < M; m += kWave) {
-                    const int w = at_lanes + 4 * kWave + m;
+                    const int w = at_lanes + 5 * kWave + m;
                     const uint32_t at = queues + (uint32_t)m * 16u;
                     lds_put<uint32_t>(at, lds_get<uint32_t>(at) + (uint32_t)(e[w] - (whole ? 0ull : b[w])));
                 }
@@ -837,7 +852,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         from_w = (int64_t)end * kWave;
     }
 
-    for (int k = 1; k < 8; k *= 2) lat_sum += __hiloint2double(__shfl_xor(__double2hiint(lat_sum), k), __shfl_xor(__double2loint(lat_sum), k));
+    for (int k = 1; k < 8; k *= 2) {
+        auto theirs = [&](double x) -> double { return __hiloint2double(__shfl_xor(__double2hiint(x), k), __shfl_xor(__double2loint(x), k)); };
+        if constexpr (SPANS) lat_rest += theirs(lat_rest);
+        add_latency(theirs(lat_sum));
+    }
+    if constexpr (SPANS) lat_sum += lat_sum < inf ? lat_rest : 0.0;
     if (lane == 0) {
         const size_t out = (size_t)wave;
         a.n_good[out] = n_good;

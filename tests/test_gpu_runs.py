@@ -113,6 +113,7 @@ def test_runs_of_the_batching_simulator(depths, uniform, groups, hosts, M, span)
                 assert np.array_equal(out["n_good"][k], ref["n_good"]), (B, k)
                 for key in ("model_num_good", "group_num_requests", "group_num_good") if flags else ():
                     assert np.array_equal(out[key][k], ref[key]), (B, k, key)
+                assert np.array_equal(out["latency_sum"][k], outs[0]["latency_sum"][k]), (B, k)   # wherever the runs met
                 assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=1e-12, atol=0), (B, k)
     for dw in dws:
         dw.close()
