@@ -147,3 +147,23 @@ def test_clocks_that_no_request_can_tell_apart():
         batch.close()
         assert_batch_matches(out, oracle_batch(st, table, packed), 0, packed[0], where=f"uneven {uneven}")
         dw.close()
+
+
+@pytest.mark.parametrize("faster,cut", [(1.0, True), (60.0, False)])
+def test_streams_that_overload_the_groups_are_not_cut(faster, cut):
+    """Several groups for every model and far more requests than they can take: the same results, one wavefront to a simulation."""
+    eng = E.Engine.default()
+    profiles, sols = _problem(3, (1, 2, 4), True, 9, 6, 12, 4)
+    table = E.LatencyTable(profiles, [1])
+    packed = E.pack_placements(sols, table)
+    st = _with_pauses(11, 12000, 9, 0.8, 120)
+    st.tstamps = st.tstamps / faster
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, 9)
+    batch = E.Batch(eng, [dw], table, packed, COUNTS)
+    assert (batch.kernel_name().count(",") == 6) == cut
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    assert_batch_matches(out, oracle_batch(st, table, packed), 0, packed[0], where=f"faster {faster}")
+    dw.close()
