@@ -364,7 +364,8 @@ typedef struct {
     int32_t launches;         /* kernel launches of one mmsim_batch_run                             */
     int32_t waves_per_group;  /* wavefronts of a workgroup that simulate side by side               */
     int32_t event_slots;      /* batching simulator: idle-event slots per simulation; 0 otherwise   */
-    int32_t reserved;
+    int32_t runs_met_again;       /* simulations cut into runs: how often in the last run one that was given up and taken
+                                     up again met another; 0 otherwise                                      */
 } mmsim_batch_info;
 int mmsim_batch_get_info(const mmsim_batch *batch, mmsim_batch_info *out);
 /* Name of the kernel template instance mmsim_batch_run launches for this batch, as a profiler prints it

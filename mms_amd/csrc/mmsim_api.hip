@@ -1955,7 +1955,16 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {
     out->launches = 1;
     out->waves_per_group = b->waves_per_block;
     out->event_slots = (b->flags & MMSIM_BATCHING) ? b->bargs.heap_cap : 0;
-    out->reserved = 0;
+    out->runs_met_again = 0;
+    if (b->window && b->wargs.spans > 1) {
+        const size_t row = (size_t)b->wargs.spans + kSyncWords;
+        std::vector<uint32_t> words((size_t)b->wargs.tiles * b->out_seeds * row);
+        HIP_TRY(hipSetDevice(b->ctx->device));
+        StreamWait copy(b->ctx->stream);
+        HIP_TRY(hipMemcpyAsync(words.data(), b->wargs.span_sync, sizeof(uint32_t) * words.size(), hipMemcpyDeviceToHost, b->ctx->stream));
+        HIP_TRY(copy.now());
+        for (size_t at = row - 1; at < words.size(); at += row) out->runs_met_again += (int32_t)words[at];
+    }
     return MMSIM_OK;
 } catch (...) {
     return caught();

@@ -258,7 +258,8 @@ struct WindowArgs {
     int32_t marks, state_words;      // most marks of a span, 64-bit words of a state
     int32_t alike;                   // clocks that differ before the next arrival may count as equal: arrivals ascend, no latency is negative, up to 64 groups
     int64_t run_cap, true_cap;       // values of a run: 64 * (span_blocks + ext_blocks), and of a whole stream
-    uint32_t *span_sync;             // [L][spans + 1] marks that every run has published, and how many runs have ended: 0 before a launch and after
+    uint32_t *span_sync;             // [L][spans + kSyncWords] marks that every run has published, how many runs have ended (0 before a launch and
+                                     // after), and how often a run that was taken up again met another
     uint64_t *mark_state;            // [L][spans][marks][state_words]
     uint64_t *end_state;             // [L][spans][state_words + kEndWords]
     double *run_vals;                // [L][true_cap + (spans - 1) * run_cap] latencies of the requests of a run (finish times, if wanted)
@@ -276,6 +277,7 @@ struct WindowArgs {
 __host__ __device__ constexpr int window_ring_bytes(int lanes) { return lanes == kWave ? 0 : 2 * kWave * (int)sizeof(Req); }
 constexpr int kMaxWindowWaves = 4;  // wavefronts of a workgroup
 constexpr int kEndWords = 2;        // of end_state: end block, link
+constexpr int kSyncWords = 2;       // of span_sync, beside the runs'
 constexpr int kSumWaves = 4;        // wavefronts that put a simulation's runs together
 constexpr int kMaxSpans = 64;       // most runs of a simulation (their records are a lane's each)
 constexpr int32_t kLeastSpan = 20, kLeastExt = 48;  // blocks of a span, and what a run may go on behind its span, at least

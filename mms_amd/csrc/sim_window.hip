@@ -544,7 +544,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
     // Something happens before block `at`: a mark of this run, one of a later run or the block ahead of it, the end of the run (true).
     auto published = [&](int r) {
         ColdArgs *q = cold_args<WindowArgs>();
-        return q->span_sync + (size_t)sim * (q->spans + 1) + r;
+        return q->span_sync + (size_t)sim * (q->spans + kSyncWords) + r;
     };
     uint64_t peeked = 0;
     auto event = [&](uint32_t at) -> bool {
@@ -603,6 +603,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
     double *run_vals = SPANS ? values_of(cold_args<WindowArgs>(), sim, own) : nullptr;  // by place in the stream
     uint32_t num_pieces = 0;
     bool last = false;  // this wavefront puts the simulation together
+    uint32_t met_again = 0;
     for (;;) {
         if (from < R) start_at(from);
         for (blk = from; blk < R; blk += W) {
@@ -938,12 +939,11 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             uint32_t before_me = 0;
             if (lane == 0)
-                before_me = __hip_atomic_fetch_add(q->span_sync + (size_t)sim * (q->spans + 1) + q->spans, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                before_me = __hip_atomic_fetch_add(published(q->spans), 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
             if (__builtin_amdgcn_readfirstlane(before_me) + 1u != (uint32_t)q->spans) return;
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // All runs have ended: this wavefront follows them from the first on.
             last = true;
-            for (int k = j; k <= q->spans; k += W) tell(q->span_sync + (size_t)sim * (q->spans + 1) + k, 0u);  // for the next launch
             n_good = 0;
             if constexpr (OUTPUTS) {
                 for (int k = j; k < q->nslots; k += W) lds_put<uint64_t>(clk + (uint32_t)k * 8u + cnt_rel, 0ull);
@@ -953,6 +953,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
             if (lane == 0) piece(num_pieces, from / 64u, blk < R ? blk / 64u : (R + 63u) / 64u, 0);
             num_pieces += 1;
             if (!runs.met) break;
+            met_again += 1;
             first = runs.in;
             first_mark = runs.mark;
         }
@@ -1013,8 +1014,14 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         run_vals = values_of(q, sim, 0);
     }
 
-    if constexpr (!SPANS)
+    if constexpr (SPANS) {
+        // For the next launch; not before: a run that is taken up again looks at the marks.
+        ColdArgs *q = cold_args<WindowArgs>();
+        for (int k = j; k <= q->spans; k += W) tell(published(k), 0u);
+        if (j == 0) tell(published(q->spans + 1), met_again);
+    } else {
         for (int d = 1; d < W; d *= 2) n_good += shfl_xor<W>(n_good, d);
+    }
     if (!mine) return;
     if (j == 0) {
         a.n_good[row] = n_good;

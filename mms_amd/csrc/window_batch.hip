@@ -126,7 +126,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     const size_t at_lat = in.take(sizeof(float) * (cl.lat.size() + MMSIM_MAX_STAGES));  // (the walk reads past a shallow group's row)
     const int64_t blocks = (longest + kWave - 1) / kWave;
     const bool may_cut = !g_arena && (o.window_lanes > 0 ? o.segment_requests > 0 : blocks >= 6 * kLeastSpan);
-    const size_t at_sync = in.take(may_cut ? sizeof(uint32_t) * (size_t)(sims + std::min<int64_t>(kMaxRuns, sims * kMaxSpans)) : 0);
+    const size_t at_sync = in.take(may_cut ? sizeof(uint32_t) * (size_t)(sims * kSyncWords + std::min<int64_t>(kMaxRuns, sims * kMaxSpans)) : 0);
     HIP_TRY(hipSetDevice(ctx->device));
     std::vector<unsigned char> plain;  // (read until the wait below)
     if (g_arena)
@@ -395,7 +395,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     }
     std::memcpy(host + at_lat, cl.lat.data(), sizeof(float) * cl.lat.size());
 
-    std::memset(host + at_sync, 0, spans > 1 ? sizeof(uint32_t) * (size_t)(units * (spans + 1)) : 0);
+    std::memset(host + at_sync, 0, spans > 1 ? sizeof(uint32_t) * (size_t)(units * (spans + kSyncWords)) : 0);
 
     // ---- outputs: one buffer, laid out as the caller's arrays
     Layout res;

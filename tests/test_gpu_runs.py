@@ -23,6 +23,56 @@ def _with_pauses(seed, R, M, load, every, pause=4.0, quiet_until=1.0):
     return st
 
 
+def _busy_between(seed, R, M, load, first, end):
+    """Pauses in which the groups catch up, but for the requests [first, end), which come ``load`` times as fast."""
+    st = _with_pauses(seed, R, M, 0.6, 10 ** 9)
+    rng = np.random.default_rng(seed + 2)
+    gaps = np.diff(st.tstamps, prepend=0.0)
+    busy = (np.arange(R) >= first) & (np.arange(R) < end)
+    gaps[busy] *= 0.6 / load
+    gaps[(rng.random(R) < 1.0 / 150) & ~busy] += 4.0
+    st.tstamps = np.cumsum(gaps)
+    st.slos = np.where(np.isfinite(st.slos), st.slos, np.float32(0.5))        # (a clock that an infinite one drove up stays up)
+    return st
+
+
+@pytest.mark.parametrize("depths,uniform,groups,hosts", [((1,), True, 6, 7), ((1, 2, 4), True, 6, 8), ((1, 3, 4), False, 9, 7)])
+def test_runs_taken_up_again_meet_others(depths, uniform, groups, hosts):
+    """Requests that overload several groups of every model for longer than a run may go on behind its span, twice, and pauses before,
+    between and behind: runs are given up and taken up again, and those meet the runs that started in the pauses."""
+    eng = E.Engine.default()
+    M, span = 9, 512
+    streams = [_busy_between(31 + k, 300 * 64 + 17, M, 3.0, 60 * 64, 170 * 64) for k in range(2)] + [_with_pauses(40, 200 * 64, M, 0.6, 100)]
+    streams.append(_busy_between(33, 400 * 64, M, 3.0, 40 * 64, 130 * 64))
+    late = _busy_between(34, 400 * 64, M, 3.0, 200 * 64, 290 * 64)
+    gaps = np.diff(streams[3].tstamps, prepend=0.0)
+    gaps[180 * 64:] = np.diff(late.tstamps, prepend=0.0)[180 * 64:]
+    streams[3].tstamps = np.cumsum(gaps)
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    for B, flags in ((24, COUNTS), (9, COUNTS | _lib.WANT_PER_REQUEST), (40, 0)):
+        profiles, sols = _problem(B + sum(depths), depths, uniform, M, groups, B, hosts)
+        table = E.LatencyTable(profiles, [1])
+        packed = E.pack_placements(sols, table)
+        batch = E.Batch(eng, dws, table, packed, flags, options=dict(window_lanes=64, segment_requests=span))
+        assert batch.kernel_name().count(",") == 6            # (the last one: cut into runs)
+        outs = []
+        for _ in range(3):
+            batch.run()
+            batch.sync()
+            assert batch.info()["runs_met_again"] > 0
+            outs.append(batch.fetch())
+        batch.close()
+        for k, st in enumerate(streams):
+            ref = oracle_batch(st, table, packed, want_per_request=bool(flags & _lib.WANT_PER_REQUEST))
+            for out in outs:
+                if flags & _lib.WANT_PER_REQUEST:
+                    R = len(st.tstamps)
+                    assert np.array_equal(out["good"][k][:, :R], ref["good"]) and np.array_equal(out["finish"][k][:, :R], ref["finish"])
+                assert_batch_matches(out, ref, k, packed[0], where=f"B={B}, stream {k}")
+    for dw in dws:
+        dw.close()
+
+
 @pytest.mark.parametrize("depths,uniform,groups,hosts,M", [((1,), True, 6, 4, 9), ((1,), True, 40, 5, 5), ((1, 2, 4), True, 5, 4, 9),
                                                            ((1, 3, 4), False, 9, 5, 5), ((1, 2, 4, 8, 16), True, 7, 4, 9), ((8, 32), True, 6, 4, 9)])
 @pytest.mark.parametrize("span", [512, 1024])
