@@ -1376,7 +1376,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
             for (const float l : lat_nb)
                 if (!(l >= 0.0f)) q.alike = 0;
             const size_t marks = 8 * n * (size_t)q.marks * (size_t)q.state_words, ends = 8 * n * (size_t)(q.state_words + kEndWords),
-                         sync = 4 * L * (size_t)(runs_of + 1);
+                         sync = 4 * L * (size_t)(runs_of + kSyncWords);
             HIP_TRY(b->run_memory.alloc(marks + ends + sync));
             HIP_TRY(hipMemsetAsync(b->run_memory.p + marks + ends, 0, sync, st));
             q.mark_state = reinterpret_cast<uint64_t *>(b->run_memory.p);
@@ -1956,12 +1956,14 @@ int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {
     out->waves_per_group = b->waves_per_block;
     out->event_slots = (b->flags & MMSIM_BATCHING) ? b->bargs.heap_cap : 0;
     out->runs_met_again = 0;
-    if (b->window && b->wargs.spans > 1) {
-        const size_t row = (size_t)b->wargs.spans + kSyncWords;
-        std::vector<uint32_t> words((size_t)b->wargs.tiles * b->out_seeds * row);
+    const int32_t spans = b->window ? b->wargs.spans : (b->flags & MMSIM_BATCHING) ? b->bargs.spans : 1;
+    if (spans > 1) {
+        const uint32_t *sync = b->window ? b->wargs.span_sync : b->bargs.span_sync;
+        const size_t row = (size_t)spans + kSyncWords;
+        std::vector<uint32_t> words((size_t)b->tiles * b->out_seeds * row);
         HIP_TRY(hipSetDevice(b->ctx->device));
         StreamWait copy(b->ctx->stream);
-        HIP_TRY(hipMemcpyAsync(words.data(), b->wargs.span_sync, sizeof(uint32_t) * words.size(), hipMemcpyDeviceToHost, b->ctx->stream));
+        HIP_TRY(hipMemcpyAsync(words.data(), sync, sizeof(uint32_t) * words.size(), hipMemcpyDeviceToHost, b->ctx->stream));
         HIP_TRY(copy.now());
         for (size_t at = row - 1; at < words.size(); at += row) out->runs_met_again += (int32_t)words[at];
     }

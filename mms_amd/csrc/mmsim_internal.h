@@ -217,7 +217,7 @@ struct BatchingArgs {
     uint32_t flags;
     // simulations cut into runs (solo), as in WindowArgs
     int32_t spans, span_blocks, ext_blocks, marks, state_words, alike;
-    uint32_t *span_sync;
+    uint32_t *span_sync;         // as there
     uint64_t *mark_state, *end_state;
     // outputs
     int32_t *n_good;             // [n_seeds][tiles*row]

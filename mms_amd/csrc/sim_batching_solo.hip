@@ -574,7 +574,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     };
     auto published = [&](int r) {
         ColdArgs *q = cold_args<BatchingArgs>();
-        return q->span_sync + (size_t)wave * (q->spans + 1) + r;
+        return q->span_sync + (size_t)wave * (q->spans + kSyncWords) + r;
     };
     const int at_queues = 2 + a.nslots, at_lanes = at_queues + M;  // where the queues and the lanes' words begin
     auto save = [&](uint64_t *st) {
@@ -663,6 +663,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     };
     int64_t from_w = start, w0 = start;
     bool last_one = false;  // this wavefront puts the simulation together
+    uint32_t met_again = 0;
     for (;;) {
         bool cut = false;
         if (from_w < R) start_at(from_w);
@@ -788,12 +789,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // All runs have ended: this wavefront follows them from the first on.
             last_one = true;
-            for (int k = lane; k <= q->spans; k += kWave) tell(published(k), 0u);  // for the next launch
             n_good = requests_of_group = good_of_group = 0;
             lat_sum = lat_rest = 0.0;
             for (int m = lane; m < M; m += kWave) lds_put<uint32_t>(queues + (uint32_t)m * 16u, 0u);
         } else {
             if (!runs.met) break;
+            met_again += 1;
             first = runs.in;
             first_mark = runs.mark;
         }
@@ -850,6 +851,12 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
         wave_order();
         runs.resume(q, end);
         from_w = (int64_t)end * kWave;
+    }
+    if constexpr (SPANS) {
+        // For the next launch; not before: a run that is taken up again looks at the marks.
+        ColdArgs *q = cold_args<BatchingArgs>();
+        for (int k = lane; k <= q->spans; k += kWave) tell(published(k), 0u);
+        if (lane == 0) tell(published(q->spans + 1), met_again);
     }
 
     for (int k = 1; k < 8; k *= 2) {

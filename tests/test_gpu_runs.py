@@ -217,3 +217,42 @@ def test_streams_that_overload_the_groups_are_not_cut(faster, cut):
     batch.close()
     assert_batch_matches(out, oracle_batch(st, table, packed), 0, packed[0], where=f"faster {faster}")
     dw.close()
+
+
+@pytest.mark.parametrize("depths,uniform,groups,hosts,M", [((1,), True, 6, 7, 9), ((1, 2, 4), True, 6, 8, 9), ((1, 3, 5), False, 12, 9, 70)])
+def test_runs_of_the_batching_simulator_taken_up_again(depths, uniform, groups, hosts, M):
+    """As test_runs_taken_up_again_meet_others; latency sums within the bound above (25600 requests: 2.9e-12)."""
+    eng = E.Engine.default()
+    span, sizes = 512, [1, 2, 4, 8]
+    streams = [_busy_between(51 + k, 300 * 64 + 17, M, 12.0, 60 * 64, 170 * 64) for k in range(2)] + [_busy_between(53, 400 * 64, M, 12.0, 40 * 64, 130 * 64)]
+    late = _busy_between(54, 400 * 64, M, 12.0, 200 * 64, 290 * 64)
+    gaps = np.diff(streams[2].tstamps, prepend=0.0)
+    gaps[180 * 64:] = np.diff(late.tstamps, prepend=0.0)[180 * 64:]
+    streams[2].tstamps = np.cumsum(gaps)
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    for B, flags in ((24, COUNTS), (40, 0)):
+        profiles, sols = _problem(B + sum(depths), depths, uniform, M, groups, B, hosts)
+        for p in profiles:
+            for d in p.para_dict.values():
+                for b in sizes[1:]:
+                    d.latency[b] = [x * (1 + 0.15 * (b - 1)) for x in d.latency[1]]
+        table = E.LatencyTable(profiles, sizes)
+        packed = E.pack_placements(sols, table)
+        batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING, options=dict(segment_requests=span))
+        outs = []
+        for _ in range(3):
+            batch.run()
+            batch.sync()
+            assert batch.info()["runs_met_again"] > 0
+            outs.append(batch.fetch())
+        batch.close()
+        for k, st in enumerate(streams):
+            ref = oracle_batch(st, table, packed, batching=True)
+            for out in outs:
+                assert not out["status"].any() and np.array_equal(out["n_good"][k], ref["n_good"]), (B, k)
+                for key in ("model_num_good", "group_num_requests", "group_num_good") if flags else ():
+                    assert np.array_equal(out[key][k], ref[key]), (B, k, key)
+                assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=3e-12, atol=0), (B, k)
+                assert np.array_equal(out["latency_sum"][k], outs[0]["latency_sum"][k]), (B, k)
+    for dw in dws:
+        dw.close()
