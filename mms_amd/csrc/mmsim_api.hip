@@ -1924,7 +1924,9 @@ void mmsim_batch_destroy(mmsim_batch *b) {
         (void)hipStreamSynchronize(b->ctx->stream);
         if (b->window && !b->in_scratch) b->ctx->staging.trim();  // (of a call that failed on the way)
     }
+    mmsim_ctx *ctx = b->ctx;
     delete b;
+    if (ctx) ctx->runs.trim();
 }
 
 int mmsim_batch_get_info(const mmsim_batch *b, mmsim_batch_info *out) try {

@@ -149,6 +149,36 @@ struct Staging {
     }
 };
 
+// What a launch of simulations that are cut into runs has of device memory beside its batch's: no launch needs what another left
+// there, and those of a context follow one another on its stream, so all of its batches share one buffer.
+struct RunMemory {
+    // Most bytes of a launch, and most that are kept while no batch is there that may be run again (a gigabyte costs 0.3 ms to
+    // allocate and free).  A launch takes no more than a quarter of what is free either: it can do without.
+    static constexpr size_t kMost = (size_t)16 << 30, kMostKept = (size_t)2 << 30;
+    DevBuf<uint8_t> buf;
+    int batches = 0;  // that may be run again
+    bool fits(size_t bytes) const {
+        if (bytes <= buf.n) return true;
+        size_t free = 0, total = 0;
+        if (bytes > kMost || hipMemGetInfo(&free, &total) != hipSuccess) return false;
+        return bytes <= (free + buf.n) / 4;
+    }
+    // nullptr: there is no room, simulations are not cut
+    uint8_t *ensure(size_t bytes, hipStream_t stream) {
+        if (bytes <= buf.n) return buf.p;
+        if (!fits(bytes) || hipStreamSynchronize(stream) != hipSuccess) return nullptr;  // (a launch before this one may still use it)
+        if (buf.alloc(bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            buf.release();
+            return nullptr;
+        }
+        return buf.p;
+    }
+    void trim() {
+        if (batches == 0 && buf.n > kMostKept) buf.release();
+    }
+};
+
 // Runs fn(lo, hi) on slices of [0, n) on up to 16 host threads (one slice per thread; the caller's
 // slices write disjoint memory).  Small ranges run on the calling thread.  What a slice throws is thrown to the caller
 // when all have ended; a slice for which there is no thread runs on the calling one.
@@ -189,7 +219,7 @@ void parallel_slices(int64_t n, int64_t min_per_thread, F &&fn) {
 
 struct mmsim_ctx {
     Staging staging;
-    mmsim::DevBuf<uint8_t> runs;           // of simulations that are cut into runs (window_batch.hip): no launch needs another's
+    RunMemory runs;
     int device = 0;
     hipStream_t stream = nullptr;
     hipDeviceProp_t prop{};
@@ -345,7 +375,9 @@ struct mmsim_batch {
     // Requests side by side (window_batch.hip): all inputs in one buffer, all outputs in another
     bool window = false;
     WindowArgs wargs{};
-    DevBuf<uint8_t> win_in, win_out, win_runs;
+    DevBuf<uint8_t> win_in, win_out;
+    size_t run_bytes = 0, run_ends = 0, run_pieces = 0, run_vals = 0;  // simulations cut into runs: of RunMemory, and offsets there
+    RunMemory *runs_again = nullptr;                                   // ... of a batch that may be run again
     DevBuf<uint8_t> run_memory;  // batching simulator: of simulations cut into runs
     std::vector<std::shared_ptr<DevBuf<Req>>> win_streams;
     size_t win_lat_sum = 0, win_model = 0, win_group = 0, win_finish = 0, win_good = 0;  // offsets in win_out (n_good: 0)
@@ -357,9 +389,14 @@ struct mmsim_batch {
     bool ran = false;
     mmsim_options opt{};     // the options the batch was built with
 
+    void run_again(RunMemory *runs) {
+        runs_again = runs;
+        runs->batches += 1;
+    }
     ~mmsim_batch() {
         if (own_events && ev_start) (void)hipEventDestroy(ev_start);
         if (own_events && ev_stop) (void)hipEventDestroy(ev_stop);
+        if (runs_again) --runs_again->batches;
     }
 };
 

@@ -63,10 +63,6 @@ struct Shape {
 
 }  // namespace
 
-// How many bytes the runs of a launch may take, and how many a context keeps for the next call (a gigabyte costs 0.3 ms to
-// allocate and free).
-constexpr size_t kMostRunBytes = (size_t)16 << 30, kMostRunsKept = (size_t)2 << 30;
-
 int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_seeds, const mmsim_tables *t,
                  const mmsim_placements *p, const int32_t *stream_of, uint32_t flags, const mmsim_options &o, bool events,
                  mmsim_batch **out) {
@@ -333,25 +329,13 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         if (o.window_lanes > 0) spans = blocks / std::max<int64_t>(8, o.segment_requests / kWave);
     }
     cut(std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / units))));
-    DevBuf<uint8_t> own_runs;  // of a batch that is kept; a call that runs its batch once borrows the context's
-    DevBuf<uint8_t> &run_memory = events ? own_runs : ctx->runs;
-    if (a.spans > 1 && (runs.used > kMostRunBytes || (run_memory.n < runs.used && run_memory.alloc(runs.used) != hipSuccess))) {
-        (void)hipGetLastError();
-        run_memory.release();
-        cut(1);
-    }
+    if (a.spans > 1 && !ctx->runs.fits(runs.used)) cut(1);
     spans = a.spans;
     a.alike = Gmax <= kWave ? 1 : 0;
     for (int s = 0; s < n_seeds; ++s)
         if (!wls[s]->sorted) a.alike = 0;
     for (const float l : cl.lat)
         if (!(l >= 0.0f)) a.alike = 0;
-    if (spans > 1) {
-        a.mark_state = reinterpret_cast<uint64_t *>(run_memory.p);
-        a.end_state = reinterpret_cast<uint64_t *>(run_memory.p + at_ends);
-        a.pieces = reinterpret_cast<uint32_t *>(run_memory.p + at_pieces);
-        a.run_vals = reinterpret_cast<double *>(run_memory.p + at_vals);
-    }
     const int64_t wave_units = units * spans;
     int waves = spans > 1 ? (int)std::min<int64_t>(kMaxWindowWaves, std::max<int64_t>(1, (wave_units + cus - 1) / cus)) : waves_for(lanes);
     while (spans > 1 && waves > 1 && lat_lds + wave_lds(lanes) * (size_t)waves > lds) --waves;
@@ -461,10 +445,12 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
     a.finish = reinterpret_cast<double *>(r + b->win_finish);
     a.good = r + b->win_good;
     b->wargs = a;
-    if (events && spans > 1) {
-        b->win_runs.p = own_runs.p;
-        b->win_runs.n = own_runs.n;
-        own_runs.owned = false;
+    if (spans > 1) {
+        b->run_bytes = runs.used;
+        b->run_ends = at_ends;
+        b->run_pieces = at_pieces;
+        b->run_vals = at_vals;
+        if (events) b->run_again(&ctx->runs);
     }
     unless_made.staging = nullptr;
     *out = b.release();
@@ -478,6 +464,18 @@ std::string sim_window_kernel_name(const WindowArgs &a) {
 }
 
 int run_window(mmsim_batch *b) {
+    WindowArgs &a = b->wargs;
+    if (a.spans > 1) {
+        if (uint8_t *at = b->ctx->runs.ensure(b->run_bytes, b->ctx->stream)) {
+            a.mark_state = reinterpret_cast<uint64_t *>(at);
+            a.end_state = reinterpret_cast<uint64_t *>(at + b->run_ends);
+            a.pieces = reinterpret_cast<uint32_t *>(at + b->run_pieces);
+            a.run_vals = reinterpret_cast<double *>(at + b->run_vals);
+        } else {  // not cut from here on
+            b->waves /= a.spans;
+            a.spans = 1;
+        }
+    }
     if (b->ev_start) HIP_TRY(hipEventRecord(b->ev_start, b->ctx->stream));
     const hipError_t e = launch_window(b->wargs, b->waves_per_block, b->lds_bytes, b->ctx->stream);
     if (e == hipErrorInvalidKernelFile) return fail(MMSIM_E_HIP, "simulation kernel: dynamic LDS does not start at address 0");
@@ -523,7 +521,6 @@ int fetch_window(mmsim_batch *b, mmsim_result *out) {
         std::memcpy(out->group_num_good, host + b->win_group + sizeof(int32_t) * L * G, sizeof(int32_t) * L * G);
     }
     if (!b->in_scratch) stage.trim();
-    if (b->ctx->runs.n > kMostRunsKept) b->ctx->runs.release();
     return MMSIM_OK;
 }
 

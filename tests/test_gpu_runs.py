@@ -2,6 +2,8 @@
 with pauses, in which neighbouring runs come to agree, streams that overload the groups all along, where none do and the first
 run goes through the whole stream, and streams of both, where runs are given up and taken up again; streams that end inside a
 span, at its edge and before it; all outputs."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -256,3 +258,68 @@ def test_runs_of_the_batching_simulator_taken_up_again(depths, uniform, groups, 
                 assert np.array_equal(out["latency_sum"][k], outs[0]["latency_sum"][k]), (B, k)
     for dw in dws:
         dw.close()
+
+
+def _hip():
+    """The HIP runtime that the library runs on (torch brings another one)."""
+    with open("/proc/self/maps") as f:
+        return C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_batches_share_the_memory_of_their_runs():
+    """The runs of a batch that is kept are in memory of the context: three batches hold as much of it as the largest, they may be run
+    in any order, and what one call needed beyond 2 GiB is given back."""
+    eng = E.Engine(0)                                     # (no memory of other tests' runs)
+    profiles, sols = _problem(3, (1, 2, 4), True, 9, 6, 200, 4)
+    table = E.LatencyTable(profiles, [1])
+    st = _with_pauses(71, 60000, 9, 0.8, 120)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, 9)
+    packed = [E.pack_placements(sols[:n], table) for n in (60, 200, 120)]
+    refs = [oracle_batch(st, table, p) for p in packed]
+    before = _free_bytes()
+    batches = [E.Batch(eng, [dw], table, p, COUNTS) for p in packed]
+    for b in batches:
+        assert b.kernel_name().count(",") == 6            # (the last one: cut into runs)
+    for k in (0, 1, 2, 0, 1):
+        batches[k].run()
+    for k in (0, 1, 2):
+        assert_batch_matches(batches[k].fetch(), refs[k], 0, packed[k][0], where=f"batch {k}")
+    # 60000 requests have 2.5 values of eight bytes at most each in 200 simulations (240 MB), marks and ends a tenth of that
+    assert before - _free_bytes() < 300 << 20
+    for b in batches:
+        b.close()
+    dw.close()
+    eng.close()
+
+
+def test_simulations_are_not_cut_where_there_is_no_memory_for_their_runs():
+    eng = E.Engine(0)
+    profiles, sols = _problem(3, (1, 2, 4), True, 9, 6, 300, 4)
+    table = E.LatencyTable(profiles, [1])
+    st = _with_pauses(71, 60000, 9, 0.8, 120)
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, 9)
+    packed = E.pack_placements(sols, table)
+    ref = oracle_batch(st, table, packed)
+    batch = E.Batch(eng, [dw], table, packed, COUNTS)
+    assert batch.kernel_name().count(",") == 6
+    taken = C.c_void_p()                                  # (a quarter of the rest: 100 MiB)
+    assert _hip().hipMalloc(C.byref(taken), C.c_size_t(_free_bytes() - (400 << 20))) == 0
+    try:
+        late = E.Batch(eng, [dw], table, packed, COUNTS)
+        assert late.kernel_name().count(",") == 5
+        for b in (batch, late):
+            b.run()
+            b.sync()
+            assert b.kernel_name().count(",") == 5
+            assert_batch_matches(b.fetch(), ref, 0, packed[0])
+            b.close()
+    finally:
+        assert _hip().hipFree(taken) == 0
+    dw.close()
+    eng.close()
