@@ -932,7 +932,7 @@ hipError_t launch_sim_batching_solo<kRuns>(const BatchingArgs &args, int wpb, si
 #ifndef MMSIM_SOLO_RUNS
 std::string sim_batching_solo_kernel_name(const BatchingArgs &args) {
     return std::string("sim_batching_solo_kernel<") + (args.lat_lds_bytes > 0 ? "true, " : "false, ") +
-           (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.solo == 2 ? "0>" : args.M <= 64 ? "1>" : args.M <= 128 ? "2>" : args.M <= 256 ? "4>" : "8>");
+           (args.uniform_stages != 0 ? "true, " : "false, ") + (solo_outputs(args) ? "true, " : "false, ") + (args.solo == 2 ? "0" : args.M <= 64 ? "1" : args.M <= 128 ? "2" : args.M <= 256 ? "4" : "8") + (args.spans > 1 ? ", true>" : ">");
 }
 #endif
 

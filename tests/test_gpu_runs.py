@@ -151,7 +151,7 @@ def test_runs_of_the_batching_simulator(depths, uniform, groups, hosts, M, span)
         table = E.LatencyTable(profiles, sizes)
         packed = E.pack_placements(sols, table)
         batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING, options=dict(segment_requests=span))
-        assert batch.kernel_name().startswith("sim_batching_solo_kernel<") and batch.info()["workgroups"] >= 0
+        assert batch.kernel_name().startswith("sim_batching_solo_kernel<") and batch.kernel_name().count(",") == 4    # (the last one: cut into runs)
         outs = []
         for _ in range(3):
             batch.run()
@@ -241,6 +241,7 @@ def test_runs_of_the_batching_simulator_taken_up_again(depths, uniform, groups, 
         table = E.LatencyTable(profiles, sizes)
         packed = E.pack_placements(sols, table)
         batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING, options=dict(segment_requests=span))
+        assert batch.kernel_name().count(",") == 4            # (the last one: cut into runs)
         outs = []
         for _ in range(3):
             batch.run()
@@ -256,6 +257,46 @@ def test_runs_of_the_batching_simulator_taken_up_again(depths, uniform, groups, 
                     assert np.array_equal(out[key][k], ref[key]), (B, k, key)
                 assert np.allclose(out["latency_sum"][k], ref["latency_sum"], rtol=3e-12, atol=0), (B, k)
                 assert np.array_equal(out["latency_sum"][k], outs[0]["latency_sum"][k]), (B, k)
+    for dw in dws:
+        dw.close()
+
+
+def test_where_simulations_of_the_batching_simulator_are_cut_by_themselves():
+    """Few simulations of long streams, on every stream and paired; not with per-request outputs, and not short streams."""
+    eng = E.Engine.default()
+    M, sizes = 9, [1, 2, 4, 8]
+    profiles, sols = _problem(3, (1, 2, 4), True, M, 6, 12, 4)
+    for p in profiles:
+        for d in p.para_dict.values():
+            for b in sizes[1:]:
+                d.latency[b] = [x * (1 + 0.15 * (b - 1)) for x in d.latency[1]]
+    table = E.LatencyTable(profiles, sizes)
+    packed = E.pack_placements(sols, table)
+    streams = [_with_pauses(11, 20000, M, 0.8, 120), _with_pauses(12, 9000, M, 0.8, 120)]
+    for s in streams:
+        s.slos = np.where(np.isfinite(s.slos), s.slos, np.float32(0.4))
+    dws = [E.DeviceWorkload(eng, s.tstamps, s.model_ids, s.slos, M) for s in streams]
+    refs = [oracle_batch(s, table, packed, batching=True) for s in streams]
+    for flags in (0, COUNTS):
+        batch = E.Batch(eng, dws, table, packed, flags | _lib.BATCHING)
+        assert batch.kernel_name().count(",") == 4            # (the last one: cut into runs)
+        batch.run()
+        batch.sync()
+        out = batch.fetch()
+        batch.close()
+        for k in range(2):
+            assert np.array_equal(out["n_good"][k], refs[k]["n_good"])
+            assert np.allclose(out["latency_sum"][k], refs[k]["latency_sum"], rtol=3e-12, atol=0)     # (20000 requests, see above)
+            for key in ("model_num_good", "group_num_requests", "group_num_good") if flags else ():
+                assert np.array_equal(out[key][k], refs[k][key]), key
+    of = np.arange(len(sols)) % 2
+    got = E.eval_pairs(eng, dws, table, packed, of, COUNTS | _lib.BATCHING)
+    for key in ("n_good", "model_num_good", "group_num_requests", "group_num_good"):
+        assert np.array_equal(got[key], np.where((of == 0).reshape((-1,) + (1,) * (refs[0][key].ndim - 1)), refs[0][key], refs[1][key])), key
+    for loads, flags in ((dws, COUNTS | _lib.WANT_PER_REQUEST), ([E.DeviceWorkload(eng, streams[0].tstamps[:7616], streams[0].model_ids[:7616], streams[0].slos[:7616], M)], 0)):
+        batch = E.Batch(eng, loads, table, packed, flags | _lib.BATCHING)
+        assert batch.kernel_name().count(",") == 3
+        batch.close()
     for dw in dws:
         dw.close()
 
