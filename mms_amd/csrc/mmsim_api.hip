@@ -1093,7 +1093,8 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
     //      idle SIMD loses more than one that reads these tables through the caches.
     size_t batching_lat_lds = 0;
     int batching_g2m_lds = 0, runs_of = 1;  // runs_of: a simulation's
-    int64_t span_blocks = 1;
+    int32_t span_blocks = 1, span_marks = 0;
+    const int32_t state_words = 2 + nslots + M + 5 * kWave + M;
     if (batching) {
         const size_t lat_b = (lat_nb.size() * sizeof(float) + 15) & ~(size_t)15;
         const size_t g2m_b = solo ? (solo_masks ? 0 : ((size_t)members_max * 2 + 15) & ~(size_t)15) : ((size_t)(Gmax + 1) * blanes * 2 + (size_t)members_max * blanes * 2 + 15) & ~(size_t)15;
@@ -1108,8 +1109,13 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
                                   : blocks >= 6 * kLeastSpan ? std::min((12 * cus + cus / 2) / b->waves, blocks / kLeastSpan)
                                                              : 1;
             runs_of = (int)std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / b->waves)));
-            span_blocks = std::max<int64_t>((blocks + runs_of - 1) / runs_of, 1);
+            span_blocks = (int32_t)std::max<int64_t>((blocks + runs_of - 1) / runs_of, 1);
             runs_of = (int)std::max<int64_t>((blocks + span_blocks - 1) / span_blocks, 1);
+            while (span_mark(span_marks) < span_blocks) ++span_marks;
+            const size_t n = (size_t)b->waves * (size_t)runs_of;
+            b->run_ends = 8 * n * (size_t)span_marks * (size_t)state_words;
+            b->run_bytes = b->run_ends + 8 * n * (size_t)(state_words + kEndWords);
+            if (runs_of > 1 && !ctx->runs.fits(b->run_bytes)) runs_of = 1;
         }
         const int64_t wavefronts = (int64_t)b->waves * runs_of;
         // (no more wavefronts to a CU than there are for it: few of them take a CU each, and all its LDS)
@@ -1365,23 +1371,19 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
         q.solo = !solo ? 0 : solo_masks ? 1 : 2;
         q.spans = runs_of;
         if (runs_of > 1) {
-            const size_t L = (size_t)b->waves, n = L * (size_t)runs_of;
-            q.span_blocks = (int32_t)span_blocks;
+            q.span_blocks = span_blocks;
             q.ext_blocks = std::max(q.span_blocks / 2, kLeastExt);
-            for (q.marks = 0; span_mark(q.marks) < q.span_blocks;) ++q.marks;
-            q.state_words = 2 + nslots + M + 5 * kWave + M;
+            q.marks = span_marks;
+            q.state_words = state_words;
             q.alike = t->fixed_overhead >= 0.0 ? 1 : 0;
             for (int s = 0; s < n_seeds; ++s)
                 if (!wls[s]->sorted) q.alike = 0;
             for (const float l : lat_nb)
                 if (!(l >= 0.0f)) q.alike = 0;
-            const size_t marks = 8 * n * (size_t)q.marks * (size_t)q.state_words, ends = 8 * n * (size_t)(q.state_words + kEndWords),
-                         sync = 4 * L * (size_t)(runs_of + kSyncWords);
-            HIP_TRY(b->run_memory.alloc(marks + ends + sync));
-            HIP_TRY(hipMemsetAsync(b->run_memory.p + marks + ends, 0, sync, st));
-            q.mark_state = reinterpret_cast<uint64_t *>(b->run_memory.p);
-            q.end_state = reinterpret_cast<uint64_t *>(b->run_memory.p + marks);
-            q.span_sync = reinterpret_cast<uint32_t *>(b->run_memory.p + marks + ends);
+            HIP_TRY(b->run_sync.alloc((size_t)b->waves * (size_t)(runs_of + kSyncWords)));
+            HIP_TRY(hipMemsetAsync(b->run_sync.p, 0, b->run_sync.bytes(), st));
+            q.span_sync = b->run_sync.p;
+            b->run_again(&ctx->runs);
         }
         q.uniform_stages = uniform_stages ? 1 : 0;
         q.tile_seed = b->tile_seed.p;
@@ -1646,6 +1648,14 @@ int mmsim_batch_run(mmsim_batch *b) try {
     mmsim_ctx *ctx = b->ctx;
     HIP_TRY(hipSetDevice(ctx->device));
     if (b->window) return run_window(b);
+    if ((b->flags & MMSIM_BATCHING) && b->bargs.spans > 1) {
+        if (uint8_t *at = ctx->runs.ensure(b->run_bytes, ctx->stream)) {
+            b->bargs.mark_state = reinterpret_cast<uint64_t *>(at);
+            b->bargs.end_state = reinterpret_cast<uint64_t *>(at + b->run_ends);
+        } else {
+            b->bargs.spans = 1;  // not cut from here on
+        }
+    }
     if (b->flags & MMSIM_WANT_MODEL_COUNTS)
         HIP_TRY(hipMemsetAsync(b->model_good.p, 0, b->model_good.bytes(), ctx->stream));
     if (b->group_by_slot) {

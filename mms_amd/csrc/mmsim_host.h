@@ -378,7 +378,7 @@ struct mmsim_batch {
     DevBuf<uint8_t> win_in, win_out;
     size_t run_bytes = 0, run_ends = 0, run_pieces = 0, run_vals = 0;  // simulations cut into runs: of RunMemory, and offsets there
     RunMemory *runs_again = nullptr;                                   // ... of a batch that may be run again
-    DevBuf<uint8_t> run_memory;  // batching simulator: of simulations cut into runs
+    DevBuf<uint32_t> run_sync;                                         // ... batching simulator
     std::vector<std::shared_ptr<DevBuf<Req>>> win_streams;
     size_t win_lat_sum = 0, win_model = 0, win_group = 0, win_finish = 0, win_good = 0;  // offsets in win_out (n_good: 0)
 

@@ -3,6 +3,7 @@ with pauses, in which neighbouring runs come to agree, streams that overload the
 run goes through the whole stream, and streams of both, where runs are given up and taken up again; streams that end inside a
 span, at its edge and before it; all outputs."""
 import ctypes as C
+from contextlib import contextmanager
 
 import numpy as np
 import pytest
@@ -313,6 +314,19 @@ def _free_bytes():
     return free.value
 
 
+@contextmanager
+def _no_more_free_than(most):
+    taken = []
+    try:
+        while _free_bytes() > most + (16 << 20) and len(taken) < 8:        # (of a large piece the runtime takes less than asked for)
+            taken.append(C.c_void_p())
+            assert _hip().hipMalloc(C.byref(taken[-1]), C.c_size_t(_free_bytes() - most)) == 0
+        yield
+    finally:
+        for p in taken:
+            assert _hip().hipFree(p) == 0
+
+
 def test_batches_share_the_memory_of_their_runs():
     """The runs of a batch that is kept are in memory of the context: three batches hold as much of it as the largest, they may be run
     in any order, and what one call needed beyond 2 GiB is given back."""
@@ -349,9 +363,7 @@ def test_simulations_are_not_cut_where_there_is_no_memory_for_their_runs():
     ref = oracle_batch(st, table, packed)
     batch = E.Batch(eng, [dw], table, packed, COUNTS)
     assert batch.kernel_name().count(",") == 6
-    taken = C.c_void_p()                                  # (a quarter of the rest: 100 MiB)
-    assert _hip().hipMalloc(C.byref(taken), C.c_size_t(_free_bytes() - (400 << 20))) == 0
-    try:
+    with _no_more_free_than(400 << 20):                   # (a quarter of that: 100 MiB)
         late = E.Batch(eng, [dw], table, packed, COUNTS)
         assert late.kernel_name().count(",") == 5
         for b in (batch, late):
@@ -360,7 +372,37 @@ def test_simulations_are_not_cut_where_there_is_no_memory_for_their_runs():
             assert b.kernel_name().count(",") == 5
             assert_batch_matches(b.fetch(), ref, 0, packed[0])
             b.close()
-    finally:
-        assert _hip().hipFree(taken) == 0
+    dw.close()
+    eng.close()
+
+
+def test_batching_simulations_are_not_cut_where_there_is_no_memory_for_their_runs():
+    """Marks and ends of 3200 runs of 400 models, 146 MB, do not fit into 120 MB."""
+    eng = E.Engine(0)
+    M, sizes = 400, [1, 2, 4, 8]
+    profiles, sols = _problem(3, (1, 2, 4), True, M, 6, 64, 40)
+    for p in profiles:
+        for d in p.para_dict.values():
+            for b in sizes[1:]:
+                d.latency[b] = [x * (1 + 0.15 * (b - 1)) for x in d.latency[1]]
+    table = E.LatencyTable(profiles, sizes)
+    st = _with_pauses(71, 66000, M, 0.8, 120)
+    st.slos = np.where(np.isfinite(st.slos), st.slos, np.float32(0.4))
+    dw = E.DeviceWorkload(eng, st.tstamps, st.model_ids, st.slos, M)
+    packed = E.pack_placements(sols, table)
+    ref = oracle_batch(st, table, packed, batching=True)
+    batch = E.Batch(eng, [dw], table, packed, _lib.BATCHING)
+    assert batch.kernel_name().count(",") == 4
+    with _no_more_free_than(120 << 20):
+        late = E.Batch(eng, [dw], table, packed, _lib.BATCHING)
+        assert late.kernel_name().count(",") == 3
+        for b in (batch, late):
+            b.run()
+            b.sync()
+            assert b.kernel_name().count(",") == 3
+            out = b.fetch()
+            assert np.array_equal(out["n_good"][0], ref["n_good"])
+            assert np.allclose(out["latency_sum"][0], ref["latency_sum"], rtol=8e-12, atol=0)      # (66000 requests, see above)
+            b.close()
     dw.close()
     eng.close()
