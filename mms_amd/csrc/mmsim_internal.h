@@ -257,13 +257,13 @@ struct WindowArgs {
     int32_t span_blocks, ext_blocks; // blocks of a span, and how many a run goes on behind its own
     int32_t marks, state_words;      // most marks of a span, 64-bit words of a state
     int32_t alike;                   // clocks that differ before the next arrival may count as equal: arrivals ascend, no latency is negative, up to 64 groups
-    int64_t run_cap, true_cap;       // values of a run: 64 * (span_blocks + ext_blocks), and of a whole stream
+    int64_t run_cap;                 // values of a run: 64 * (span_blocks + ext_blocks)
     uint32_t *span_sync;             // [L][spans + kSyncWords] marks that every run has published, how many runs have ended (0 before a launch and
                                      // after), and how often a run that was taken up again met another
     uint64_t *mark_state;            // [L][spans][marks][state_words]
     uint64_t *end_state;             // [L][spans][state_words + kEndWords]
-    double *run_vals;                // [L][true_cap + (spans - 1) * run_cap] latencies of the requests of a run (finish times, if wanted)
-    uint32_t *pieces;                // [L][2 * kMaxSpans][4] blocks [first, end) of the stream are run [2]'s; the last word: how many pieces
+    double *run_vals;                // [L][spans - 1][run_cap] latencies of the requests of a run, but the first (finish times, if wanted)
+    uint32_t *pieces;                // [L][kPieceWords / 4][4] blocks [first, end) of the stream are among the values of run [2]; the last word: how many pieces
     // outputs, laid out as the caller's: simulation = seed * B + placement
     int32_t *n_good;
     double *lat_sum;
@@ -280,6 +280,7 @@ constexpr int kEndWords = 2;        // of end_state: end block, link
 constexpr int kSyncWords = 2;       // of span_sync, beside the runs'
 constexpr int kSumWaves = 4;        // wavefronts that put a simulation's runs together
 constexpr int kMaxSpans = 64;       // most runs of a simulation (their records are a lane's each)
+constexpr int kPieceWords = 16 * kMaxSpans;  // each run that is followed is a piece, and those that are taken up again have one for every span they go through
 constexpr int32_t kLeastSpan = 20, kLeastExt = 48;  // blocks of a span, and what a run may go on behind its span, at least
 constexpr int kMaxRuns = 4096;      // most runs of a launch, if its simulations are cut
 // Where the k-th mark of a span is, in blocks from its beginning: 4, 8, 12, 16, 24, 32, 48, 64, 96, ...

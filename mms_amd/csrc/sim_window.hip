@@ -315,12 +315,12 @@ template <int I>
 struct Int {
     static constexpr int value = I;
 };
-// Where a run's latencies are (finish times, if wanted), by place in the stream: those of runs that are taken up again in an array of
-// the whole stream.  (Run 0 adds up its own and writes its outputs.)
+// Where a run's latencies are (finish times, if wanted), by place in the stream.  Run 0 adds up its own and writes its outputs.  One
+// that is taken up again puts them where the run of the span that it is in has its own: if anybody takes over from that one, then behind
+// where the two meet.
 typedef const __attribute__((address_space(4))) WindowArgs ColdArgs;
 __device__ __forceinline__ double *values_of(ColdArgs *q, int sim, int r) {
-    double *v = q->run_vals + (size_t)sim * (size_t)(q->true_cap + (q->spans - 1) * q->run_cap);
-    return r == 0 ? v : v + q->true_cap + (r - 1) * q->run_cap - (int64_t)r * q->span_blocks * kWave;
+    return q->run_vals + ((int64_t)sim * (q->spans - 1) + (r - 1)) * q->run_cap - (int64_t)r * q->span_blocks * kWave;
 }
 
 // Wavefronts of a SIMD that the registers have to leave room for, with simulations cut into runs.
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         runs.go_on(q, at);
         return false;
     };
-    auto q_pieces = [&](int of) { return cold_args<WindowArgs>()->pieces + (size_t)of * (8 * kMaxSpans); };
+    auto q_pieces = [&](int of) { return cold_args<WindowArgs>()->pieces + (size_t)of * kPieceWords; };
     auto piece = [&](uint32_t at, uint32_t first, uint32_t end, int src) {
         uint32_t *w = q_pieces(sim) + at * 4u;
         w[0] = first;
@@ -920,8 +920,10 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
             nxt = nn;
             q = nrep;
             look();
-            if (SPANS && runs.own != 0) run_vals[blk + (uint32_t)j] = OUTPUTS && want_req ? (good ? t + overhead : __builtin_nan("")) : took;
-            else if (accepted != 0ull) lat_sum = ordered_sum<W>(lat_sum, took, accepted);
+            if (SPANS && runs.own != 0) {
+                if (runs.own < 0) run_vals = values_of(cold_args<WindowArgs>(), sim, (int)(blk / 64u / (uint32_t)cold_args<WindowArgs>()->span_blocks));
+                run_vals[blk + (uint32_t)j] = OUTPUTS && want_req ? (good ? t + overhead : __builtin_nan("")) : took;
+            } else if (accepted != 0ull) lat_sum = ordered_sum<W>(lat_sum, took, accepted);
         }
         if constexpr (!SPANS) break;
         // ---- the end of a run
@@ -950,8 +952,13 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
                 for (int m = j; m < M; m += W) lds_put<uint32_t>(mcnt + (uint32_t)m * 4u, 0u);
             }
         } else {
-            if (lane == 0) piece(num_pieces, from / 64u, blk < R ? blk / 64u : (R + 63u) / 64u, 0);
-            num_pieces += 1;
+            const uint32_t span = (uint32_t)q->span_blocks, stop = blk < R ? blk / 64u : (R + 63u) / 64u;
+            for (uint32_t at = from / 64u; at < stop;) {
+                const uint32_t in = at / span, next = (in + 1u) * span < stop ? (in + 1u) * span : stop;
+                if (lane == 0) piece(num_pieces, at, next, (int)in);
+                num_pieces += 1;
+                at = next;
+            }
             if (!runs.met) break;
             met_again += 1;
             first = runs.in;
@@ -1011,7 +1018,6 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
         wave_order();
         runs.resume(q, resume);
         from = resume * 64u;
-        run_vals = values_of(q, sim, 0);
     }
 
     if constexpr (SPANS) {
@@ -1025,7 +1031,7 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
     if (!mine) return;
     if (j == 0) {
         a.n_good[row] = n_good;
-        if constexpr (SPANS) q_pieces(sim)[8 * kMaxSpans - 1] = num_pieces;
+        if constexpr (SPANS) q_pieces(sim)[kPieceWords - 1] = num_pieces;
         else a.lat_sum[row] = lat_sum;
     }
     if constexpr (OUTPUTS) {
@@ -1049,14 +1055,14 @@ __global__ __launch_bounds__(kMaxWindowWaves *kWave, SPANS ? least_waves(SMAX, O
 // here, 0.23 -> 0.22 ms (450 MB of latencies; a copy reads them in 0.1), 600 placements 0.34 -> 0.24, five of 82000 0.20 -> 0.12, one of 30000 with outputs 0.10 -> 0.08.
 __global__ __launch_bounds__(kSumWaves *kWave) void window_sum_kernel(const WindowArgs a) {
     constexpr int N = 16;
-    __shared__ uint32_t pieces[8 * kMaxSpans];
+    __shared__ uint32_t pieces[kPieceWords];
     __shared__ double added[kSumWaves], more_if_odd[kSumWaves], exact;
     __shared__ int negative[kSumWaves];
     const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = (int)(blockDim.x >> 6), sim = (int)blockIdx.x;
     ColdArgs *q = cold_args<WindowArgs>();
-    for (int k = (int)threadIdx.x; k < 8 * kMaxSpans; k += (int)blockDim.x) pieces[k] = a.pieces[(size_t)sim * (8 * kMaxSpans) + k];
+    for (int k = (int)threadIdx.x; k < kPieceWords; k += (int)blockDim.x) pieces[k] = a.pieces[(size_t)sim * kPieceWords + k];
     __syncthreads();
-    const int num = __builtin_amdgcn_readfirstlane((int)pieces[8 * kMaxSpans - 1]);
+    const int num = __builtin_amdgcn_readfirstlane((int)pieces[kPieceWords - 1]);
     const bool want_req = (a.flags & MMSIM_WANT_PER_REQUEST) != 0;
     const int seed = __builtin_amdgcn_readfirstlane(a.stream_of ? a.stream_of[sim] : sim / a.tiles);
     const Req *__restrict__ reqs = a.stream_ptr[seed];

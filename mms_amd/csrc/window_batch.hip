@@ -298,14 +298,13 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         a.spans = (int32_t)std::max<int64_t>((blocks + a.span_blocks - 1) / a.span_blocks, 1);
         a.ext_blocks = std::max(a.span_blocks / 2, kLeastExt);
         a.run_cap = (int64_t)kWave * (a.span_blocks + a.ext_blocks);
-        a.true_cap = (int64_t)kWave * blocks;
         for (a.marks = 0; span_mark(a.marks) < a.span_blocks;) ++a.marks;
         const size_t n = a.spans > 1 ? (size_t)(units * a.spans) : 0;
         runs = Layout{};
         runs.take(8 * n * (size_t)a.marks * (size_t)a.state_words);
         at_ends = runs.take(8 * n * (size_t)(a.state_words + kEndWords));
-        at_pieces = runs.take(4 * (n > 0 ? (size_t)units : 0) * 8 * kMaxSpans);
-        at_vals = runs.take(n > 0 ? 8 * (size_t)units * (size_t)(a.true_cap + (a.spans - 1) * a.run_cap) : 0);
+        at_pieces = runs.take(4 * (n > 0 ? (size_t)units : 0) * kPieceWords);
+        at_vals = runs.take(n > 0 ? 8 * (size_t)units * (size_t)((a.spans - 1) * a.run_cap) : 0);
     };
     // sixteen replicas in registers, which leaves two or three wavefronts to a SIMD: sim_window.hip has both sides
     const bool sixteen = lanes == kWave && shape.rmax > 8 && units <= 8 * cus;
