@@ -73,6 +73,8 @@ const char *mmsim_last_error(void);
 
 /* Binds a context to HIP device `device` and creates its stream. */
 int mmsim_ctx_create(int device, mmsim_ctx **out);
+/* Ends the caller's use of the context.  What it holds is given back when the last workload and batch made of it are destroyed, which
+ * may be later. */
 void mmsim_ctx_destroy(mmsim_ctx *ctx);
 
 /*

@@ -1510,13 +1510,8 @@ int mmsim_ctx_create(int device, mmsim_ctx **out) try {
 void mmsim_ctx_destroy(mmsim_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
-    if (ctx->stream) {
-        (void)hipStreamSynchronize(ctx->stream);
-        (void)hipStreamDestroy(ctx->stream);
-    }
-    for (hipEvent_t e : ctx->ev_static)
-        if (e) (void)hipEventDestroy(e);
-    delete ctx;
+    if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    ctx->drop();
 }
 
 int mmsim_ctx_device_info(mmsim_ctx *ctx, mmsim_device_info *out) try {
@@ -1934,7 +1929,8 @@ void mmsim_batch_destroy(mmsim_batch *b) {
         (void)hipStreamSynchronize(b->ctx->stream);
         if (b->window && !b->in_scratch) b->ctx->staging.trim();  // (of a call that failed on the way)
     }
-    mmsim_ctx *ctx = b->ctx;
+    CtxRef ctx;
+    ctx = b->ctx.p;
     delete b;
     if (ctx) ctx->runs.trim();
 }

@@ -227,12 +227,40 @@ struct mmsim_ctx {
     unsigned char *scratch = nullptr;     // this device's copy of the static scratch (mmsim_eval_batch_static)
     hipEvent_t ev_static[2] = {};         // timing events of batches that live in the static scratch
     mmsim_options opt{};                  // what batches made without options of their own use (mmsim_ctx_set_options)
+    std::atomic<int> users{1};            // its owner, and the workloads and batches that were made of it
+    void drop() {
+        if (users.fetch_sub(1) != 1) return;
+        (void)hipSetDevice(device);
+        if (stream) (void)hipStreamDestroy(stream);
+        for (hipEvent_t e : ev_static)
+            if (e) (void)hipEventDestroy(e);
+        delete this;
+    }
+};
+
+// The context of a workload or batch, which lives until they are gone as well (a garbage collector may end it first).
+struct CtxRef {
+    mmsim_ctx *p = nullptr;
+    CtxRef() = default;
+    CtxRef(const CtxRef &) = delete;
+    ~CtxRef() {
+        if (p) p->drop();
+    }
+    CtxRef &operator=(const CtxRef &) = delete;
+    CtxRef &operator=(mmsim_ctx *ctx) {
+        if (ctx) ctx->users.fetch_add(1);
+        if (p) p->drop();
+        p = ctx;
+        return *this;
+    }
+    operator mmsim_ctx *() const { return p; }
+    mmsim_ctx *operator->() const { return p; }
 };
 
 inline std::atomic<uint64_t> g_next_workload_id{1};
 
 struct mmsim_workload {
-    mmsim_ctx *ctx = nullptr;
+    CtxRef ctx;
     uint64_t id = 0;  // unique per mmsim_workload_create: a batch remembers which streams it was made from
     int64_t R = 0;
     int32_t M = 0;
@@ -308,7 +336,7 @@ inline double replicas_of_a_request(const mmsim_workload *const *wls, int32_t n_
 }
 
 struct mmsim_batch {
-    mmsim_ctx *ctx = nullptr;
+    CtxRef ctx;
     uint32_t flags = 0;
     int32_t n_seeds = 0, B = 0, M = 0, Gmax = 0, tiles = 0, waves = 0;
     int32_t smax_bucket = 0, rmax_all = 0, nslots = 0, waves_per_block = 1;
