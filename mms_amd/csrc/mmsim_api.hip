@@ -1109,6 +1109,9 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
                                   : blocks >= 6 * kLeastSpan ? std::min((12 * cus + cus / 2) / b->waves, blocks / kLeastSpan)
                                                              : 1;
             runs_of = (int)std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / b->waves)));
+            if (runs_of > 1 && o.segment_requests == 0 &&
+                !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()), replicas_of_a_request(wls, n_seeds, rl)))
+                runs_of = 1;
             span_blocks = (int32_t)std::max<int64_t>((blocks + runs_of - 1) / runs_of, 1);
             runs_of = (int)std::max<int64_t>((blocks + span_blocks - 1) / span_blocks, 1);
             while (span_mark(span_marks) < span_blocks) ++span_marks;
@@ -1596,6 +1599,20 @@ int mmsim_workload_create(mmsim_ctx *ctx, int64_t R, int32_t M, const double *ts
                 e.rank = rank[(size_t)i];
                 e.pad[0] = e.pad[1] = 0;
             }
+    }
+    if (R >= 6 * kLeastSpan * kWave) {
+        double models = 0.0, burst = 0.0;
+        for (int32_t m = 0; m < M; ++m) {
+            const MqEntry *e = mq.data() + w->mq_off[m];
+            const int64_t n = w->model_num_requests[m] - 1;
+            double squares = 0.0;
+            for (int64_t i = 0; i < n; ++i) squares += (e[i + 1].t - e[i].t) * (e[i + 1].t - e[i].t);
+            const double mean = n < 5 ? 0.0 : (e[n].t - e[0].t) / (double)n, variance = squares / (double)std::max<int64_t>(n, 1) - mean * mean;
+            if (!(mean > 0.0) || !(variance < 1e300)) continue;
+            models += (double)n;
+            burst += (double)n * std::sqrt(std::max(0.0, variance)) / mean;
+        }
+        if (models > 0.0) w->burst = burst / models;
     }
     HIP_TRY(hipSetDevice(ctx->device));
     HIP_TRY(w->reqs->alloc((size_t)R));

@@ -317,14 +317,9 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         // with four runs); below 120 blocks there is little to gain (5757 requests 155 us, with a second kernel 190).
         const int64_t per_cu = blocks < 384 ? 4 : sixteen || a.smax_bucket == 32 ? 8 : 12;
         spans = std::min((per_cu * cus + cus / 2) / units, blocks / kLeastSpan);
-        // Streams that overload the groups and find several of them for every model: a group is never idle, and two runs that once chose
-        // differently go on doing so.  106 batches of 16 to 1100 placements, not cut against cut: of the 40 beyond this line 39 are slower cut, by 3 to 31 %
-        // (1.24 -> 1.78 ms at load 8 with 1.5 replicas to a model), and one is faster (1.73 -> 1.34 ms); of the 66 others 49 are faster (up to
-        // 7.4 -> 0.42 ms) and 12 slower, by up to a quarter (3.35 -> 4.40 ms), with loads and replicas like those of the 49.
-        if (o.window_lanes == 0 && spans > 1) {
-            const double load = offered_load(wls, n_seeds, t, B, Gmax, p->num_groups, p->group_cfg);
-            if (load >= 2.5 && load * (double)replicas >= 2.2 * (double)B * (double)M) spans = 1;
-        }
+        if (o.window_lanes == 0 && spans > 1 &&
+            !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, p->num_groups, p->group_cfg), replicas_of_a_request(wls, n_seeds, p, M)))
+            spans = 1;
         if (o.window_lanes > 0) spans = blocks / std::max<int64_t>(8, o.segment_requests / kWave);
     }
     cut(std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / units))));

@@ -4,11 +4,14 @@ run goes through the whole stream, and streams of both, where runs are given up 
 span, at its edge and before it; all outputs."""
 import ctypes as C
 from contextlib import contextmanager
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
 
 from mms_amd import _lib, engine as E
+from mms_amd.placement_policy import ModelPlacement
+from mms_amd.profiling import ParallelConfig
 from helpers import assert_batch_matches, oracle_batch
 from test_gpu_window import COUNTS, _problem, _stream
 
@@ -220,6 +223,38 @@ def test_streams_that_overload_the_groups_are_not_cut(faster, cut):
     batch.close()
     assert_batch_matches(out, oracle_batch(st, table, packed), 0, packed[0], where=f"faster {faster}")
     dw.close()
+
+
+@pytest.mark.parametrize("bursty", [False, True])
+@pytest.mark.parametrize("batching", [0, _lib.BATCHING])
+def test_where_runs_would_not_agree_simulations_are_not_cut(batching, bursty):
+    """Four groups for every model that are half busy: cut where arrivals come in bursts, not where they come evenly (a request
+    each time goes to another group then, and runs that once chose differently go on doing so)."""
+    eng = E.Engine.default()
+    rng = np.random.default_rng(8)
+    M, R, sizes = 9, 12000, [1, 2, 4, 8] if batching else [1]
+    profiles, _ = _problem(8, (1,), True, M, 1, 1, 1)
+    for p in profiles:
+        for d in p.para_dict.values():
+            for b in sizes[1:]:
+                d.latency[b] = [x * (1 + 0.15 * (b - 1)) for x in d.latency[1]]
+    sols = [ModelPlacement([ParallelConfig(1, 1, 1)] * 6, [[int(x) for x in rng.choice(M, 6, replace=False)] for _ in range(6)]) for _ in range(12)]
+    table = E.LatencyTable(profiles, sizes)
+    packed = E.pack_placements(sols, table)
+    gaps = rng.gamma(1 / 64, 64, R) if bursty else rng.exponential(1.0, R)
+    times = np.cumsum(gaps * (R / gaps.sum() / 15.0))             # 15 a second, of the 34 that six groups can do
+    ids, slos = rng.integers(0, M, R).astype(np.int32), rng.uniform(0.1, 0.8, R).astype(np.float32)
+    dw = E.DeviceWorkload(eng, times, ids, slos, M)
+    batch = E.Batch(eng, [dw], table, packed, batching)
+    assert (batch.kernel_name().count(",") == (4 if batching else 6)) == bursty
+    batch.run()
+    batch.sync()
+    out = batch.fetch()
+    batch.close()
+    dw.close()
+    ref = oracle_batch(SimpleNamespace(tstamps=times, model_ids=ids, slos=slos), table, packed, batching=bool(batching))
+    assert np.array_equal(out["n_good"][0], ref["n_good"])
+    assert np.allclose(out["latency_sum"][0], ref["latency_sum"], rtol=1.4e-12 if batching else 0, atol=0)     # (12000 * 2^-53, as above)
 
 
 @pytest.mark.parametrize("depths,uniform,groups,hosts,M", [((1,), True, 6, 7, 9), ((1, 2, 4), True, 6, 8, 9), ((1, 3, 5), False, 12, 9, 70)])
