@@ -1110,7 +1110,7 @@ int build_batch_with(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n
                                                              : 1;
             runs_of = (int)std::max<int64_t>(1, std::min<int64_t>(spans, std::min<int64_t>(kMaxSpans, kMaxRuns / b->waves)));
             if (runs_of > 1 && o.segment_requests == 0 &&
-                !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()), replicas_of_a_request(wls, n_seeds, rl)))
+                !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, rl.num_groups.data(), rl.group_cfg.data()), replicas_of_a_request(wls, n_seeds, rl), 2.0))
                 runs_of = 1;
             span_blocks = (int32_t)std::max<int64_t>((blocks + runs_of - 1) / runs_of, 1);
             runs_of = (int)std::max<int64_t>((blocks + span_blocks - 1) / span_blocks, 1);

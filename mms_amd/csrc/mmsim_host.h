@@ -323,18 +323,19 @@ inline double replicas_of_a_request(const mmsim_workload *const *wls, int32_t n_
 }
 
 // Whether it pays to cut simulations into runs: groups that are busy all along, and requests that may go to several of them, keep runs
-// that once chose differently apart; pauses between a model's bursts bring them together.  Random batches of 1 to 1100 placements, 7700 to
-// 121000 requests, loads of 0.3 to 8, times between arrivals that vary by 1 to 8 times their mean, cut against not cut (where there is room for two runs).
-// Plain, 403 batches: all cut 147 are more than 5 % slower; with the line at load x replicas >= burst 36 of the 231 that are cut (the worst 3.5 -> 4.7
-// ms), and of the 162 that cutting makes a quarter or more faster 7 are not cut; a line at three quarters of that leaves 24 and 14.  (The line before, load >= 2.5 and
-// load x replicas >= 2.2, 61 of 283, 11.)  Batching, 195 batches: all cut 38 are more than 5 % slower (at most 13 %), with this line 7 of 122, and 4 of 89 are missed.
-inline bool runs_agree_early(const mmsim_workload *const *wls, int32_t n_streams, double load, double replicas) {
+// that once chose differently apart; pauses between a model's bursts bring them together.  Cut against not cut, random batches of 1 to 1100
+// placements, 7700 to 121000 requests, loads of 0.3 to 8, times between arrivals that vary by 1 to 8 times their mean, lines at
+// load x replicas = most x burst.  Plain, 806 batches, most = 1: 70 of the 462 that are cut are more than 5 % slower for it (worst 2.8 -> 4.3 ms), and 13
+// of the 326 that cutting makes a quarter or more faster are not cut; most = 2: 143 of 572, and 2; all cut 298; a line at load >= 2.5 and load x
+// replicas >= 2.2 128 of 574, and 20.  Batching, 413 batches, where runs that never agree cost less (13 % at most): most = 1 16 of 259, and 11 of the 196 not
+// cut, some of which take 8 times as long for it; 2: 34 of 324, and 2; all cut 76.
+inline bool runs_agree_early(const mmsim_workload *const *wls, int32_t n_streams, double load, double replicas, double most) {
     double requests = 0.0, burst = 0.0;
     for (int s = 0; s < n_streams; ++s) {
         requests += (double)wls[s]->R;
         burst += (double)wls[s]->R * wls[s]->burst;
     }
-    return load * replicas * requests < burst || burst == 0.0;
+    return load * replicas * requests < most * burst;
 }
 
 // Ordered replica lists per (placement, model): the rows of m_id2g_id.

@@ -318,7 +318,7 @@ int build_window(mmsim_ctx *ctx, const mmsim_workload *const *wls, int32_t n_see
         const int64_t per_cu = blocks < 384 ? 4 : sixteen || a.smax_bucket == 32 ? 8 : 12;
         spans = std::min((per_cu * cus + cus / 2) / units, blocks / kLeastSpan);
         if (o.window_lanes == 0 && spans > 1 &&
-            !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, p->num_groups, p->group_cfg), replicas_of_a_request(wls, n_seeds, p, M)))
+            !runs_agree_early(wls, n_seeds, offered_load(wls, n_seeds, t, B, Gmax, p->num_groups, p->group_cfg), replicas_of_a_request(wls, n_seeds, p, M), 1.0))
             spans = 1;
         if (o.window_lanes > 0) spans = blocks / std::max<int64_t>(8, o.segment_requests / kWave);
     }

@@ -228,7 +228,7 @@ def test_streams_that_overload_the_groups_are_not_cut(faster, cut):
 @pytest.mark.parametrize("bursty", [False, True])
 @pytest.mark.parametrize("batching", [0, _lib.BATCHING])
 def test_where_runs_would_not_agree_simulations_are_not_cut(batching, bursty):
-    """Four groups for every model that are half busy: cut where arrivals come in bursts, not where they come evenly (a request
+    """Four groups for every model that are half busy (three quarters with batching): cut where arrivals come in bursts, not where they come evenly (a request
     each time goes to another group then, and runs that once chose differently go on doing so)."""
     eng = E.Engine.default()
     rng = np.random.default_rng(8)
@@ -242,7 +242,7 @@ def test_where_runs_would_not_agree_simulations_are_not_cut(batching, bursty):
     table = E.LatencyTable(profiles, sizes)
     packed = E.pack_placements(sols, table)
     gaps = rng.gamma(1 / 64, 64, R) if bursty else rng.exponential(1.0, R)
-    times = np.cumsum(gaps * (R / gaps.sum() / 15.0))             # 15 a second, of the 34 that six groups can do
+    times = np.cumsum(gaps * (R / gaps.sum() / (25.0 if batching else 15.0)))       # a second, of the 34 that six groups can do
     ids, slos = rng.integers(0, M, R).astype(np.int32), rng.uniform(0.1, 0.8, R).astype(np.float32)
     dw = E.DeviceWorkload(eng, times, ids, slos, M)
     batch = E.Batch(eng, [dw], table, packed, batching)
