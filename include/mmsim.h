@@ -104,7 +104,8 @@ typedef struct {
                                      their own pace more than 8192 are taken up to a multiple of 8192.  With
                                      window_lanes 64: a simulation is cut into runs of so many requests (512 at
                                      least, 64 runs at most) that are simulated at the same time; 0: not cut,
-                                     and with window_lanes 0 as many as the chip has room for.  The same in the
+                                     and with window_lanes 0 as many as the chip has room for, where arrivals
+                                     are bursty enough for that to pay.  The same in the
                                      batching simulator where a wavefront simulates one placement (up to 512
                                      models, no per-request outputs; 0: as many as there is room for)          */
     int32_t sched_spin_limit;     /* looks in a row after which a wavefront that finds only busy items leaves;

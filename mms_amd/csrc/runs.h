@@ -7,6 +7,9 @@ namespace mmsim {
 namespace {
 
 // What wavefronts of different workgroups tell one another while the kernel runs: stores and loads that all of the device sees.
+// A mark is told, the wavefront waits until its stores have been carried out, and only then tells that the mark is there; who is told so
+// asks for the mark afterwards.  (The waits are instructions of this hardware.  A release and an acquire at device scope would say the same in the
+// language's terms, but write back and throw away caches at every mark: 179 placements of 25094 requests 0.335 -> 0.557 ms, 79 of 98901 0.87 -> 1.20.)
 __device__ __forceinline__ void tell(uint64_t *p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void tell(uint32_t *p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ uint64_t told(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }

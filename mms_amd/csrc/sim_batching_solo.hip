@@ -12,7 +12,8 @@
 //           AND, and only when several of its models wait are the ranks of their heads looked at (:654-664).
 //   lane j  entry j of the queue a batch is taken from, sixteen of them, and latency column j (:666-704).
 //
-// Latency sums are kept by place in the queue, as the octets there keep them, so that they are equal bit for bit.
+// Latency sums are kept by place in the queue, as the octets there keep them, so that they are equal bit for bit (but where simulations are
+// cut into runs: add_latency).
 //
 // Arrivals are looked at eight at a time, one to an octet of lanes (lane 8 i + j: the j-th replica of arrival i's model):
 // those at which nothing happens but a place in a queue cost no more than that.  Events that are due are seen to before
@@ -41,7 +42,8 @@
 // Few simulations of long streams without per-request outputs are cut into runs (SPANS), as sim_window.hip cuts its own: a run starts a span
 // with idle clocks and empty queues, and ends where its clocks, the queues of the models that some group lists and its idle events equal those that
 // the next run had there (or its clocks differ where nothing looks any more).  30000 requests, 128 placements, runs agree after 192 requests in the median, 704 at most of 24: 24 runs
-// each, calls 14.3 -> 2.03 ms; 105000 requests of 10 models on 30 single devices, 309 placements, of which some never agree, 126 -> 101 ms.
+// each, 15.4 -> 1.76 ms.  This instance is 3 to 5 % slower by itself (scalar registers that are kept in vector registers), and runs that never agree cost
+// up to 13 % (105000 requests of 10 models on 30 single devices, 309 placements, 259 -> 270 ms): runs_agree_early says where the line is.
 //
 // LDS: the latency table (per workgroup, if it fits), and per wavefront the stage clocks and, per model, its queue: places of
 // its head and of its next arrival in the stream's lists, rank of the head, requests accepted; up to 128 models also their replicas; without
@@ -250,7 +252,9 @@ __global__ __launch_bounds__(kMaxWavesPerBlockBatching *kWave) void sim_batching
     int32_t requests_of_group = 0, good_of_group = 0;  // lane g (a count in global memory would be waited for in every batch)
     int32_t n_good = 0;
     // Of the batch members this lane accounts for.  SPANS: and what its roundings left out (Knuth's two-sum).  Where one run takes over from
-    // another depends on which marks were there in time: with 106 bits the sum of all of them is the same wherever that was.
+    // another depends on which marks were there in time, and so does the order of the additions: with 106 bits the sum of all of them comes out the same
+    // wherever that was (unless what lat_rest itself leaves out decides a rounding, which no launch has shown).  It is the exact sum, rounded once, but for that;
+    // that of a simulation that is not cut has its own roundings, so the last bits of a sum depend on how many placements there are beside it.
     double lat_sum = 0.0, lat_rest = 0.0;
     auto add_latency = [&](double x) {
         const double sum = lat_sum + x;

@@ -63,7 +63,10 @@
 // that are all idle most of the time, whose requests go round in the order the groups were used.
 // Kernels, 108000 requests: 700 placements of single devices, four runs each, 5.2 -> 2.9 + 0.2 ms (three wavefronts to a SIMD take 1.9 times
 // as long as one: issue); 600 of four-stage pipelines, five, 9.6 -> 3.4 + 0.3; 1025 up to 16 deep, three, 13.1 -> 8.4 + 0.3; one placement, 30000
-// requests, 24 runs, 1.85 -> 0.21 + 0.10 ms.  Where no runs agree: five placements, 82000 requests, 64 runs, 2.71 -> 2.84 ms.
+// requests, 24 runs, 1.85 -> 0.21 + 0.10 ms.  A run that is taken up again looks for the marks of the others as the first one does (five even streams of 82000 requests
+// at load 0.4, three replicas to a model, 20 such meetings: 4.9 -> 1.4 and 5.5 -> 3.1 ms, and 30 % slower with more wavefronts to a SIMD: runs_agree_early).  Where no
+// runs agree ten placements of 115532 requests, cut into 2 to 64 runs, take 4.7 -> 5.0 to 5.2 ms: this instance keeps scalar registers in vector registers and is up to 8 %
+// slower by itself; the wavefronts' priorities (s_setprio for the first run and one taken up again) change nothing.
 //
 // LDS of one placement (byte offsets in WindowArgs, built by the wavefront itself from the packed placement):
 //   clk  [slots+SMAX] f64   stage clocks, a placement's groups laid end to end, and SMAX slots for what does not count
