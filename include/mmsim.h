@@ -372,7 +372,8 @@ typedef struct {
 } mmsim_batch_info;
 int mmsim_batch_get_info(const mmsim_batch *batch, mmsim_batch_info *out);
 /* Name of the kernel template instance mmsim_batch_run launches for this batch, as a profiler prints it
- * (e.g. "sim_mixed_kernel<16, true, true, true, 0, true>"); measurement aid, no counterpart in the reference. */
+ * (e.g. "sim_mixed_kernel<16, true, true, true, 0, true>"), but without the last argument of kernels that are not cut
+ * into runs, `false`; measurement aid, no counterpart in the reference. */
 int mmsim_batch_kernel_name(const mmsim_batch *batch, char *buf, size_t size);
 
 /* create + run + sync + fetch + destroy.  With MMSIM_BATCHING, a simulation that runs out of idle-event slots
